@@ -22,27 +22,14 @@
 #include <cstdio>
 #include <cstdlib>
 
-#include <map>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
-#include "cfg_kernels.hpp"
-#include "cfg_math.hpp"
+#include "cfg_dev.hpp"
 #include "cfg_wave.hpp"
 
 namespace cfg {
-
-constexpr double PI = 3.14159265358979323846;
-
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double2 imul(double s, double2 a) { return make_double2(-(s * a.y), s * a.x); }  // (i s) a
-
-__device__ __forceinline__ int kx_of(const Geom& g, int ikx) { return ikx <= g.kxd ? ikx : ikx - g.nkx; }
 
 // LDS layout of FFT lines: element i of a line sits at pidx(i) = i + i/8 (one
 // pad slot per 8 complex values spreads the power-of-two strides of the
@@ -283,629 +270,6 @@ __device__ __forceinline__ void stage_tw(double2* dst, const FFTPlan& P) {
 }
 
 // ===========================================================================
-// Tau solver kernels: one thread per live mode (tausolver.cpp, nse.cpp:479)
-// ===========================================================================
-__device__ TauView make_view(const Geom& g, const TauSet& s, int m, double nu, bool taucorr) {
-    const int ikx = m % g.nkx, ikz = m / g.nkx;
-    const int kx = kx_of(g, ikx), kz = ikz;
-    const double pi2 = PI * PI;
-    const double kappa2 = 4 * pi2 * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
-    const double c = 4.0 * pi2 * nu;
-    const double lambda = s.lambda_t + c * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
-    double* cm = s.coef + (long)m * TAU_NA * g.Ny;
-    auto A = [&](int k) { return SV{cm + (long)k * g.Ny, 1}; };
-    TauView t;
-    t.ph = HelmholtzView{A(0), A(1), A(2), kappa2, g.Ny};
-    t.vh = HelmholtzView{A(3), A(4), A(5), lambda, g.Ny};
-    t.Pp = A(6);
-    t.Pm = A(7);
-    t.vp = A(8);
-    t.vm = A(9);
-    t.P0 = A(10);
-    t.v0 = A(11);
-    t.scal = s.scal + (long)m * 6;
-    t.sstride = 1;
-    t.nu = nu;
-    t.a = g.a;
-    t.b = g.b;
-    t.kx2pi = 2 * PI * kx / g.Lx;
-    t.kz2pi = 2 * PI * kz / g.Lz;
-    t.zero_mode = (kx == 0 && kz == 0);
-    t.taucorrection = taucorr;
-    return t;
-}
-
-// TauSolver constructor per mode (tausolver.cpp:81-176), T modes per block,
-// one thread each. ALL: the mode's whole working set in LDS, its 12 tau
-// profiles (array a at element (a*Ny + n)*T + t), 6 scalars and 2 scratch
-// profiles, copied to the mode-major tau set with contiguous writes at the end.
-// Otherwise (tall grids, where a block of 64 KB would hold fewer than 8 such
-// working sets) the profiles and scalars are built in place in the tau set and
-// only the 2 scratch profiles are in LDS. The arithmetic is tau_setup's either
-// way (the sequential set-up, bit for bit the oracle's); only the memory the
-// recurrences store to and reload from moves.
-template <bool ALL>
-__global__ void k_tau_setup(Geom g, TauSet s, double nu, int taucorr) {
-    extern __shared__ double sl[];
-    const int T = blockDim.x, t = threadIdx.x;
-    const int m0 = blockIdx.x * T, m = m0 + t;
-    const int Ny = g.Ny;
-    const long arr = (long)Ny * T;  // one profile of the block's modes
-    if (m < g.M) {
-        TauView v = make_view(g, s, m, nu, taucorr != 0);
-        auto A = [&](int a) { return SV{sl + a * arr + t, T}; };
-        if constexpr (ALL) {
-            v.ph.band = A(0);
-            v.ph.up = A(1);
-            v.ph.invd = A(2);
-            v.vh.band = A(3);
-            v.vh.up = A(4);
-            v.vh.invd = A(5);
-            v.Pp = A(6);
-            v.Pm = A(7);
-            v.vp = A(8);
-            v.vm = A(9);
-            v.P0 = A(10);
-            v.v0 = A(11);
-            v.scal = sl + 14 * arr + t;
-            v.sstride = T;
-            tau_setup(v, A(12), A(13));
-        } else {
-            tau_setup(v, A(0), A(1));
-        }
-    }
-    if constexpr (ALL) {
-        __syncthreads();
-        const int nm = min(T, g.M - m0);
-        __attribute__((address_space(1))) double* coef = gmem_w(s.coef) + (long)m0 * TAU_NA * Ny;
-        for (int i = t; i < nm * TAU_NA * Ny; i += T) {
-            const int mm = i / (TAU_NA * Ny), r = i - mm * (TAU_NA * Ny), a = r / Ny, n = r - a * Ny;
-            coef[i] = sl[a * arr + (long)n * T + mm];
-        }
-        __attribute__((address_space(1))) double* scal = gmem_w(s.scal) + (long)m0 * 6;
-        for (int i = t; i < nm * 6; i += T) scal[i] = sl[14 * arr + (long)(i % 6) * T + i / 6];
-    }
-}
-
-// modes per block of the set-up within 64 KB of LDS, at most 64: whole working
-// sets (14 profiles and 6 scalars each) where 8 or more fit, else scratch
-// profiles only (2 each)
-static int tau_setup_modes(int Ny, bool* all) {
-    const long whole = (14L * Ny + 6) * (long)sizeof(double), scratch = 2L * Ny * (long)sizeof(double);
-    const long T = (64L * 1024) / whole;
-    *all = T >= 8;
-    return (int)std::max(1L, std::min(64L, (64L * 1024) / (*all ? whole : scratch)));
-}
-
-void launch_tau_setup(const Geom& g, const TauSet& s, double nu, bool taucorr, hipStream_t st) {
-    bool all = false;
-    const int T = tau_setup_modes(g.Ny, &all);
-    const dim3 grid((g.M + T - 1) / T);
-    if (all) {
-        const size_t lds = (size_t)(14L * g.Ny + 6) * T * sizeof(double);
-        k_tau_setup<true><<<grid, T, lds, st>>>(g, s, nu, taucorr ? 1 : 0);
-    } else {
-        const size_t lds = (size_t)2 * g.Ny * T * sizeof(double);
-        k_tau_setup<false><<<grid, T, lds, st>>>(g, s, nu, taucorr ? 1 : 0);
-    }
-}
-
-__device__ __forceinline__ CV cview(double* base, const Geom& g, int comp, int m) {
-    const long S2 = 2L * g.M;
-    double* p = base + 2L * ((long)comp * g.Ny * g.M + m);
-    return CV{SV{p, S2}, SV{p + 1, S2}};
-}
-
-// Tau solve with one W-lane segment of a wavefront per live mode (NSE::solve, nse.cpp:479-575;
-// TauSolver::solve, tausolver.cpp:347-450, with solve_P_and_v :193-251).
-
-// solve_P_and_v for the real and imaginary parts at once (NR = 2 right-hand
-// sides per scan); per part the same arithmetic as the one-RHS routines
-// (tausolver.cpp:193-251).
-// Ry is read again from its LDS row (re, im per coefficient) where it is
-// needed, instead of being held in registers through the pressure solve.
-template <int K, int W>
-__device__ __forceinline__ void tau_P_and_v_wave2(const WCtx& c, gcdouble cm, gcdouble sc, double kappa2,
-                                                  double lambda, double nu, bool taucorr, const WV<K> (&r)[2],
-                                                  const double2* Ryrow, WV<K> (&P)[2], WV<K> (&v)[2]) {
-    const long Ny = c.N;
-    const double z2[2] = {0.0, 0.0};
-    whelm_n<K, W, 2>(r, cm + 0 * Ny, cm + 1 * Ny, cm + 2 * Ny, kappa2, z2, z2, c, P);
-    WV<K> tmp[2];
-    wdiff_n<K, W, 2>(P, c, tmp);
-    double rtop[2], rtop1[2];  // Ry's top coefficients, for the tau correction
-    {
-        WV<K> Ry[2];
-        wload_c<K, W>(Ryrow, c, Ry[0], Ry[1]);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                tmp[p].e[k] -= Ry[p].e[k];
-                tmp[p].o[k] -= Ry[p].o[k];
-            }
-            rtop[p] = wtop<K, W>(Ry[p], c);
-            rtop1[p] = wtop1<K, W>(Ry[p], c);
-        }
-    }
-    whelm_n<K, W, 2>(tmp, cm + 3 * Ny, cm + 4 * Ny, cm + 5 * Ny, lambda, z2, z2, c, v);
-    // influence-matrix correction (tausolver.cpp:178-191)
-    double dvb[2], dva[2];
-    wdiff_n<K, W, 2>(v, c, tmp);
-    wends_n<K, W, 2>(tmp, c, dvb, dva);
-    {
-        const WV<K> Pp = wload<K, W>(cm + 6 * Ny, c), Pm = wload<K, W>(cm + 7 * Ny, c);
-        const WV<K> vp = wload<K, W>(cm + 8 * Ny, c), vm = wload<K, W>(cm + 9 * Ny, c);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const double dplus = -sc[0] * dvb[p] - sc[1] * dva[p];
-            const double dminus = -sc[2] * dvb[p] - sc[3] * dva[p];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                P[p].e[k] += dplus * Pp.e[k] + dminus * Pm.e[k];
-                P[p].o[k] += dplus * Pp.o[k] + dminus * Pm.o[k];
-                v[p].e[k] += dplus * vp.e[k] + dminus * vm.e[k];
-                v[p].o[k] += dplus * vp.o[k] + dminus * vm.o[k];
-            }
-        }
-    }
-    if (!taucorr) return;
-    const int Nb = c.Nb;
-    const WV<K> P0 = wload<K, W>(cm + 10 * Ny, c), v0 = wload<K, W>(cm + 11 * Ny, c);
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        double sigma1_Nb = lambda * wtop<K, W>(v[p], c) - nu * 0.0 - rtop[p];
-        double sigma1_Nb1 = lambda * wtop1<K, W>(v[p], c) - nu * 0.0 - rtop1[p];
-        sigma1_Nb1 += (4.0 / c.L) * Nb * wtop<K, W>(P[p], c);
-        const double sigmaNb = sigma1_Nb / (1.0 - sc[5]);
-        const double sigmaNb1 = sigma1_Nb1 / (1.0 - sc[4]);
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            P[p].e[k] += sigmaNb1 * P0.e[k];
-            P[p].o[k] += sigmaNb * P0.o[k];
-            v[p].e[k] += sigmaNb * v0.e[k];
-            v[p].o[k] += sigmaNb1 * v0.o[k];
-        }
-    }
-}
-
-// The right-hand-side rows [c][n][m0..m0+MPB) of a block: sum_j coef_j in_j
-// (the multistep / Runge-Kutta combination, dnsalgo.cpp:218-224, 668-673),
-// stored to LDS as [mode][c][n]. The term count is a template parameter and
-// UNR elements are loaded per pass, so the NT x UNR loads of a pass are all in
-// flight before the first is summed.
-template <int NT, int MPB>
-__device__ __forceinline__ void tau_stage_rhs(const TauMember& me, const Geom& g, int m0, int nthr, double2* lds) {
-    constexpr int UNR = NT <= 2 ? 8 : (NT <= 4 ? 4 : 2);  // 16 loads in flight at most
-    const __attribute__((address_space(1))) dvec2* in[NT];
-    double coef[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        in[j] = gmem(reinterpret_cast<const dvec2*>(me.in[j]));
-        coef[j] = me.coef[j];
-    }
-    const int Ny = g.Ny;
-    const int total = 3 * Ny * MPB;
-    for (int base = threadIdx.x; base < total; base += UNR * nthr) {
-        dvec2 v[UNR][NT];
-        int slot[UNR];
-#pragma unroll
-        for (int r = 0; r < UNR; ++r) {
-            const int idx = base + r * nthr;
-            const int ww = idx % MPB, rest = idx / MPB, n = rest % Ny, comp = rest / Ny;
-            const int mm = m0 + ww;
-            const bool ok = idx < total && mm < g.M;
-            slot[r] = idx < total ? (ww * 3 + comp) * Ny + n : -1;
-            // element 0 stands in for an element past the block (then zeroed),
-            // so that every load is issued unconditionally
-            const long off = ok ? ((long)comp * Ny + n) * g.M + mm : 0;
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                v[r][j] = in[j][off];
-                if (!ok) v[r][j] = dvec2{0.0, 0.0};
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < UNR; ++r) {
-            double2 acc = make_double2(0.0, 0.0);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                acc.x += coef[j] * v[r][j].x;
-                acc.y += coef[j] * v[r][j].y;
-            }
-            if (slot[r] >= 0) lds[slot[r]] = acc;
-        }
-    }
-}
-
-// waves per SIMD a tau-solve variant is compiled for: two 16-lane coefficient
-// blocks fit in the 168 registers of three waves
-constexpr int tau_waves(int K, int W) { return (W == 16 && K == 2) ? 3 : 1; }
-constexpr int NXCD = 8;
-
-// Block order of a launch over (mode block, member) pairs: the dispatcher
-// hands consecutive workgroups to the 8 XCDs in turn, so the linear block
-// index is renumbered to put a contiguous range of pairs on each XCD, members
-// fastest. The members of a launch share their tau factors, which one XCD
-// then reads from its own L2 for every member after the first.
-// The launch's block (x, y, z) renumbered so that each XCD runs a contiguous
-// range of the linear block order (x fastest): the dispatcher deals
-// consecutive workgroups to the NXCD XCDs in turn, so without it neighbouring
-// blocks, which share the cache lines at their edges, fetch those lines into
-// different L2s. A permutation of the blocks: the work of each is unchanged.
-struct BlockId {
-    int x, y, z;
-};
-__device__ __forceinline__ BlockId xcd_grid() {
-    const unsigned gx = gridDim.x, gy = gridDim.y;
-    const unsigned T = gx * gy * gridDim.z;
-    const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const unsigned q = T / NXCD, r = T % NXCD, x = L % NXCD;
-    const unsigned p = x * q + (x < r ? x : r) + L / NXCD;
-    const unsigned t = p / gx;
-    return BlockId{(int)(p - t * gx), (int)(t % gy), (int)(t / gy)};
-}
-
-__device__ __forceinline__ void xcd_block(int nmem, int& mode_block, int& member) {
-    const int T = gridDim.x;  // mode blocks x members
-    const int L = blockIdx.x;
-    const int q = T / NXCD, r = T % NXCD, x = L % NXCD;
-    const int p = x * q + (x < r ? x : r) + L / NXCD;
-    mode_block = p / nmem;
-    member = p - mode_block * nmem;
-}
-
-// Block of MPB consecutive modes of one member. Each wave solves its modes in
-// registers from the right-hand sides staged in LDS, and u, v, w, q leave
-// through LDS the same way.
-template <int K, int W, int MPB>
-__global__ void __launch_bounds__(W * MPB) __attribute__((amdgpu_waves_per_eu(tau_waves(K, W))))
-k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMember* __restrict__ tab) {
-    extern __shared__ double2 lds[];  // [MPB][3][Ny] right-hand sides, then the B rows [3][Ny]
-    int mblk, mem;
-    xcd_block(nmem, mblk, mem);
-    const TauMember& me = tab[mem];
-    const TauSet s = me.set;
-    const double nu = me.nu;
-    const int taucorr = me.taucorr;
-    const SolveConst zc = me.sc;
-    __attribute__((address_space(1))) dvec2* __restrict__ u = gmem_w(reinterpret_cast<dvec2*>(me.u));
-    __attribute__((address_space(1))) dvec2* __restrict__ q = gmem_w(reinterpret_cast<dvec2*>(me.q));
-    const int Ny = g.Ny;
-    const int nthr = W * MPB;
-    const int m0 = mblk * MPB;
-    const int w = threadIdx.x / W;  // mode slot of this lane's segment
-    const int m = m0 + w;
-    const bool valid = m < g.M;
-    double* hbl = reinterpret_cast<double*>(lds + 3 * Ny * MPB);
-    for (int i = threadIdx.x; i < 3 * Ny; i += nthr) hbl[i] = hb[i];
-    switch (me.nterms) {
-        case 1: tau_stage_rhs<1, MPB>(me, g, m0, nthr, lds); break;
-        case 2: tau_stage_rhs<2, MPB>(me, g, m0, nthr, lds); break;
-        case 3: tau_stage_rhs<3, MPB>(me, g, m0, nthr, lds); break;
-        case 4: tau_stage_rhs<4, MPB>(me, g, m0, nthr, lds); break;
-        case 5: tau_stage_rhs<5, MPB>(me, g, m0, nthr, lds); break;
-        case 6: tau_stage_rhs<6, MPB>(me, g, m0, nthr, lds); break;
-        case 7: tau_stage_rhs<7, MPB>(me, g, m0, nthr, lds); break;
-        default: tau_stage_rhs<MAX_TERMS, MPB>(me, g, m0, nthr, lds); break;
-    }
-    __syncthreads();
-    WCtx c;
-    c.N = Ny;
-    c.Me = (Ny + 1) / 2;
-    c.Mo = (Ny - 1) / 2;
-    c.Nb = Ny - 1;
-    c.Nc = Ny - 1;
-    c.lane = threadIdx.x % W;
-    c.L = g.b - g.a;
-    c.hb = hbl;
-    const int ikx = m % g.nkx, ikz = m / g.nkx;
-    const int kx = kx_of(g, ikx), kz = ikz;
-    const bool zero = (kx == 0 && kz == 0);
-    const double pi2 = PI * PI;
-    const double kk = (kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz);
-    const double kappa2 = 4 * pi2 * kk;
-    const double lambda = s.lambda_t + (4.0 * pi2 * nu) * kk;
-    const double kx2pi = 2 * PI * kx / g.Lx, kz2pi = 2 * PI * kz / g.Lz;
-    const gcdouble cm = gmem(s.coef) + (long)(valid ? m : 0) * TAU_NA * Ny;
-    const gcdouble sc = gmem(s.scal) + (long)(valid ? m : 0) * 6;
-    // LDS rows of this mode: Rx, Ry, Rz as staged. Each is read where it is
-    // needed rather than held in registers across the solves (the registers
-    // bound the waves per SIMD); the rows are then reused for the outputs.
-    double2* const Sx = lds + (w * 3 + 0) * Ny;
-    double2* const Sy = lds + (w * 3 + 1) * Ny;
-    double2* const Sz = lds + (w * 3 + 2) * Ny;
-    // Rx or Rz of this mode; kx = kz = 0 (nse.cpp:505-527) adds nu U'' (nu W'')
-    // and, with a fixed pressure gradient, the mean gradient
-    auto load_R = [&](const double2* S, const gcdouble base, double dPref, WV<K>& re, WV<K>& im) {
-        wload_c<K, W>(S, c, re, im);
-        if (zero) {
-            const WV<K> Byy = wload<K, W>(base, c);
-            for (int k = 0; k < K; ++k) {
-                re.e[k] += Byy.e[k];
-                re.o[k] += Byy.o[k];
-            }
-            if (!zc.bulk && c.lane == 0) re.e[0] -= dPref;
-        }
-    };
-    const gcdouble nuUyy = gmem(zc.nuUbaseyy), nuWyy = gmem(zc.nuWbaseyy);
-    WV<K> Pr, Pi, vr, vi;
-    if (valid) {
-        if (zero) {  // solve_P_and_v for kx = kz = 0: P from the pressure Helmholtz, v = 0
-            WV<K> Ryr, Ryi;
-            wload_c<K, W>(Sy, c, Ryr, Ryi);
-            Pr = whelm<K, W>(wdiff<K, W>(Ryr, c), cm, cm + Ny, cm + 2L * Ny, kappa2, 0.0, 0.0, c);
-            vr = wzero<K, W>();
-            vi = wzero<K, W>();
-            Pi = wzero<K, W>();  // real parts only (nse.cpp:555-563)
-        } else {  // real and imaginary parts together
-            WV<K> rr[2], P2[2], v2[2];
-            {
-                WV<K> Ry2[2];
-                wload_c<K, W>(Sy, c, Ry2[0], Ry2[1]);
-                wdiff_n<K, W, 2>(Ry2, c, rr);
-            }
-            {
-                WV<K> Rxr, Rxi, Rzr, Rzi;
-                wload_c<K, W>(Sx, c, Rxr, Rxi);
-                wload_c<K, W>(Sz, c, Rzr, Rzi);
-                for (int k = 0; k < K; ++k) {
-                    rr[0].e[k] -= kx2pi * Rxi.e[k] + kz2pi * Rzi.e[k];
-                    rr[0].o[k] -= kx2pi * Rxi.o[k] + kz2pi * Rzi.o[k];
-                    rr[1].e[k] += kx2pi * Rxr.e[k] + kz2pi * Rzr.e[k];
-                    rr[1].o[k] += kx2pi * Rxr.o[k] + kz2pi * Rzr.o[k];
-                }
-            }
-            tau_P_and_v_wave2<K, W>(c, cm, sc, kappa2, lambda, nu, taucorr != 0, rr, Sy, P2, v2);
-            Pr = P2[0];
-            Pi = P2[1];
-            vr = v2[0];
-            vi = v2[1];
-        }
-        wstore_c<K, W>(Sy, c, vr, vi);  // Ry's row is free: v goes out through it
-    }
-    // rows [slot][n] of the block's modes -> global component array dst (stride M)
-    auto drain = [&](int slot, __attribute__((address_space(1))) dvec2* dst) {
-        for (int idx = threadIdx.x; idx < Ny * MPB; idx += nthr) {
-            const int ww = idx % MPB, n = idx / MPB;
-            const int mm = m0 + ww;
-            if (mm < g.M) {
-                const double2 v = lds[(ww * 3 + slot) * Ny + n];
-                dst[(long)n * g.M + mm] = dvec2{v.x, v.y};
-            }
-        }
-    };
-    __syncthreads();
-    drain(1, u + (long)Ny * g.M);  // v
-    __syncthreads();
-    if (valid) wstore_c<K, W>(Sy, c, Pr, Pi);
-    __syncthreads();
-    drain(1, q);  // q = P
-    if (valid) {
-        const gcdouble vb = cm + 3L * Ny;
-        const gcdouble vu = cm + 4L * Ny;
-        const gcdouble vd = cm + 5L * Ny;
-        // u (row Sx) and w (row Sz) from the velocity Helmholtz operator. Called
-        // with explicit register arrays: selecting between them at run time
-        // would put them in scratch memory.
-        auto solve_uw = [&](double k2, const WV<K>& Rr, const WV<K>& Ri, double umean, double* mu_out,
-                            double2* row) {
-            WV<K> fr, fi;
-            for (int k = 0; k < K; ++k) {
-                fr.e[k] = -(k2 * Pi.e[k]) - Rr.e[k];
-                fr.o[k] = -(k2 * Pi.o[k]) - Rr.o[k];
-                fi.e[k] = k2 * Pr.e[k] - Ri.e[k];
-                fi.o[k] = k2 * Pr.o[k] - Ri.o[k];
-            }
-            WV<K> xr, xi;
-            if (zc.bulk) {  // bulk-velocity constraint (tausolver.cpp:404-450)
-                const double mu = whelm_mean<K, W>(fr, vb, vu, vd, lambda, nu, umean, c, xr);
-                if (c.lane == 0) *mu_out = mu;
-            } else {
-                xr = whelm<K, W>(fr, vb, vu, vd, lambda, 0.0, 0.0, c);
-            }
-            xi = wzero<K, W>();
-            wstore_c<K, W>(row, c, xr, xi);
-        };
-        if (zero) {  // kx = kz = 0: real parts only
-            {
-                WV<K> Rxr, Rxi;
-                load_R(Sx, nuUyy, zc.dPdxRef, Rxr, Rxi);
-                solve_uw(kx2pi, Rxr, Rxi, zc.umean, zc.dPdx_out, Sx);
-            }
-            WV<K> Rzr, Rzi;
-            load_R(Sz, nuWyy, zc.dPdzRef, Rzr, Rzi);
-            solve_uw(kz2pi, Rzr, Rzi, zc.wmean, zc.dPdz_out, Sz);
-        } else {  // u and w, real and imaginary parts: four right-hand sides of one operator
-            WV<K> f4[4], x4[4];
-            {
-                WV<K> Rxr, Rxi, Rzr, Rzi;
-                wload_c<K, W>(Sx, c, Rxr, Rxi);
-                wload_c<K, W>(Sz, c, Rzr, Rzi);
-                for (int k = 0; k < K; ++k) {
-                    f4[0].e[k] = -(kx2pi * Pi.e[k]) - Rxr.e[k];
-                    f4[0].o[k] = -(kx2pi * Pi.o[k]) - Rxr.o[k];
-                    f4[1].e[k] = kx2pi * Pr.e[k] - Rxi.e[k];
-                    f4[1].o[k] = kx2pi * Pr.o[k] - Rxi.o[k];
-                    f4[2].e[k] = -(kz2pi * Pi.e[k]) - Rzr.e[k];
-                    f4[2].o[k] = -(kz2pi * Pi.o[k]) - Rzr.o[k];
-                    f4[3].e[k] = kz2pi * Pr.e[k] - Rzi.e[k];
-                    f4[3].o[k] = kz2pi * Pr.o[k] - Rzi.o[k];
-                }
-            }
-            const double z4[4] = {0.0, 0.0, 0.0, 0.0};
-            whelm_n<K, W, 4>(f4, vb, vu, vd, lambda, z4, z4, c, x4);
-            wstore_c<K, W>(Sx, c, x4[0], x4[1]);
-            wstore_c<K, W>(Sz, c, x4[2], x4[3]);
-        }
-    }
-    __syncthreads();
-    drain(0, u);                     // u
-    drain(2, u + 2L * Ny * g.M);     // w
-}
-
-// PressureSolver::solve (poissonsolver.cpp:326-431) per mode, after the
-// nonlinear term f of u + U: p'' - kappa^2 p = -div f with p = 0 at the walls,
-// solved with the pressure factors of the tau data (the same Helmholtz operator,
-// nu = 1), then for every mode but (0,0) the wall correction
-// g = c exp(-mu (y-a)) + d exp(mu (y-b)), mu^2 = kappa^2, that makes
-// dp/dy = nu v'' at y = a, b; g's coefficients are Ti times its values at the
-// Chebyshev points.
-template <int K, int W, int MPB>
-__global__ void __launch_bounds__(W * MPB) k_pressure_wave(Geom g, YMats ym, PressArgs pa, const double* __restrict__ hb) {
-    extern __shared__ double2 lds[];  // [MPB][4][Ny]: f0, f1, f2, v; then the B rows [3][Ny]
-    const int Ny = g.Ny;
-    double* hbl = reinterpret_cast<double*>(lds + 4 * Ny * MPB);
-    for (int i = threadIdx.x; i < 3 * Ny; i += W * MPB) hbl[i] = hb[i];
-    const long M = g.M;
-    const int m0 = blockIdx.x * MPB, w = threadIdx.x / W;
-    const long m = m0 + w;
-    const bool valid = m < M;
-    const double2* __restrict__ f = reinterpret_cast<const double2*>(pa.f);
-    const double2* __restrict__ u = reinterpret_cast<const double2*>(pa.u);
-    double2* __restrict__ q = reinterpret_cast<double2*>(pa.q);
-    for (int idx = threadIdx.x; idx < 4 * Ny * MPB; idx += W * MPB) {
-        const int ww = idx % MPB, rest = idx / MPB, n = rest % Ny, comp = rest / Ny;
-        const long mm = m0 + ww;
-        double2 v = make_double2(0.0, 0.0);
-        if (mm < M) v = comp < 3 ? f[((long)comp * Ny + n) * M + mm] : u[((long)Ny + n) * M + mm];
-        lds[(ww * 4 + comp) * Ny + n] = v;
-    }
-    __syncthreads();
-    WCtx c;
-    c.N = Ny;
-    c.Me = (Ny + 1) / 2;
-    c.Mo = (Ny - 1) / 2;
-    c.Nb = Ny - 1;
-    c.Nc = Ny - 1;
-    c.lane = threadIdx.x % W;
-    c.L = g.b - g.a;
-    c.hb = hbl;
-    if (valid) {
-        const int ikx = (int)(m % g.nkx), ikz = (int)(m / g.nkx);
-        const int kx = kx_of(g, ikx), kz = ikz;
-        const bool zero = (kx == 0 && kz == 0);
-        const double pi2 = PI * PI;
-        const double kappa2 = 4 * pi2 * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
-        const double ax = 2 * PI * kx / g.Lx, az = 2 * PI * kz / g.Lz;
-        const double* cm = pa.set.coef + m * TAU_NA * Ny;
-        WV<K> Fxr, Fxi, Fyr, Fyi, Fzr, Fzi;
-        wload_c<K, W>(lds + (w * 4 + 0) * Ny, c, Fxr, Fxi);
-        wload_c<K, W>(lds + (w * 4 + 1) * Ny, c, Fyr, Fyi);
-        wload_c<K, W>(lds + (w * 4 + 2) * Ny, c, Fzr, Fzi);
-        const WV<K> Dr = wdiff<K, W>(Fyr, c), Di = wdiff<K, W>(Fyi, c);
-        WV<K> Rr, Ri;  // -div f (diffops.cpp:2488-2516)
-        for (int k = 0; k < K; ++k) {
-            Rr.e[k] = -((-ax * Fxi.e[k] - az * Fzi.e[k]) + Dr.e[k]);
-            Rr.o[k] = -((-ax * Fxi.o[k] - az * Fzi.o[k]) + Dr.o[k]);
-            Ri.e[k] = -((ax * Fxr.e[k] + az * Fzr.e[k]) + Di.e[k]);
-            Ri.o[k] = -((ax * Fxr.o[k] + az * Fzr.o[k]) + Di.o[k]);
-        }
-        WV<K> Pr = whelm<K, W>(Rr, cm, cm + Ny, cm + 2L * Ny, kappa2, 0.0, 0.0, c);
-        WV<K> Pi = whelm<K, W>(Ri, cm, cm + Ny, cm + 2L * Ny, kappa2, 0.0, 0.0, c);
-        if (!zero) {  // dp/dy = nu v'' at the walls (poissonsolver.cpp:356-427)
-            WV<K> Vr, Vi;
-            wload_c<K, W>(lds + (w * 4 + 3) * Ny, c, Vr, Vi);
-            double pbr, par_, pbi, pai, vbr, var_, vbi, vai;
-            wends<K, W>(wdiff<K, W>(Pr, c), c, pbr, par_);
-            wends<K, W>(wdiff<K, W>(Pi, c), c, pbi, pai);
-            wends<K, W>(wdiff<K, W>(wdiff<K, W>(Vr, c), c), c, vbr, var_);
-            wends<K, W>(wdiff<K, W>(wdiff<K, W>(Vi, c), c), c, vbi, vai);
-            const double alr = pa.nu * var_ - par_, ali = pa.nu * vai - pai;
-            const double ber = pa.nu * vbr - pbr, bei = pa.nu * vbi - pbi;
-            const double mu = sqrt(kappa2), H = g.b - g.a, e = exp(-mu * H);
-            const double delta = mu * (1 - exp(-2 * mu * H));
-            const double ccr = (-alr + ber * e) / delta, cci = (-ali + bei * e) / delta;
-            const double ddr = (ber - alr * e) / delta, ddi = (bei - ali * e) / delta;
-            const double piN = PI / (Ny - 1), rad = (g.b - g.a) / 2, cen = (g.b + g.a) / 2;  // chebypoints
-            for (int par = 0; par < 2; ++par)
-                for (int k = 0; k < K; ++k) {
-                    const int n = 2 * (K * c.lane + k) + par;
-                    if (n >= Ny) continue;
-                    double sr = 0.0, si = 0.0;
-                    for (int j = 0; j < Ny; ++j) {
-                        const double y = cen + rad * cos(j * piN);
-                        const double e1 = exp(-mu * (y - g.a)), e2 = exp(mu * (y - g.b));
-                        const double t = ym.Ti[(long)n * Ny + j];
-                        sr += t * (ccr * e1 + ddr * e2);
-                        si += t * (cci * e1 + ddi * e2);
-                    }
-                    if (par == 0) {
-                        Pr.e[k] += sr;
-                        Pi.e[k] += si;
-                    } else {
-                        Pr.o[k] += sr;
-                        Pi.o[k] += si;
-                    }
-                }
-        }
-        wstore_c<K, W>(lds + (w * 4 + 0) * Ny, c, Pr, Pi);
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < Ny * MPB; idx += W * MPB) {
-        const int ww = idx % MPB, n = idx / MPB;
-        const long mm = m0 + ww;
-        if (mm < M) q[(long)n * M + mm] = lds[(ww * 4 + 0) * Ny + n];
-    }
-}
-
-// Raises a kernel's dynamic-LDS limit once per (kernel, size), so that launches
-// recorded into a graph make no attribute calls.
-template <class K>
-static void allow_lds(K kernel, size_t bytes) {
-    if (bytes <= 64 * 1024) return;
-    static std::map<const void*, size_t> done;
-    size_t& d = done[(const void*)kernel];
-    if (d >= bytes) return;
-    const hipError_t e =
-        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess)  // the launch that follows would fail without saying why
-        throw std::runtime_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize, " + std::to_string(bytes) +
-                                 " B): " + hipGetErrorString(e));
-    d = bytes;
-}
-
-void launch_pressure(const Geom& g, const YMats& ym, const double* hb, const PressArgs& pa, hipStream_t st) {
-    const int Me = (g.Ny + 1) / 2;
-    auto go = [&](auto kern, int w) {
-        const int mpb = 256 / w;
-        const dim3 grid((unsigned)((g.M + mpb - 1) / mpb));
-        const size_t lds = (size_t)4 * g.Ny * mpb * sizeof(double2) + (size_t)3 * g.Ny * sizeof(double);
-        allow_lds(kern, lds);
-        kern<<<grid, 256, lds, st>>>(g, ym, pa, hb);
-    };
-    if (Me <= 16) go(k_pressure_wave<1, 16, 16>, 16);
-    else if (Me <= 32) go(k_pressure_wave<1, 32, 8>, 32);
-    else if (Me <= 64) go(k_pressure_wave<1, 64, 4>, 64);
-    else if (Me <= 128) go(k_pressure_wave<2, 64, 4>, 64);
-    else go(k_pressure_wave<3, 64, 4>, 64);
-}
-
-void launch_tau_solve(const Geom& g, const double* hb, int n, const TauMember* tab, hipStream_t st) {
-    const int Me = (g.Ny + 1) / 2;  // even coefficients: at most K per lane of a W-lane segment
-    // 256-thread blocks: several per CU, so that one block's HBM staging overlaps
-    // another's scans
-    auto go = [&](auto kern, int w) {
-        const int mpb = 256 / w;
-        const long nblk = (long)((g.M + mpb - 1) / mpb) * n;
-        if (nblk > 0x7fffffffL) throw std::runtime_error("tau solve: too many blocks in one launch");
-        const size_t lds = (size_t)3 * g.Ny * mpb * sizeof(double2) + (size_t)3 * g.Ny * sizeof(double);
-        allow_lds(kern, lds);
-        kern<<<dim3((unsigned)nblk), 256, lds, st>>>(g, hb, n, tab);
-    };
-    // Up to 48 even coefficients: 16-lane segments (four modes per wave, every
-    // shuffle a DPP row move) with up to three coefficients per lane. Above:
-    // one or two modes per wave, shuffles through LDS permutes.
-    if (Me <= 16) go(k_tau_solve_wave<1, 16, 16>, 16);
-    else if (Me <= 32) go(k_tau_solve_wave<2, 16, 16>, 16);
-    else if (Me <= 48) go(k_tau_solve_wave<3, 16, 16>, 16);
-    else if (Me <= 64) go(k_tau_solve_wave<1, 64, 4>, 64);
-    else if (Me <= 96) go(k_tau_solve_wave<3, 32, 8>, 32);
-    else if (Me <= 128) go(k_tau_solve_wave<2, 64, 4>, 64);
-    else go(k_tau_solve_wave<3, 64, 4>, 64);
-}
-
-// ===========================================================================
 // Elementwise combination (dnsalgo.cpp:218-224, 668-673)
 // ===========================================================================
 struct CombineArgs {
@@ -952,112 +316,6 @@ void launch_nonfinite(int nfields, const double* const* fields, long n, double* 
     const long want = (n + blk * 8L - 1) / (blk * 8L);  // about 8 values per thread
     const unsigned gx = (unsigned)std::max(1L, std::min(want, 1024L));
     k_nonfinite<<<dim3(gx, (unsigned)nfields), blk, 0, st>>>(fields, n, flags);
-}
-
-// ===========================================================================
-// NSE::linear on live modes (nse.cpp:393-477), one thread per mode
-// ===========================================================================
-// NSE::linear (nse.cpp:393-477) with one W-lane segment of a wavefront per
-// mode, MPB modes per block, member blockIdx.y: for each velocity component
-// L = nu (u'' - kappa^2 u) - grad q, plus on kx = kz = 0 nu U'', nu W'' and
-// the mean pressure gradient (the bulk-velocity branch takes dPdx from
-// nu (du/dy(b) - du/dy(a)) / Ly, nse.cpp:437-472). Real and imaginary parts
-// share each derivative scan.
-template <int K, int W, int MPB>
-__global__ void __launch_bounds__(W * MPB) k_linear_wave(Geom g, const LinearMember* __restrict__ tab) {
-    const LinearMember& me = tab[blockIdx.y];
-    const int m = blockIdx.x * MPB + threadIdx.x / W;
-    if (m >= g.M) return;  // whole segments leave together
-    const double nu = me.nu;
-    const LinearConst lc = me.c;
-    const gcdouble u = gmem(me.u), q = gmem(me.q);
-    __attribute__((address_space(1))) double* out = gmem_w(me.out);
-    const int Ny = g.Ny;
-    WCtx c;
-    c.N = Ny;
-    c.Me = (Ny + 1) / 2;
-    c.Mo = (Ny - 1) / 2;
-    c.Nb = Ny - 1;
-    c.Nc = Ny - 1;
-    c.lane = threadIdx.x % W;
-    c.L = g.b - g.a;
-    c.hb = nullptr;
-    const int ikx = m % g.nkx, kz = m / g.nkx, kx = kx_of(g, ikx);
-    const bool zero = kx == 0 && kz == 0;
-    const double kappa2 = 4 * PI * PI * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
-    const long rs = 2L * g.M;  // doubles between consecutive Chebyshev rows
-    auto row0 = [&](int comp) { return 2L * ((long)comp * Ny * g.M + m); };
-    WV<K> Pq[2] = {wload_s<K, W>(q + row0(0), rs, c), wload_s<K, W>(q + row0(0) + 1, rs, c)};
-    double dPd[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int comp = 0; comp < 3; ++comp) {
-        WV<K> s0[2] = {wload_s<K, W>(u + row0(comp), rs, c), wload_s<K, W>(u + row0(comp) + 1, rs, c)};
-        for (int p = 0; p < 2; ++p)
-            for (int k = 0; k < K; ++k) {
-                s0[p].e[k] *= nu;  // nu u
-                s0[p].o[k] *= nu;
-            }
-        WV<K> s1[2], s2[2];
-        wdiff_n<K, W, 2>(s0, c, s1);
-        if (zero && lc.bulk && comp != 1) {
-            double eb, ea;
-            wends<K, W>(s1[0], c, eb, ea);
-            dPd[comp] = (eb - ea) / c.L;
-        }
-        wdiff_n<K, W, 2>(s1, c, s2);  // nu u''
-        WV<K> o[2];
-        for (int p = 0; p < 2; ++p)
-            for (int k = 0; k < K; ++k) {
-                o[p].e[k] = s2[p].e[k] - kappa2 * s0[p].e[k];
-                o[p].o[k] = s2[p].o[k] - kappa2 * s0[p].o[k];
-            }
-        if (comp == 1) {  // - dq/dy
-            WV<K> dq[2];
-            wdiff_n<K, W, 2>(Pq, c, dq);
-            for (int p = 0; p < 2; ++p)
-                for (int k = 0; k < K; ++k) {
-                    o[p].e[k] = o[p].e[k] - dq[p].e[k];
-                    o[p].o[k] = o[p].o[k] - dq[p].o[k];
-                }
-        } else {  // - (i k) q: (0, d) * (Pr, Pi) = (-(d Pi), d Pr)
-            const double d = comp == 0 ? 2 * PI * kx / g.Lx : 2 * PI * kz / g.Lz;
-            for (int k = 0; k < K; ++k) {
-                o[0].e[k] = o[0].e[k] - (0.0 * Pq[0].e[k] - d * Pq[1].e[k]);
-                o[0].o[k] = o[0].o[k] - (0.0 * Pq[0].o[k] - d * Pq[1].o[k]);
-                o[1].e[k] = o[1].e[k] - (0.0 * Pq[1].e[k] + d * Pq[0].e[k]);
-                o[1].o[k] = o[1].o[k] - (0.0 * Pq[1].o[k] + d * Pq[0].o[k]);
-            }
-        }
-        if (zero && comp != 1) {
-            const WV<K> base = wload<K, W>(gmem(comp == 0 ? lc.nuUbaseyy : lc.nuWbaseyy), c);
-            for (int k = 0; k < K; ++k) {
-                o[0].e[k] += base.e[k];
-                o[0].o[k] += base.o[k];
-            }
-            if (c.lane == 0) {
-                if (!lc.bulk) o[0].e[0] -= comp == 0 ? lc.dPdxRef : lc.dPdzRef;
-                else o[0].e[0] -= dPd[comp] + (comp == 0 ? lc.nuUbase_slope : lc.nuWbase_slope);
-            }
-        }
-        wstore_s<K, W>(out + row0(comp), rs, o[0], c);
-        wstore_s<K, W>(out + row0(comp) + 1, rs, o[1], c);
-    }
-}
-
-void launch_linear(const Geom& g, int n, const LinearMember* tab, hipStream_t st) {
-    const int Me = (g.Ny + 1) / 2;
-    auto go = [&](auto kern, int w) {
-        const int mpb = 256 / w;
-        kern<<<dim3((g.M + mpb - 1) / mpb, n), 256, 0, st>>>(g, tab);
-    };
-    if (Me <= 16) go(k_linear_wave<1, 16, 16>, 16);
-    else if (Me <= 32) go(k_linear_wave<2, 16, 16>, 16);
-    else if (Me <= 48) go(k_linear_wave<3, 16, 16>, 16);
-    else if (Me <= 64) go(k_linear_wave<1, 64, 4>, 64);
-    else if (Me <= 96) go(k_linear_wave<3, 32, 8>, 32);
-    else if (Me <= 128) go(k_linear_wave<2, 64, 4>, 64);
-    else if (Me <= 192) go(k_linear_wave<3, 64, 4>, 64);
-    else throw std::runtime_error("NSE::linear: Ny above 383 is not supported");
 }
 
 // ===========================================================================

@@ -1,4 +1,5 @@
-// Kernel launchers of the MI355X DNS time step (implemented in cfg_kernels.hip).
+// Kernel launchers of the MI355X DNS time step (cfg_kernels.hip: the nonlinear
+// term; cfg_tau.hip: the tau solver).
 // All buffers are device pointers; all arithmetic is FP64.
 #pragma once
 

@@ -1,0 +1,695 @@
+// Tau-solver kernels of the MI355X DNS time step (gfx950, FP64): the per-mode
+// set-up, NSE::solve, PressureSolver::solve and NSE::linear, one (kx, kz) mode
+// (or one real part of it) per segment of a wavefront.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "cfg_dev.hpp"
+#include "cfg_math.hpp"
+#include "cfg_wave.hpp"
+
+namespace cfg {
+
+// Block order of a launch over (mode block, member) pairs: the dispatcher
+// hands consecutive workgroups to the 8 XCDs in turn, so the linear block
+// index is renumbered to put a contiguous range of pairs on each XCD, members
+// fastest. The members of a launch share their tau factors, which one XCD
+// then reads from its own L2 for every member after the first.
+__device__ __forceinline__ void xcd_block(int nmem, int& mode_block, int& member) {
+    const int T = gridDim.x;  // mode blocks x members
+    const int L = blockIdx.x;
+    const int q = T / NXCD, r = T % NXCD, x = L % NXCD;
+    const int p = x * q + (x < r ? x : r) + L / NXCD;
+    mode_block = p / nmem;
+    member = p - mode_block * nmem;
+}
+
+// ===========================================================================
+// Tau solver kernels: one thread per live mode (tausolver.cpp, nse.cpp:479)
+// ===========================================================================
+__device__ TauView make_view(const Geom& g, const TauSet& s, int m, double nu, bool taucorr) {
+    const int ikx = m % g.nkx, ikz = m / g.nkx;
+    const int kx = kx_of(g, ikx), kz = ikz;
+    const double pi2 = PI * PI;
+    const double kappa2 = 4 * pi2 * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
+    const double c = 4.0 * pi2 * nu;
+    const double lambda = s.lambda_t + c * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
+    double* cm = s.coef + (long)m * TAU_NA * g.Ny;
+    auto A = [&](int k) { return SV{cm + (long)k * g.Ny, 1}; };
+    TauView t;
+    t.ph = HelmholtzView{A(0), A(1), A(2), kappa2, g.Ny};
+    t.vh = HelmholtzView{A(3), A(4), A(5), lambda, g.Ny};
+    t.Pp = A(6);
+    t.Pm = A(7);
+    t.vp = A(8);
+    t.vm = A(9);
+    t.P0 = A(10);
+    t.v0 = A(11);
+    t.scal = s.scal + (long)m * 6;
+    t.sstride = 1;
+    t.nu = nu;
+    t.a = g.a;
+    t.b = g.b;
+    t.kx2pi = 2 * PI * kx / g.Lx;
+    t.kz2pi = 2 * PI * kz / g.Lz;
+    t.zero_mode = (kx == 0 && kz == 0);
+    t.taucorrection = taucorr;
+    return t;
+}
+
+// TauSolver constructor per mode (tausolver.cpp:81-176), T modes per block,
+// one thread each. ALL: the mode's whole working set in LDS, its 12 tau
+// profiles (array a at element (a*Ny + n)*T + t), 6 scalars and 2 scratch
+// profiles, copied to the mode-major tau set with contiguous writes at the end.
+// Otherwise (tall grids, where a block of 64 KB would hold fewer than 8 such
+// working sets) the profiles and scalars are built in place in the tau set and
+// only the 2 scratch profiles are in LDS. The arithmetic is tau_setup's either
+// way (the sequential set-up, bit for bit the oracle's); only the memory the
+// recurrences store to and reload from moves.
+template <bool ALL>
+__global__ void k_tau_setup(Geom g, TauSet s, double nu, int taucorr) {
+    extern __shared__ double sl[];
+    const int T = blockDim.x, t = threadIdx.x;
+    const int m0 = blockIdx.x * T, m = m0 + t;
+    const int Ny = g.Ny;
+    const long arr = (long)Ny * T;  // one profile of the block's modes
+    if (m < g.M) {
+        TauView v = make_view(g, s, m, nu, taucorr != 0);
+        auto A = [&](int a) { return SV{sl + a * arr + t, T}; };
+        if constexpr (ALL) {
+            v.ph.band = A(0);
+            v.ph.up = A(1);
+            v.ph.invd = A(2);
+            v.vh.band = A(3);
+            v.vh.up = A(4);
+            v.vh.invd = A(5);
+            v.Pp = A(6);
+            v.Pm = A(7);
+            v.vp = A(8);
+            v.vm = A(9);
+            v.P0 = A(10);
+            v.v0 = A(11);
+            v.scal = sl + 14 * arr + t;
+            v.sstride = T;
+            tau_setup(v, A(12), A(13));
+        } else {
+            tau_setup(v, A(0), A(1));
+        }
+    }
+    if constexpr (ALL) {
+        __syncthreads();
+        const int nm = min(T, g.M - m0);
+        __attribute__((address_space(1))) double* coef = gmem_w(s.coef) + (long)m0 * TAU_NA * Ny;
+        for (int i = t; i < nm * TAU_NA * Ny; i += T) {
+            const int mm = i / (TAU_NA * Ny), r = i - mm * (TAU_NA * Ny), a = r / Ny, n = r - a * Ny;
+            coef[i] = sl[a * arr + (long)n * T + mm];
+        }
+        __attribute__((address_space(1))) double* scal = gmem_w(s.scal) + (long)m0 * 6;
+        for (int i = t; i < nm * 6; i += T) scal[i] = sl[14 * arr + (long)(i % 6) * T + i / 6];
+    }
+}
+
+// modes per block of the set-up within 64 KB of LDS, at most 64: whole working
+// sets (14 profiles and 6 scalars each) where 8 or more fit, else scratch
+// profiles only (2 each)
+static int tau_setup_modes(int Ny, bool* all) {
+    const long whole = (14L * Ny + 6) * (long)sizeof(double), scratch = 2L * Ny * (long)sizeof(double);
+    const long T = (64L * 1024) / whole;
+    *all = T >= 8;
+    return (int)std::max(1L, std::min(64L, (64L * 1024) / (*all ? whole : scratch)));
+}
+
+void launch_tau_setup(const Geom& g, const TauSet& s, double nu, bool taucorr, hipStream_t st) {
+    bool all = false;
+    const int T = tau_setup_modes(g.Ny, &all);
+    const dim3 grid((g.M + T - 1) / T);
+    if (all) {
+        const size_t lds = (size_t)(14L * g.Ny + 6) * T * sizeof(double);
+        k_tau_setup<true><<<grid, T, lds, st>>>(g, s, nu, taucorr ? 1 : 0);
+    } else {
+        const size_t lds = (size_t)2 * g.Ny * T * sizeof(double);
+        k_tau_setup<false><<<grid, T, lds, st>>>(g, s, nu, taucorr ? 1 : 0);
+    }
+}
+
+__device__ __forceinline__ CV cview(double* base, const Geom& g, int comp, int m) {
+    const long S2 = 2L * g.M;
+    double* p = base + 2L * ((long)comp * g.Ny * g.M + m);
+    return CV{SV{p, S2}, SV{p + 1, S2}};
+}
+
+// Tau solve (NSE::solve, nse.cpp:479-575; TauSolver::solve, tausolver.cpp:347-450,
+// with solve_P_and_v :193-251). The operators of a mode are real, and the real
+// and imaginary parts of its equations couple only as (v, P real; u, w
+// imaginary) and (v, P imaginary; u, w real): two independent real problems
+//   P'' - kappa^2 P = Ry' - s (kx Rx + kz Rz),  v from P' - Ry,
+//   u from s kx P - Rx,  w from s kz P - Rz,
+// s = +1 with (Ry.re, Rx.im, Rz.im) and s = -1 with (Ry.im, Rx.re, Rz.re). Each
+// runs on its own W-lane segment of a wavefront.
+
+// The right-hand-side rows of a block's modes, [comp][n] at rows row0 .. row0 +
+// nrow (row = comp Ny + n): sum_j coef_j in_j (the multistep / Runge-Kutta
+// combination, dnsalgo.cpp:218-224, 668-673), handed to put(mode slot, row, re,
+// im). The term count is a template parameter and UNR rows are loaded per pass,
+// so the NT x UNR loads of a pass are all in flight before the first is summed
+// (36 or 54 in flight were no faster: 192x129x192 136-138 us against 130).
+template <int NT, int MPB, class Put>
+__device__ __forceinline__ void tau_stage_rhs(const TauMember& me, const Geom& g, int m0, int nthr, Put&& put) {
+    constexpr int UNR = NT <= 2 ? 8 : 16 / NT;  // 16 loads in flight at most
+    const __attribute__((address_space(1))) dvec2* in[NT];
+    double coef[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        in[j] = gmem(reinterpret_cast<const dvec2*>(me.in[j]));
+        coef[j] = me.coef[j];
+    }
+    const int ww = threadIdx.x % MPB, nrow = 3 * g.Ny, step = nthr / MPB;
+    const int mm = min(m0 + ww, g.M - 1);  // slots past the last mode repeat it
+    for (int row = threadIdx.x / MPB; row < nrow; row += UNR * step) {
+        dvec2 v[UNR][NT];
+#pragma unroll
+        for (int r = 0; r < UNR; ++r) {
+            // rows past the end repeat the last one, so that every load is issued unconditionally
+            const long off = (long)min(row + r * step, nrow - 1) * g.M + mm;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) v[r][j] = in[j][off];
+        }
+#pragma unroll
+        for (int r = 0; r < UNR; ++r) {
+            dvec2 acc = dvec2{0.0, 0.0};
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                acc.x += coef[j] * v[r][j].x;
+                acc.y += coef[j] * v[r][j].y;
+            }
+            if (row + r * step < nrow) put(ww, row + r * step, acc);
+        }
+    }
+}
+template <int MPB, class Put>
+__device__ __forceinline__ void tau_stage(const TauMember& me, const Geom& g, int m0, int nthr, Put&& put) {
+    switch (me.nterms) {
+        case 1: tau_stage_rhs<1, MPB>(me, g, m0, nthr, put); break;
+        case 2: tau_stage_rhs<2, MPB>(me, g, m0, nthr, put); break;
+        case 3: tau_stage_rhs<3, MPB>(me, g, m0, nthr, put); break;
+        case 4: tau_stage_rhs<4, MPB>(me, g, m0, nthr, put); break;
+        case 5: tau_stage_rhs<5, MPB>(me, g, m0, nthr, put); break;
+        case 6: tau_stage_rhs<6, MPB>(me, g, m0, nthr, put); break;
+        case 7: tau_stage_rhs<7, MPB>(me, g, m0, nthr, put); break;
+        default: tau_stage_rhs<MAX_TERMS, MPB>(me, g, m0, nthr, put); break;
+    }
+}
+
+// LDS of a tau-solve block of MPB modes: the rows of its 2 MPB real problems,
+// [mode][part][comp] of tau_pitch(Ny) doubles, then the rows of B (3 of 2KW
+// doubles, zero past Ny).
+__host__ __device__ constexpr int tau_pitch(int Ny) { return Ny + 1; }  // even (Ny is odd): 16-byte pairs
+constexpr size_t tau_lds(int Ny, int K, int W, int MPB) {
+    return ((size_t)MPB * 6 * tau_pitch(Ny) + (size_t)3 * 2 * K * W) * sizeof(double);
+}
+
+// Waves per SIMD a variant is compiled for, where its registers fit without
+// spilling more than a few values (K = 5: 256 registers; a third wave at K = 3
+// spills 164 bytes, one 64^3 field 14.6 -> 21.3 us).
+constexpr int tau_waves(int K, int W) { return W == 16 && K <= 5 ? (K == 1 ? 4 : K == 2 ? 3 : 2) : 1; }
+
+// Blocks of a launch, in XCD order: per member the block of the kx = kz = 0
+// mode alone (its mean-flow solves would run one after the other with the
+// general path of the modes beside it), then blocks of MPB consecutive modes;
+// the general path also passes over mode 0, and its result there is dropped.
+//
+// What bounds it: for one field the instruction chain of a wave, for a batch
+// HBM and that chain (24 x 32^3: 63 MB in 20.8 us, one round of blocks), for
+// one large field HBM (192x129x192: 450 MB in 120.8 us, 3.7 TB/s, of which the
+// right-hand-side rows are 256-byte pieces 130 KB apart). Against a segment per
+// complex mode with the scan multipliers recomputed for every right-hand side
+// and every lane past a system masked (8557 instructions at K = 3, now about
+// 2200): one 32^3 field 20.5 -> 9.2 us, 64^3 31.3 -> 14.6, 96^3 39.5 -> 23.5,
+// 128^3 66.7 -> 48.0, 192x129x192 138.7 -> 120.8, 24 x 32^3 26.8 -> 20.8.
+template <int K, int W, int MPB>
+__global__ void __launch_bounds__(2 * W * MPB) __attribute__((amdgpu_waves_per_eu(tau_waves(K, W))))
+k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMember* __restrict__ tab) {
+    extern __shared__ double2 lds2[];
+    double* const lds = reinterpret_cast<double*>(lds2);
+    constexpr int nthr = 2 * W * MPB, HP = 2 * K * W;
+    int mblk, mem;
+    xcd_block(nmem, mblk, mem);
+    const TauMember& me = tab[mem];
+    const TauSet s = me.set;
+    const double nu = me.nu;
+    const int taucorr = me.taucorr;
+    __attribute__((address_space(1))) dvec2* __restrict__ u = gmem_w(reinterpret_cast<dvec2*>(me.u));
+    __attribute__((address_space(1))) dvec2* __restrict__ q = gmem_w(reinterpret_cast<dvec2*>(me.q));
+    const int Ny = g.Ny, RP = tau_pitch(Ny);
+    double* const hbl = lds + MPB * 6 * RP;
+    for (int i = threadIdx.x; i < 3 * HP; i += nthr) {
+        const int r = i / HP, n = i % HP;
+        hbl[i] = n < Ny ? hb[r * Ny + n] : 0.0;
+    }
+    for (int i = threadIdx.x; i < 6 * MPB; i += nthr) lds[i * RP + Ny] = 0.0;  // the rows' padding
+    WCtx c;
+    c.N = Ny;
+    c.Me = (Ny + 1) / 2;
+    c.Mo = (Ny - 1) / 2;
+    c.Nb = Ny - 1;
+    c.Nc = Ny - 1;
+    c.lane = threadIdx.x % W;
+    c.L = g.b - g.a;
+    c.hb = hbl;
+    const int seg = threadIdx.x / W;
+    const gcdouble coef = gmem(s.coef);
+    const double pi2 = PI * PI;
+
+    if (mblk == 0) {  // kx = kz = 0: P from Ry', v = 0, u and w from the velocity operator; real parts only
+        double* const R = lds;  // [comp][RP]
+        for (int row = threadIdx.x; row < 3 * Ny; row += nthr) {
+            double acc = 0.0;
+            for (int j = 0; j < me.nterms; ++j) acc += me.coef[j] * gmem(me.in[j])[2L * row * g.M];
+            R[row + row / Ny * (RP - Ny)] = acc;
+        }
+        __syncthreads();
+        const SolveConst zc = me.sc;
+        // segment 0 solves for P, the first two of the next wavefront for u and w
+        constexpr int U0 = 64 / W;
+        static_assert(U0 >= 2 && 2 * MPB >= U0 + 2, "two segments in a wavefront, two wavefronts in a block");
+        if (seg == 0) {
+            const HelmOp<K, W> op(wfac3<K, W>(coef, Ny, 0, 0u, c), 0.0, c);
+            WV<K> y[1], f[1], x[1];
+            y[0] = wrow_load<K, W>(R + RP, c);
+            wdiff_n<K, W, 1>(y, c, f);
+            op.template solve<1>(f, c, x);
+            wrow_store<K, W>(R + RP, c, x[0]);
+        } else if (seg == U0 || seg == U0 + 1) {
+            const int cc = seg - U0;
+            double* const S = R + 2 * cc * RP;
+            const HelmOp<K, W> op(wfac3<K, W>(coef, Ny, 3, 0u, c), s.lambda_t, c);
+            const WV<K> r = wrow_load<K, W>(S, c);
+            const WV<K> Byy = wload<K, W>(gmem(cc == 0 ? zc.nuUbaseyy : zc.nuWbaseyy), c);
+            WV<K> f[1], x[1];  // nse.cpp:505-527: nu U'' (nu W''), and a fixed mean gradient
+            for (int i = 0; i < K; ++i) {
+                f[0].e[i] = -(r.e[i] + Byy.e[i]);
+                f[0].o[i] = -(r.o[i] + Byy.o[i]);
+            }
+            if (zc.bulk) {  // bulk-velocity constraint (tausolver.cpp:404-450, helmholtz.cpp:158-213)
+                WV<K> two[2], sol[2];
+                two[0] = f[0];
+                two[1] = wzero<K, W>();
+                if (c.lane == 0) two[1].e[0] = nu;
+                op.template solve<2>(two, c, sol);
+                const double uamean = wmean<K, W>(sol[0], c), ucmean = wmean<K, W>(sol[1], c);
+                const double mu = nu * ((cc == 0 ? zc.umean : zc.wmean) - uamean) / ucmean;
+                if (c.lane == 0) {
+                    f[0].e[0] += mu;
+                    *(cc == 0 ? zc.dPdx_out : zc.dPdz_out) = mu;
+                }
+            } else if (c.lane == 0) {
+                f[0].e[0] += cc == 0 ? zc.dPdxRef : zc.dPdzRef;
+            }
+            op.template solve<1>(f, c, x);
+            wrow_store<K, W>(S, c, x[0]);
+        }
+        __syncthreads();
+        for (int row = threadIdx.x; row < 3 * Ny; row += nthr) {
+            const double v = R[row + row / Ny * (RP - Ny)];
+            const bool mid = row >= Ny && row < 2 * Ny;
+            if (mid) q[(long)(row - Ny) * g.M] = dvec2{v, 0.0};
+            u[(long)row * g.M] = dvec2{mid ? 0.0 : v, 0.0};
+        }
+        return;
+    }
+
+    const int m0 = (mblk - 1) * MPB;
+    const int w = seg >> 1, part = seg & 1;
+    const int m = min(m0 + w, g.M - 1);
+    // part 0 takes Ry.re, Rx.im, Rz.im; part 1 Ry.im, Rx.re, Rz.re
+    auto slot = [&](int ww, int pt, int row) {
+        const int comp = (row >= Ny) + (row >= 2 * Ny);
+        return ((ww * 2 + pt) * 3 + comp) * RP + row - comp * Ny;
+    };
+    const unsigned fo = (unsigned)m * (TAU_NA * Ny);  // this mode's factors
+    tau_stage<MPB>(me, g, m0, nthr, [&](int ww, int row, dvec2 v) {
+        const bool mid = row >= Ny && row < 2 * Ny;
+        lds[slot(ww, 0, row)] = mid ? v.x : v.y;
+        lds[slot(ww, 1, row)] = mid ? v.y : v.x;
+    });
+    __syncthreads();
+    const int ikx = m % g.nkx, ikz = m / g.nkx;
+    const int kx = kx_of(g, ikx), kz = ikz;
+    const double kk = (kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz);
+    const double kappa2 = 4 * pi2 * kk;
+    const double lambda = s.lambda_t + (4.0 * pi2 * nu) * kk;
+    const double sgn = part ? -1.0 : 1.0;
+    const double ax = sgn * (2 * PI * kx / g.Lx), az = sgn * (2 * PI * kz / g.Lz);
+    double* const Sx = lds + (seg * 3 + 0) * RP;
+    double* const Sy = lds + (seg * 3 + 1) * RP;
+    double* const Sz = lds + (seg * 3 + 2) * RP;
+    WV<K> P[1], v[1];
+    {
+        WV<K> f[1], t[1];
+        t[0] = wrow_load<K, W>(Sy, c);
+        wdiff_n<K, W, 1>(t, c, f);
+        const WV<K> X = wrow_load<K, W>(Sx, c), Z = wrow_load<K, W>(Sz, c);
+        for (int k = 0; k < K; ++k) {
+            f[0].e[k] -= ax * X.e[k] + az * Z.e[k];
+            f[0].o[k] -= ax * X.o[k] + az * Z.o[k];
+        }
+        const HelmOp<K, W> op(wfac3<K, W>(coef, Ny, 0, fo, c), kappa2, c);
+        op.template solve<1>(f, c, P);
+    }
+    const HelmOp<K, W> vop(wfac3<K, W>(coef, Ny, 3, fo, c), lambda, c);  // velocity operator: v, then u and w
+    {
+        WV<K> f[1], t[1];
+        wdiff_n<K, W, 1>(P, c, f);
+        t[0] = wrow_load<K, W>(Sy, c);
+        for (int k = 0; k < K; ++k) {
+            f[0].e[k] -= t[0].e[k];
+            f[0].o[k] -= t[0].o[k];
+        }
+        vop.template solve<1>(f, c, v);
+        // influence-matrix correction (tausolver.cpp:178-191)
+        double dvb[1], dva[1];
+        wdiff_n<K, W, 1>(v, c, f);
+        wends_n<K, W, 1>(f, c, dvb, dva);
+        const gcdouble sc = gmem(s.scal) + 6L * m;
+        const double dplus = -sc[0] * dvb[0] - sc[1] * dva[0];
+        const double dminus = -sc[2] * dvb[0] - sc[3] * dva[0];
+        const WV<K> Pp = wfac<K, W>(coef, Ny, 6, fo, c), Pm = wfac<K, W>(coef, Ny, 7, fo, c);
+        const WV<K> vp = wfac<K, W>(coef, Ny, 8, fo, c), vm = wfac<K, W>(coef, Ny, 9, fo, c);
+        for (int k = 0; k < K; ++k) {
+            P[0].e[k] += dplus * Pp.e[k] + dminus * Pm.e[k];
+            P[0].o[k] += dplus * Pp.o[k] + dminus * Pm.o[k];
+            v[0].e[k] += dplus * vp.e[k] + dminus * vm.e[k];
+            v[0].o[k] += dplus * vp.o[k] + dminus * vm.o[k];
+        }
+        if (taucorr) {
+            const int Nb = c.Nb;
+            const WV<K> P0 = wfac<K, W>(coef, Ny, 10, fo, c), v0 = wfac<K, W>(coef, Ny, 11, fo, c);
+            const double sigma1_Nb = lambda * wtop<K, W>(v[0], c) - Sy[Nb];
+            double sigma1_Nb1 = lambda * wtop1<K, W>(v[0], c) - Sy[Nb - 1];
+            sigma1_Nb1 += (4.0 / c.L) * Nb * wtop<K, W>(P[0], c);
+            const double sigmaNb = sigma1_Nb / (1.0 - sc[5]);
+            const double sigmaNb1 = sigma1_Nb1 / (1.0 - sc[4]);
+            for (int k = 0; k < K; ++k) {
+                P[0].e[k] += sigmaNb1 * P0.e[k];
+                P[0].o[k] += sigmaNb * P0.o[k];
+                v[0].e[k] += sigmaNb * v0.e[k];
+                v[0].o[k] += sigmaNb1 * v0.o[k];
+            }
+        }
+    }
+    wrow_store<K, W>(Sy, c, v[0]);  // the rows are this segment's alone
+    // u and w, one parity at a time (fewer live registers)
+    auto solve_uw = [&](const HelmPar<K, W>& op, const double (&Pk)[K], int par, int M) {
+        double f[2][K], x[2][K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int n = 2 * min(K * c.lane + k, M - 1) + par;
+            f[0][k] = ax * Pk[k] - Sx[n];
+            f[1][k] = az * Pk[k] - Sz[n];
+        }
+        op.template solve<2>(f, hbl + 2 * K * c.lane + par, HP, c, x);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int i = K * c.lane + k;
+            if (i < M) {
+                Sx[2 * i + par] = x[0][k];
+                Sz[2 * i + par] = x[1][k];
+            }
+        }
+    };
+    solve_uw(vop.e, P[0].e, 0, c.Me);
+    solve_uw(vop.o, P[0].o, 1, c.Mo);
+    __syncthreads();
+    const int ww = threadIdx.x % MPB, mm = m0 + ww;
+    const bool out = mm > 0 && mm < g.M;
+    for (int row = threadIdx.x / MPB; row < 3 * Ny; row += nthr / MPB) {
+        const double a = lds[slot(ww, 0, row)], b = lds[slot(ww, 1, row)];
+        const bool mid = row >= Ny && row < 2 * Ny;
+        if (out) u[(long)row * g.M + mm] = mid ? dvec2{a, b} : dvec2{b, a};
+    }
+    __syncthreads();
+    wrow_store<K, W>(Sy, c, P[0]);
+    __syncthreads();
+    for (int row = Ny + threadIdx.x / MPB; row < 2 * Ny; row += nthr / MPB) {
+        const double a = lds[slot(ww, 0, row)], b = lds[slot(ww, 1, row)];
+        if (out) q[(long)(row - Ny) * g.M + mm] = dvec2{a, b};
+    }
+}
+
+// PressureSolver::solve (poissonsolver.cpp:326-431) per mode, after the
+// nonlinear term f of u + U: p'' - kappa^2 p = -div f with p = 0 at the walls,
+// solved with the pressure factors of the tau data (the same Helmholtz operator,
+// nu = 1), then for every mode but (0,0) the wall correction
+// g = c exp(-mu (y-a)) + d exp(mu (y-b)), mu^2 = kappa^2, that makes
+// dp/dy = nu v'' at y = a, b; g's coefficients are Ti times its values at the
+// Chebyshev points.
+template <int K, int W, int MPB>
+__global__ void __launch_bounds__(W * MPB) k_pressure_wave(Geom g, YMats ym, PressArgs pa, const double* __restrict__ hb) {
+    extern __shared__ double2 lds[];  // [MPB][4][Ny]: f0, f1, f2, v; then the B rows [3][Ny]
+    const int Ny = g.Ny;
+    double* hbl = reinterpret_cast<double*>(lds + 4 * Ny * MPB);
+    for (int i = threadIdx.x; i < 3 * Ny; i += W * MPB) hbl[i] = hb[i];
+    const long M = g.M;
+    const int m0 = blockIdx.x * MPB, w = threadIdx.x / W;
+    const long m = m0 + w;
+    const bool valid = m < M;
+    const double2* __restrict__ f = reinterpret_cast<const double2*>(pa.f);
+    const double2* __restrict__ u = reinterpret_cast<const double2*>(pa.u);
+    double2* __restrict__ q = reinterpret_cast<double2*>(pa.q);
+    for (int idx = threadIdx.x; idx < 4 * Ny * MPB; idx += W * MPB) {
+        const int ww = idx % MPB, rest = idx / MPB, n = rest % Ny, comp = rest / Ny;
+        const long mm = m0 + ww;
+        double2 v = make_double2(0.0, 0.0);
+        if (mm < M) v = comp < 3 ? f[((long)comp * Ny + n) * M + mm] : u[((long)Ny + n) * M + mm];
+        lds[(ww * 4 + comp) * Ny + n] = v;
+    }
+    __syncthreads();
+    WCtx c;
+    c.N = Ny;
+    c.Me = (Ny + 1) / 2;
+    c.Mo = (Ny - 1) / 2;
+    c.Nb = Ny - 1;
+    c.Nc = Ny - 1;
+    c.lane = threadIdx.x % W;
+    c.L = g.b - g.a;
+    c.hb = hbl;
+    if (valid) {
+        const int ikx = (int)(m % g.nkx), ikz = (int)(m / g.nkx);
+        const int kx = kx_of(g, ikx), kz = ikz;
+        const bool zero = (kx == 0 && kz == 0);
+        const double pi2 = PI * PI;
+        const double kappa2 = 4 * pi2 * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
+        const double ax = 2 * PI * kx / g.Lx, az = 2 * PI * kz / g.Lz;
+        const double* cm = pa.set.coef + m * TAU_NA * Ny;
+        WV<K> Fxr, Fxi, Fyr, Fyi, Fzr, Fzi;
+        wload_c<K, W>(lds + (w * 4 + 0) * Ny, c, Fxr, Fxi);
+        wload_c<K, W>(lds + (w * 4 + 1) * Ny, c, Fyr, Fyi);
+        wload_c<K, W>(lds + (w * 4 + 2) * Ny, c, Fzr, Fzi);
+        const WV<K> Dr = wdiff<K, W>(Fyr, c), Di = wdiff<K, W>(Fyi, c);
+        WV<K> Rr, Ri;  // -div f (diffops.cpp:2488-2516)
+        for (int k = 0; k < K; ++k) {
+            Rr.e[k] = -((-ax * Fxi.e[k] - az * Fzi.e[k]) + Dr.e[k]);
+            Rr.o[k] = -((-ax * Fxi.o[k] - az * Fzi.o[k]) + Dr.o[k]);
+            Ri.e[k] = -((ax * Fxr.e[k] + az * Fzr.e[k]) + Di.e[k]);
+            Ri.o[k] = -((ax * Fxr.o[k] + az * Fzr.o[k]) + Di.o[k]);
+        }
+        WV<K> Pr = whelm<K, W>(Rr, cm, cm + Ny, cm + 2L * Ny, kappa2, 0.0, 0.0, c);
+        WV<K> Pi = whelm<K, W>(Ri, cm, cm + Ny, cm + 2L * Ny, kappa2, 0.0, 0.0, c);
+        if (!zero) {  // dp/dy = nu v'' at the walls (poissonsolver.cpp:356-427)
+            WV<K> Vr, Vi;
+            wload_c<K, W>(lds + (w * 4 + 3) * Ny, c, Vr, Vi);
+            double pbr, par_, pbi, pai, vbr, var_, vbi, vai;
+            wends<K, W>(wdiff<K, W>(Pr, c), c, pbr, par_);
+            wends<K, W>(wdiff<K, W>(Pi, c), c, pbi, pai);
+            wends<K, W>(wdiff<K, W>(wdiff<K, W>(Vr, c), c), c, vbr, var_);
+            wends<K, W>(wdiff<K, W>(wdiff<K, W>(Vi, c), c), c, vbi, vai);
+            const double alr = pa.nu * var_ - par_, ali = pa.nu * vai - pai;
+            const double ber = pa.nu * vbr - pbr, bei = pa.nu * vbi - pbi;
+            const double mu = sqrt(kappa2), H = g.b - g.a, e = exp(-mu * H);
+            const double delta = mu * (1 - exp(-2 * mu * H));
+            const double ccr = (-alr + ber * e) / delta, cci = (-ali + bei * e) / delta;
+            const double ddr = (ber - alr * e) / delta, ddi = (bei - ali * e) / delta;
+            const double piN = PI / (Ny - 1), rad = (g.b - g.a) / 2, cen = (g.b + g.a) / 2;  // chebypoints
+            for (int par = 0; par < 2; ++par)
+                for (int k = 0; k < K; ++k) {
+                    const int n = 2 * (K * c.lane + k) + par;
+                    if (n >= Ny) continue;
+                    double sr = 0.0, si = 0.0;
+                    for (int j = 0; j < Ny; ++j) {
+                        const double y = cen + rad * cos(j * piN);
+                        const double e1 = exp(-mu * (y - g.a)), e2 = exp(mu * (y - g.b));
+                        const double t = ym.Ti[(long)n * Ny + j];
+                        sr += t * (ccr * e1 + ddr * e2);
+                        si += t * (cci * e1 + ddi * e2);
+                    }
+                    if (par == 0) {
+                        Pr.e[k] += sr;
+                        Pi.e[k] += si;
+                    } else {
+                        Pr.o[k] += sr;
+                        Pi.o[k] += si;
+                    }
+                }
+        }
+        wstore_c<K, W>(lds + (w * 4 + 0) * Ny, c, Pr, Pi);
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < Ny * MPB; idx += W * MPB) {
+        const int ww = idx % MPB, n = idx / MPB;
+        const long mm = m0 + ww;
+        if (mm < M) q[(long)n * M + mm] = lds[(ww * 4 + 0) * Ny + n];
+    }
+}
+
+void launch_pressure(const Geom& g, const YMats& ym, const double* hb, const PressArgs& pa, hipStream_t st) {
+    const int Me = (g.Ny + 1) / 2;
+    auto go = [&](auto kern, int w) {
+        const int mpb = 256 / w;
+        const dim3 grid((unsigned)((g.M + mpb - 1) / mpb));
+        const size_t lds = (size_t)4 * g.Ny * mpb * sizeof(double2) + (size_t)3 * g.Ny * sizeof(double);
+        allow_lds(kern, lds);
+        kern<<<grid, 256, lds, st>>>(g, ym, pa, hb);
+    };
+    if (Me <= 16) go(k_pressure_wave<1, 16, 16>, 16);
+    else if (Me <= 32) go(k_pressure_wave<1, 32, 8>, 32);
+    else if (Me <= 64) go(k_pressure_wave<1, 64, 4>, 64);
+    else if (Me <= 128) go(k_pressure_wave<2, 64, 4>, 64);
+    else go(k_pressure_wave<3, 64, 4>, 64);
+}
+
+void launch_tau_solve(const Geom& g, const double* hb, int n, const TauMember* tab, hipStream_t st) {
+    const int Me = (g.Ny + 1) / 2;  // even coefficients: at most K per lane of a W-lane segment
+    auto go = [&](auto kern, int k, int w, int mpb) {
+        const long nblk = ((long)((g.M + mpb - 1) / mpb) + 1) * n;
+        if (nblk > 0x7fffffffL) throw std::runtime_error("tau solve: too many blocks in one launch");
+        const size_t lds = tau_lds(g.Ny, k, w, mpb);
+        allow_lds(kern, lds);
+        kern<<<dim3((unsigned)nblk), 2 * w * mpb, lds, st>>>(g, hb, n, tab);
+    };
+    // 16-lane segments (every shuffle a DPP row move) as far as their
+    // coefficients fit the registers, 32 lanes above. 8 modes per block: with 16
+    // a lone 32^3 field took 12.4 us, not 9.2, 64^3 17.1, not 14.6, and 24 of
+    // 32^3 26.7, not 20.8. At 65-80 coefficients, where a block of 8 leaves
+    // half-filled 256-byte runs of every row, 16 modes per block are faster once
+    // one field fills the chip with them (192x129x192 122.5 -> 120.8 us, 128^3,
+    // 224 blocks, 53.3 -> 48.0). The rule looks at the grid alone: a member's
+    // result must not depend on which instance its batch runs.
+    if (Me <= 16) go(k_tau_solve_wave<1, 16, 8>, 1, 16, 8);
+    else if (Me <= 32) go(k_tau_solve_wave<2, 16, 8>, 2, 16, 8);
+    else if (Me <= 48) go(k_tau_solve_wave<3, 16, 8>, 3, 16, 8);
+    else if (Me <= 64) go(k_tau_solve_wave<4, 16, 8>, 4, 16, 8);
+    else if (Me <= 80 && g.M >= 192 * 16) go(k_tau_solve_wave<5, 16, 16>, 5, 16, 16);
+    else if (Me <= 80) go(k_tau_solve_wave<5, 16, 8>, 5, 16, 8);
+    else if (Me <= 96) go(k_tau_solve_wave<6, 16, 8>, 6, 16, 8);
+    else if (Me <= 128) go(k_tau_solve_wave<4, 32, 4>, 4, 32, 4);
+    else go(k_tau_solve_wave<6, 32, 4>, 6, 32, 4);
+}
+
+// ===========================================================================
+// NSE::linear on live modes (nse.cpp:393-477), one thread per mode
+// ===========================================================================
+// NSE::linear (nse.cpp:393-477) with one W-lane segment of a wavefront per
+// mode, MPB modes per block, member blockIdx.y: for each velocity component
+// L = nu (u'' - kappa^2 u) - grad q, plus on kx = kz = 0 nu U'', nu W'' and
+// the mean pressure gradient (the bulk-velocity branch takes dPdx from
+// nu (du/dy(b) - du/dy(a)) / Ly, nse.cpp:437-472). Real and imaginary parts
+// share each derivative scan.
+template <int K, int W, int MPB>
+__global__ void __launch_bounds__(W * MPB) k_linear_wave(Geom g, const LinearMember* __restrict__ tab) {
+    const LinearMember& me = tab[blockIdx.y];
+    const int m = blockIdx.x * MPB + threadIdx.x / W;
+    if (m >= g.M) return;  // whole segments leave together
+    const double nu = me.nu;
+    const LinearConst lc = me.c;
+    const gcdouble u = gmem(me.u), q = gmem(me.q);
+    __attribute__((address_space(1))) double* out = gmem_w(me.out);
+    const int Ny = g.Ny;
+    WCtx c;
+    c.N = Ny;
+    c.Me = (Ny + 1) / 2;
+    c.Mo = (Ny - 1) / 2;
+    c.Nb = Ny - 1;
+    c.Nc = Ny - 1;
+    c.lane = threadIdx.x % W;
+    c.L = g.b - g.a;
+    c.hb = nullptr;
+    const int ikx = m % g.nkx, kz = m / g.nkx, kx = kx_of(g, ikx);
+    const bool zero = kx == 0 && kz == 0;
+    const double kappa2 = 4 * PI * PI * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
+    const long rs = 2L * g.M;  // doubles between consecutive Chebyshev rows
+    auto row0 = [&](int comp) { return 2L * ((long)comp * Ny * g.M + m); };
+    WV<K> Pq[2] = {wload_s<K, W>(q + row0(0), rs, c), wload_s<K, W>(q + row0(0) + 1, rs, c)};
+    double dPd[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int comp = 0; comp < 3; ++comp) {
+        WV<K> s0[2] = {wload_s<K, W>(u + row0(comp), rs, c), wload_s<K, W>(u + row0(comp) + 1, rs, c)};
+        for (int p = 0; p < 2; ++p)
+            for (int k = 0; k < K; ++k) {
+                s0[p].e[k] *= nu;  // nu u
+                s0[p].o[k] *= nu;
+            }
+        WV<K> s1[2], s2[2];
+        wdiff_n<K, W, 2>(s0, c, s1);
+        if (zero && lc.bulk && comp != 1) {
+            double eb, ea;
+            wends<K, W>(s1[0], c, eb, ea);
+            dPd[comp] = (eb - ea) / c.L;
+        }
+        wdiff_n<K, W, 2>(s1, c, s2);  // nu u''
+        WV<K> o[2];
+        for (int p = 0; p < 2; ++p)
+            for (int k = 0; k < K; ++k) {
+                o[p].e[k] = s2[p].e[k] - kappa2 * s0[p].e[k];
+                o[p].o[k] = s2[p].o[k] - kappa2 * s0[p].o[k];
+            }
+        if (comp == 1) {  // - dq/dy
+            WV<K> dq[2];
+            wdiff_n<K, W, 2>(Pq, c, dq);
+            for (int p = 0; p < 2; ++p)
+                for (int k = 0; k < K; ++k) {
+                    o[p].e[k] = o[p].e[k] - dq[p].e[k];
+                    o[p].o[k] = o[p].o[k] - dq[p].o[k];
+                }
+        } else {  // - (i k) q: (0, d) * (Pr, Pi) = (-(d Pi), d Pr)
+            const double d = comp == 0 ? 2 * PI * kx / g.Lx : 2 * PI * kz / g.Lz;
+            for (int k = 0; k < K; ++k) {
+                o[0].e[k] = o[0].e[k] - (0.0 * Pq[0].e[k] - d * Pq[1].e[k]);
+                o[0].o[k] = o[0].o[k] - (0.0 * Pq[0].o[k] - d * Pq[1].o[k]);
+                o[1].e[k] = o[1].e[k] - (0.0 * Pq[1].e[k] + d * Pq[0].e[k]);
+                o[1].o[k] = o[1].o[k] - (0.0 * Pq[1].o[k] + d * Pq[0].o[k]);
+            }
+        }
+        if (zero && comp != 1) {
+            const WV<K> base = wload<K, W>(gmem(comp == 0 ? lc.nuUbaseyy : lc.nuWbaseyy), c);
+            for (int k = 0; k < K; ++k) {
+                o[0].e[k] += base.e[k];
+                o[0].o[k] += base.o[k];
+            }
+            if (c.lane == 0) {
+                if (!lc.bulk) o[0].e[0] -= comp == 0 ? lc.dPdxRef : lc.dPdzRef;
+                else o[0].e[0] -= dPd[comp] + (comp == 0 ? lc.nuUbase_slope : lc.nuWbase_slope);
+            }
+        }
+        wstore_s<K, W>(out + row0(comp), rs, o[0], c);
+        wstore_s<K, W>(out + row0(comp) + 1, rs, o[1], c);
+    }
+}
+
+void launch_linear(const Geom& g, int n, const LinearMember* tab, hipStream_t st) {
+    const int Me = (g.Ny + 1) / 2;
+    auto go = [&](auto kern, int w) {
+        const int mpb = 256 / w;
+        kern<<<dim3((g.M + mpb - 1) / mpb, n), 256, 0, st>>>(g, tab);
+    };
+    if (Me <= 16) go(k_linear_wave<1, 16, 16>, 16);
+    else if (Me <= 32) go(k_linear_wave<2, 16, 16>, 16);
+    else if (Me <= 48) go(k_linear_wave<3, 16, 16>, 16);
+    else if (Me <= 64) go(k_linear_wave<1, 64, 4>, 64);
+    else if (Me <= 96) go(k_linear_wave<3, 32, 8>, 32);
+    else if (Me <= 128) go(k_linear_wave<2, 64, 4>, 64);
+    else if (Me <= 192) go(k_linear_wave<3, 64, 4>, 64);
+    else throw std::runtime_error("NSE::linear: Ny above 383 is not supported");
+}
+
+}  // namespace cfg

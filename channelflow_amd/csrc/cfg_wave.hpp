@@ -225,17 +225,6 @@ __device__ __forceinline__ double wtop(const WV<K>& v, const WCtx& c) { return w
 template <int K, int W>
 __device__ __forceinline__ double wtop1(const WV<K>& v, const WCtx& c) { return wpick<K, W>(v.o, c.Mo - 1, c); }
 
-// a*x + b*y elementwise
-template <int K, int W>
-__device__ __forceinline__ WV<K> waxpby(double a, const WV<K>& x, double b, const WV<K>& y) {
-    WV<K> r;
-    for (int k = 0; k < K; ++k) {
-        r.e[k] = a * x.e[k] + b * y.e[k];
-        r.o[k] = a * x.o[k] + b * y.o[k];
-    }
-    return r;
-}
-
 // suffix sums of t over the blocked index: out[i] = sum_{j >= i} t[j]
 // (inclusive) and excl[i] = sum_{j > i} t[j]
 template <int K, int W>
@@ -576,23 +565,6 @@ __device__ __forceinline__ double wmean(const WV<K>& v, const WCtx& c) {
     return wbc<W>(v.e[0], 0) - wsum<W>(part, c.lane);
 }
 
-// Helmholtz solve with unknown constant forcing mu and mean(u) = umean
-// (helmholtz.cpp:158-213); returns mu.
-template <int K, int W, class P>
-__device__ __forceinline__ double whelm_mean(const WV<K>& f, P band, P up, P invd, double lambda, double nu,
-                                             double umean, const WCtx& c, WV<K>& u) {
-    const double uamean = wmean<K, W>(whelm<K, W>(f, band, up, invd, lambda, 0.0, 0.0, c), c);
-    WV<K> r = wzero<K, W>();
-    if (c.lane == 0) r.e[0] = nu;
-    const double ucmean = wmean<K, W>(whelm<K, W>(r, band, up, invd, lambda, 0.0, 0.0, c), c);
-    const double mu = nu * (umean - uamean) / ucmean;
-    r = f;
-    if (c.lane == 0) r.e[0] += mu;
-    u = whelm<K, W>(r, band, up, invd, lambda, 0.0, 0.0, c);
-    return mu;
-}
-
-
 // suffix sums of NR arrays at once (as wsuffix)
 template <int K, int W, int NR>
 __device__ __forceinline__ void wsuffix_n(const double (&t)[NR][K], double (&incl)[NR][K], double (&excl)[NR][K],
@@ -679,6 +651,241 @@ __device__ __forceinline__ void wends_n(const WV<K> (&v)[NR], const WCtx& c, dou
         at_a[r] = s2[2 * r] - s2[2 * r + 1];
     }
 }
+
+// ---- one operator, several solves ----------------------------------------------
+// A profile in a row of doubles: pairs (row[2i], row[2i+1]), the row 16-byte
+// aligned and row[N] (N is odd) finite. Lanes past the profile hold its last
+// pair: finite values that the operators' zero entries cancel (HelmPar).
+template <int K, int W>
+__device__ __forceinline__ WV<K> wrow_load(const double* row, const WCtx& c) {
+    WV<K> v;
+    const dvec2* p = reinterpret_cast<const dvec2*>(row);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const dvec2 a = p[min(K * c.lane + k, c.Me - 1)];
+        v.e[k] = a.x;
+        v.o[k] = a.y;
+    }
+    return v;
+}
+template <int K, int W>
+__device__ __forceinline__ void wrow_store(double* row, const WCtx& c, const WV<K>& v) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = K * c.lane + k;
+        if (i < c.Me) row[2 * i] = v.e[k];
+        if (i < c.Mo) row[2 * i + 1] = v.o[k];
+    }
+}
+// Array k of a tau set's mode (coef + off: the mode's first array), loaded at a
+// uniform base with a 32-bit offset per lane. Lanes past the profile hold its
+// last entries.
+template <int K, int W>
+__device__ __forceinline__ WV<K> wfac(const gcdouble coef, int Ny, int arr, unsigned off, const WCtx& c) {
+    const gcdouble b = coef + (long)arr * Ny;
+    WV<K> v;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = K * c.lane + k;
+        v.e[k] = b[off + (unsigned)(2 * min(i, c.Me - 1))];
+        v.o[k] = b[off + (unsigned)(2 * min(i, c.Mo - 1) + 1)];
+    }
+    return v;
+}
+
+// the factors of one Helmholtz operator as loaded: arrays arr, arr + 1, arr + 2
+// (band, up, 1/diag) of a mode
+template <int K>
+struct HelmRaw {
+    WV<K> band, up, invd;
+};
+template <int K, int W>
+__device__ __forceinline__ HelmRaw<K> wfac3(const gcdouble coef, int Ny, int arr, unsigned off, const WCtx& c) {
+    return HelmRaw<K>{wfac<K, W>(coef, Ny, arr, off, c), wfac<K, W>(coef, Ny, arr + 1, off, c),
+                      wfac<K, W>(coef, Ny, arr + 2, off, c)};
+}
+
+constexpr int wlog2(int w) {
+    int l = 0;
+    while ((1 << l) < w) ++l;
+    return l;
+}
+
+// One parity system of nu u'' - lambda u = f with u = 0 at both ends, from its
+// UL factors (whelm_par_n's solve), the multipliers of its scans' steps formed
+// once for every solve with it. Zero are: invd and band past the system and on
+// row 0 (band_0 sits in b0), up on row 0 and on the last row (where the factors
+// hold 0). Then rows past the system contribute nothing whatever their finite
+// right-hand sides are, row 0 of B f is 0, and no scan step needs a condition.
+template <int K, int W>
+struct HelmPar {
+    double up[K], band[K], invd[K], xs[wlog2(W)], xp[wlog2(W)];
+    double b0, rb, lam;
+
+    __device__ __forceinline__ void init(double lambda, const double* bl, int stride, int M, const WCtx& c) {
+        lam = lambda;
+        b0 = band[0];
+        rb = 1.0 / b0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const bool in = K * c.lane + k < M && (k > 0 || c.lane > 0);
+            band[k] = in ? band[k] : 0.0;
+            invd[k] = in ? invd[k] : 0.0;
+        }
+        if (c.lane == 0) up[0] = 0.0;
+        double xa = 1.0, ya = 1.0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            xa *= -up[k];
+            ya *= lambda * bl[stride * k] * invd[k];
+        }
+        int s = 0;
+#pragma unroll
+        for (int d = 1; d < W; d <<= 1, ++s) {
+            xs[s] = (wrow<W>() || c.lane + d < W) ? xa : 0.0;
+            xp[s] = (wrow<W>() || c.lane >= d) ? ya : 0.0;
+            const double x1 = wdn1<W>(xa, d), y1 = wup1<W>(ya, d);
+            xa = (wrow<W>() || c.lane + d < W) ? xa * x1 : xa;
+            ya = (wrow<W>() || c.lane >= d) ? ya * y1 : ya;
+        }
+    }
+
+    // x = A^{-1} (B f) for NR right-hand sides; hb: this parity's B rows of the
+    // lane's coefficients (lower, diagonal, upper at hstride doubles, k at stride 2)
+    template <int NR>
+    __device__ __forceinline__ void solve(const double (&f)[NR][K], const double* hb, int hstride, const WCtx& c,
+                                          double (&x)[NR][K]) const {
+        const int lane = c.lane;
+        double bl[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) bl[k] = hb[2 * k];
+        double xc[NR];
+        double Fa[K];
+        {
+            double bd[K], bu[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                bd[k] = hb[hstride + 2 * k];
+                bu[k] = hb[2 * hstride + 2 * k];
+            }
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const double prev = wup<W>(f[r][K - 1], 1), next = wdn<W>(f[r][0], 1);
+                xc[r] = 0.0;
+#pragma unroll
+                for (int k = K - 1; k >= 0; --k) {
+                    const double fm = k > 0 ? f[r][k - 1] : prev, fp = k + 1 < K ? f[r][k + 1] : next;
+                    const double u = bl[k] * fm + bd[k] * f[r][k] + bu[k] * fp;
+                    xc[r] = u - up[k] * xc[r];
+                    x[r][k] = xc[r];
+                }
+            }
+            double a = 1.0;
+#pragma unroll
+            for (int k = K - 1; k >= 0; --k) {
+                a *= -up[k];
+                Fa[k] = a;
+            }
+        }
+        int s = 0;
+#pragma unroll
+        for (int d = 1; d < W; d <<= 1, ++s)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) xc[r] = fma(xs[s], wdn<W>(xc[r], d), xc[r]);
+        double part[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            double ec = wdn<W>(xc[r], 1);
+            if (!wrow<W>() && lane == W - 1) ec = 0.0;
+            part[r] = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                x[r][k] = x[r][k] + Fa[k] * ec;
+                part[r] += band[k] * x[r][k];
+                x[r][k] *= invd[k];
+            }
+        }
+        wsum_n<W, NR>(part, lane);
+        // row 0 (lane 0): x0 = -sum_{j>=1} band_j x_j / band_0, the quotient from
+        // the reciprocal with one correction
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const double t = -part[r] * rb;
+            const double x0 = fma(fma(-t, b0, -part[r]), rb, t);
+            x[r][0] = lane == 0 ? x0 : x[r][0];
+        }
+        double ap[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) ap[k] = lam * bl[k] * invd[k];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            double y = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                y = x[r][k] + ap[k] * y;
+                x[r][k] = y;
+            }
+            xc[r] = y;
+        }
+        s = 0;
+#pragma unroll
+        for (int d = 1; d < W; d <<= 1, ++s)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) xc[r] = fma(xp[s], wup<W>(xc[r], d), xc[r]);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            double ec = wup<W>(xc[r], 1);
+            if (!wrow<W>() && lane == 0) ec = 0.0;
+            double a = 1.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                a *= ap[k];
+                x[r][k] += a * ec;
+            }
+        }
+    }
+};
+
+// Both parity systems of one Helmholtz operator
+template <int K, int W>
+struct HelmOp {
+    HelmPar<K, W> e, o;
+    __device__ __forceinline__ HelmOp(const HelmRaw<K>& f, double lambda, const WCtx& c) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            e.band[k] = f.band.e[k];
+            e.up[k] = f.up.e[k];
+            e.invd[k] = f.invd.e[k];
+            o.band[k] = f.band.o[k];
+            o.up[k] = f.up.o[k];
+            o.invd[k] = f.invd.o[k];
+        }
+        const double* hb = c.hb + 2 * K * c.lane;
+        e.init(lambda, hb, 2, c.Me, c);
+        o.init(lambda, hb + 1, 2, c.Mo, c);
+    }
+    template <int NR>
+    __device__ __forceinline__ void solve(const WV<K> (&f)[NR], const WCtx& c, WV<K> (&x)[NR]) const {
+        double fe[NR][K], fo[NR][K], xe[NR][K], xo[NR][K];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                fe[r][k] = f[r].e[k];
+                fo[r][k] = f[r].o[k];
+            }
+        const double* hb = c.hb + 2 * K * c.lane;
+        e.template solve<NR>(fe, hb, 2 * K * W, c, xe);
+        o.template solve<NR>(fo, hb + 1, 2 * K * W, c, xo);
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                x[r].e[k] = xe[r][k];
+                x[r].o[k] = xo[r][k];
+            }
+    }
+};
 
 // complex profile <-> LDS row of double2 (re, im) per coefficient n
 template <int K, int W>

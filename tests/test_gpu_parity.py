@@ -117,6 +117,34 @@ def test_solve_single_call(gpu, constraint, taucorr, grid):
         assert abs(dp_gpu - dp_ref) <= 1e-12 * max(1.0, abs(dp_ref))
 
 
+@pytest.mark.parametrize("constraint", ["PressureGradient", "BulkVelocity"])
+@pytest.mark.parametrize("grid", [(6, 5, 6), (8, 31, 12), (12, 63, 8), (8, 95, 8), (8, 127, 8), (8, 159, 8), (6, 161, 6),
+                                  (6, 191, 6), (6, 255, 6), (6, 383, 6), (96, 129, 72)])
+def test_solve_segment_edges(gpu, constraint, grid):
+    """One solve at the sizes where the tau solve changes: the last (and first)
+    Ny of each number of coefficients per lane, the smallest and largest Ny,
+    mode counts that leave a block partly empty, and (96x129x72 without
+    dealiasing, 3420 modes) 16 modes per block. Same bar as
+    test_solve_single_call, one call against the oracle."""
+    Nx, Ny, Nz = grid
+    g = R.Grid(Nx, Ny, Nz, LX_C, LZ_C)
+    rng = np.random.default_rng(15)
+    rhs = rng.standard_normal((3, Ny, Nx, Nz // 2 + 1)) + 1j * rng.standard_normal((3, Ny, Nx, Nz // 2 + 1))
+    rhs *= 0.8 ** np.arange(Ny)[None, :, None, None]
+    u0 = g.zeros(3)
+    fl = dict(constraint=constraint, nu=1 / 400, dPdx=-0.01, Ubulk=0.6, Wbulk=0.1, baseflow="LaminarBase",
+              dealiasing="NoDealiasing")
+    lam = (11.0 / 6.0) / 0.02
+    u_ref, q_ref, dp_ref = R.solve(g, R.make_flags(**fl), lam, u0, rhs)
+    u_gpu, q_gpu, dp_gpu = cfa.solve(cfa.FlowField(Nx, Ny, Nz, 3, LX_C, LZ_C), rhs, cfa.DNSFlags(**fl), lam)
+    eu = rel_l2_per_component(g, u_gpu, u_ref)
+    eq = rel_l2_per_component(g, q_gpu, q_ref)
+    print(constraint, grid, "u", eu, "q", eq, "dPdx", dp_gpu, dp_ref, flush=True)
+    assert np.all(eu <= 1e-12) and np.all(eq <= 1e-12)
+    if constraint == "BulkVelocity":
+        assert abs(dp_gpu - dp_ref) <= 1e-12 * max(1.0, abs(dp_ref))
+
+
 C1_FLAGS = dict(baseflow="LaminarBase", ulowerwall=-1.0, uupperwall=1.0, constraint="BulkVelocity", Ubulk=0.0,
                 timestepping="SBDF3", initstepping="SMRK2", nonlinearity="SkewSymmetric", dealiasing="DealiasXZ",
                 taucorrection=True, nu=1 / 400, dt=0.02)
