@@ -155,7 +155,7 @@ def live(grid):
     return Ny * (2 * (Nx // 3) - 1) * (Nz // 3)  # complex values per component
 
 
-WAVE_FFT_LENGTHS = (16, 32, 48, 64, 96, 128, 192, 256)  # x/z lengths of the wavefront-local FFT kernels
+WAVE_FFT_LENGTHS = (16, 18, 24, 32, 36, 48, 54, 64, 72, 96, 108, 128, 144, 162, 192, 256)  # x/z lengths of the wavefront-local FFT kernels
 
 
 def kernel_bytes(grid, method):

@@ -90,6 +90,25 @@ def test_nonlinear_chebyshev_sizes(gpu, method, Ny):
     assert np.all(err <= 1e-12), err
 
 
+@pytest.mark.parametrize("method", ["Rotational", "Convection", "Divergence", "SkewSymmetric"])
+@pytest.mark.parametrize("N", [18, 24, 36, 54, 72, 108, 144, 162])
+def test_nonlinear_ragged_lengths(gpu, method, N):
+    """One NL call with x- and z-lines of the FFT lengths 2^a 3^b between the
+    powers of two, with and without dealiasing (line counts that do and do not
+    fill a wavefront); the same 1e-12 bar as test_nonlinear_single_call."""
+    for grid, dealias in (((N, 9, 18), "DealiasXZ"), ((16, 9, N), "NoDealiasing"), ((24, 9, N), "DealiasXZ")):
+        Nx, Ny, Nz = grid
+        g = R.Grid(Nx, Ny, Nz, LX_C, LZ_C)
+        u = random_field(Nx, Ny, Nz, LX_C, LZ_C, norm=1.0, decay=0.7, seed=N, dealias=(dealias == "DealiasXZ"))
+        fl = dict(nonlinearity=method, dealiasing=dealias, baseflow="LaminarBase", ulowerwall=-1.0, uupperwall=1.0,
+                  nu=1 / 400, rotation=0.3 if method in ("Rotational", "SkewSymmetric") else 0.0)
+        f_ref, _ = R.nonlinear(g, R.make_flags(**fl), u)
+        f_gpu = cfa.nonlinear(cfa.FlowField(Nx, Ny, Nz, 3, LX_C, LZ_C, data=u), cfa.DNSFlags(**fl))
+        e = rel_l2_per_component(g, f_gpu, f_ref)
+        print(method, grid, dealias, "rel L2", e, flush=True)
+        assert np.all(e <= 1e-12), e
+
+
 @pytest.mark.parametrize("constraint", ["PressureGradient", "BulkVelocity"])
 @pytest.mark.parametrize("taucorr", [True, False])
 @pytest.mark.parametrize("grid", [(16, 33, 16), (8, 25, 8), (8, 65, 8), (8, 97, 8), (8, 129, 8), (6, 193, 6),
