@@ -286,13 +286,46 @@ constexpr int pow2_at_least(int n) {
     return p;
 }
 
+// A line of N values on G lanes of a wavefront, 64/G lines per wavefront:
+//   spectral layout  lane s < SL holds Z[s + SL r], r < SV;
+//   physical layout  lane p < PL holds x[p + PL m], m < PV.
 template <int NZ>
 struct ZW {
     static constexpr int N1 = ZWShape<NZ>::N1, N2 = ZWShape<NZ>::N2, N = N1 * N2;
+    static constexpr int SL = N1, SV = N2, PL = N2, PV = N1;
     static constexpr int NMAX = N1 > N2 ? N1 : N2;
     static constexpr int G = pow2_at_least(NMAX);  // lanes per line
     static constexpr int LPW = 64 / G;             // lines per wavefront
     static constexpr int LBUF = N + NMAX;          // LDS slots per line (transposes, padded rows)
+};
+
+// The same in three steps, N = A B C with the physical values A per lane: two
+// transposes, but fewer values per lane and transform. QG: groups of B values a
+// lane holds in the middle step.
+template <int NZ>
+struct ZW3Shape {
+    static constexpr int A = 0, B = 0, C = 0, QG = 1;
+};
+template <> struct ZW3Shape<72> { static constexpr int A = 3, B = 4, C = 6, QG = 1; };
+template <> struct ZW3Shape<96> { static constexpr int A = 3, B = 4, C = 8, QG = 1; };
+template <> struct ZW3Shape<108> { static constexpr int A = 6, B = 3, C = 6, QG = 2; };
+template <> struct ZW3Shape<128> { static constexpr int A = 4, B = 4, C = 8, QG = 1; };
+template <> struct ZW3Shape<144> { static constexpr int A = 6, B = 4, C = 6, QG = 2; };
+template <> struct ZW3Shape<162> { static constexpr int A = 6, B = 3, C = 9, QG = 3; };
+template <> struct ZW3Shape<192> { static constexpr int A = 6, B = 4, C = 8, QG = 2; };
+template <> struct ZW3Shape<256> { static constexpr int A = 8, B = 4, C = 8, QG = 2; };
+
+template <int NZ>
+struct ZW3 {
+    static constexpr int A = ZW3Shape<NZ>::A, B = ZW3Shape<NZ>::B, C = ZW3Shape<NZ>::C, QG = ZW3Shape<NZ>::QG;
+    static constexpr int N = A * B * C;
+    static constexpr int SL = A * B, SV = C, PL = B * C, PV = A, QL = A * C / QG;
+    static constexpr int G = pow2_at_least(PL > SL ? PL : SL);
+    static constexpr int LPW = 64 / G;
+    static constexpr int AP = A | 1, BP = B | 1, CP = C | 1;  // row pitches, odd
+    static constexpr int max3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
+    static constexpr int LBUF = max3(A * C * BP, A * B * CP, B * C * AP);
+    static_assert(QL <= G && A * C % QG == 0, "the middle step's lanes");
 };
 
 // the lengths with a wavefront FFT
@@ -502,6 +535,116 @@ __device__ __forceinline__ void zw_b2a(double2 (&u)[ZW<N>::N1], double2 (&v)[ZW<
 #pragma unroll
     for (int i = 0; i < N2; ++i) v[i] = T[row * (N2 + 1) + i];
     dft_reg<N2, SIGN>(v);
+}
+
+// The three-step transforms, between the same layouts. With n = s + SL c,
+// s = j + A b (j < A, b < B, c < C) and k = k1 + PL k2, k1 = m1 + C m2:
+// X[k] = sum_j w_A^(j k2) w_N^(j k1) sum_b w_B^(b m2) w_PL^(b m1) sum_c Z w_C^(c m1).
+template <int NZ, int SIGN>
+__device__ __forceinline__ void zw3_s2p(double2 (&v)[ZW3<NZ>::SV], double2 (&u)[ZW3<NZ>::PV], int l, double2* T,
+                                        const double2* tw) {
+    using S = ZW3<NZ>;
+    constexpr int A = S::A, B = S::B, C = S::C;
+    auto turn = [&](double2 x, int i) {
+        double2 t = tw[i];
+        if (SIGN > 0) t.y = -t.y;
+        return cmul(x, t);
+    };
+    dft_reg<C, SIGN>(v);
+    const int s = l < S::SL ? l : S::SL - 1, b = s / A, j = s - b * A;
+    wave_lds_sync();
+    if (l < S::SL) {
+        T[j * S::BP + b] = v[0];
+#pragma unroll
+        for (int m1 = 1; m1 < C; ++m1) T[(m1 * A + j) * S::BP + b] = turn(v[m1], A * b * m1);
+    }
+    wave_lds_sync();
+    double2 w[S::QG][B];
+    const int q0 = l < S::QL ? l : S::QL - 1;
+#pragma unroll
+    for (int g = 0; g < S::QG; ++g) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) w[g][i] = T[(q0 + S::QL * g) * S::BP + i];
+        dft_reg<B, SIGN>(w[g]);
+    }
+    wave_lds_sync();
+    if (l < S::QL) {
+#pragma unroll
+        for (int g = 0; g < S::QG; ++g) {
+            const int q = q0 + S::QL * g, m1 = q / A, jq = q - m1 * A;
+#pragma unroll
+            for (int m2 = 0; m2 < B; ++m2) {
+                const int k1 = m1 + C * m2;
+                T[k1 * S::AP + jq] = turn(w[g][m2], jq * k1);
+            }
+        }
+    }
+    wave_lds_sync();
+    const int p = l < S::PL ? l : S::PL - 1;
+#pragma unroll
+    for (int i = 0; i < A; ++i) u[i] = T[p * S::AP + i];
+    dft_reg<A, SIGN>(u);
+}
+
+template <int NZ, int SIGN>
+__device__ __forceinline__ void zw3_p2s(double2 (&u)[ZW3<NZ>::PV], double2 (&v)[ZW3<NZ>::SV], int l, double2* T,
+                                        const double2* tw) {
+    using S = ZW3<NZ>;
+    constexpr int A = S::A, B = S::B, C = S::C;
+    auto turn = [&](double2 x, int i) {
+        double2 t = tw[i];
+        if (SIGN > 0) t.y = -t.y;
+        return cmul(x, t);
+    };
+    dft_reg<A, SIGN>(u);
+    const int p = l < S::PL ? l : S::PL - 1;
+    wave_lds_sync();
+    if (l < S::PL) {
+        const int i1 = p % C, i2 = p / C;
+        T[i1 * A * S::BP + i2] = u[0];
+#pragma unroll
+        for (int q = 1; q < A; ++q) T[(i1 * A + q) * S::BP + i2] = turn(u[q], p * q);
+    }
+    wave_lds_sync();
+    double2 w[S::QG][B];
+    const int q0 = l < S::QL ? l : S::QL - 1;
+#pragma unroll
+    for (int g = 0; g < S::QG; ++g) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) w[g][i] = T[(q0 + S::QL * g) * S::BP + i];
+        dft_reg<B, SIGN>(w[g]);
+    }
+    wave_lds_sync();
+    if (l < S::QL) {
+#pragma unroll
+        for (int g = 0; g < S::QG; ++g) {
+            const int vq = q0 + S::QL * g, i1 = vq / A, q = vq - i1 * A;
+            T[q * S::CP + i1] = w[g][0];
+#pragma unroll
+            for (int p1 = 1; p1 < B; ++p1) T[(p1 * A + q) * S::CP + i1] = turn(w[g][p1], A * i1 * p1);
+        }
+    }
+    wave_lds_sync();
+    const int s = l < S::SL ? l : S::SL - 1;
+#pragma unroll
+    for (int i = 0; i < C; ++i) v[i] = T[s * S::CP + i];
+    dft_reg<C, SIGN>(v);
+}
+
+// spectral -> physical and back by either kind of line
+template <class S>
+constexpr bool three_step = false;
+template <int N>
+constexpr bool three_step<ZW3<N>> = true;
+template <class S, int SIGN>
+__device__ __forceinline__ void line_s2p(double2 (&v)[S::SV], double2 (&u)[S::PV], int l, double2* T, const double2* tw) {
+    if constexpr (three_step<S>) zw3_s2p<S::N, SIGN>(v, u, l, T, tw);
+    else zw_a2b<S::N, SIGN>(v, u, l, T, tw);
+}
+template <class S, int SIGN>
+__device__ __forceinline__ void line_p2s(double2 (&u)[S::PV], double2 (&v)[S::SV], int l, double2* T, const double2* tw) {
+    if constexpr (three_step<S>) zw3_p2s<S::N, SIGN>(u, v, l, T, tw);
+    else zw_b2a<S::N, SIGN>(u, v, l, T, tw);
 }
 
 #define CFG_FFT_SIZES(X) \

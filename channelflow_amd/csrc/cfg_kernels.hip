@@ -1132,9 +1132,9 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
     NLTune out;
     std::vector<NLTune> zc;
     if (zwave_size(g.Nz)) {  // wavefront z pass: the staged form, or wavefronts per block
-        // the grid's and form's choice (zwave_staged), or the one CFGPU_ZWAVE_STAGED=1 / 0 names
+        // the grid's choice (zwave_staged), or the one CFGPU_ZWAVE_STAGED=1 / 0 names
         const char* force = std::getenv("CFGPU_ZWAVE_STAGED");
-        const bool staged = force ? force[0] != '0' : zwave_stages(method, g.Nz), unstaged = !staged;
+        const bool staged = force ? force[0] != '0' : zwave_stages(g.Nz), unstaged = !staged;
         NLTune c;
         if (staged) {
             c.zwb = ZWAVE_WB;

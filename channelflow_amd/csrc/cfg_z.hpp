@@ -11,8 +11,8 @@ size_t lds_budget();
 int zpass_nphys(int method);
 // largest LDS z-pass lines per block that fit the LDS budget
 int zpass_xb_max(const Geom& g, int nphys);
-// whether the z pass of a form at length nz stages its inputs in LDS
-bool zwave_stages(int method, int nz);
+// whether the z pass at length nz stages its inputs in LDS
+bool zwave_stages(int nz);
 // wavefronts per block of the staged wavefront z pass
 constexpr int ZWAVE_WB = 1;
 

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "cfg_fft.hpp"
 #include "cfg_wave.hpp"
@@ -282,7 +283,6 @@ struct ZWCtx {
 // to its base + 16 i; lanes past the run copy nothing). The data are in LDS
 // once the wavefront's vector-memory count has drained; the compiler waits for
 // it before the first LDS read of the staging array.
-template <int NZ>
 __device__ __forceinline__ void zw_stage(const ZWCtx& c, const double2* __restrict__ xp, int f, int slot) {
     const __attribute__((address_space(1))) double2* src = gmem(xp) + (long)f * c.fsz + c.wbase;
     double2* dst = c.S + slot * c.sstride;
@@ -299,19 +299,19 @@ __device__ __forceinline__ void zw_stage(const ZWCtx& c, const double2* __restri
 // slots 0 (fa) and 1 (fb), and once these are read the copies of fields na and
 // nb (< 0: none) into them start, to land while this transform and what
 // follows it run.
-template <int NZ, bool STAGED>
+template <class S, bool STAGED>
 __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
-                                       bool dzb, double (&pa)[ZW<NZ>::N1], double (&pb)[ZW<NZ>::N1], int na = -1,
+                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV], int na = -1,
                                        int nb = -1) {
-    constexpr int N1 = ZW<NZ>::N1, N2 = ZW<NZ>::N2, N = ZW<NZ>::N;
+    constexpr int SL = S::SL, SV = S::SV, PV = S::PV, N = S::N;
     const int j = c.gi;
-    const bool act = c.line_ok && j < N1;
+    const bool act = c.line_ok && j < SL;
     const double2* Sa = c.S + c.sline;
     const double2* Sb = Sa + c.sstride;
-    double2 v[N2];
+    double2 v[SV];
 #pragma unroll
-    for (int r = 0; r < N2; ++r) {
-        const int n = j + N1 * r;
+    for (int r = 0; r < SV; ++r) {
+        const int n = j + SL * r;
         const bool lo = n < c.nkz, hi = n > N - c.nkz;
         const int k = lo ? n : N - n;
         double2 A = make_double2(0.0, 0.0), B = make_double2(0.0, 0.0);
@@ -333,13 +333,13 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
     if (STAGED && na >= 0) {
         // every lane's reads of the slots have returned before the copies may overwrite them
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        zw_stage<NZ>(c, xp, na, 0);
-        if (nb >= 0) zw_stage<NZ>(c, xp, nb, 1);
+        zw_stage(c, xp, na, 0);
+        if (nb >= 0) zw_stage(c, xp, nb, 1);
     }
-    double2 u[N1];
-    zw_a2b<NZ, +1>(v, u, j, c.T, c.tw);
+    double2 u[PV];
+    line_s2p<S, +1>(v, u, j, c.T, c.tw);
 #pragma unroll
-    for (int m = 0; m < N1; ++m) {
+    for (int m = 0; m < PV; ++m) {
         pa[m] = u[m].x;
         pb[m] = u[m].y;
     }
@@ -348,26 +348,26 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
 // r2c of pa (and pb when TWO) -> zo fields ga (and gb), bins kz < nkz.
 // fold != 0 (with TWO): field ga receives A + fold i kz B instead of A, with
 // kz = 2 pi k / Lz, A and B the spectra of pa and pb; gb < 0 then drops B.
-template <int NZ, bool TWO>
-__device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo, const double (&pa)[ZW<NZ>::N1],
-                                       const double (&pb)[ZW<NZ>::N1], int ga, int gb, double fold = 0.0) {
-    constexpr int N1 = ZW<NZ>::N1, N2 = ZW<NZ>::N2, N = ZW<NZ>::N;
+template <class S, bool TWO>
+__device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo, const double (&pa)[S::PV],
+                                       const double (&pb)[S::PV], int ga, int gb, double fold = 0.0) {
+    constexpr int SL = S::SL, SV = S::SV, PV = S::PV, N = S::N;
     const int j = c.gi;
-    double2 v[N1];
+    double2 v[PV];
 #pragma unroll
-    for (int m = 0; m < N1; ++m) v[m] = make_double2(pa[m], TWO ? pb[m] : 0.0);
-    double2 w[N2];
-    zw_b2a<NZ, -1>(v, w, j, c.T, c.tw);  // w[p] = X[j + N1 p]
+    for (int m = 0; m < PV; ++m) v[m] = make_double2(pa[m], TWO ? pb[m] : 0.0);
+    double2 w[SV];
+    line_p2s<S, -1>(v, w, j, c.T, c.tw);  // w[p] = X[j + SL p]
     wave_lds_sync();
-    if (j < N1) {
+    if (j < SL) {
 #pragma unroll
-        for (int p = 0; p < N2; ++p) c.T[j + N1 * p] = w[p];
+        for (int p = 0; p < SV; ++p) c.T[j + SL * p] = w[p];
     }
     wave_lds_sync();
-    if (c.line_ok && j < N1) {
+    if (c.line_ok && j < SL) {
 #pragma unroll
-        for (int p = 0; p < N2; ++p) {
-            const int k = j + N1 * p;
+        for (int p = 0; p < SV; ++p) {
+            const int k = j + SL * p;
             if (k < c.nkz) {
                 const double2 Zk = w[p];
                 const double2 Zn = c.T[(N - k) % N];
@@ -385,40 +385,47 @@ __device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo,
     }
 }
 
-// The z pass stages its inputs at Nz = 64, and at Nz = 128 for the rotational
-// form. The choice depends on the grid and form alone (never on the member
-// count), so a member's result is the same alone and in a batch: the two forms
-// contract multiply-adds differently (the compiler fuses either product of
-// a*b + c*d depending on the code around it) and differ in the last bits. At
-// Nz = 64 the staged form wins where it matters, in batches (16 members of
-// 64x65x64, skew-symmetric: 104 against 122 us per launch) and loses 2.6 us on
-// a lone field; at 32 and 48 (24 members) and for lone 96^3 and 192^3 fields
-// the unstaged one is faster. The rotational form at Nz = 128 runs the staged
-// kernel at 2 waves per SIMD (zwave_min_waves; 256 VGPRs and a 60-byte spill,
-// where the unstaged one needs 277 + 21 and runs 1): a lone 128^3 field 56.4
-// -> 47.5 us. The same cap on the skew-symmetric form spills 232-692 bytes at
-// 96-128 and on the rotational one 200 bytes at 192, and those were slower.
-constexpr bool zwave_staged(int method, int nz) { return nz == 64 || (nz == 128 && method == NL_ROT); }
-// lengths the staged form is compiled for
-constexpr bool zwave_has_staged(int nz) { return nz == 16 || nz == 32 || nz == 48 || nz == 64 || nz == 128; }
-constexpr int zwave_min_waves(int method, int nz, bool staged) {
-    return (staged && nz == 128 && method == NL_ROT) ? 2 : 1;
-}
+// The z pass stages its inputs at Nz = 64. The choice depends on the grid alone
+// (never on the member count), so a member's result is the same alone and in a
+// batch: the two forms contract multiply-adds differently (the compiler fuses
+// either product of a*b + c*d depending on the code around it) and differ in the
+// last bits. At Nz = 64 the staged form wins where it matters, in batches (16
+// members of 64x65x64, skew-symmetric: 104 against 122 us per launch) and loses
+// 2.6 us on a lone field; at 32 and 48 (24 members) and at the three-step
+// lengths (one 128^3 field: rotational 39.2 us staged, 35.0 not, convection 73.2
+// and 70.1) the unstaged one is faster.
+constexpr bool zwave_staged(int nz) { return nz == 64; }
 
+// Three steps per transform (ZW3) at Nz = 72 and from 96 on. What bounds the z
+// pass there is how few wavefronts a SIMD holds: with 6 physical values per lane
+// instead of 8 to 16 and transforms of at most 9 values, 2 or 3 of them fit the
+// registers where 1 did (skew-symmetric 96: 341 -> 162 registers, rotational
+// 192: 297 -> 131), at the price of a second transpose through LDS. us per
+// launch, two steps -> three: one 96^3 skew-symmetric field 59 -> 44, 128^3
+// convection 92 -> 70, rotational 49 -> 35, 192x129x192 rotational 95 -> 76,
+// 256x33x256 52 -> 48, 64x49x162 skew-symmetric 61 -> 32, 8 members of 32x49x72
+// 72 -> 53. At 48 and 64, where 2 wavefronts fit anyway, the second transpose
+// costs more than it gives in a batch (16 of 64^3 113 -> 127, 24 of 48^3 82 -> 88).
+constexpr bool zwave_three(int nz) { return nz == 72 || nz >= 96; }
+template <int NZ>
+using ZLine = std::conditional_t<zwave_three(NZ), ZW3<NZ>, ZW<NZ>>;
+
+// lengths the staged form is compiled for
+constexpr bool zwave_has_staged(int nz) { return nz == 16 || nz == 32 || nz == 48 || nz == 64; }
 // The z pass of k_zpass with one wavefront per 64/G lines (same fields, same
 // products in the same order). A block is independent wavefronts: any number
 // up to 4 (LDS sized at launch), or, STAGED, ZWAVE_WB of them, each staging
 // the next transform's two input fields in LDS while it works on the current
 // one. Staging hides the loads' latency where many wavefronts share a CU;
 // with few wavefronts per SIMD the extra LDS round trip costs more than it
-// hides (zwave_staged picks the form per grid and nonlinear form).
+// hides (zwave_staged picks the form per grid).
 template <int METHOD, int NZ, bool STAGED>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(zwave_min_waves(METHOD, NZ, STAGED), 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8)))
 k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ tab,
                                                int want_g, const double2* __restrict__ xp0, double2* __restrict__ zo0,
                                                long sx) {
-    using S = ZW<NZ>;
-    constexpr int N1 = S::N1, SLOT = S::LPW * (NZ / 2);
+    using S = ZLine<NZ>;
+    constexpr int N1 = S::PV, SLOT = S::LPW * (NZ / 2);
     double2 *tw_l, *T_l, *in_l = nullptr;
     if constexpr (STAGED) {
         // Separate LDS arrays (not one dynamic block) let the compiler tell the
@@ -463,14 +470,14 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
     const double2* __restrict__ xp = xp0 + blockIdx.y * sx;
     double2* __restrict__ zo = zo0 + blockIdx.y * sx;
     if constexpr (STAGED) {
-        zw_stage<NZ>(c, xp, 0, 0);  // u, v: the first transform's pair
-        zw_stage<NZ>(c, xp, 1, 1);
+        zw_stage(c, xp, 0, 0);  // u, v: the first transform's pair
+        zw_stage(c, xp, 1, 1);
     }
     if constexpr (METHOD == NL_ROT) {
         double u0[N1], u1[N1], u2[N1], w0[N1], w1[N1], w2[N1];
-        zw_c2r<NZ, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2, 3);
-        zw_c2r<NZ, STAGED>(c, xp, 2, false, 3, false, u2, w0, 4, 5);
-        zw_c2r<NZ, STAGED>(c, xp, 4, false, 5, false, w1, w2);
+        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2, 3);
+        zw_c2r<S, STAGED>(c, xp, 2, false, 3, false, u2, w0, 4, 5);
+        zw_c2r<S, STAGED>(c, xp, 4, false, 5, false, w1, w2);
         double f0[N1], f1[N1], f2[N1];
 #pragma unroll
         for (int m = 0; m < N1; ++m) {  // cross(vort, u) (diffops.cpp:2598-2605)
@@ -483,8 +490,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
                 f1[m] += rotation * a0;
             }
         }
-        zw_r2c<NZ, true>(c, zo, f0, f1, 0, 1);
-        zw_r2c<NZ, false>(c, zo, f2, f2, 2, -1);
+        zw_r2c<S, true>(c, zo, f0, f1, 0, 1);
+        zw_r2c<S, false>(c, zo, f2, f2, 2, -1);
     } else if constexpr (METHOD == NL_CONV || METHOD == NL_SKEW) {
         // f_i = sum_j (s u_j) du_i/dx_j, terms added in the order j = x, y, z
         // (diffops.cpp:3192-3199, 3626-3633). The skew-symmetric form keeps
@@ -500,8 +507,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         constexpr bool SK = (METHOD == NL_SKEW);
         constexpr double s = SK ? 0.5 : 1.0, us = SK ? 2.0 : 1.0;
         double h0[N1], h1[N1], h2[N1], pa[N1], pb[N1], fa[N1], fb[N1];
-        zw_c2r<NZ, STAGED>(c, xp, 0, false, 1, false, h0, h1, 2, 6);   // u, v
-        zw_c2r<NZ, STAGED>(c, xp, 2, false, 6, false, h2, pa, 3, 0);   // w, du/dx
+        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, h0, h1, 2, 6);   // u, v
+        zw_c2r<S, STAGED>(c, xp, 2, false, 6, false, h2, pa, 3, 0);   // w, du/dx
         if constexpr (SK) {
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
@@ -512,7 +519,7 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         }
 #pragma unroll
         for (int m = 0; m < N1; ++m) fa[m] = 0.0 + h0[m] * pa[m];
-        zw_c2r<NZ, STAGED>(c, xp, 3, false, 0, true, pa, pb, 7, 4);    // du/dy, du/dz
+        zw_c2r<S, STAGED>(c, xp, 3, false, 0, true, pa, pb, 7, 4);    // du/dy, du/dz
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] += h1[m] * pa[m];
@@ -520,22 +527,22 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
             if (rotation != 0.0) fa[m] -= rotation * (us * h1[m]);  // nse.cpp:61-80
             if (SK) pb[m] = 4.0 * (h0[m] * h2[m]);
         }
-        if constexpr (SK) zw_r2c<NZ, true>(c, zo, fa, pb, 0, 5, 0.5);  // f0 + i kz u0u2 / 2, and u0u2
-        else zw_r2c<NZ, false>(c, zo, fa, pb, 0, -1);                  // f0
-        zw_c2r<NZ, STAGED>(c, xp, 7, false, 4, false, pa, pb, 1, 8);   // dv/dx, dv/dy
+        if constexpr (SK) zw_r2c<S, true>(c, zo, fa, pb, 0, 5, 0.5);  // f0 + i kz u0u2 / 2, and u0u2
+        else zw_r2c<S, false>(c, zo, fa, pb, 0, -1);                  // f0
+        zw_c2r<S, STAGED>(c, xp, 7, false, 4, false, pa, pb, 1, 8);   // dv/dx, dv/dy
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] = 0.0 + h0[m] * pa[m];
             fa[m] += h1[m] * pb[m];
         }
-        zw_c2r<NZ, STAGED>(c, xp, 1, true, 8, false, pa, pb, 5, 2);    // dv/dz, dw/dx
+        zw_c2r<S, STAGED>(c, xp, 1, true, 8, false, pa, pb, 5, 2);    // dv/dz, dw/dx
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] += h2[m] * pa[m];
             if (rotation != 0.0) fa[m] += rotation * (us * h0[m]);
             fb[m] = 0.0 + h0[m] * pb[m];
         }
-        zw_c2r<NZ, STAGED>(c, xp, 5, false, 2, true, pa, pb);    // dw/dy, dw/dz
+        zw_c2r<S, STAGED>(c, xp, 5, false, 2, true, pa, pb);    // dw/dy, dw/dz
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fb[m] += h1[m] * pa[m];
@@ -544,37 +551,37 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         if constexpr (SK) {
 #pragma unroll
             for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h1[m] * h2[m]);
-            zw_r2c<NZ, true>(c, zo, fa, pa, 1, 7, 0.5);   // f1 + i kz u1u2 / 2, and u1u2
+            zw_r2c<S, true>(c, zo, fa, pa, 1, 7, 0.5);   // f1 + i kz u1u2 / 2, and u1u2
 #pragma unroll
             for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h2[m] * h2[m]);
-            zw_r2c<NZ, true>(c, zo, fb, pa, 2, -1, 0.5);  // f2 + i kz u2u2 / 2
+            zw_r2c<S, true>(c, zo, fb, pa, 2, -1, 0.5);  // f2 + i kz u2u2 / 2
             // remaining entries of outer(u, u) (diffops.cpp:2336-2388)
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
                 pa[m] = 4.0 * (h0[m] * h0[m]);
                 pb[m] = 4.0 * (h0[m] * h1[m]);
             }
-            zw_r2c<NZ, true>(c, zo, pa, pb, 3, 4);
+            zw_r2c<S, true>(c, zo, pa, pb, 3, 4);
 #pragma unroll
             for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h1[m] * h1[m]);
-            zw_r2c<NZ, false>(c, zo, pa, pa, 6, -1);
+            zw_r2c<S, false>(c, zo, pa, pa, 6, -1);
         } else {
-            zw_r2c<NZ, true>(c, zo, fa, fb, 1, 2);            // f1, f2
+            zw_r2c<S, true>(c, zo, fa, fb, 1, 2);            // f1, f2
         }
     } else {
         double u0[N1], u1[N1], u2[N1], pa[N1], pb[N1];
-        zw_c2r<NZ, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2);
-        zw_c2r<NZ, STAGED>(c, xp, 2, false, -1, false, u2, pa);
+        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2);
+        zw_c2r<S, STAGED>(c, xp, 2, false, -1, false, u2, pa);
         if (want_g) {  // DIV with rotation: g = rotation terms only
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
                 pa[m] = -(rotation * u1[m]);
                 pb[m] = rotation * u0[m];
             }
-            zw_r2c<NZ, true>(c, zo, pa, pb, 0, 1);
+            zw_r2c<S, true>(c, zo, pa, pb, 0, 1);
 #pragma unroll
             for (int m = 0; m < N1; ++m) pa[m] = 0.0;
-            zw_r2c<NZ, false>(c, zo, pa, pa, 2, -1);
+            zw_r2c<S, false>(c, zo, pa, pa, 2, -1);
         }
         // outer(u, u) (diffops.cpp:2336-2388), two entries per r2c
 #pragma unroll
@@ -582,19 +589,19 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
             pa[m] = u0[m] * u0[m];
             pb[m] = u0[m] * u1[m];
         }
-        zw_r2c<NZ, true>(c, zo, pa, pb, 3, 4);
+        zw_r2c<S, true>(c, zo, pa, pb, 3, 4);
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             pa[m] = u0[m] * u2[m];
             pb[m] = u1[m] * u1[m];
         }
-        zw_r2c<NZ, true>(c, zo, pa, pb, 5, 6);
+        zw_r2c<S, true>(c, zo, pa, pb, 5, 6);
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             pa[m] = u1[m] * u2[m];
             pb[m] = u2[m] * u2[m];
         }
-        zw_r2c<NZ, true>(c, zo, pa, pb, 7, 8);
+        zw_r2c<S, true>(c, zo, pa, pb, 7, 8);
     }
 }
 
@@ -604,10 +611,10 @@ template <int METHOD, int NZ>
 void launch_z_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, int want_g, const double2* xp,
                        double2* zo, long sx, const NLTune& tn, hipStream_t st) {
     if constexpr (zwave_size(NZ)) {
-        using S = ZW<NZ>;
+        using S = ZLine<NZ>;
         const long waves = (long)g.Ny * ((g.Nx + S::LPW - 1) / S::LPW);
         if constexpr (zwave_has_staged(NZ)) {
-            if (tn.zstage < 0 ? zwave_staged(METHOD, NZ) : tn.zstage != 0) {
+            if (tn.zstage < 0 ? zwave_staged(NZ) : tn.zstage != 0) {
                 if (g.nkz > NZ / 2) throw std::runtime_error("z pass: more live kz bins than Nz/2");
                 const dim3 grid((unsigned)((waves + ZWAVE_WB - 1) / ZWAVE_WB), n);
                 k_zwave<METHOD, NZ, true><<<grid, 64 * ZWAVE_WB, 0, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
