@@ -1122,8 +1122,8 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
         if (std::getenv("CFGPU_TUNE_LOG")) {
             std::fprintf(stderr, "cfg tune %s %dx%dx%d form %d members %d:", what, g.Nx, g.Ny, g.Nz, method, n);
             for (size_t i = 0; i < cands.size(); ++i)
-                std::fprintf(stderr, " [zwb %d zstage %d zxb %d xwb %d xwbf %d xl %d] %.1f us%s", cands[i].zwb,
-                             cands[i].zstage, cands[i].zxb, cands[i].xwb, cands[i].xwbf, cands[i].xl, best[i] * 1e3f,
+                std::fprintf(stderr, " [zwb %d zxb %d xwb %d xwbf %d xl %d] %.1f us%s", cands[i].zwb,
+                             cands[i].zxb, cands[i].xwb, cands[i].xwbf, cands[i].xl, best[i] * 1e3f,
                              i == k ? " *" : "");
             std::fprintf(stderr, "\n");
         }
@@ -1131,19 +1131,10 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
     };
     NLTune out;
     std::vector<NLTune> zc;
-    if (zwave_size(g.Nz)) {  // wavefront z pass: the staged form, or wavefronts per block
-        // the grid's choice (zwave_staged), or the one CFGPU_ZWAVE_STAGED=1 / 0 names
-        const char* force = std::getenv("CFGPU_ZWAVE_STAGED");
-        const bool staged = force ? force[0] != '0' : zwave_stages(g.Nz), unstaged = !staged;
-        NLTune c;
-        if (staged) {
-            c.zwb = ZWAVE_WB;
-            c.zstage = 1;
-            zc.push_back(c);
-        }
-        for (int wb = 1; unstaged && wb <= 4; wb *= 2) {
+    if (zwave_size(g.Nz)) {  // wavefront z pass: wavefronts per block
+        for (int wb = 1; wb <= 4; wb *= 2) {
+            NLTune c;
             c.zwb = wb;
-            c.zstage = 0;
             zc.push_back(c);
         }
     } else {  // LDS z pass: lines per block
@@ -1157,7 +1148,6 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
         const NLTune z = pick(zc, [&](const NLTune& c) { launch_z_any(method, g, pz, n, tab, want_g, xp, zo, sx, c, st); },
                               "z");
         out.zwb = z.zwb;
-        out.zstage = z.zstage;
         out.zxb = z.zxb;
     }
     std::vector<NLTune> xc;  // x-FFTs, timed on the inverse

@@ -33,6 +33,19 @@ template <class T>
 __device__ __forceinline__ __attribute__((address_space(1))) T* gmem_w(T* p) {
     return (__attribute__((address_space(1))) T*)p;
 }
+// A 16-byte access at a uniform base and a 32-bit byte offset per lane: the base
+// stays in scalar registers, constant distances in the instruction.
+using gbytes = const __attribute__((address_space(1))) char*;
+using gbytes_w = __attribute__((address_space(1))) char*;
+__device__ __forceinline__ double2 gload(gbytes base, unsigned off) {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 v = *reinterpret_cast<const __attribute__((address_space(1))) d2*>(base + off);
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void gstore(gbytes_w base, unsigned off, double2 v) {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    *reinterpret_cast<__attribute__((address_space(1))) d2*>(base + off) = d2{v.x, v.y};
+}
 using gcdouble = const __attribute__((address_space(1))) double*;
 // a complex value as a native two-double vector (one 16-byte load or store)
 typedef double dvec2 __attribute__((ext_vector_type(2)));

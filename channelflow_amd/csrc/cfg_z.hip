@@ -93,8 +93,6 @@ int zpass_xb(const Geom& g, int nphys, const NLTune& tn) {
     return tn.zxb > 0 ? std::min(tn.zxb, m) : m;
 }
 
-bool zwave_stages(int nz) { return zwave_staged(nz); }
-
 #define CFG_Z_EXTERN(F)                                                                                            \
     extern template void launch_z<F>(const Geom&, const FFTPlan&, int, const NLMember*, int, const double2*, double2*, \
                                      long, const NLTune&, hipStream_t);

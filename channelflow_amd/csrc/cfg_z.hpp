@@ -11,11 +11,6 @@ size_t lds_budget();
 int zpass_nphys(int method);
 // largest LDS z-pass lines per block that fit the LDS budget
 int zpass_xb_max(const Geom& g, int nphys);
-// whether the z pass at length nz stages its inputs in LDS
-bool zwave_stages(int nz);
-// wavefronts per block of the staged wavefront z pass
-constexpr int ZWAVE_WB = 1;
-
 // z pass of n members (strides sx in double2): fields of xp to fields of zo
 void launch_z_any(int method, const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, int want_g,
                   const double2* xp, double2* zo, long sx, const NLTune& tn, hipStream_t st);

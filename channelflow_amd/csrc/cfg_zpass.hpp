@@ -269,75 +269,66 @@ struct ZWCtx {
     double dk;         // 2 pi / Lz
     double2* T;        // the line's LDS rows
     const double2* tw; // exp(-2 pi i m / N), m < N, in LDS
-    // input staging: the wavefront's lines are one contiguous run of the
-    // [field][y][x][kz] arrays (wcount values from wbase); two fields of it sit
-    // in LDS (slots 0 and 1 from S, slot stride sstride), this line's bins at
-    // L * nkz within a slot
-    long wbase;
-    int wcount, lane, sline, sstride;
-    double2* S;
 };
 
-// Starts the copy of field f of the wavefront's lines into staging slot
-// `slot` (global_load_lds_dwordx4: lane i of a copy instruction moves 16 bytes
-// to its base + 16 i; lanes past the run copy nothing). The data are in LDS
-// once the wavefront's vector-memory count has drained; the compiler waits for
-// it before the first LDS read of the staging array.
-__device__ __forceinline__ void zw_stage(const ZWCtx& c, const double2* __restrict__ xp, int f, int slot) {
-    const __attribute__((address_space(1))) double2* src = gmem(xp) + (long)f * c.fsz + c.wbase;
-    double2* dst = c.S + slot * c.sstride;
-    for (int t = 0; t < c.wcount; t += 64) {
-        if (t + c.lane < c.wcount)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + t + c.lane),
-                                             (__attribute__((address_space(3))) void*)(dst + t), 16, 0, 0);
-    }
+// A lane's live bins: those of the lower half (s + SL r with SL r < lo) and the
+// mirrored ones (SL - s + SL q with SL q < hi), and the byte offsets of bins s and
+// SL - s of its line within a field.
+struct Bins {
+    int lo, hi;
+    unsigned at, at_hi;
+};
+template <class S>
+__device__ __forceinline__ Bins zw_bins(const ZWCtx& c) {
+    const bool act = c.line_ok && c.gi < S::SL;
+    return Bins{act ? c.nkz - c.gi : 0, act ? c.nkz - S::SL + c.gi : 0, (unsigned)(c.base + c.gi) * 16u,
+                (unsigned)(c.base + (S::SL - c.gi)) * 16u};
 }
 
 // c2r of two real fields at once (fa -> pa, fb -> pb; fb < 0: none), from the
 // live bins kz < nkz of xp; dza / dzb apply d/dz. As in FFTW's c2r, the
-// imaginary part of bin 0 is ignored. STAGED: the bins come from staging
-// slots 0 (fa) and 1 (fb), and once these are read the copies of fields na and
-// nb (< 0: none) into them start, to land while this transform and what
-// follows it run.
-template <class S, bool STAGED>
+// imaginary part of bin 0 is ignored.
+template <class S>
 __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
-                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV], int na = -1,
-                                       int nb = -1) {
-    constexpr int SL = S::SL, SV = S::SV, PV = S::PV, N = S::N;
-    const int j = c.gi;
-    const bool act = c.line_ok && j < SL;
-    const double2* Sa = c.S + c.sline;
-    const double2* Sb = Sa + c.sstride;
+                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV]) {
+    constexpr int SL = S::SL, SV = S::SV, PV = S::PV;
+    const int s = c.gi;
+    // Value r of lane s is bin n = s + SL r. In the lower half of the r it can
+    // only be a live bin k = n, in the upper half only the mirror of k = N - n =
+    // SL - s + SL (SV - 1 - r) (nkz <= N/2); an odd SV has a middle r that can be
+    // either. So each load is at a fixed distance from one of two lane addresses.
+    const Bins bins = zw_bins<S>(c);
+    double2 A[SV], B[SV];
+    auto fetch = [&](int f, double2 (&X)[SV]) {
+        const gbytes fld = reinterpret_cast<gbytes>(gmem(xp) + (long)f * c.fsz);
+#pragma unroll
+        for (int r = 0; r < SV; ++r) {
+            X[r] = make_double2(0.0, 0.0);
+            if (2 * r < SV && SL * r < bins.lo) X[r] = gload(fld + 16 * SL * r, bins.at);
+            if (2 * r + 1 >= SV && SL * (SV - 1 - r) < bins.hi)
+                X[r] = gload(fld + 16 * SL * (SV - 1 - r), bins.at_hi);
+        }
+    };
+    fetch(fa, A);
+    if (fb >= 0) fetch(fb, B);
     double2 v[SV];
+    const double sd = s;
 #pragma unroll
     for (int r = 0; r < SV; ++r) {
-        const int n = j + SL * r;
-        const bool lo = n < c.nkz, hi = n > N - c.nkz;
-        const int k = lo ? n : N - n;
-        double2 A = make_double2(0.0, 0.0), B = make_double2(0.0, 0.0);
-        if (act && (lo || hi)) {
-            if constexpr (STAGED) {
-                A = Sa[k];
-                if (fb >= 0) B = Sb[k];
-            } else {
-                A = xp[(long)fa * c.fsz + c.base + k];
-                if (fb >= 0) B = xp[(long)fb * c.fsz + c.base + k];
-            }
+        const bool up = 2 * r + 1 > SV || (2 * r + 1 == SV && SL * r >= bins.lo);  // the mirror of bin k
+        const double k = up ? (double)(SL * (SV - r)) - sd : sd + (double)(SL * r);
+        double2 a = A[r], b = fb >= 0 ? B[r] : make_double2(0.0, 0.0);
+        if (dza) a = imul(c.dk * k, a);
+        if (dzb) b = imul(c.dk * k, b);
+        if (up) {
+            v[r] = make_double2(a.x + b.y, b.x - a.y);  // conj(A) + i conj(B) (zero in the gap)
+        } else {
+            v[r] = make_double2(a.x - b.y, a.y + b.x);  // A + iB
+            if (r == 0 && s == 0) v[r] = make_double2(a.x, b.x);
         }
-        if (dza) A = imul(c.dk * k, A);
-        if (dzb) B = imul(c.dk * k, B);
-        if (n == 0) v[r] = make_double2(A.x, B.x);
-        else if (lo) v[r] = make_double2(A.x - B.y, A.y + B.x);  // A + iB
-        else v[r] = make_double2(A.x + B.y, B.x - A.y);          // conj(A) + i conj(B) (zero in the gap)
-    }
-    if (STAGED && na >= 0) {
-        // every lane's reads of the slots have returned before the copies may overwrite them
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        zw_stage(c, xp, na, 0);
-        if (nb >= 0) zw_stage(c, xp, nb, 1);
     }
     double2 u[PV];
-    line_s2p<S, +1>(v, u, j, c.T, c.tw);
+    line_s2p<S, +1>(v, u, s, c.T, c.tw);
 #pragma unroll
     for (int m = 0; m < PV; ++m) {
         pa[m] = u[m].x;
@@ -351,50 +342,42 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
 template <class S, bool TWO>
 __device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo, const double (&pa)[S::PV],
                                        const double (&pb)[S::PV], int ga, int gb, double fold = 0.0) {
-    constexpr int SL = S::SL, SV = S::SV, PV = S::PV, N = S::N;
-    const int j = c.gi;
+    constexpr int SL = S::SL, SV = S::SV, PV = S::PV;
+    const int s = c.gi;
     double2 v[PV];
 #pragma unroll
     for (int m = 0; m < PV; ++m) v[m] = make_double2(pa[m], TWO ? pb[m] : 0.0);
     double2 w[SV];
-    line_p2s<S, -1>(v, w, j, c.T, c.tw);  // w[p] = X[j + SL p]
+    line_p2s<S, -1>(v, w, s, c.T, c.tw);  // w[p] = X[s + SL p]
+    const Bins bins = zw_bins<S>(c);
+    // the mirrors of the live bins meet them through the line's LDS rows; bin 0 is its own
     wave_lds_sync();
-    if (j < SL) {
+    if (s < SL) {
 #pragma unroll
-        for (int p = 0; p < SV; ++p) c.T[j + SL * p] = w[p];
+        for (int p = SV / 2; p < SV; ++p) c.T[s + SL * p] = w[p];
     }
     wave_lds_sync();
-    if (c.line_ok && j < SL) {
+    const double sd = s;
+    const gbytes_w oa = reinterpret_cast<gbytes_w>(gmem_w(zo) + (long)ga * c.fsz);
+    const gbytes_w ob = reinterpret_cast<gbytes_w>(gmem_w(zo) + (long)(TWO && gb >= 0 ? gb : ga) * c.fsz);
 #pragma unroll
-        for (int p = 0; p < SV; ++p) {
-            const int k = j + SL * p;
-            if (k < c.nkz) {
-                const double2 Zk = w[p];
-                const double2 Zn = c.T[(N - k) % N];
-                const double2 A = make_double2(0.5 * (Zk.x + Zn.x), 0.5 * (Zk.y - Zn.y));
-                const double2 B = make_double2(0.5 * (Zk.y + Zn.y), -0.5 * (Zk.x - Zn.x));
-                if (TWO && fold != 0.0) {
-                    const double fk = fold * (c.dk * k);
-                    zo[(long)ga * c.fsz + c.base + k] = make_double2(A.x - fk * B.y, A.y + fk * B.x);
-                } else {
-                    zo[(long)ga * c.fsz + c.base + k] = A;
-                }
-                if (TWO && gb >= 0) zo[(long)gb * c.fsz + c.base + k] = B;
+    for (int p = 0; 2 * p < SV; ++p) {
+        if (SL * p < bins.lo) {
+            const double2 Zk = w[p];
+            double2 Zn = c.T[SL - s + SL * (SV - 1 - p) - (p == 0 && s == 0 ? 1 : 0)];
+            if (p == 0 && s == 0) Zn = Zk;
+            const double2 A = make_double2(0.5 * (Zk.x + Zn.x), 0.5 * (Zk.y - Zn.y));
+            const double2 B = make_double2(0.5 * (Zk.y + Zn.y), -0.5 * (Zk.x - Zn.x));
+            if (TWO && fold != 0.0) {
+                const double fk = fold * (c.dk * (sd + (double)(SL * p)));
+                gstore(oa + 16 * SL * p, bins.at, make_double2(A.x - fk * B.y, A.y + fk * B.x));
+            } else {
+                gstore(oa + 16 * SL * p, bins.at, A);
             }
+            if (TWO && gb >= 0) gstore(ob + 16 * SL * p, bins.at, B);
         }
     }
 }
-
-// The z pass stages its inputs at Nz = 64. The choice depends on the grid alone
-// (never on the member count), so a member's result is the same alone and in a
-// batch: the two forms contract multiply-adds differently (the compiler fuses
-// either product of a*b + c*d depending on the code around it) and differ in the
-// last bits. At Nz = 64 the staged form wins where it matters, in batches (16
-// members of 64x65x64, skew-symmetric: 104 against 122 us per launch) and loses
-// 2.6 us on a lone field; at 32 and 48 (24 members) and at the three-step
-// lengths (one 128^3 field: rotational 39.2 us staged, 35.0 not, convection 73.2
-// and 70.1) the unstaged one is faster.
-constexpr bool zwave_staged(int nz) { return nz == 64; }
 
 // Three steps per transform (ZW3) at Nz = 72 and from 96 on. What bounds the z
 // pass there is how few wavefronts a SIMD holds: with 6 physical values per lane
@@ -410,38 +393,25 @@ constexpr bool zwave_three(int nz) { return nz == 72 || nz >= 96; }
 template <int NZ>
 using ZLine = std::conditional_t<zwave_three(NZ), ZW3<NZ>, ZW<NZ>>;
 
-// lengths the staged form is compiled for
-constexpr bool zwave_has_staged(int nz) { return nz == 16 || nz == 32 || nz == 48 || nz == 64; }
 // The z pass of k_zpass with one wavefront per 64/G lines (same fields, same
-// products in the same order). A block is independent wavefronts: any number
-// up to 4 (LDS sized at launch), or, STAGED, ZWAVE_WB of them, each staging
-// the next transform's two input fields in LDS while it works on the current
-// one. Staging hides the loads' latency where many wavefronts share a CU;
-// with few wavefronts per SIMD the extra LDS round trip costs more than it
-// hides (zwave_staged picks the form per grid).
-template <int METHOD, int NZ, bool STAGED>
+// products in the same order). A block is independent wavefronts, any number up
+// to 4 (LDS sized at launch). Every access is at a field's uniform base, one of
+// two 32-bit lane offsets and a constant distance: with 64-bit addresses and the
+// bin tests formed per access the kernel was bound by those instructions. us per
+// launch, before -> after: one 128^3 convection field 70 -> 50, rotational 35 ->
+// 32, 96^3 skew-symmetric 44 -> 39, 192x129x192 rotational 76 -> 64, 24 members of
+// 48^3 skew-symmetric 83 -> 71, of 32^3 32 -> 29. A form that staged its inputs in
+// LDS one transform ahead is slower than this one at every length (16 members of
+// 64^3 skew-symmetric 108 against 99, rotational 52 against 42).
+template <int METHOD, int NZ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8)))
 k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ tab,
                                                int want_g, const double2* __restrict__ xp0, double2* __restrict__ zo0,
                                                long sx) {
     using S = ZLine<NZ>;
-    constexpr int N1 = S::PV, SLOT = S::LPW * (NZ / 2);
-    double2 *tw_l, *T_l, *in_l = nullptr;
-    if constexpr (STAGED) {
-        // Separate LDS arrays (not one dynamic block) let the compiler tell the
-        // staging copies apart from the transposes: an LDS read waits for the
-        // copies in flight only when it reads the staging array.
-        __shared__ double2 tw_s[NZ];
-        __shared__ double2 T_s[ZWAVE_WB * S::LPW * S::LBUF];
-        __shared__ double2 in_s[ZWAVE_WB * 2 * SLOT];
-        tw_l = tw_s;
-        T_l = T_s;
-        in_l = in_s;
-    } else {
-        extern __shared__ double2 lds[];
-        tw_l = lds;
-        T_l = lds + NZ;
-    }
+    constexpr int N1 = S::PV;
+    extern __shared__ double2 lds[];
+    double2 *const tw_l = lds, *const T_l = lds + NZ;
     for (int i = threadIdx.x; i < NZ; i += blockDim.x) tw_l[i] = twg[i];
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
@@ -460,24 +430,14 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
     c.dk = 2 * PI / g.Lz;
     c.T = T_l + (wave * S::LPW + L) * S::LBUF;
     c.tw = tw_l;
-    c.wbase = ((long)y * g.Nx + x0) * g.nkz;
-    c.wcount = min(S::LPW, g.Nx - x0) * g.nkz;
-    c.lane = lane;
-    c.sline = L * g.nkz;
-    c.sstride = SLOT;
-    c.S = in_l + wave * 2 * SLOT;
     const double rotation = tab[blockIdx.y].rotation;
     const double2* __restrict__ xp = xp0 + blockIdx.y * sx;
     double2* __restrict__ zo = zo0 + blockIdx.y * sx;
-    if constexpr (STAGED) {
-        zw_stage(c, xp, 0, 0);  // u, v: the first transform's pair
-        zw_stage(c, xp, 1, 1);
-    }
     if constexpr (METHOD == NL_ROT) {
         double u0[N1], u1[N1], u2[N1], w0[N1], w1[N1], w2[N1];
-        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2, 3);
-        zw_c2r<S, STAGED>(c, xp, 2, false, 3, false, u2, w0, 4, 5);
-        zw_c2r<S, STAGED>(c, xp, 4, false, 5, false, w1, w2);
+        zw_c2r<S>(c, xp, 0, false, 1, false, u0, u1);
+        zw_c2r<S>(c, xp, 2, false, 3, false, u2, w0);
+        zw_c2r<S>(c, xp, 4, false, 5, false, w1, w2);
         double f0[N1], f1[N1], f2[N1];
 #pragma unroll
         for (int m = 0; m < N1; ++m) {  // cross(vort, u) (diffops.cpp:2598-2605)
@@ -507,8 +467,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         constexpr bool SK = (METHOD == NL_SKEW);
         constexpr double s = SK ? 0.5 : 1.0, us = SK ? 2.0 : 1.0;
         double h0[N1], h1[N1], h2[N1], pa[N1], pb[N1], fa[N1], fb[N1];
-        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, h0, h1, 2, 6);   // u, v
-        zw_c2r<S, STAGED>(c, xp, 2, false, 6, false, h2, pa, 3, 0);   // w, du/dx
+        zw_c2r<S>(c, xp, 0, false, 1, false, h0, h1);   // u, v
+        zw_c2r<S>(c, xp, 2, false, 6, false, h2, pa);   // w, du/dx
         if constexpr (SK) {
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
@@ -519,7 +479,7 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         }
 #pragma unroll
         for (int m = 0; m < N1; ++m) fa[m] = 0.0 + h0[m] * pa[m];
-        zw_c2r<S, STAGED>(c, xp, 3, false, 0, true, pa, pb, 7, 4);    // du/dy, du/dz
+        zw_c2r<S>(c, xp, 3, false, 0, true, pa, pb);    // du/dy, du/dz
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] += h1[m] * pa[m];
@@ -529,20 +489,20 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         }
         if constexpr (SK) zw_r2c<S, true>(c, zo, fa, pb, 0, 5, 0.5);  // f0 + i kz u0u2 / 2, and u0u2
         else zw_r2c<S, false>(c, zo, fa, pb, 0, -1);                  // f0
-        zw_c2r<S, STAGED>(c, xp, 7, false, 4, false, pa, pb, 1, 8);   // dv/dx, dv/dy
+        zw_c2r<S>(c, xp, 7, false, 4, false, pa, pb);   // dv/dx, dv/dy
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] = 0.0 + h0[m] * pa[m];
             fa[m] += h1[m] * pb[m];
         }
-        zw_c2r<S, STAGED>(c, xp, 1, true, 8, false, pa, pb, 5, 2);    // dv/dz, dw/dx
+        zw_c2r<S>(c, xp, 1, true, 8, false, pa, pb);    // dv/dz, dw/dx
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fa[m] += h2[m] * pa[m];
             if (rotation != 0.0) fa[m] += rotation * (us * h0[m]);
             fb[m] = 0.0 + h0[m] * pb[m];
         }
-        zw_c2r<S, STAGED>(c, xp, 5, false, 2, true, pa, pb);    // dw/dy, dw/dz
+        zw_c2r<S>(c, xp, 5, false, 2, true, pa, pb);    // dw/dy, dw/dz
 #pragma unroll
         for (int m = 0; m < N1; ++m) {
             fb[m] += h1[m] * pa[m];
@@ -570,8 +530,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         }
     } else {
         double u0[N1], u1[N1], u2[N1], pa[N1], pb[N1];
-        zw_c2r<S, STAGED>(c, xp, 0, false, 1, false, u0, u1, 2);
-        zw_c2r<S, STAGED>(c, xp, 2, false, -1, false, u2, pa);
+        zw_c2r<S>(c, xp, 0, false, 1, false, u0, u1);
+        zw_c2r<S>(c, xp, 2, false, -1, false, u2, pa);
         if (want_g) {  // DIV with rotation: g = rotation terms only
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
@@ -613,19 +573,11 @@ void launch_z_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, in
     if constexpr (zwave_size(NZ)) {
         using S = ZLine<NZ>;
         const long waves = (long)g.Ny * ((g.Nx + S::LPW - 1) / S::LPW);
-        if constexpr (zwave_has_staged(NZ)) {
-            if (tn.zstage < 0 ? zwave_staged(NZ) : tn.zstage != 0) {
-                if (g.nkz > NZ / 2) throw std::runtime_error("z pass: more live kz bins than Nz/2");
-                const dim3 grid((unsigned)((waves + ZWAVE_WB - 1) / ZWAVE_WB), n);
-                k_zwave<METHOD, NZ, true><<<grid, 64 * ZWAVE_WB, 0, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
-                return;
-            }
-        }
         const int wb = tn.zwb > 0 ? tn.zwb : 4;
         const size_t lds = (size_t)(NZ + wb * S::LPW * S::LBUF) * sizeof(double2);
         const dim3 grid((unsigned)((waves + wb - 1) / wb), n);
-        allow_lds(k_zwave<METHOD, NZ, false>, lds);
-        k_zwave<METHOD, NZ, false><<<grid, 64 * wb, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
+        allow_lds(k_zwave<METHOD, NZ>, lds);
+        k_zwave<METHOD, NZ><<<grid, 64 * wb, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
     } else {
         const int nphys = zpass_nphys(METHOD);
         const int XB = zpass_xb(g, nphys, tn);
