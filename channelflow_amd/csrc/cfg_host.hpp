@@ -272,6 +272,48 @@ inline YTables y_tables(int N, double a, double b) {
     return yt;
 }
 
+// T, TD and Ti, DTi in the order in which the matrix-core transforms stage them in
+// LDS (k_yinv_w, k_yfwd_w), so that a chunk is one contiguous copy: [chunk][matrix]
+// of yinv_tile (per row split) / yfwd_tile doubles, zero past the operator. Empty above the largest
+// row-tile class.
+struct YTiles {
+    std::vector<double> inv, fwd;
+};
+inline YTiles y_tiles(int N, const YTables& yt) {
+    YTiles o;
+    const int cls = yw_class(N), nm = N / 2, nh = (N + 1) / 2;
+    const bool odd = N & 1;
+    if (cls == 0) return o;
+    const int ci = (N + YINV_KC - 1) / YINV_KC, ns = yinv_split(cls), rows = yinv_rows(cls) * 16;
+    const int ti = yinv_tile(yinv_rows(cls));
+    o.inv.assign((size_t)ns * ci * 2 * ti, 0.0);
+    for (int sp = 0; sp < ns; ++sp)
+        for (int c = 0; c < ci; ++c)
+            for (int a = 0; a < 2; ++a)
+                for (int slot = 0; slot <= rows; ++slot)
+                    for (int kk = 0; kk < YINV_KC; ++kk) {
+                        const int k = c * YINV_KC + kk, row = slot < rows ? sp * rows + slot : nm;
+                        if (k >= N || (slot < rows ? row >= nm : !odd)) continue;
+                        // the chunk's even columns before its odd ones
+                        o.inv[(((size_t)sp * ci + c) * 2 + a) * ti + slot * (YINV_KC + 1) + (kk & 1) * (YINV_KC / 2) +
+                              (kk >> 1)] = (a == 0 ? yt.T : yt.TD)[(size_t)row * N + k];
+                    }
+    const int cf = (nh + YFWD_KC - 1) / YFWD_KC, tf = yfwd_tile(cls);
+    o.fwd.assign((size_t)cf * 2 * tf, 0.0);
+    for (int c = 0; c < cf; ++c)
+        for (int a = 0; a < 2; ++a)
+            for (int slot = 0; slot <= 2 * cls * 16; ++slot)
+                for (int kk = 0; kk < YFWD_KC; ++kk) {
+                    // rows: even coefficients, odd ones, then the last one of an odd Ny
+                    const int par = slot / (cls * 16), r = slot % (cls * 16), y = c * YFWD_KC + kk;
+                    const int k = par < 2 ? 2 * r + par : N - 1;
+                    if (y >= nh || (par < 2 ? r >= nm : !odd)) continue;
+                    o.fwd[((size_t)c * 2 + a) * tf + slot * (YFWD_KC + 1) + kk] =
+                        (a == 0 ? yt.Ti : yt.DTi)[(size_t)k * N + y];
+                }
+    return o;
+}
+
 // y values of a coefficient profile and of its derivative (long double sums)
 inline std::vector<double> eval_profile(const Geom& g, const std::vector<long double>& tcheb,
                                         const std::vector<double>& c, bool deriv) {
@@ -302,11 +344,11 @@ struct Geometry {
     Geom g{};
     int dealias = 0;
     FFTTable fx, fz;
-    DBuf T, TD, Ti, DTi;
+    DBuf T, TD, Ti, DTi, Tinv, Tfwd;
     DBuf HB;  // rows of the Chebyshev-tau operator B of the Helmholtz systems, [3][Ny]
     std::vector<long double> tcheb;  // T_k(y_n) = cos(pi n k / (Ny-1)), [n][k], for host profile evaluation
 
-    YMats ymats() const { return YMats{T.p, TD.p, Ti.p, DTi.p}; }
+    YMats ymats() const { return YMats{T.p, TD.p, Ti.p, DTi.p, Tinv.p, Tfwd.p}; }
 
     void build(const cfg_grid& gr, bool dealias_xz) {
         dealias = dealias_xz ? 1 : 0;
@@ -318,8 +360,11 @@ struct Geometry {
         tcheb = yt.tcheb;
         auto up = [&](DBuf& b, const std::vector<double>& h) {
             b.alloc(h.size());
-            HIPCHK(hipMemcpy(b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+            if (!h.empty()) HIPCHK(hipMemcpy(b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
         };
+        const YTiles tiles = y_tiles(N, yt);
+        up(Tinv, tiles.inv);
+        up(Tfwd, tiles.fwd);
         up(T, yt.T);
         up(TD, yt.TD);
         up(Ti, yt.Ti);

@@ -24,6 +24,7 @@
 
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "cfg_fft.hpp"
@@ -524,9 +525,19 @@ __global__ void __launch_bounds__(256) k_yfwd_t(Geom g, YMats ym, int have_g, co
 //
 // A block is three waves per transform matrix; wave c handles velocity
 // component c of YW_MODES = 8 consecutive modes, i.e. 16 real columns (real,
-// imaginary part of each mode), over all output rows. Each lane's B operand
-// streams from HBM straight into registers, one chunk ahead; the chunk of the
-// transform matrices, shared by the waves, is staged in LDS.
+// imaginary part of each mode), over all output rows of the block. Each lane's B
+// operand streams from HBM straight into registers, one chunk ahead; the chunk of
+// the transform matrices, shared by the waves, is staged in LDS. The matrices come
+// in the order in which they are staged (y_tiles): a chunk is one contiguous copy in
+// 16-byte pieces. Picked entry by entry out of the row-major matrices, with the row,
+// column and bounds formed for each, the staging took half the kernels' VALU
+// instructions; us per launch, before -> after (inverse, forward): one 32^3 field
+// 5.4 -> 4.8, 6.0 -> 4.7; 64^3 10.8 -> 6.9 (with the row split), 11.6 -> 8.6; 96^3
+// 17.0 -> 14.4, 19.1 -> 13.8; 128^3 convection 41 -> 35, 22 -> 19; 192x129x192 81 ->
+// 63, 44 -> 35; 16 of 64^3 52 -> 46, 51 -> 44. The inverse at 192x129x192 then takes
+// 24 us for its loads alone, 23 us of matrix products at their peak rate and writes
+// 96 MB (20 us at the copy rate), one after the other in each block; loading two or
+// three chunks ahead, or four waves per SIMD, changes nothing.
 //
 // Both transforms use the mirror symmetry of the Chebyshev points,
 // y_{Ny-1-j} = -y_j: T[Ny-1-j][k] = (-1)^k T[j][k], and the derivative flips
@@ -557,25 +568,28 @@ constexpr int yw_waves_fwd(bool divf, int nrt) { return nrt <= 1 ? 4 : (nrt <= (
 // p_{Ny-1-j} = E - O, q_j = E + O, q_{Ny-1-j} = O - E. The middle point of an
 // odd Ny is a dot product per lane, summed over the lane groups. NRT: row
 // tiles of 16 upper points.
-template <int METHOD, int NRT>
+template <int METHOD, int NRT, int NSP>
 __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((amdgpu_waves_per_eu(yw_waves(NRT))))
     k_yinv_w(Geom g, YMats ym, const NLMember* __restrict__ tab, double2* __restrict__ yp0, long sy) {
     const BlockId bid = xcd_grid();  // neighbouring blocks on one XCD
     constexpr int NMAT = (METHOD == NL_DIV) ? 1 : 2, NT = 192 * NMAT;
-    constexpr int KC = 16, AP = KC + 1, EP = 17;  // chunk columns: 8 even k, then 8 odd k
-    constexpr int RS = NRT * 16 + 1;              // LDS rows per matrix: tiles, middle point
+    constexpr int KC = YINV_KC, AP = KC + 1, EP = 17;  // chunk columns: 8 even k, then 8 odd k
+    constexpr int RS = NRT * 16 + 1;                   // LDS rows per matrix: tiles, middle point
     // two matrix chunk buffers: chunk i + 1 is loaded into registers while
-    // chunk i is multiplied, and stored to the other buffer after it
-    constexpr int SA = NMAT * RS * AP, SE = NMAT * 3 * 2 * 16 * EP;
-    constexpr int NSTG = NMAT * RS * KC, NST = (NSTG + NT - 1) / NT;  // staged entries per chunk, per thread
-    __shared__ double sm[2 * SA > SE ? 2 * SA : SE];
+    // chunk i is multiplied, and stored to the other buffer after it. A chunk is
+    // one contiguous piece of ym.inv, laid out as it lies in LDS.
+    constexpr int SM = yinv_tile(NRT), SA = NMAT * SM, SE = NMAT * 3 * 2 * 16 * EP;
+    constexpr int NST = (SA / 2 + NT - 1) / NT;  // 16-byte pieces per thread
+    static_assert(SM == RS * AP + 1 && SM % 2 == 0, "the staged chunk's layout");
+    __shared__ __align__(16) double sm[2 * SA > SE ? 2 * SA : SE];
     const NLMember& me = tab[bid.y];
     double2* __restrict__ yp = yp0 + bid.y * sy;
     const int Ny = g.Ny, nm = Ny / 2, mid = (Ny & 1) ? nm : -1;
     const long M = g.M;
     const int nrt = (nm + 15) / 16;
-    const int w = threadIdx.x >> 6, c = w % 3, am = w / 3, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
-    const long m0 = (long)bid.x * YW_MODES;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = w % 3, am = w / 3, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+    const int sp = bid.x % NSP, rt0 = sp * NRT;  // this block's row tiles
+    const long m0 = (long)(bid.x / NSP) * YW_MODES;
     const long mcol = m0 + (lr >> 1);
     const bool mok = mcol < M;
     const gcdouble ucol = gmem(me.u) + 2 * ((long)c * Ny * M + mcol) + (l & 1);
@@ -591,18 +605,11 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
             bn[i] = (mok && k < Ny) ? ucol[2L * k * M] : 0.0;
         }
     };
-    // matrix entries of chunk k0: entry i = (matrix a, row slot, column kk),
-    // stored with the 8 even columns before the 8 odd ones
-    double mv[NST];
+    dvec2 mv[NST];
     auto load_mat = [&](int k0) {
+        const auto src = gmem(reinterpret_cast<const dvec2*>(ym.inv + ((long)sp * ((Ny + KC - 1) / KC) + k0 / KC) * 2 * SM));
 #pragma unroll
-        for (int s = 0; s < NST; ++s) {
-            const int i = threadIdx.x + s * NT;
-            const int kk = i % KC, slot = (i / KC) % RS, a = i / (KC * RS);
-            const int k = k0 + kk, row = slot < NRT * 16 ? slot : mid;
-            const bool ok = i < NSTG && (slot < NRT * 16 ? slot < nm : mid >= 0) && k < Ny;
-            mv[s] = ok ? (a == 0 ? ym.T : ym.TD)[(long)row * Ny + k] : 0.0;
-        }
+        for (int s = 0; s < NST; ++s) mv[s] = src[min((int)threadIdx.x + s * NT, SA / 2 - 1)];
     };
     fetch(0);
     load_mat(0);
@@ -616,16 +623,16 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
 #pragma unroll
         for (int s = 0; s < NST; ++s) {
             const int i = threadIdx.x + s * NT;
-            const int kk = i % KC, slot = (i / KC) % RS, a = i / (KC * RS);
-            if (i < NSTG) sb[(a * RS + slot) * AP + (kk & 1) * 8 + (kk >> 1)] = mv[s];
+            if (i < SA / 2) reinterpret_cast<dvec2*>(sb)[i] = mv[s];
         }
         __syncthreads();
         if (k0 + KC < Ny) {
             fetch(k0 + KC);
             load_mat(k0 + KC);
         }
-        const double* __restrict__ arow = sb + (am * RS + lr) * AP + lk;
-        const double* __restrict__ amid = sb + (am * RS + NRT * 16) * AP + lk;
+        const double* __restrict__ arow = sb + am * SM + lr * AP + lk;
+        const double* __restrict__ amid = sb + am * SM + NRT * 16 * AP + lk;
+        if (METHOD == NL_ROT && w == 4) continue;  // dv/dy, which no vorticity component needs (uniform)
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
             // unconditional: staged rows and columns past the grid are zero,
@@ -680,7 +687,7 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
     // row tiles: the components and both halves meet in LDS
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
-        if (rt >= nrt) continue;  // uniform
+        if (rt0 + rt >= nrt) continue;  // uniform
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -691,12 +698,12 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
         __syncthreads();
         for (int pt = threadIdx.x; pt < 256; pt += NT) {
             const int half = pt >> 7, pr = (pt >> 3) & 15;
-            const int yt = rt * 16 + pr;
+            const int yt = (rt0 + rt) * 16 + pr;
             if (yt >= nm || m >= M) continue;
             emit(half ? Ny - 1 - yt : yt, sm + (half * 16 + pr) * EP + 2 * pm, 2 * 16 * EP);
         }
     }
-    if (mid < 0) return;  // uniform
+    if (mid < 0 || sp != NSP - 1) return;  // uniform
     dmid += __shfl_xor(dmid, 16);
     dmid += __shfl_xor(dmid, 32);
     __syncthreads();
@@ -720,14 +727,14 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     const BlockId bid = xcd_grid();  // neighbouring blocks on one XCD
     constexpr bool DIVF = (METHOD == NL_DIV || METHOD == NL_SKEW);
     constexpr int NMAT = DIVF ? 2 : 1;
-    constexpr int KC = 8, AP = KC + 1, NS = KC / 4;
-    constexpr int RS = 2 * NRT * 16 + 1;  // LDS rows per matrix: even, odd coefficients, last one
+    constexpr int KC = YFWD_KC, AP = KC + 1, NS = KC / 4;
     // two matrix chunk buffers, as in k_yinv_w, unless the chunk in flight
     // would not fit the registers (two matrices of 6 or 8 row tiles): then one
     // buffer, loaded and stored between two barriers
-    constexpr int SA = NMAT * RS * AP, NSTG = NMAT * RS * KC, NST = (NSTG + 191) / 192;
+    constexpr int SM = yfwd_tile(NRT), SA = NMAT * SM, NST = (SA / 2 + 191) / 192;
+    static_assert(SM % 2 == 0, "16-byte pieces");
     constexpr bool DB = !(DIVF && NRT >= 6);
-    __shared__ double sm[(DB ? 2 : 1) * SA];
+    __shared__ __align__(16) double sm[(DB ? 2 : 1) * SA];
     const double* __restrict__ fo = reinterpret_cast<const double*>(fo0 + bid.y * sy);
     __attribute__((address_space(1))) double* __restrict__ f = gmem_w(tab[bid.y].f);
     const int Ny = g.Ny, nh = (Ny + 1) / 2, nm = Ny / 2;
@@ -798,18 +805,12 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
         if (DIVF && XTERM) G += ZTERM ? sdx * r[4 + i] + sdz * r[6 + i] : sdx * r[4 + i];
         return G;
     };
-    // matrix entries of chunk y0: entry i = (matrix a, row slot, column kk)
-    double mv[NST];
+    dvec2 mv[NST];
+    auto mat = [&](int y0) { return gmem(reinterpret_cast<const dvec2*>(ym.fwd + (long)(y0 / KC) * 2 * SM)); };
     auto load_mat = [&](int y0) {
+        const auto src = mat(y0);
 #pragma unroll
-        for (int s = 0; s < NST; ++s) {
-            const int i = threadIdx.x + s * 192;
-            const int kk = i % KC, slot = (i / KC) % RS, a = i / (KC * RS);
-            const int par = slot / (NRT * 16), r = slot % (NRT * 16), y = y0 + kk;  // par 2: the last coefficient
-            const int k = par < 2 ? 2 * r + par : Ny - 1;
-            const bool ok = i < NSTG && (par < 2 ? r < nm : odd) && y < nh;
-            mv[s] = ok ? (a == 0 ? ym.Ti : ym.DTi)[(long)k * Ny + y] : 0.0;
-        }
+        for (int s = 0; s < NST; ++s) mv[s] = src[min((int)threadIdx.x + s * 192, SA / 2 - 1)];
     };
     fetch(0);
     if (DB) load_mat(0);
@@ -839,18 +840,12 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
 #pragma unroll
             for (int s = 0; s < NST; ++s) {
                 const int i = threadIdx.x + s * 192;
-                const int kk = i % KC, slot = (i / KC) % RS, a = i / (KC * RS);
-                if (i < NSTG) sb[(a * RS + slot) * AP + kk] = mv[s];
+                if (i < SA / 2) reinterpret_cast<dvec2*>(sb)[i] = mv[s];
             }
         } else {
             __syncthreads();  // the previous chunk's matrix reads are done
-            for (int i = threadIdx.x; i < NSTG; i += 192) {
-                const int kk = i % KC, slot = (i / KC) % RS, a = i / (KC * RS);
-                const int par = slot / (NRT * 16), r = slot % (NRT * 16), y = y0 + kk;
-                const int k = par < 2 ? 2 * r + par : Ny - 1;
-                const bool ok = (par < 2 ? r < nm : odd) && y < nh;
-                sb[(a * RS + slot) * AP + kk] = ok ? (a == 0 ? ym.Ti : ym.DTi)[(long)k * Ny + y] : 0.0;
-            }
+            const auto src = mat(y0);
+            for (int i = threadIdx.x; i < SA / 2; i += 192) reinterpret_cast<dvec2*>(sb)[i] = src[i];
         }
         __syncthreads();
         if (y0 + KC < nh) {
@@ -867,13 +862,13 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
                 ae[rt] = mfma16x16x4(A[0], sg[s], ae[rt]);
                 ao[rt] = mfma16x16x4(A[NRT * 16 * AP], dg[s], ao[rt]);
                 if (DIVF) {
-                    ae[rt] = mfma16x16x4(A[RS * AP], dh[s], ae[rt]);
-                    ao[rt] = mfma16x16x4(A[(RS + NRT * 16) * AP], sh[s], ao[rt]);
+                    ae[rt] = mfma16x16x4(A[SM], dh[s], ae[rt]);
+                    ao[rt] = mfma16x16x4(A[SM + NRT * 16 * AP], sh[s], ao[rt]);
                 }
             }
             const double* A = sb + 2 * NRT * 16 * AP + 4 * s + lk;
             dlast = fma(A[0], sg[s], dlast);
-            if (DIVF) dlast = fma(A[RS * AP], dh[s], dlast);
+            if (DIVF) dlast = fma(A[SM], dh[s], dlast);
             __builtin_amdgcn_sched_barrier(0);  // keep each step's operand reads next to its MFMAs
         }
     }
@@ -900,14 +895,18 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
 template <int METHOD>
 static void launch_yinv(const Geom& g, const YMats& ym, int n, const NLMember* tab, double2* yp, long sy,
                         hipStream_t st) {
-    const int nrt = (g.Ny / 2 + 15) / 16, nt = METHOD == NL_DIV ? 192 : 384;
-    const dim3 grid((unsigned)((g.M + YW_MODES - 1) / YW_MODES), n);
-    if (nrt <= 1) k_yinv_w<METHOD, 1><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
-    else if (nrt <= 2) k_yinv_w<METHOD, 2><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
-    else if (nrt <= 3) k_yinv_w<METHOD, 3><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
-    else if (nrt <= 4) k_yinv_w<METHOD, 4><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
-    else if (nrt <= 6) k_yinv_w<METHOD, 6><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
-    else if (nrt <= 8) k_yinv_w<METHOD, 8><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
+    const int cls = yw_class(g.Ny), nt = METHOD == NL_DIV ? 192 : 384;
+    auto go = [&](auto c) {
+        constexpr int C = decltype(c)::value, NSP = yinv_split(C);
+        const dim3 grid((unsigned)((g.M + YW_MODES - 1) / YW_MODES * NSP), n);
+        k_yinv_w<METHOD, yinv_rows(C), NSP><<<grid, nt, 0, st>>>(g, ym, tab, yp, sy);
+    };
+    if (cls == 1) go(std::integral_constant<int, 1>{});
+    else if (cls == 2) go(std::integral_constant<int, 2>{});
+    else if (cls == 3) go(std::integral_constant<int, 3>{});
+    else if (cls == 4) go(std::integral_constant<int, 4>{});
+    else if (cls == 6) go(std::integral_constant<int, 6>{});
+    else if (cls == 8) go(std::integral_constant<int, 8>{});
     else {
         const dim3 tg((unsigned)(((g.M + YB_M - 1) / YB_M) * ((g.Ny + YB_R - 1) / YB_R)), n);
         k_yinv_t<METHOD><<<tg, 256, 0, st>>>(g, ym, tab, yp, sy);

@@ -100,7 +100,28 @@ struct YMats {            // y-direction operators, row-major [row][col], Ny x N
     const double* TD;     // T * (d/dy)
     const double* Ti;     // values -> coefficients
     const double* DTi;    // (d/dy) * Ti
+    const double* inv;    // T and TD, Ti and DTi as the matrix-core transforms stage
+    const double* fwd;    // them, chunk by chunk (y_tiles)
 };
+
+// Row-tile class of the matrix-core y transforms (16 rows of the upper half of
+// the points per tile), 0 above the largest
+constexpr int yw_class(int Ny) {
+    const int n = (Ny / 2 + 15) / 16;
+    return n <= 1 ? 1 : n <= 4 ? n : n <= 6 ? 6 : n <= 8 ? 8 : 0;
+}
+// Blocks per mode group of the inverse transform, and row tiles per block: fewer
+// accumulators per wave and more blocks where the tile count is even (one 64^3
+// field 8.9 -> 6.9 us, 192x129x192 67.6 -> 63.4, 16 of 64^3 45.9 -> 46.0; one tile
+// per block at three tiles: one 96^3 field 14.4 -> 14.9). Every block reads all the
+// coefficients of its modes, the second time from L2.
+constexpr int yinv_split(int cls) { return cls == 2 || cls >= 4 ? 2 : 1; }
+constexpr int yinv_rows(int cls) { return cls / yinv_split(cls); }
+// A chunk of one staged matrix: rows of the class's tiles and one more (the middle
+// point; the last coefficient) of KC columns at an odd pitch, one double of padding
+constexpr int YINV_KC = 16, YFWD_KC = 8;
+constexpr int yinv_tile(int cls) { return (cls * 16 + 1) * (YINV_KC + 1) + 1; }
+constexpr int yfwd_tile(int cls) { return (2 * cls * 16 + 1) * (YFWD_KC + 1) + 1; }
 
 // Per-mode tau data for one lambda_t, mode-major: array k (TAU_NA of them:
 // pband pup pinvd vband vup vinvd Pp Pm vp vm P0 v0) of mode m is the Ny-vector

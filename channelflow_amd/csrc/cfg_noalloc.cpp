@@ -73,6 +73,10 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
         const size_t o_twz = carve(off, 2 * (size_t)g.Nz);
         const size_t nyy = (size_t)g.Ny * g.Ny;
         const size_t o_T = carve(off, nyy), o_TD = carve(off, nyy), o_Ti = carve(off, nyy), o_DTi = carve(off, nyy);
+        const int cls = yw_class(g.Ny);
+        const size_t n_inv = cls ? (size_t)((g.Ny + YINV_KC - 1) / YINV_KC) * 2 * yinv_split(cls) * yinv_tile(yinv_rows(cls)) : 0;
+        const size_t n_fwd = cls ? (size_t)(((g.Ny + 1) / 2 + YFWD_KC - 1) / YFWD_KC) * 2 * yfwd_tile(cls) : 0;
+        const size_t o_inv = carve(off, n_inv), o_fwd = carve(off, n_fwd);
         const size_t o_base = carve(off, 4 * (size_t)g.Ny);
         const size_t ny = (size_t)nlwork_y_doubles(g), nx = (size_t)nlwork_x_doubles(g);
         const size_t o_yp = carve(off, ny), o_fo = carve(off, ny), o_xp = carve(off, nx), o_zo = carve(off, nx);
@@ -105,6 +109,11 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
         put(o_TD, yt.TD.data(), nyy * 8);
         put(o_Ti, yt.Ti.data(), nyy * 8);
         put(o_DTi, yt.DTi.data(), nyy * 8);
+        const YTiles tiles = y_tiles(g.Ny, yt);
+        if (cls) {
+            put(o_inv, tiles.inv.data(), tiles.inv.size() * 8);
+            put(o_fwd, tiles.fwd.data(), tiles.fwd.size() * 8);
+        }
         put(o_base, h.base.data(), h.base.size() * 8);
         int method;  // NSE::nonlinear's form for one call (nse.cpp:12-91)
         switch (flags->nonlinearity) {
@@ -115,7 +124,7 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
             case CFG_Alternating: method = NL_DIV; break;
             default: method = NL_CONV; break;
         }
-        const YMats ym{S + o_T, S + o_TD, S + o_Ti, S + o_DTi};
+        const YMats ym{S + o_T, S + o_TD, S + o_Ti, S + o_DTi, S + o_inv, S + o_fwd};
         const NLWork w{S + o_yp, S + o_xp, S + o_zo, S + o_fo};
         launch_nonlinear(g, ym, h.px, h.pz, method, 1, reinterpret_cast<const NLMember*>(S + o_tab),
                          flags->rotation != 0.0, w, NLTune{}, st, nullptr);

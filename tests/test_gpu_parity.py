@@ -91,6 +91,25 @@ def test_nonlinear_chebyshev_sizes(gpu, method, Ny):
 
 
 @pytest.mark.parametrize("method", ["Rotational", "Convection", "Divergence", "SkewSymmetric"])
+@pytest.mark.parametrize("Ny", [35, 67, 99, 127, 131, 191, 195, 255])
+def test_nonlinear_row_tile_edges(gpu, method, Ny):
+    """The y transforms at the smallest and largest Ny of their row-tile counts
+    (with one and with two blocks per mode group, the middle point alone in the last
+    one's hands), 18 x 10 modes: groups of eight with a remainder. The same 1e-12 bar
+    as test_nonlinear_chebyshev_sizes."""
+    Nx, Nz = 18, 18
+    g = R.Grid(Nx, Ny, Nz, LX_C, LZ_C)
+    u = random_field(Nx, Ny, Nz, LX_C, LZ_C, norm=0.3, decay=0.5, seed=Ny, dealias=False)
+    fl = dict(nonlinearity=method, dealiasing="NoDealiasing", baseflow="LaminarBase", uupperwall=1.0,
+              ulowerwall=-1.0, constraint="BulkVelocity", nu=1 / 400, Vsuck=0.0)
+    f_ref, _ = R.nonlinear(g, R.make_flags(**fl), u)
+    f_gpu = cfa.nonlinear(cfa.FlowField(Nx, Ny, Nz, 3, LX_C, LZ_C, data=u), cfa.DNSFlags(**fl))
+    err = rel_l2_per_component(g, f_gpu, f_ref)
+    print(Ny, method, "rel L2 per component", err, flush=True)
+    assert np.all(err <= 1e-12), err
+
+
+@pytest.mark.parametrize("method", ["Rotational", "Convection", "Divergence", "SkewSymmetric"])
 @pytest.mark.parametrize("N", [18, 24, 36, 54, 72, 108, 144, 162])
 def test_nonlinear_ragged_lengths(gpu, method, N):
     """One NL call with x- and z-lines of the FFT lengths 2^a 3^b between the
