@@ -274,8 +274,8 @@ inline YTables y_tables(int N, double a, double b) {
 
 // T, TD and Ti, DTi in the order in which the matrix-core transforms stage them in
 // LDS (k_yinv_w, k_yfwd_w), so that a chunk is one contiguous copy: [chunk][matrix]
-// of yinv_tile (per row split) / yfwd_tile doubles, zero past the operator. Empty above the largest
-// row-tile class.
+// of yinv_tile (per row split) / yfwd_tile doubles, then the tails (per row split,
+// [matrix]), zero past the operator. Empty above the largest row-tile class.
 struct YTiles {
     std::vector<double> inv, fwd;
 };
@@ -284,9 +284,9 @@ inline YTiles y_tiles(int N, const YTables& yt) {
     const int cls = yw_class(N), nm = N / 2, nh = (N + 1) / 2;
     const bool odd = N & 1;
     if (cls == 0) return o;
-    const int ci = (N + YINV_KC - 1) / YINV_KC, ns = yinv_split(cls), rows = yinv_rows(cls) * 16;
-    const int ti = yinv_tile(yinv_rows(cls));
-    o.inv.assign((size_t)ns * ci * 2 * ti, 0.0);
+    const int ci = yinv_chunks(N), ns = yinv_split(cls), rows = yinv_rows(cls) * 16;
+    const int ti = yinv_tile(yinv_rows(cls)), li = yinv_tail(yinv_rows(cls));
+    o.inv.assign((size_t)ns * 2 * (ci * ti + li), 0.0);
     for (int sp = 0; sp < ns; ++sp)
         for (int c = 0; c < ci; ++c)
             for (int a = 0; a < 2; ++a)
@@ -298,8 +298,18 @@ inline YTiles y_tiles(int N, const YTables& yt) {
                         o.inv[(((size_t)sp * ci + c) * 2 + a) * ti + slot * (YINV_KC + 1) + (kk & 1) * (YINV_KC / 2) +
                               (kk >> 1)] = (a == 0 ? yt.T : yt.TD)[(size_t)row * N + k];
                     }
-    const int cf = (nh + YFWD_KC - 1) / YFWD_KC, tf = yfwd_tile(cls);
-    o.fwd.assign((size_t)cf * 2 * tf, 0.0);
+    for (int sp = 0; sp < ns; ++sp)
+        for (int a = 0; a < 2; ++a)
+            for (int slot = 0; slot <= rows; ++slot)
+                for (int k = ci * YINV_KC; k < N; ++k) {
+                    const int row = slot < rows ? sp * rows + slot : nm, par = k & 1, lk = (k - ci * YINV_KC) >> 1;
+                    if (slot < rows ? row >= nm : !odd) continue;
+                    const int at = slot < rows ? ((slot / 16) * 2 + par) * 64 + lk * 16 + slot % 16 : 8 * rows + 4 * par + lk;
+                    o.inv[(size_t)ns * ci * 2 * ti + (size_t)(sp * 2 + a) * li + at] =
+                        (a == 0 ? yt.T : yt.TD)[(size_t)row * N + k];
+                }
+    const int cf = yfwd_chunks(nh), tf = yfwd_tile(cls), lf = yfwd_tail(cls);
+    o.fwd.assign((size_t)2 * (cf * tf + lf), 0.0);
     for (int c = 0; c < cf; ++c)
         for (int a = 0; a < 2; ++a)
             for (int slot = 0; slot <= 2 * cls * 16; ++slot)
@@ -311,6 +321,15 @@ inline YTiles y_tiles(int N, const YTables& yt) {
                     o.fwd[((size_t)c * 2 + a) * tf + slot * (YFWD_KC + 1) + kk] =
                         (a == 0 ? yt.Ti : yt.DTi)[(size_t)k * N + y];
                 }
+    for (int a = 0; a < 2; ++a)
+        for (int slot = 0; slot <= 2 * cls * 16; ++slot)
+            for (int y = cf * YFWD_KC; y < nh; ++y) {
+                const int par = slot / (cls * 16), r = slot % (cls * 16), lk = y - cf * YFWD_KC;
+                const int k = par < 2 ? 2 * r + par : N - 1;
+                if (par < 2 ? r >= nm : !odd) continue;
+                const int at = par < 2 ? ((r / 16) * 2 + par) * 64 + lk * 16 + r % 16 : 2 * 64 * cls + lk;
+                o.fwd[(size_t)cf * 2 * tf + (size_t)a * lf + at] = (a == 0 ? yt.Ti : yt.DTi)[(size_t)k * N + y];
+            }
     return o;
 }
 

@@ -593,9 +593,8 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
     const long mcol = m0 + (lr >> 1);
     const bool mok = mcol < M;
     const gcdouble ucol = gmem(me.u) + 2 * ((long)c * Ny * M + mcol) + (l & 1);
+    const int nch = yinv_chunks(Ny), kend = nch * KC;
     mfma4d ae[NRT], ao[NRT];
-#pragma unroll
-    for (int rt = 0; rt < NRT; ++rt) ae[rt] = ao[rt] = mfma4d{0.0, 0.0, 0.0, 0.0};
     double dmid = 0.0;
     double bn[4];  // [parity * 2 + step]: k = k0 + 2 (4 step + lane / 16) + parity
     auto fetch = [&](int k0) {
@@ -607,13 +606,34 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
     };
     dvec2 mv[NST];
     auto load_mat = [&](int k0) {
-        const auto src = gmem(reinterpret_cast<const dvec2*>(ym.inv + ((long)sp * ((Ny + KC - 1) / KC) + k0 / KC) * 2 * SM));
+        const auto src = gmem(reinterpret_cast<const dvec2*>(ym.inv + ((long)sp * nch + k0 / KC) * 2 * SM));
 #pragma unroll
         for (int s = 0; s < NST; ++s) mv[s] = src[min((int)threadIdx.x + s * NT, SA / 2 - 1)];
     };
+    // the remainder of the contraction, straight from the caches (zero without one)
+    double ta[NRT][2], tm[2] = {0.0, 0.0}, tb[2] = {0.0, 0.0};
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) ta[rt][0] = ta[rt][1] = 0.0;
+    if (kend < Ny) {
+        const gcdouble tail = gmem(ym.inv) + (long)NSP * nch * 2 * SM + (sp * 2 + am) * yinv_tail(NRT);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int k = kend + 2 * lk + p;
+            tb[p] = (mok && k < Ny) ? ucol[2L * k * M] : 0.0;
+            tm[p] = tail[2 * 64 * NRT + 4 * p + lk];
+#pragma unroll
+            for (int rt = 0; rt < NRT; ++rt) ta[rt][p] = tail[(rt * 2 + p) * 64 + l];
+        }
+    }
     fetch(0);
     load_mat(0);
-    for (int k0 = 0, buf = 0; k0 < Ny; k0 += KC, buf ^= 1) {
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) {
+        ae[rt] = mfma16x16x4(ta[rt][0], tb[0], mfma4d{0.0, 0.0, 0.0, 0.0});
+        ao[rt] = mfma16x16x4(ta[rt][1], tb[1], mfma4d{0.0, 0.0, 0.0, 0.0});
+    }
+    dmid = fma(tm[0], tb[0], tm[1] * tb[1]);
+    for (int k0 = 0, buf = 0; k0 < kend; k0 += KC, buf ^= 1) {
         double b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) b[i] = bn[i];
@@ -626,7 +646,7 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
             if (i < SA / 2) reinterpret_cast<dvec2*>(sb)[i] = mv[s];
         }
         __syncthreads();
-        if (k0 + KC < Ny) {
+        if (k0 + KC < kend) {
             fetch(k0 + KC);
             load_mat(k0 + KC);
         }
@@ -767,9 +787,8 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     const double* __restrict__ p0 = fo + 2 * ((long)f0 * Ny * M + mcl) + (1 - part);
     const double* __restrict__ p1 = fo + 2 * ((long)f1 * Ny * M + mcl) + part;
     const double* __restrict__ p2 = fo + 2 * ((long)f2 * Ny * M + mcl) + (1 - part);
+    const int nch = yfwd_chunks(nh), yend = nch * KC;
     mfma4d ae[NRT], ao[NRT];
-#pragma unroll
-    for (int rt = 0; rt < NRT; ++rt) ae[rt] = ao[rt] = mfma4d{0.0, 0.0, 0.0, 0.0};
     double dlast = 0.0;
     // Raw values of a chunk, per step: g at the upper point and its mirror,
     // then (divergence forms) uu_c1, then the x and z terms of G. They are
@@ -779,31 +798,49 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     // serialized instead of in flight behind the previous chunk's products.
     constexpr int NR = DIVF ? 8 : 2;
     double rv[NS][NR];
-    auto fetch = [&](int y0) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const int y = min(y0 + 4 * s + lk, nh - 1), ymr = Ny - 1 - y;
-            rv[s][0] = pg[y * rowst];
-            rv[s][1] = pg[ymr * rowst];
-            if (DIVF) {
-                rv[s][2] = p1[y * rowst];
-                rv[s][3] = p1[ymr * rowst];
-                if (XTERM) {
-                    rv[s][4] = p0[y * rowst];
-                    rv[s][5] = p0[ymr * rowst];
-                }
-                if (ZTERM) {
-                    rv[s][6] = p2[y * rowst];
-                    rv[s][7] = p2[ymr * rowst];
-                }
+    auto fetch1 = [&](int y0, double (&r)[NR]) {
+        const int y = min(y0 + lk, nh - 1), ymr = Ny - 1 - y;
+        r[0] = pg[y * rowst];
+        r[1] = pg[ymr * rowst];
+        if (DIVF) {
+            r[2] = p1[y * rowst];
+            r[3] = p1[ymr * rowst];
+            if (XTERM) {
+                r[4] = p0[y * rowst];
+                r[5] = p0[ymr * rowst];
+            }
+            if (ZTERM) {
+                r[6] = p2[y * rowst];
+                r[7] = p2[ymr * rowst];
             }
         }
+    };
+    auto fetch = [&](int y0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) fetch1(y0 + 4 * s, rv[s]);
     };
     // G at a point from its raw values (i: 0 the upper point, 1 its mirror)
     auto gval = [&](const double* r, int i) {
         double G = have_g ? r[i] : 0.0;
         if (DIVF && XTERM) G += ZTERM ? sdx * r[4 + i] + sdz * r[6 + i] : sdx * r[4 + i];
         return G;
+    };
+    // sums and differences of G and H at an upper point and its mirror
+    auto comb = [&](int y, const double (&r)[NR], double& sg, double& dg, double& sh, double& dh) {
+        const int ymr = Ny - 1 - y;
+        double G = 0, Gm = 0, H = 0, Hm = 0;
+        if (mok && y < nh) {
+            G = gval(r, 0);
+            if (DIVF) H = beta * r[2];
+            if (ymr != y) {
+                Gm = gval(r, 1);
+                if (DIVF) Hm = beta * r[3];
+            }
+        }
+        sg = G + Gm;
+        dg = G - Gm;
+        sh = H + Hm;
+        dh = H - Hm;
     };
     dvec2 mv[NST];
     auto mat = [&](int y0) { return gmem(reinterpret_cast<const dvec2*>(ym.fwd + (long)(y0 / KC) * 2 * SM)); };
@@ -812,27 +849,47 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
 #pragma unroll
         for (int s = 0; s < NST; ++s) mv[s] = src[min((int)threadIdx.x + s * 192, SA / 2 - 1)];
     };
+    // the remainder of the contraction, straight from the caches (zero without one)
+    double ta[NMAT][NRT][2], tl[NMAT], rt0[NR];
+#pragma unroll
+    for (int a = 0; a < NMAT; ++a) {
+        tl[a] = 0.0;
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt) ta[a][rt][0] = ta[a][rt][1] = 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) rt0[i] = 0.0;
+    if (yend < nh) {
+        fetch1(yend, rt0);
+#pragma unroll
+        for (int a = 0; a < NMAT; ++a) {
+            const gcdouble tail = gmem(ym.fwd) + (long)nch * 2 * SM + a * yfwd_tail(NRT);
+            tl[a] = tail[2 * 64 * NRT + lk];
+#pragma unroll
+            for (int i = 0; i < 2 * NRT; ++i) ta[a][i >> 1][i & 1] = tail[i * 64 + l];
+        }
+    }
     fetch(0);
     if (DB) load_mat(0);
-    for (int y0 = 0, buf = 0; y0 < nh; y0 += KC, buf ^= DB) {
+    {
+        double sg, dg, sh, dh;
+        comb(yend + lk, rt0, sg, dg, sh, dh);
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt) {
+            ae[rt] = mfma16x16x4(ta[0][rt][0], sg, mfma4d{0.0, 0.0, 0.0, 0.0});
+            ao[rt] = mfma16x16x4(ta[0][rt][1], dg, mfma4d{0.0, 0.0, 0.0, 0.0});
+            if (DIVF) {
+                ae[rt] = mfma16x16x4(ta[NMAT - 1][rt][0], dh, ae[rt]);
+                ao[rt] = mfma16x16x4(ta[NMAT - 1][rt][1], sh, ao[rt]);
+            }
+        }
+        dlast = tl[0] * sg;
+        if (DIVF) dlast = fma(tl[NMAT - 1], dh, dlast);
+    }
+    for (int y0 = 0, buf = 0; y0 < yend; y0 += KC, buf ^= DB) {
         double sg[NS], dg[NS], sh[NS], dh[NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const int y = y0 + 4 * s + lk, ymr = Ny - 1 - y;
-            double G = 0, Gm = 0, H = 0, Hm = 0;
-            if (mok && y < nh) {
-                G = gval(rv[s], 0);
-                if (DIVF) H = beta * rv[s][2];
-                if (ymr != y) {
-                    Gm = gval(rv[s], 1);
-                    if (DIVF) Hm = beta * rv[s][3];
-                }
-            }
-            sg[s] = G + Gm;
-            dg[s] = G - Gm;
-            sh[s] = H + Hm;
-            dh[s] = H - Hm;
-        }
+        for (int s = 0; s < NS; ++s) comb(y0 + 4 * s + lk, rv[s], sg[s], dg[s], sh[s], dh[s]);
         // DB: buffer buf was last read two chunks ago, before every thread
         // passed the previous chunk's barrier
         double* __restrict__ sb = sm + buf * SA;
@@ -848,7 +905,7 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
             for (int i = threadIdx.x; i < SA / 2; i += 192) reinterpret_cast<dvec2*>(sb)[i] = src[i];
         }
         __syncthreads();
-        if (y0 + KC < nh) {
+        if (y0 + KC < yend) {
             fetch(y0 + KC);
             if (DB) load_mat(y0 + KC);
         }

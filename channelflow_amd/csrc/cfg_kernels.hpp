@@ -122,6 +122,22 @@ constexpr int yinv_rows(int cls) { return cls / yinv_split(cls); }
 constexpr int YINV_KC = 16, YFWD_KC = 8;
 constexpr int yinv_tile(int cls) { return (cls * 16 + 1) * (YINV_KC + 1) + 1; }
 constexpr int yfwd_tile(int cls) { return (2 * cls * 16 + 1) * (YFWD_KC + 1) + 1; }
+// Chunks of the contraction (Ny coefficients; nh = (Ny + 1) / 2 upper points). A
+// remainder that fits one matrix-core step (4 coefficients of each parity; 4
+// points) is no chunk of its own: its operand comes from a tail in the lanes'
+// order, [matrix][row tile][parity][lane], then the extra row's 4 per parity. At
+// Ny = 2^a + 1 and 2^a 3 + 1, where the remainder is one, a chunk with its barrier
+// and its zero products was spent on it (inverse / forward, us: 48x35x48 7.8 -> 6.9 /
+// 5.3 -> 4.5, 96^3 14.6 -> 14.4 / 13.9 -> 13.2, 128^3 34.0 -> 32.8 / 19.1 -> 18.2,
+// 192x129x192 64.1 -> 62.8 / 34.4 -> 34.9; 32^3 and 64^3 unchanged).
+constexpr int yinv_chunks(int Ny) {
+    return Ny > YINV_KC && Ny % YINV_KC < YINV_KC / 2 ? Ny / YINV_KC : (Ny + YINV_KC - 1) / YINV_KC;
+}
+constexpr int yfwd_chunks(int nh) {
+    return nh > YFWD_KC && nh % YFWD_KC <= YFWD_KC / 2 ? nh / YFWD_KC : (nh + YFWD_KC - 1) / YFWD_KC;
+}
+constexpr int yinv_tail(int cls) { return 2 * 64 * cls + 8; }  // per matrix
+constexpr int yfwd_tail(int cls) { return 2 * 64 * cls + 4; }
 
 // Per-mode tau data for one lambda_t, mode-major: array k (TAU_NA of them:
 // pband pup pinvd vband vup vinvd Pp Pm vp vm P0 v0) of mode m is the Ny-vector

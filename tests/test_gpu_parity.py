@@ -91,11 +91,13 @@ def test_nonlinear_chebyshev_sizes(gpu, method, Ny):
 
 
 @pytest.mark.parametrize("method", ["Rotational", "Convection", "Divergence", "SkewSymmetric"])
-@pytest.mark.parametrize("Ny", [35, 67, 99, 127, 131, 191, 195, 255])
+@pytest.mark.parametrize("Ny", [35, 37, 55, 57, 67, 99, 127, 131, 191, 195, 255])
 def test_nonlinear_row_tile_edges(gpu, method, Ny):
     """The y transforms at the smallest and largest Ny of their row-tile counts
     (with one and with two blocks per mode group, the middle point alone in the last
-    one's hands), 18 x 10 modes: groups of eight with a remainder. The same 1e-12 bar
+    one's hands) and with the remainders of their contractions on both sides of one
+    matrix-core step (Ny % 16 = 3, 5, 7, 9, 15; (Ny + 1) / 2 % 8 = 0, 2, 3, 4, 5),
+    18 x 10 modes: groups of eight with a remainder. The same 1e-12 bar
     as test_nonlinear_chebyshev_sizes."""
     Nx, Nz = 18, 18
     g = R.Grid(Nx, Ny, Nz, LX_C, LZ_C)
