@@ -8,9 +8,9 @@
 //            U(y), W(y), -Vsuck added to the kx=kz=0 mode;
 //   k_xwinv  inverse x-FFT per (field, y, kz) line, optional d/dx (k_xinv:
 //            LDS FFTs for the lengths the wavefront FFT does not cover);
-//   k_zwave  per (y, x) line: c2r z-FFTs, pointwise products, r2c z-FFTs,
-//            a wavefront per group of lines (k_zpass: LDS FFTs, block-wide,
-//            for the lengths the wavefront FFT does not cover);
+//   k_zsplit per (y, x) line: c2r z-FFTs, pointwise products, r2c z-FFTs,
+//            three wavefronts per group of lines (k_zwave: one; k_zpass: LDS
+//            FFTs, block-wide, for the lengths the wavefront FFT does not cover);
 //   k_xwfwd  forward x-FFT, live kx kept, 1/(Nx Nz) scaling (k_xfwd);
 //   k_yfwd_t values -> Chebyshev coefficients, with the spectral divergence
 //            of u_i u_j folded in for the divergence/skew-symmetric forms.
@@ -1187,7 +1187,8 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
     };
     NLTune out;
     std::vector<NLTune> zc;
-    if (zwave_size(g.Nz)) {  // wavefront z pass: wavefronts per block
+    if (zwave_size(g.Nz) && zsplit(method, g.Nz)) {  // three wavefronts per block
+    } else if (zwave_size(g.Nz)) {                   // wavefront z pass: wavefronts per block
         for (int wb = 1; wb <= 4; wb *= 2) {
             NLTune c;
             c.zwb = wb;

@@ -7,6 +7,22 @@ namespace cfg {
 
 size_t lds_budget();
 
+// Whether a form's wavefront z pass runs a component per wavefront (k_zsplit) or
+// all three in one (k_zwave). The forms with gradients, always: a wavefront then
+// holds a third of the values and runs 4 (convection 3) transforms in a row instead
+// of 11 (8), so twice as many fit a SIMD. us per launch, one wavefront -> three:
+// skew-symmetric 32^3 11.1 -> 6.5, 64^3 14.0 -> 11.2, 96^3 38.8 -> 33.6, 128^3 66.7 ->
+// 63.7, 192x97x192 163 -> 130, 24 of 32^3 27.4 -> 22.4, 24 of 48^3 73 -> 67, 16 of
+// 64^3 100 -> 96; convection 24 of 32^3 22.0 -> 18.8, 96^3 29.6 -> 25.6, 128^3 49.3 ->
+// 48.0, 192x97x192 94 -> 75. The rotational and the divergence form have few
+// transforms to share out (the divergence form one more than alone): rotational
+// 16x33x32 4.5 -> 3.7, 32^3 5.9 -> 4.5, 24 of them 13.9 -> 14.1, but 16 of 48^3 20.7
+// -> 23.3, 16 of 64^3 43 -> 46, 192x129x192 62 -> 68; divergence 16 of 24x33x24 8.9 ->
+// 8.6, but 24 of 32^3 13.1 -> 16.6, 16 of 64^3 45 -> 83. The rule looks at the grid
+// alone: a member's result must not depend on which instance its batch runs.
+constexpr bool zsplit(int method, int nz) {
+    return method == NL_CONV || method == NL_SKEW || nz <= (method == NL_ROT ? 32 : 24);
+}
 // real physical lines per (y, x) line the LDS z-pass of a form keeps
 int zpass_nphys(int method);
 // largest LDS z-pass lines per block that fit the LDS budget

@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
             if (SK) pb[w] = u0[w] * u2[w];
         }
         __syncthreads();
-        // skew-symmetric: f0 + i kz u0u2 / 2 and u0u2 (the layout of k_zwave)
+        // skew-symmetric: f0 + i kz u0u2 / 2 and u0u2 (the layout of k_zsplit)
         zr2c_pair<NZ>(c, zo, 5, 0, SK ? 4 : -1, SK ? 5 : -1, SK ? 0.5 : 0.0);
         zc2r_pair<NZ>(c, xp, 7, false, 3, 4, false, 4);  // dv/dx, dv/dy
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
@@ -288,9 +288,9 @@ __device__ __forceinline__ Bins zw_bins(const ZWCtx& c) {
 // c2r of two real fields at once (fa -> pa, fb -> pb; fb < 0: none), from the
 // live bins kz < nkz of xp; dza / dzb apply d/dz. As in FFTW's c2r, the
 // imaginary part of bin 0 is ignored.
-template <class S>
+template <class S, class Then>
 __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
-                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV]) {
+                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV], Then&& issued) {
     constexpr int SL = S::SL, SV = S::SV, PV = S::PV;
     const int s = c.gi;
     // Value r of lane s is bin n = s + SL r. In the lower half of the r it can
@@ -311,6 +311,7 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
     };
     fetch(fa, A);
     if (fb >= 0) fetch(fb, B);
+    issued();
     double2 v[SV];
     const double sd = s;
 #pragma unroll
@@ -334,6 +335,12 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
         pa[m] = u[m].x;
         pb[m] = u[m].y;
     }
+}
+
+template <class S>
+__device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
+                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV]) {
+    zw_c2r<S>(c, xp, fa, dza, fb, dzb, pa, pb, [] {});
 }
 
 // r2c of pa (and pb when TWO) -> zo fields ga (and gb), bins kz < nkz.
@@ -387,22 +394,22 @@ __device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo,
 // launch, two steps -> three: one 96^3 skew-symmetric field 59 -> 44, 128^3
 // convection 92 -> 70, rotational 49 -> 35, 192x129x192 rotational 95 -> 76,
 // 256x33x256 52 -> 48, 64x49x162 skew-symmetric 61 -> 32, 8 members of 32x49x72
-// 72 -> 53. At 48 and 64, where 2 wavefronts fit anyway, the second transpose
+// 72 -> 53; with a component per wavefront (k_zsplit) 96^3 skew-symmetric 37 -> 34,
+// 128^3 convection 62 -> 52. At 48 and 64, where 2 wavefronts fit anyway, the second transpose
 // costs more than it gives in a batch (16 of 64^3 113 -> 127, 24 of 48^3 82 -> 88).
 constexpr bool zwave_three(int nz) { return nz == 72 || nz >= 96; }
 template <int NZ>
 using ZLine = std::conditional_t<zwave_three(NZ), ZW3<NZ>, ZW<NZ>>;
 
-// The z pass of k_zpass with one wavefront per 64/G lines (same fields, same
-// products in the same order). A block is independent wavefronts, any number up
-// to 4 (LDS sized at launch). Every access is at a field's uniform base, one of
-// two 32-bit lane offsets and a constant distance: with 64-bit addresses and the
-// bin tests formed per access the kernel was bound by those instructions. us per
-// launch, before -> after: one 128^3 convection field 70 -> 50, rotational 35 ->
-// 32, 96^3 skew-symmetric 44 -> 39, 192x129x192 rotational 76 -> 64, 24 members of
-// 48^3 skew-symmetric 83 -> 71, of 32^3 32 -> 29. A form that staged its inputs in
-// LDS one transform ahead is slower than this one at every length (16 members of
-// 64^3 skew-symmetric 108 against 99, rotational 52 against 42).
+// The z pass of k_zpass for the rotational and the divergence form, one wavefront
+// per 64/G lines (same fields, same products in the same order). A block is
+// independent wavefronts, any number up to 4 (LDS sized at launch). Every access is
+// at a field's uniform base, one of two 32-bit lane offsets and a constant distance:
+// with 64-bit addresses and the bin tests formed per access the kernel was bound by
+// those instructions. us per launch, before -> after: rotational 128^3 35 -> 32,
+// 192x129x192 76 -> 64 (228 MB, 3.6 TB/s). A form that staged its inputs in LDS one
+// transform ahead is slower than this one at every length (16 members of 64^3
+// rotational 52 against 42).
 template <int METHOD, int NZ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8)))
 k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ tab,
@@ -452,82 +459,6 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         }
         zw_r2c<S, true>(c, zo, f0, f1, 0, 1);
         zw_r2c<S, false>(c, zo, f2, f2, 2, -1);
-    } else if constexpr (METHOD == NL_CONV || METHOD == NL_SKEW) {
-        // f_i = sum_j (s u_j) du_i/dx_j, terms added in the order j = x, y, z
-        // (diffops.cpp:3192-3199, 3626-3633). The skew-symmetric form keeps
-        // h = u/2 only: halving is exact, so s u_j is h_j, u_j is 2 h_j and
-        // u_i u_j is 4 (h_i h_j), all with the bits of the unscaled products.
-        //
-        // Skew-symmetric outputs: the z-derivative part of div(u u)/2
-        // (diffops.cpp:3254-3279) is added here, in z-spectral space:
-        // field i = f_i + 1/2 i kz (u_i u_z) (i = 0, 1, 2), then u_0u_0, u_0u_1,
-        // u_0u_2, u_1u_1, u_1u_2 in fields 3-7; u_2u_2 is needed only for that
-        // z-derivative and never leaves. The forward transforms add the x and y
-        // parts of the divergence.
-        constexpr bool SK = (METHOD == NL_SKEW);
-        constexpr double s = SK ? 0.5 : 1.0, us = SK ? 2.0 : 1.0;
-        double h0[N1], h1[N1], h2[N1], pa[N1], pb[N1], fa[N1], fb[N1];
-        zw_c2r<S>(c, xp, 0, false, 1, false, h0, h1);   // u, v
-        zw_c2r<S>(c, xp, 2, false, 6, false, h2, pa);   // w, du/dx
-        if constexpr (SK) {
-#pragma unroll
-            for (int m = 0; m < N1; ++m) {
-                h0[m] *= s;
-                h1[m] *= s;
-                h2[m] *= s;
-            }
-        }
-#pragma unroll
-        for (int m = 0; m < N1; ++m) fa[m] = 0.0 + h0[m] * pa[m];
-        zw_c2r<S>(c, xp, 3, false, 0, true, pa, pb);    // du/dy, du/dz
-#pragma unroll
-        for (int m = 0; m < N1; ++m) {
-            fa[m] += h1[m] * pa[m];
-            fa[m] += h2[m] * pb[m];
-            if (rotation != 0.0) fa[m] -= rotation * (us * h1[m]);  // nse.cpp:61-80
-            if (SK) pb[m] = 4.0 * (h0[m] * h2[m]);
-        }
-        if constexpr (SK) zw_r2c<S, true>(c, zo, fa, pb, 0, 5, 0.5);  // f0 + i kz u0u2 / 2, and u0u2
-        else zw_r2c<S, false>(c, zo, fa, pb, 0, -1);                  // f0
-        zw_c2r<S>(c, xp, 7, false, 4, false, pa, pb);   // dv/dx, dv/dy
-#pragma unroll
-        for (int m = 0; m < N1; ++m) {
-            fa[m] = 0.0 + h0[m] * pa[m];
-            fa[m] += h1[m] * pb[m];
-        }
-        zw_c2r<S>(c, xp, 1, true, 8, false, pa, pb);    // dv/dz, dw/dx
-#pragma unroll
-        for (int m = 0; m < N1; ++m) {
-            fa[m] += h2[m] * pa[m];
-            if (rotation != 0.0) fa[m] += rotation * (us * h0[m]);
-            fb[m] = 0.0 + h0[m] * pb[m];
-        }
-        zw_c2r<S>(c, xp, 5, false, 2, true, pa, pb);    // dw/dy, dw/dz
-#pragma unroll
-        for (int m = 0; m < N1; ++m) {
-            fb[m] += h1[m] * pa[m];
-            fb[m] += h2[m] * pb[m];
-        }
-        if constexpr (SK) {
-#pragma unroll
-            for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h1[m] * h2[m]);
-            zw_r2c<S, true>(c, zo, fa, pa, 1, 7, 0.5);   // f1 + i kz u1u2 / 2, and u1u2
-#pragma unroll
-            for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h2[m] * h2[m]);
-            zw_r2c<S, true>(c, zo, fb, pa, 2, -1, 0.5);  // f2 + i kz u2u2 / 2
-            // remaining entries of outer(u, u) (diffops.cpp:2336-2388)
-#pragma unroll
-            for (int m = 0; m < N1; ++m) {
-                pa[m] = 4.0 * (h0[m] * h0[m]);
-                pb[m] = 4.0 * (h0[m] * h1[m]);
-            }
-            zw_r2c<S, true>(c, zo, pa, pb, 3, 4);
-#pragma unroll
-            for (int m = 0; m < N1; ++m) pa[m] = 4.0 * (h1[m] * h1[m]);
-            zw_r2c<S, false>(c, zo, pa, pa, 6, -1);
-        } else {
-            zw_r2c<S, true>(c, zo, fa, fb, 1, 2);            // f1, f2
-        }
     } else {
         double u0[N1], u1[N1], u2[N1], pa[N1], pb[N1];
         zw_c2r<S>(c, xp, 0, false, 1, false, u0, u1);
@@ -565,6 +496,174 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
     }
 }
 
+// The z pass of 64/G lines by three wavefronts, one per velocity component (zsplit:
+// where, and what it measured). Wavefront c transforms u_c and what belongs to it (its
+// gradient, or the vorticity component w_c), hands the velocity (and w) to the other
+// two through LDS and forms its part of the products. Each wavefront's transforms are
+// a serial chain through LDS, so what bounds the pass is how many wavefronts a SIMD
+// holds: 32 bins take 126 registers here against 180 in one wavefront, 64 bins 162
+// against 238, 192 bins 116 against 200. The shared values lie in the wavefronts'
+// line rows, which are free between the inverse and the forward transforms; in space
+// of their own they cost a third of the occupancy (rotational 192x129x192 93 against
+// 76 us). The first bins are requested before the twiddles are waited for. Two such
+// groups of lines per block, or blocks in XCD order, are slower (16 of 64^3 100 ->
+// 115, 107; the chain of barriers couples six wavefronts).
+// LDS of a block: the twiddles, then the line rows of the three wavefronts, which also carry the shared values
+template <int METHOD, int NZ>
+constexpr size_t zsplit_lds() {
+    using S = ZLine<NZ>;
+    const size_t rows = (size_t)3 * S::LPW * S::LBUF * sizeof(double2);
+    const size_t shared = (size_t)(METHOD == NL_ROT ? 6 : 3) * S::PV * 64 * sizeof(double);
+    return NZ * sizeof(double2) + (rows > shared ? rows : shared);
+}
+template <int METHOD, int NZ>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(1, 8)))
+k_zsplit(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ tab, int want_g,
+         const double2* __restrict__ xp0, double2* __restrict__ zo0, long sx) {
+    using S = ZLine<NZ>;
+    constexpr int PV = S::PV;
+    extern __shared__ double2 lds[];
+    double2* const T_l = lds + NZ;
+    double* const ex = reinterpret_cast<double*>(T_l);  // [shared field][value][lane]
+    constexpr int NTW = (NZ + 191) / 192;
+    dvec2 twr[NTW];
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) twr[i] = gmem(reinterpret_cast<const dvec2*>(twg))[min((int)threadIdx.x + 192 * i, NZ - 1)];
+    auto twiddles = [&] {  // behind the first loads of bins
+#pragma unroll
+        for (int i = 0; i < NTW; ++i)
+            if ((int)threadIdx.x + 192 * i < NZ) reinterpret_cast<dvec2*>(lds)[threadIdx.x + 192 * i] = twr[i];
+        __syncthreads();
+    };
+    const int cc = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int nxc = (g.Nx + S::LPW - 1) / S::LPW;
+    const int y = blockIdx.x / nxc;
+    const int L = lane / S::G;
+    const int x = (blockIdx.x - y * nxc) * S::LPW + L;
+    ZWCtx c;
+    c.gi = lane % S::G;
+    c.line_ok = x < g.Nx;
+    c.base = ((long)y * g.Nx + (c.line_ok ? x : 0)) * g.nkz;
+    c.fsz = (long)g.Ny * g.Nx * g.nkz;
+    c.nkz = g.nkz;
+    c.dk = 2 * PI / g.Lz;
+    c.T = T_l + (cc * S::LPW + L) * S::LBUF;
+    c.tw = lds;
+    const double rotation = tab[blockIdx.y].rotation;
+    const double2* __restrict__ xp = xp0 + blockIdx.y * sx;
+    double2* __restrict__ zo = zo0 + blockIdx.y * sx;
+    auto share = [&](int f, const double (&v)[PV]) {
+#pragma unroll
+        for (int m = 0; m < PV; ++m) ex[(f * PV + m) * 64 + lane] = v[m];
+    };
+    auto get = [&](int f, int m) { return ex[(f * PV + m) * 64 + lane]; };
+    if constexpr (METHOD == NL_ROT) {
+        double u[PV], w[PV];
+        zw_c2r<S>(c, xp, cc, false, 3 + cc, false, u, w, twiddles);
+        __syncthreads();
+        share(cc, u);
+        share(3 + cc, w);
+        __syncthreads();
+        // cross(vort, u) (diffops.cpp:2598-2605): wavefront 0 takes f0 and f1, 2 takes f2
+#pragma unroll
+        for (int m = 0; m < PV; ++m) {
+            if (cc == 0) {
+                const double a0 = get(0, m), a1 = get(1, m), a2 = get(2, m);
+                const double b0 = get(3, m), b1 = get(4, m), b2 = get(5, m);
+                u[m] = b1 * a2 - b2 * a1;
+                w[m] = b2 * a0 - b0 * a2;
+                if (rotation != 0.0) {  // nse.cpp:61-80
+                    u[m] -= rotation * a1;
+                    w[m] += rotation * a0;
+                }
+            } else if (cc == 2) {
+                u[m] = get(3, m) * get(1, m) - get(4, m) * get(0, m);
+            }
+        }
+        __syncthreads();
+        if (cc == 0) zw_r2c<S, true>(c, zo, u, w, 0, 1);
+        else if (cc == 2) zw_r2c<S, false>(c, zo, u, u, 2, -1);
+    } else if constexpr (METHOD == NL_CONV || METHOD == NL_SKEW) {
+        // f_i = sum_j (s u_j) du_i/dx_j, terms added in the order j = x, y, z
+        // (diffops.cpp:3192-3199, 3626-3633). The skew-symmetric form shares
+        // h = u/2: halving is exact, so s u_j is h_j, u_j is 2 h_j and u_i u_j is
+        // 4 (h_i h_j), all with the bits of the unscaled products.
+        //
+        // Skew-symmetric outputs: the z-derivative part of div(u u)/2
+        // (diffops.cpp:3254-3279) is added here, in z-spectral space:
+        // field i = f_i + 1/2 i kz (u_i u_z) (i = 0, 1, 2), then u_0u_0, u_0u_1,
+        // u_0u_2, u_1u_1, u_1u_2 in fields 3-7; u_2u_2 is needed only for that
+        // z-derivative and never leaves. The forward transforms add the x and y
+        // parts of the divergence.
+        constexpr bool SK = (METHOD == NL_SKEW);
+        constexpr double s = SK ? 0.5 : 1.0, us = SK ? 2.0 : 1.0;
+        double h[PV], dx[PV], dy[PV], dz[PV], f[PV];
+        zw_c2r<S>(c, xp, cc, false, 6 + cc, false, h, dx, twiddles);
+        zw_c2r<S>(c, xp, 3 + cc, false, cc, true, dy, dz);
+        if constexpr (SK) {
+#pragma unroll
+            for (int m = 0; m < PV; ++m) h[m] *= s;
+        }
+        __syncthreads();
+        share(cc, h);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < PV; ++m) {
+            const double h0 = get(0, m), h1 = get(1, m), h2 = get(2, m);
+            f[m] = 0.0 + h0 * dx[m];
+            f[m] += h1 * dy[m];
+            f[m] += h2 * dz[m];
+            if (rotation != 0.0) {  // nse.cpp:61-80
+                if (cc == 0) f[m] -= rotation * (us * h1);
+                if (cc == 1) f[m] += rotation * (us * h0);
+            }
+            if constexpr (SK) {  // u_i u_z; u_0u_0 and u_0u_1, or u_1u_1 (diffops.cpp:2336-2388)
+                dx[m] = 4.0 * (h[m] * h2);
+                dy[m] = 4.0 * (h[m] * h[m]);
+                dz[m] = cc == 0 ? 4.0 * (h0 * h1) : 0.0;
+            }
+        }
+        __syncthreads();
+        if constexpr (SK) {
+            zw_r2c<S, true>(c, zo, f, dx, cc, cc == 0 ? 5 : cc == 1 ? 7 : -1, 0.5);
+            if (cc < 2) zw_r2c<S, true>(c, zo, dy, dz, cc == 0 ? 3 : 6, cc == 0 ? 4 : -1);
+        } else {
+            // f0 and f1 in one transform of wavefront 0, f2 in one of wavefront 2
+            double* const hand = reinterpret_cast<double*>(T_l + S::LPW * S::LBUF) + lane;  // wavefront 1's rows
+            if (cc == 1) {
+#pragma unroll
+                for (int m = 0; m < PV; ++m) hand[64 * m] = f[m];
+            }
+            __syncthreads();
+            if (cc == 0) {
+#pragma unroll
+                for (int m = 0; m < PV; ++m) dx[m] = hand[64 * m];
+                zw_r2c<S, true>(c, zo, f, dx, 0, 1);
+            } else if (cc == 2) {
+                zw_r2c<S, false>(c, zo, f, f, 2, -1);
+            }
+        }
+    } else {
+        double u[PV], pa[PV], pb[PV], ga[PV], gb[PV];
+        zw_c2r<S>(c, xp, cc, false, -1, false, u, pa, twiddles);
+        __syncthreads();
+        share(cc, u);
+        __syncthreads();
+        // outer(u, u) (diffops.cpp:2336-2388): 00 01, 02 11, 12 22; with rotation g, the rotation terms only
+        const int i0 = cc == 2 ? 1 : 0, j0 = cc == 0 ? 0 : 2, i1 = cc == 0 ? 0 : cc, j1 = cc == 2 ? 2 : 1;
+#pragma unroll
+        for (int m = 0; m < PV; ++m) {
+            pa[m] = get(i0, m) * get(j0, m);
+            pb[m] = get(i1, m) * get(j1, m);
+            ga[m] = cc == 0 ? -(rotation * get(1, m)) : 0.0;
+            gb[m] = cc == 0 ? rotation * get(0, m) : 0.0;
+        }
+        __syncthreads();
+        if (want_g && cc < 2) zw_r2c<S, true>(c, zo, ga, gb, cc == 0 ? 0 : 2, cc == 0 ? 1 : -1);
+        zw_r2c<S, true>(c, zo, pa, pb, 3 + 2 * cc, 4 + 2 * cc);
+    }
+}
+
 int zpass_xb(const Geom& g, int nphys, const NLTune& tn);
 
 template <int METHOD, int NZ>
@@ -573,11 +672,17 @@ void launch_z_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, in
     if constexpr (zwave_size(NZ)) {
         using S = ZLine<NZ>;
         const long waves = (long)g.Ny * ((g.Nx + S::LPW - 1) / S::LPW);
-        const int wb = tn.zwb > 0 ? tn.zwb : 4;
-        const size_t lds = (size_t)(NZ + wb * S::LPW * S::LBUF) * sizeof(double2);
-        const dim3 grid((unsigned)((waves + wb - 1) / wb), n);
-        allow_lds(k_zwave<METHOD, NZ>, lds);
-        k_zwave<METHOD, NZ><<<grid, 64 * wb, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
+        if constexpr (zsplit(METHOD, NZ)) {
+            constexpr size_t lds = zsplit_lds<METHOD, NZ>();
+            allow_lds(k_zsplit<METHOD, NZ>, lds);
+            k_zsplit<METHOD, NZ><<<dim3((unsigned)waves, n), 192, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
+        } else {
+            const int wb = tn.zwb > 0 ? tn.zwb : 4;
+            const size_t lds = (size_t)(NZ + wb * S::LPW * S::LBUF) * sizeof(double2);
+            const dim3 grid((unsigned)((waves + wb - 1) / wb), n);
+            allow_lds(k_zwave<METHOD, NZ>, lds);
+            k_zwave<METHOD, NZ><<<grid, 64 * wb, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
+        }
     } else {
         const int nphys = zpass_nphys(METHOD);
         const int XB = zpass_xb(g, nphys, tn);

@@ -130,6 +130,25 @@ def test_nonlinear_ragged_lengths(gpu, method, N):
         assert np.all(e <= 1e-12), e
 
 
+@pytest.mark.parametrize("method", ["Rotational", "Convection", "Divergence", "SkewSymmetric"])
+@pytest.mark.parametrize("grid", [(12, 9, 16), (12, 9, 24), (6, 9, 32), (12, 9, 36), (4, 9, 96), (6, 9, 192)])
+def test_nonlinear_component_wavefronts(gpu, method, grid):
+    """One NL call with suction and, where the form has it, rotation on both sides of the lengths up to
+    which the rotational (32) and the divergence form (24) run a velocity component
+    per wavefront, with line counts that do not fill the last group; the same 1e-12
+    bar as test_nonlinear_single_call."""
+    Nx, Ny, Nz = grid
+    g = R.Grid(Nx, Ny, Nz, LX_C, LZ_C)
+    u = random_field(Nx, Ny, Nz, LX_C, LZ_C, norm=1.0, decay=0.7, seed=Nz, dealias=False)
+    fl = dict(nonlinearity=method, dealiasing="NoDealiasing", baseflow="LaminarBase", ulowerwall=-1.0, uupperwall=1.0,
+              nu=1 / 400, rotation=0.3 if method in ("Rotational", "SkewSymmetric") else 0.0, Vsuck=0.1)
+    f_ref, _ = R.nonlinear(g, R.make_flags(**fl), u)
+    f_gpu = cfa.nonlinear(cfa.FlowField(Nx, Ny, Nz, 3, LX_C, LZ_C, data=u), cfa.DNSFlags(**fl))
+    e = rel_l2_per_component(g, f_gpu, f_ref)
+    print(method, grid, "rel L2", e, flush=True)
+    assert np.all(e <= 1e-12), e
+
+
 @pytest.mark.parametrize("constraint", ["PressureGradient", "BulkVelocity"])
 @pytest.mark.parametrize("taucorr", [True, False])
 @pytest.mark.parametrize("grid", [(16, 33, 16), (8, 25, 8), (8, 65, 8), (8, 97, 8), (8, 129, 8), (6, 193, 6),
