@@ -587,108 +587,150 @@ void launch_tau_solve(const Geom& g, const double* hb, int n, const TauMember* t
 }
 
 // ===========================================================================
-// NSE::linear on live modes (nse.cpp:393-477), one thread per mode
+// NSE::linear on live modes (nse.cpp:393-477)
 // ===========================================================================
-// NSE::linear (nse.cpp:393-477) with one W-lane segment of a wavefront per
-// mode, MPB modes per block, member blockIdx.y: for each velocity component
-// L = nu (u'' - kappa^2 u) - grad q, plus on kx = kz = 0 nu U'', nu W'' and
-// the mean pressure gradient (the bulk-velocity branch takes dPdx from
-// nu (du/dy(b) - du/dy(a)) / Ly, nse.cpp:437-472). Real and imaginary parts
-// share each derivative scan.
+// For each velocity component L = nu (u'' - kappa^2 u) - grad q, plus on kx = kz = 0
+// nu U'', nu W'' and the mean pressure gradient (the bulk-velocity branch takes dPdx
+// from nu (du/dy(b) - du/dy(a)) / Ly, nse.cpp:437-472). The real parts couple as in
+// the tau solve, (v, q real; u, w imaginary) and (v, q imaginary; u, w real), and
+// each set runs on its own W-lane segment; MPB modes per block, member blockIdx.y.
+//
+// What bounds it: for one field the latency of a block, for a batch HBM. The rows of
+// a block's modes are staged in LDS with MPB consecutive modes per access; loaded by
+// the segments themselves, whose lanes are rows apart, every 8 bytes were a request
+// of their own. us per launch, before -> after: one 32^3 field 9.0 -> 5.4, 54x57x72
+// 11.5 -> 6.4, 64^3 10.6 -> 7.9, 96^3 16.7 -> 10.3, 128^3 22.9 -> 18.5, 192x129x192
+// 57.8 -> 36.7 (177 MB, 4.8 TB/s), 48x193x48 17.0 -> 11.3, 16 of 48^3 16.4 -> 14.3, 16
+// of 64^3 39.3 -> 36.0.
 template <int K, int W, int MPB>
-__global__ void __launch_bounds__(W * MPB) k_linear_wave(Geom g, const LinearMember* __restrict__ tab) {
+__global__ void __launch_bounds__(2 * W * MPB) k_linear_wave(Geom g, const LinearMember* __restrict__ tab) {
+    extern __shared__ double2 lds2[];
+    double* const lds = reinterpret_cast<double*>(lds2);  // [mode][part][u v w q] of tau_pitch(Ny)
+    constexpr int nthr = 2 * W * MPB, step = nthr / MPB, UNR = 8;
     const LinearMember& me = tab[blockIdx.y];
-    const int m = blockIdx.x * MPB + threadIdx.x / W;
-    if (m >= g.M) return;  // whole segments leave together
     const double nu = me.nu;
     const LinearConst lc = me.c;
-    const gcdouble u = gmem(me.u), q = gmem(me.q);
-    __attribute__((address_space(1))) double* out = gmem_w(me.out);
-    const int Ny = g.Ny;
-    WCtx c;
-    c.N = Ny;
-    c.Me = (Ny + 1) / 2;
-    c.Mo = (Ny - 1) / 2;
-    c.Nb = Ny - 1;
-    c.Nc = Ny - 1;
-    c.lane = threadIdx.x % W;
-    c.L = g.b - g.a;
-    c.hb = nullptr;
-    const int ikx = m % g.nkx, kz = m / g.nkx, kx = kx_of(g, ikx);
-    const bool zero = kx == 0 && kz == 0;
-    const double kappa2 = 4 * PI * PI * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
-    const long rs = 2L * g.M;  // doubles between consecutive Chebyshev rows
-    auto row0 = [&](int comp) { return 2L * ((long)comp * Ny * g.M + m); };
-    WV<K> Pq[2] = {wload_s<K, W>(q + row0(0), rs, c), wload_s<K, W>(q + row0(0) + 1, rs, c)};
-    double dPd[3] = {0.0, 0.0, 0.0};
+    const int Ny = g.Ny, RP = tau_pitch(Ny), nrow = 4 * Ny;
+    const int m0 = blockIdx.x * MPB;
+    const int ww = threadIdx.x % MPB, mm = m0 + ww;
+    // part 0 takes v.re, q.re, u.im, w.im; part 1 v.im, q.im, u.re, w.re
+    auto slot = [&](int pt, int comp, int n) { return ((ww * 2 + pt) * 4 + comp) * RP + n; };
+    auto comp_of = [&](int row) { return (row >= Ny) + (row >= 2 * Ny) + (row >= 3 * Ny); };
+    {
+        const auto u = gmem(reinterpret_cast<const dvec2*>(me.u));
+        const auto q = gmem(reinterpret_cast<const dvec2*>(me.q));
+        const int mc = min(mm, g.M - 1);  // slots past the last mode repeat it
+        for (int row = threadIdx.x / MPB; row < nrow; row += UNR * step) {
+            dvec2 v[UNR];
 #pragma unroll
-    for (int comp = 0; comp < 3; ++comp) {
-        WV<K> s0[2] = {wload_s<K, W>(u + row0(comp), rs, c), wload_s<K, W>(u + row0(comp) + 1, rs, c)};
-        for (int p = 0; p < 2; ++p)
-            for (int k = 0; k < K; ++k) {
-                s0[p].e[k] *= nu;  // nu u
-                s0[p].o[k] *= nu;
+            for (int r = 0; r < UNR; ++r) {
+                const int rr = min(row + r * step, nrow - 1);
+                v[r] = rr < 3 * Ny ? u[(long)rr * g.M + mc] : q[(long)(rr - 3 * Ny) * g.M + mc];
             }
-        WV<K> s1[2], s2[2];
-        wdiff_n<K, W, 2>(s0, c, s1);
-        if (zero && lc.bulk && comp != 1) {
-            double eb, ea;
-            wends<K, W>(s1[0], c, eb, ea);
-            dPd[comp] = (eb - ea) / c.L;
+#pragma unroll
+            for (int r = 0; r < UNR; ++r) {
+                const int rr = row + r * step, comp = comp_of(rr), n = rr - comp * Ny;
+                if (rr >= nrow) continue;
+                const bool odd = comp & 1;  // v, q
+                lds[slot(0, comp, n)] = odd ? v[r].x : v[r].y;
+                lds[slot(1, comp, n)] = odd ? v[r].y : v[r].x;
+            }
         }
-        wdiff_n<K, W, 2>(s1, c, s2);  // nu u''
-        WV<K> o[2];
-        for (int p = 0; p < 2; ++p)
+    }
+    const int seg = threadIdx.x / W;
+    for (int i = threadIdx.x; i < 2 * MPB * 4; i += nthr) lds[i * RP + Ny] = 0.0;  // the rows' padding
+    __syncthreads();
+    {
+        WCtx c;
+        c.N = Ny;
+        c.Me = (Ny + 1) / 2;
+        c.Mo = (Ny - 1) / 2;
+        c.Nb = Ny - 1;
+        c.Nc = Ny - 1;
+        c.lane = threadIdx.x % W;
+        c.L = g.b - g.a;
+        c.hb = nullptr;
+        const int m = min(m0 + (seg >> 1), g.M - 1), part = seg & 1;
+        const int ikx = m % g.nkx, kz = m / g.nkx, kx = kx_of(g, ikx);
+        const bool mean = kx == 0 && kz == 0 && part == 1;  // the mean flow's real parts
+        const double kappa2 = 4 * PI * PI * ((kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz));
+        const double sgn = part ? 1.0 : -1.0;
+        double* const R = lds + seg * 4 * RP;
+        const WV<K> Pq = wrow_load<K, W>(R + 3 * RP, c);
+        WV<K> s0[3], s1[3], s2[3];
+#pragma unroll
+        for (int comp = 0; comp < 3; ++comp) {
+            s0[comp] = wrow_load<K, W>(R + comp * RP, c);
+#pragma unroll
             for (int k = 0; k < K; ++k) {
-                o[p].e[k] = s2[p].e[k] - kappa2 * s0[p].e[k];
-                o[p].o[k] = s2[p].o[k] - kappa2 * s0[p].o[k];
+                s0[comp].e[k] *= nu;
+                s0[comp].o[k] *= nu;
             }
-        if (comp == 1) {  // - dq/dy
-            WV<K> dq[2];
-            wdiff_n<K, W, 2>(Pq, c, dq);
-            for (int p = 0; p < 2; ++p)
+        }
+        wdiff_n<K, W, 3>(s0, c, s1);
+        double dPd[3] = {0.0, 0.0, 0.0};
+        if (mean && lc.bulk) {
+            double eb[3], ea[3];
+            wends_n<K, W, 3>(s1, c, eb, ea);
+            for (int comp = 0; comp < 3; comp += 2) dPd[comp] = (eb[comp] - ea[comp]) / c.L;
+        }
+        wdiff_n<K, W, 3>(s1, c, s2);  // nu u''
+        WV<K> p1[1] = {Pq}, dq[1];
+        wdiff_n<K, W, 1>(p1, c, dq);
+#pragma unroll
+        for (int comp = 0; comp < 3; ++comp) {
+            // dq/dy; i k q: the real part of u meets -k q.im, the imaginary part k q.re
+            const double d = sgn * (comp == 0 ? 2 * PI * kx / g.Lx : 2 * PI * kz / g.Lz);
+            WV<K> o;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                o.e[k] = s2[comp].e[k] - kappa2 * s0[comp].e[k];
+                o.o[k] = s2[comp].o[k] - kappa2 * s0[comp].o[k];
+                o.e[k] += comp == 1 ? -dq[0].e[k] : d * Pq.e[k];
+                o.o[k] += comp == 1 ? -dq[0].o[k] : d * Pq.o[k];
+            }
+            if (mean && comp != 1) {
+                const WV<K> base = wload<K, W>(gmem(comp == 0 ? lc.nuUbaseyy : lc.nuWbaseyy), c);
                 for (int k = 0; k < K; ++k) {
-                    o[p].e[k] = o[p].e[k] - dq[p].e[k];
-                    o[p].o[k] = o[p].o[k] - dq[p].o[k];
+                    o.e[k] += base.e[k];
+                    o.o[k] += base.o[k];
                 }
-        } else {  // - (i k) q: (0, d) * (Pr, Pi) = (-(d Pi), d Pr)
-            const double d = comp == 0 ? 2 * PI * kx / g.Lx : 2 * PI * kz / g.Lz;
-            for (int k = 0; k < K; ++k) {
-                o[0].e[k] = o[0].e[k] - (0.0 * Pq[0].e[k] - d * Pq[1].e[k]);
-                o[0].o[k] = o[0].o[k] - (0.0 * Pq[0].o[k] - d * Pq[1].o[k]);
-                o[1].e[k] = o[1].e[k] - (0.0 * Pq[1].e[k] + d * Pq[0].e[k]);
-                o[1].o[k] = o[1].o[k] - (0.0 * Pq[1].o[k] + d * Pq[0].o[k]);
+                if (c.lane == 0) {
+                    if (!lc.bulk) o.e[0] -= comp == 0 ? lc.dPdxRef : lc.dPdzRef;
+                    else o.e[0] -= dPd[comp] + (comp == 0 ? lc.nuUbase_slope : lc.nuWbase_slope);
+                }
             }
+            wrow_store<K, W>(R + comp * RP, c, o);  // the rows are this segment's alone
         }
-        if (zero && comp != 1) {
-            const WV<K> base = wload<K, W>(gmem(comp == 0 ? lc.nuUbaseyy : lc.nuWbaseyy), c);
-            for (int k = 0; k < K; ++k) {
-                o[0].e[k] += base.e[k];
-                o[0].o[k] += base.o[k];
-            }
-            if (c.lane == 0) {
-                if (!lc.bulk) o[0].e[0] -= comp == 0 ? lc.dPdxRef : lc.dPdzRef;
-                else o[0].e[0] -= dPd[comp] + (comp == 0 ? lc.nuUbase_slope : lc.nuWbase_slope);
-            }
-        }
-        wstore_s<K, W>(out + row0(comp), rs, o[0], c);
-        wstore_s<K, W>(out + row0(comp) + 1, rs, o[1], c);
+    }
+    __syncthreads();
+    if (mm >= g.M) return;
+    const auto out = gmem_w(reinterpret_cast<dvec2*>(me.out));
+    for (int row = threadIdx.x / MPB; row < 3 * Ny; row += step) {
+        const int comp = comp_of(row), n = row - comp * Ny;
+        const double a = lds[slot(0, comp, n)], b = lds[slot(1, comp, n)];
+        out[(long)row * g.M + mm] = comp == 1 ? dvec2{a, b} : dvec2{b, a};
     }
 }
 
 void launch_linear(const Geom& g, int n, const LinearMember* tab, hipStream_t st) {
     const int Me = (g.Ny + 1) / 2;
-    auto go = [&](auto kern, int w) {
-        const int mpb = 256 / w;
-        kern<<<dim3((g.M + mpb - 1) / mpb, n), 256, 0, st>>>(g, tab);
+    auto go = [&](auto kern, int w, int mpb) {
+        const size_t lds = (size_t)mpb * 8 * tau_pitch(g.Ny) * sizeof(double);
+        allow_lds(kern, lds);
+        kern<<<dim3((g.M + mpb - 1) / mpb, n), 2 * w * mpb, lds, st>>>(g, tab);
     };
-    if (Me <= 16) go(k_linear_wave<1, 16, 16>, 16);
-    else if (Me <= 32) go(k_linear_wave<2, 16, 16>, 16);
-    else if (Me <= 48) go(k_linear_wave<3, 16, 16>, 16);
-    else if (Me <= 64) go(k_linear_wave<1, 64, 4>, 64);
-    else if (Me <= 96) go(k_linear_wave<3, 32, 8>, 32);
-    else if (Me <= 128) go(k_linear_wave<2, 64, 4>, 64);
-    else if (Me <= 192) go(k_linear_wave<3, 64, 4>, 64);
+    // 16-lane segments and 8 modes per block as far as in the tau solve; above, 4 modes
+    // keep a block within 100 KB of LDS, at 64-byte pieces of a row (at 65 coefficients,
+    // 32 lanes and 4 modes against 16 and 8: 128^3 26.3 -> 18.5 us, 192x129x192 54 -> 37)
+    if (Me <= 16) go(k_linear_wave<1, 16, 8>, 16, 8);
+    else if (Me <= 32) go(k_linear_wave<2, 16, 8>, 16, 8);
+    else if (Me <= 48) go(k_linear_wave<3, 16, 8>, 16, 8);
+    else if (Me <= 64) go(k_linear_wave<4, 16, 8>, 16, 8);
+    else if (Me <= 80) go(k_linear_wave<5, 16, 8>, 16, 8);
+    else if (Me <= 96) go(k_linear_wave<3, 32, 4>, 32, 4);
+    else if (Me <= 128) go(k_linear_wave<4, 32, 4>, 32, 4);
+    else if (Me <= 192) go(k_linear_wave<6, 32, 4>, 32, 4);
     else throw std::runtime_error("NSE::linear: Ny above 383 is not supported");
 }
 

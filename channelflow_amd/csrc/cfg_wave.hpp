@@ -194,28 +194,6 @@ __device__ __forceinline__ WV<K> wload(P p, const WCtx& c) {
     return v;
 }
 
-// strided coefficients c[n] at p[n * s] (a pointer to double in any address
-// space)
-template <int K, int W, class P>
-__device__ __forceinline__ WV<K> wload_s(P p, long s, const WCtx& c) {
-    WV<K> v;
-    for (int k = 0; k < K; ++k) {
-        const int i = K * c.lane + k;
-        v.e[k] = (i < c.Me) ? p[(long)(2 * i) * s] : 0.0;
-        v.o[k] = (i < c.Mo) ? p[(long)(2 * i + 1) * s] : 0.0;
-    }
-    return v;
-}
-
-template <int K, int W, class P>
-__device__ __forceinline__ void wstore_s(P p, long s, const WV<K>& v, const WCtx& c) {
-    for (int k = 0; k < K; ++k) {
-        const int i = K * c.lane + k;
-        if (i < c.Me) p[(long)(2 * i) * s] = v.e[k];
-        if (i < c.Mo) p[(long)(2 * i + 1) * s] = v.o[k];
-    }
-}
-
 // coefficient n of v, broadcast to all lanes
 // Blocked entry i of one parity array, broadcast to all lanes. Each candidate
 // passes through an empty asm operand: without it the select chain is folded

@@ -247,6 +247,22 @@ def test_dns_schemes(gpu, method, stepping, init):
     assert np.all(eu <= 1e-10), eu
 
 
+@pytest.mark.parametrize("constraint", ["PressureGradient", "BulkVelocity"])
+@pytest.mark.parametrize("Ny", [9, 31, 33, 63, 65, 95, 97, 127, 129, 159, 161, 191, 193, 255, 257])
+def test_dns_linear_segments(gpu, constraint, Ny):
+    """Runge-Kutta steps, each substep of which takes NSE::linear, at the edges of
+    that kernel's segment shapes (16 lanes with 1 to 5 even coefficients each up to
+    Ny = 159, 32 lanes with 3, 4, 6 above); 7 x 4 modes, so that the last block is not
+    full. The same 1e-10 bar as test_dns_schemes."""
+    flags = dict(C1_FLAGS, nonlinearity="Rotational", timestepping="CNRK2", initstepping="CNRK2", dt=0.01,
+                 constraint=constraint)
+    u0 = random_field(12, Ny, 12, LX_C, LZ_C, norm=0.1, decay=0.3, seed=Ny)
+    g, ur, qr, ug, qg, ref, dns = run_pair(12, Ny, 12, LX_C, LZ_C, flags, u0, 4)
+    eu = rel_l2_per_component(g, ug, ur)
+    print(constraint, Ny, "rel L2", eu, flush=True)
+    assert np.all(eu <= 1e-10), eu
+
+
 CFL_CASES = {
     "couette_skew": (C1_FLAGS, (24, 25, 24)),
     "poiseuille_rot_nodealias": (dict(baseflow="LaminarBase", constraint="PressureGradient", dPdx=-3.0 / 2000,
