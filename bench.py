@@ -769,7 +769,8 @@ def combine_calibration(cfa, steps=2):
 
 
 # device kernels that fill a step slot of another name (wavefront-local FFT passes)
-KERNEL_ALIAS = {"k_zwave": "k_zpass", "k_zsplit": "k_zpass", "k_xwinv": "k_xinv", "k_xwfwd": "k_xfwd"}
+KERNEL_ALIAS = {"k_zwave": "k_zpass", "k_zsplit": "k_zpass", "k_xwinv": "k_xinv", "k_xwfwd": "k_xfwd",
+                "k_xwfold": "k_xfwd"}
 
 
 def _counter_rows(path, counter):

@@ -11,7 +11,8 @@
 //   k_zsplit per (y, x) line: c2r z-FFTs, pointwise products, r2c z-FFTs,
 //            three wavefronts per group of lines (k_zwave: one; k_zpass: LDS
 //            FFTs, block-wide, for the lengths the wavefront FFT does not cover);
-//   k_xwfwd  forward x-FFT, live kx kept, 1/(Nx Nz) scaling (k_xfwd);
+//   k_xwfwd  forward x-FFT, live kx kept, 1/(Nx Nz) scaling (k_xfwd; k_xwfold: the
+//            skew-symmetric form's, with the x part of its divergence);
 //   k_yfwd_t values -> Chebyshev coefficients, with the spectral divergence
 //            of u_i u_j folded in for the divergence/skew-symmetric forms.
 // Only non-aliased modes |kx| <= kxd, kz <= kzd are ever stored, so the
@@ -165,6 +166,36 @@ __global__ void __launch_bounds__(256) k_xfwd(Geom g, FFTPlan px, int XL, const 
 // FFT as in the wave-local z pass. Consecutive lanes of a group hold
 // consecutive kx (contiguous reads of yp / writes of fo); the lines of a
 // wavefront are consecutive kz (128-byte runs of xp / zo).
+//
+// Value r of lane j is bin n = j + N1 r, live as kx = n in the lower half of the r
+// and as kx = n - NX in the upper half (kxd < NX/2); an odd N2 has a middle r that can
+// be either. Every access is at a uniform base, one of two 32-bit lane offsets and a
+// constant or uniform distance; with 64-bit addresses and the bin tests formed per
+// access those were half of the instructions. us per launch, before -> after: inverse
+// 24 of 32^3 14.6 -> 12.7, 128^3 rotational 24.5 -> 22.6, convection 32.5 -> 30.6 (118
+// MB, 3.9 TB/s); forward 128^3 15.9 -> 13.0, 48x35x48 4.4 -> 4.1, 54x57x72 6.2 -> 5.8;
+// at 192x129x192, at the copy rate, 52.5 -> 53.8 and 36.4 -> 35.4.
+struct XBins {
+    int lo, hi;            // kx = j + N1 r is live if N1 r < lo, kx = j - N1 q if N1 q < hi
+    unsigned at, at_hi;    // byte offsets of kx = j and of the slot N1 N2 past the line's upper half
+};
+__device__ __forceinline__ XBins x_bins(const Geom& g, int ikz, int j, bool act) {
+    const unsigned row = (unsigned)ikz * (unsigned)g.nkx;
+    return XBins{act ? g.kxd + 1 - j : 0, act ? g.kxd + 1 + j : 0, (row + (unsigned)j) * 16u,
+                 (row + (unsigned)(j + g.nkx)) * 16u};
+}
+// the wavefront's place: its (y, kz chunk) and the lane's line and position in it
+struct XPlace {
+    int y, L, j, ikz;
+    bool line_ok;
+};
+template <class S>
+__device__ __forceinline__ XPlace x_place(const Geom& g, int wg) {
+    const int lane = threadIdx.x % 64, nzc = (g.nkz + S::LPW - 1) / S::LPW;
+    const int y = wg / nzc, L = lane / S::G;
+    const int ikz = (wg - y * nzc) * S::LPW + L;
+    return XPlace{y, L, lane % S::G, ikz, ikz < g.nkz};
+}
 
 // inverse x-FFT: yp [F][Ny][nkz][nkx] -> xp [Fo][Ny][Nx][nkz]; output f >= nsrc
 // is d/dx of source field f - nsrc
@@ -178,61 +209,67 @@ __global__ void __launch_bounds__(256) k_xwinv(Geom g, const double2* __restrict
     extern __shared__ double2 lds[];
     for (int i = threadIdx.x; i < NX; i += blockDim.x) lds[i] = twg[i];
     __syncthreads();
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int nkz = g.nkz, nkx = g.nkx, Ny = g.Ny;
-    const int nzc = (nkz + S::LPW - 1) / S::LPW;
-    const int wg = bid.x * (blockDim.x / 64) + wave;
-    const int y = wg / nzc;
-    if (y >= Ny) return;
-    const int L = lane / S::G, j = lane % S::G;
-    const int ikz = (wg - y * nzc) * S::LPW + L;
-    const bool line_ok = ikz < nkz;
-    const int fo = bid.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const XPlace w = x_place<S>(g, bid.x * (blockDim.x / 64) + wave);
+    if (w.y >= g.Ny) return;
+    const int j = w.j, fo = bid.y;
     const bool deriv = fo >= nsrc;
     const int fs = deriv ? fo - nsrc : fo;
-    const double2* __restrict__ src = yp0 + bid.z * sy + (((long)fs * Ny + y) * nkz + (line_ok ? ikz : 0)) * nkx;
-    const double dk = 2 * PI / g.Lx;
-    // All of a lane's loads are issued before any is used (bins it does not
-    // hold read bin 0 and are zeroed after): a load under the lane condition
-    // whose value was scaled at once got its own wait, one HBM round trip per
-    // load.
+    const gbytes src = reinterpret_cast<gbytes>(gmem(yp0) + bid.z * sy + ((long)fs * g.Ny + w.y) * g.M);
+    const XBins bins = x_bins(g, w.ikz, j, w.line_ok && j < N1);
     double2 v[N2];
-    int ikr[N2];
 #pragma unroll
     for (int r = 0; r < N2; ++r) {
-        const int n = j + N1 * r;
-        int ikx = -1;
-        if (n <= g.kxd) ikx = n;
-        else if (n >= NX - g.kxd) ikx = n - NX + nkx;
-        ikr[r] = (line_ok && j < N1) ? ikx : -1;
-        v[r] = src[ikr[r] >= 0 ? ikr[r] : 0];
+        v[r] = make_double2(0.0, 0.0);
+        if (2 * r < N2 && N1 * r < bins.lo) v[r] = gload(src + 16 * N1 * r, bins.at);
+        if (2 * r + 1 >= N2 && N1 * (N2 - r) < bins.hi) v[r] = gload(src - 16 * N1 * (N2 - r), bins.at_hi);
     }
+    if (deriv) {
+        const double dk = 2 * PI / g.Lx, sj = j;
 #pragma unroll
-    for (int r = 0; r < N2; ++r) {
-        double2 z = make_double2(0.0, 0.0);
-        if (ikr[r] >= 0) {
-            z = v[r];
-            if (deriv) z = imul(dk * kx_of(g, ikr[r]), z);
+        for (int r = 0; r < N2; ++r) {
+            const bool up = 2 * r + 1 > N2 || (2 * r + 1 == N2 && N1 * r >= bins.lo);
+            v[r] = imul(dk * (up ? sj - (double)(N1 * (N2 - r)) : sj + (double)(N1 * r)), v[r]);
         }
-        v[r] = z;
     }
     double2 u[N1];
-    zw_a2b<NX, +1>(v, u, j, lds + NX + (wave * S::LPW + L) * S::LBUF, lds);
-    if (line_ok && j < N2) {
-        double2* __restrict__ out = xp0 + bid.z * sx + ((long)fo * Ny + y) * NX * (long)nkz + ikz;
+    zw_a2b<NX, +1>(v, u, j, lds + NX + (wave * S::LPW + w.L) * S::LBUF, lds);
+    if (w.line_ok && j < N2) {
+        const gbytes_w out = reinterpret_cast<gbytes_w>(gmem_w(xp0) + bid.z * sx + ((long)fo * g.Ny + w.y) * NX * (long)g.nkz);
+        const unsigned at = ((unsigned)j * (unsigned)g.nkz + (unsigned)w.ikz) * 16u;
 #pragma unroll
-        for (int m = 0; m < N1; ++m) out[(long)(j + N2 * m) * nkz] = u[m];
+        for (int m = 0; m < N1; ++m) gstore(out + (long)m * (N2 * 16) * g.nkz, at, u[m]);
+    }
+}
+
+// one line's forward transform: field f of zo at (y, kz) into v[p] = X[j + N1 p]
+template <int NX>
+__device__ __forceinline__ void x_forward(const Geom& g, const double2* __restrict__ zo, int f, const XPlace& w,
+                                          double2* T, const double2* tw, double2 (&v)[ZW<NX>::N2]) {
+    constexpr int N1 = ZW<NX>::N1, N2 = ZW<NX>::N2;
+    const gbytes in = reinterpret_cast<gbytes>(gmem(zo) + ((long)f * g.Ny + w.y) * NX * (long)g.nkz);
+    const bool act = w.line_ok && w.j < N2;
+    const unsigned at = act ? ((unsigned)w.j * (unsigned)g.nkz + (unsigned)w.ikz) * 16u : 0u;
+    double2 u[N1];
+#pragma unroll
+    for (int m = 0; m < N1; ++m) {
+        u[m] = make_double2(0.0, 0.0);
+        if (act) u[m] = gload(in + (long)m * (N2 * 16) * g.nkz, at);
+    }
+    zw_b2a<NX, -1>(u, v, w.j, T, tw);
+}
+// calls put(value p, distance, offset, kx) for the live values of a lane
+template <int NX, class Put>
+__device__ __forceinline__ void x_live(const XBins& b, int j, Put&& put) {
+    constexpr int N1 = ZW<NX>::N1, N2 = ZW<NX>::N2;
+#pragma unroll
+    for (int p = 0; p < N2; ++p) {
+        if (2 * p < N2 && N1 * p < b.lo) put(p, 16 * N1 * p, b.at, j + N1 * p);
+        if (2 * p + 1 >= N2 && N1 * (N2 - p) < b.hi) put(p, -16 * N1 * (N2 - p), b.at_hi, j - N1 * (N2 - p));
     }
 }
 
 // forward x-FFT: zo [G][Ny][Nx][nkz] -> fo [G][Ny][nkz][nkx], scaled by 1/(Nx Nz).
-// fold (the skew-symmetric form): the x-derivative part of its divergence is
-// added here, in x-spectral space, and the launch has 5 line tasks, not 8:
-// task c < 3 writes field c as f_c + 1/2 i kx (u_c u_0) (u_c u_0 is z-pass
-// field 3 + c), task 1 also u_0u_1 as field 3, tasks 3 and 4 u_1u_1 (z-pass
-// field 6) and u_1u_2 (7) as fields 4 and 5. The y-forward transform then
-// reads f_c and u_c u_1 only. The added term is formed exactly as the
-// y-forward transform formed it before (the same products in the same order).
 // xcd: blocks in XCD order (xcd_grid), for grids whose rows of nkz bins are
 // not a whole number of 128-byte lines, so that neighbouring kz chunks, which
 // share the lines at their edges, read them through one L2; where the rows
@@ -240,65 +277,75 @@ __global__ void __launch_bounds__(256) k_xwinv(Geom g, const double2* __restrict
 template <int NX>
 __global__ void __launch_bounds__(256) k_xwfwd(Geom g, const double2* __restrict__ twg,
                                                const double2* __restrict__ zo0, long sx, double2* __restrict__ fo0,
-                                               long sy, int fold, int xcd) {
+                                               long sy, int xcd) {
+    const BlockId bid = xcd ? xcd_grid() : BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+    using S = ZW<NX>;
+    extern __shared__ double2 lds[];
+    for (int i = threadIdx.x; i < NX; i += blockDim.x) lds[i] = twg[i];
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const XPlace w = x_place<S>(g, bid.x * (blockDim.x / 64) + wave);
+    if (w.y >= g.Ny) return;
+    double2 v[S::N2];
+    x_forward<NX>(g, zo0 + bid.z * sx, bid.y, w, lds + NX + (wave * S::LPW + w.L) * S::LBUF, lds, v);
+    const double scale = 1.0 / ((double)g.Nx * g.Nz);
+    const gbytes_w out = reinterpret_cast<gbytes_w>(gmem_w(fo0) + bid.z * sy + ((long)bid.y * g.Ny + w.y) * g.M);
+    x_live<NX>(x_bins(g, w.ikz, w.j, w.line_ok && w.j < S::N1), w.j,
+               [&](int p, int dist, unsigned at, int) { gstore(out + dist, at, make_double2(v[p].x * scale, v[p].y * scale)); });
+}
+
+// The same for the skew-symmetric form's 8 fields, with the x-derivative part of
+// its divergence added here, in x-spectral space: task c < 3 writes field c as
+// f_c + 1/2 i kx (u_c u_0) (u_c u_0 is z-pass field 3 + c), task 1 also u_0u_1 as
+// field 3, task 3 writes u_1u_1 (z-pass field 6) and u_1u_2 (7) as fields 4 and 5.
+// The y-forward transform then reads f_c and u_c u_1 only. A task is a pair of
+// wavefronts with a field each; the second hands its spectrum to the first through
+// its LDS rows. One wavefront with both fields in turn held twice the registers and
+// ran twice the chain (us per launch, before -> after, with the accesses as above
+// after: one 32^3 field 5.5 -> 4.2, 64^3 7.1 -> 6.2, 96^3 17.6 -> 16.1, 24 of 32^3
+// 13.3 -> 11.5, 4 of 96^3 54.9 -> 52.6; 16 of 64^3, 254 MB, 63.3 -> 64.6).
+template <int NX>
+__global__ void __launch_bounds__(256) k_xwfold(Geom g, const double2* __restrict__ twg,
+                                                const double2* __restrict__ zo0, long sx, double2* __restrict__ fo0,
+                                                long sy, int xcd) {
     const BlockId bid = xcd ? xcd_grid() : BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
     using S = ZW<NX>;
     constexpr int N1 = S::N1, N2 = S::N2;
     extern __shared__ double2 lds[];
     for (int i = threadIdx.x; i < NX; i += blockDim.x) lds[i] = twg[i];
     __syncthreads();
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int nkz = g.nkz, nkx = g.nkx, Ny = g.Ny;
-    const int nzc = (nkz + S::LPW - 1) / S::LPW;
-    const int wg = bid.x * (blockDim.x / 64) + wave;
-    const int y = wg / nzc;
-    if (y >= Ny) return;
-    const int L = lane / S::G, j = lane % S::G;
-    const int ikz = (wg - y * nzc) * S::LPW + L;
-    const bool line_ok = ikz < nkz;
-    const int t = bid.y;
-    int fa = t, oa = t, fb = -1, ob = -1;
-    if (fold) {
-        fa = t < 3 ? t : t + 3;
-        oa = t < 3 ? t : t + 1;
-        if (t < 3) fb = 3 + t;
-        if (t == 1) ob = 3;
-    }
-    double2* const T = lds + NX + (wave * S::LPW + L) * S::LBUF;
-    auto line = [&](int f, double2 (&v)[N2]) {
-        const double2* __restrict__ in =
-            zo0 + bid.z * sx + ((long)f * Ny + y) * NX * (long)nkz + (line_ok ? ikz : 0);
-        double2 u[N1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), half = wave & 1;
+    const XPlace w = x_place<S>(g, bid.x * (blockDim.x / 128) + wave / 2);
+    const bool have = w.y < g.Ny;  // of the whole wavefront
+    const int t = bid.y, j = w.j;
+    double2* const T = lds + NX + (wave * S::LPW + w.L) * S::LBUF;
+    double2 v[N2];
+    if (have) x_forward<NX>(g, zo0 + bid.z * sx, t < 3 ? t + 3 * half : 6 + half, w, T, lds, v);
+    const double scale = 1.0 / ((double)g.Nx * g.Nz);
 #pragma unroll
-        for (int m = 0; m < N1; ++m)
-            u[m] = (line_ok && j < N2) ? in[(long)(j + N2 * m) * nkz] : make_double2(0.0, 0.0);
-        zw_b2a<NX, -1>(u, v, j, T, lds);
-    };
-    double2 va[N2], vb[N2];
-    line(fa, va);
-    if (fb >= 0) line(fb, vb);
-    if (line_ok && j < N1) {
-        const double scale = 1.0 / ((double)g.Nx * g.Nz), beta = 0.5;
-        double2* __restrict__ base = fo0 + bid.z * sy;
-        double2* __restrict__ outa = base + (((long)oa * Ny + y) * nkz + ikz) * nkx;
-        double2* __restrict__ outb = base + (((long)(ob < 0 ? oa : ob) * Ny + y) * nkz + ikz) * nkx;
+    for (int p = 0; p < N2; ++p) v[p] = make_double2(v[p].x * scale, v[p].y * scale);
+    if (t < 3) {
+        wave_lds_sync();
+        if (half && j < N1) {
 #pragma unroll
-        for (int p = 0; p < N2; ++p) {
-            const int n = j + N1 * p;
-            int ikx = -1;
-            if (n <= g.kxd) ikx = n;
-            else if (n >= NX - g.kxd) ikx = n - NX + nkx;
-            if (ikx < 0) continue;
-            double2 a = make_double2(va[p].x * scale, va[p].y * scale);
-            if (fb >= 0) {
-                const double2 b = make_double2(vb[p].x * scale, vb[p].y * scale);
-                const int kx = kx_of(g, ikx);
-                const double s0 = -beta * 2 * PI * kx / g.Lx, s1 = beta * 2 * PI * kx / g.Lx;
-                a = make_double2(fma(s0, b.y, a.x), fma(s1, b.x, a.y));  // a + beta i kx b
-                if (ob >= 0) outb[ikx] = b;
-            }
-            outa[ikx] = a;
+            for (int p = 0; p < N2; ++p) T[j + N1 * p] = v[p];
         }
+        __syncthreads();
+    }
+    if (!have || (half && t != 1 && t != 3)) return;
+    const XBins bins = x_bins(g, w.ikz, j, w.line_ok && j < N1);
+    const int o = t == 3 ? 4 + half : half ? 3 : t;
+    const gbytes_w out = reinterpret_cast<gbytes_w>(gmem_w(fo0) + bid.z * sy + ((long)o * g.Ny + w.y) * g.M);
+    const double2* const Tb = T + S::LPW * S::LBUF;  // the second wavefront's rows
+    if (t < 3 && !half) {
+        const double dk = PI / g.Lx;
+        x_live<NX>(bins, j, [&](int p, int dist, unsigned at, int kx) {
+            const double2 b = Tb[j + N1 * p];
+            const double hk = dk * kx;  // f_c + 1/2 i (2 pi kx / Lx) b
+            gstore(out + dist, at, make_double2(fma(-hk, b.y, v[p].x), fma(hk, b.x, v[p].y)));
+        });
+    } else {
+        x_live<NX>(bins, j, [&](int p, int dist, unsigned at, int) { gstore(out + dist, at, v[p]); });
     }
 }
 
@@ -970,7 +1017,7 @@ static void launch_yinv(const Geom& g, const YMats& ym, int n, const NLMember* t
     }
 }
 
-// xfold: the skew-symmetric fields come folded from k_xwfwd (f_c with its
+// xfold: the skew-symmetric fields come folded from k_xwfold (f_c with its
 // x-derivative term in fields 0-2, u_cu_1 in 3 + c)
 template <int METHOD>
 static void launch_yfwd(const Geom& g, const YMats& ym, int n, int have_g, const double2* fo, long sy,
@@ -1003,7 +1050,7 @@ static int xfft_lines(const Geom& g, const NLTune& tn) {
     return tn.xl > 0 ? std::min(tn.xl, m) : std::min(4, m);
 }
 
-// fold (forward only): the skew-symmetric layout of k_xwfwd (8 z-pass fields in,
+// fold (forward only): the skew-symmetric layout of k_xwfold (8 z-pass fields in,
 // 6 out, the x-derivative part of the divergence added); only the wavefront
 // FFT lengths have it. Returns whether it folded.
 template <int NX>
@@ -1020,10 +1067,18 @@ static bool launch_x(bool inverse, const Geom& g, const FFTPlan& px, int nsrc, i
             k_xwinv<NX><<<grid, 64 * wb, lds, st>>>(g, px.tw, nsrc, in, sin, out, sout);
         } else {
             if (fold && nf != 8) throw std::runtime_error("x-FFT fold: the skew-symmetric layout has 8 fields");
-            const dim3 grid((unsigned)((waves + wb - 1) / wb), fold ? 5 : nf, n);
-            allow_lds(k_xwfwd<NX>, lds);
             const int xcd = (g.nkz * (int)sizeof(double2)) % 128 != 0;
-            k_xwfwd<NX><<<grid, 64 * wb, lds, st>>>(g, px.tw, in, sin, out, sout, fold ? 1 : 0, xcd);
+            if (fold) {  // pairs of wavefronts
+                const int np = wb > 2 ? 2 : 1;
+                const size_t ldsp = (size_t)(NX + 2 * np * S::LPW * S::LBUF) * sizeof(double2);
+                allow_lds(k_xwfold<NX>, ldsp);
+                k_xwfold<NX><<<dim3((unsigned)((waves + np - 1) / np), 4, n), 128 * np, ldsp, st>>>(
+                    g, px.tw, in, sin, out, sout, xcd);
+            } else {
+                allow_lds(k_xwfwd<NX>, lds);
+                k_xwfwd<NX><<<dim3((unsigned)((waves + wb - 1) / wb), nf, n), 64 * wb, lds, st>>>(g, px.tw, in, sin,
+                                                                                               out, sout, xcd);
+            }
         }
         return fold && !inverse;
     } else {
@@ -1113,7 +1168,7 @@ void launch_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
     // skew-symmetric one; one launch when both exist (the fields are
     // contiguous)
     const bool uu = method == NL_DIV || method == NL_SKEW;
-    bool xfold = false;  // the skew-symmetric x-derivative terms already in fields 0-2 (k_xwfwd)
+    bool xfold = false;  // the skew-symmetric x-derivative terms already in fields 0-2 (k_xwfold)
     if (want_g)
         xfold = launch_xfft(false, g, px, 0, method == NL_SKEW ? 8 : (uu ? 9 : 3), n, zo, sx, fo, sy, tn, st,
                             method == NL_SKEW);
