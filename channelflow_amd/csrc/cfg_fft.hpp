@@ -297,35 +297,52 @@ struct ZW {
     static constexpr int G = pow2_at_least(NMAX);  // lanes per line
     static constexpr int LPW = 64 / G;             // lines per wavefront
     static constexpr int LBUF = N + NMAX;          // LDS slots per line (transposes, padded rows)
+    static constexpr int TWN = N;                  // twiddles: w_N^i
+    static __device__ __forceinline__ int tw_power(int i) { return i; }
 };
 
 // The same in three steps, N = A B C with the physical values A per lane: two
 // transposes, but fewer values per lane and transform. QG: groups of B values a
-// lane holds in the middle step.
+// lane holds in the middle step. P1, P2: LDS pitches of the transposes, [C][B A] and
+// [A][B C]. The middle step's lanes run over C first, so that every access is
+// contiguous or at the odd pitch P1 across lanes; P2 keeps the A-groups of a
+// 16-lane read on different banks. With rows of A or B values instead, lanes a row
+// apart, conflicts took a quarter of the rotational 192-bin z pass (9.4 M cycles, now
+// 2.0 M). us per launch, before -> after: 192x129x192 rotational 63 -> 57, 128^3
+// convection 48 -> 44, rotational 31.4 -> 30.6, skew-symmetric 64x49x108 19.5 -> 17.9,
+// 64x49x144 21.8 -> 20.4, 64x33x256 24.5 -> 20.9; at 72 and 96 the same.
 template <int NZ>
 struct ZW3Shape {
-    static constexpr int A = 0, B = 0, C = 0, QG = 1;
+    static constexpr int A = 0, B = 0, C = 0, QG = 1, P1 = 1, P2 = 1;
 };
-template <> struct ZW3Shape<72> { static constexpr int A = 3, B = 4, C = 6, QG = 1; };
-template <> struct ZW3Shape<96> { static constexpr int A = 3, B = 4, C = 8, QG = 1; };
-template <> struct ZW3Shape<108> { static constexpr int A = 6, B = 3, C = 6, QG = 2; };
-template <> struct ZW3Shape<128> { static constexpr int A = 4, B = 4, C = 8, QG = 1; };
-template <> struct ZW3Shape<144> { static constexpr int A = 6, B = 4, C = 6, QG = 2; };
-template <> struct ZW3Shape<162> { static constexpr int A = 6, B = 3, C = 9, QG = 3; };
-template <> struct ZW3Shape<192> { static constexpr int A = 6, B = 4, C = 8, QG = 2; };
-template <> struct ZW3Shape<256> { static constexpr int A = 8, B = 4, C = 8, QG = 2; };
+template <> struct ZW3Shape<72> { static constexpr int A = 3, B = 4, C = 6, QG = 1, P1 = 13, P2 = 30; };
+template <> struct ZW3Shape<96> { static constexpr int A = 3, B = 4, C = 8, QG = 1, P1 = 13, P2 = 40; };
+template <> struct ZW3Shape<108> { static constexpr int A = 6, B = 3, C = 6, QG = 2, P1 = 19, P2 = 22; };
+template <> struct ZW3Shape<128> { static constexpr int A = 4, B = 4, C = 8, QG = 1, P1 = 17, P2 = 40; };
+template <> struct ZW3Shape<144> { static constexpr int A = 6, B = 4, C = 6, QG = 2, P1 = 25, P2 = 30; };
+template <> struct ZW3Shape<162> { static constexpr int A = 6, B = 3, C = 9, QG = 3, P1 = 19, P2 = 41; };
+template <> struct ZW3Shape<192> { static constexpr int A = 6, B = 4, C = 8, QG = 2, P1 = 25, P2 = 40; };
+template <> struct ZW3Shape<256> { static constexpr int A = 8, B = 4, C = 8, QG = 2, P1 = 33, P2 = 40; };
 
 template <int NZ>
 struct ZW3 {
     static constexpr int A = ZW3Shape<NZ>::A, B = ZW3Shape<NZ>::B, C = ZW3Shape<NZ>::C, QG = ZW3Shape<NZ>::QG;
+    static constexpr int P1 = ZW3Shape<NZ>::P1, P2 = ZW3Shape<NZ>::P2, PT = C | 1;
     static constexpr int N = A * B * C;
     static constexpr int SL = A * B, SV = C, PL = B * C, PV = A, QL = A * C / QG;
     static constexpr int G = pow2_at_least(PL > SL ? PL : SL);
     static constexpr int LPW = 64 / G;
-    static constexpr int AP = A | 1, BP = B | 1, CP = C | 1;  // row pitches, odd
     static constexpr int max3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
-    static constexpr int LBUF = max3(A * C * BP, A * B * CP, B * C * AP);
-    static_assert(QL <= G && A * C % QG == 0, "the middle step's lanes");
+    static constexpr int LBUF = max3(C * P1, A * P2, N);
+    // twiddles: w_N^(j k) at j P2 + k (j < A, k < PL), then w_PL^(b m) at b PT + m (b < B, m < C)
+    static constexpr int TWN = A * P2 + B * PT;
+    static_assert(QL <= G && A % QG == 0 && P1 >= SL && P2 >= PL, "the middle step's lanes and the pitches");
+    // entry i as a power of w_N
+    static __device__ __forceinline__ int tw_power(int i) {
+        if (i < A * P2) return i / P2 * (i % P2 < PL ? i % P2 : 0);
+        i -= A * P2;
+        return A * (i / PT) * (i % PT < C ? i % PT : 0);
+    }
 };
 
 // the lengths with a wavefront FFT
@@ -544,45 +561,43 @@ template <int NZ, int SIGN>
 __device__ __forceinline__ void zw3_s2p(double2 (&v)[ZW3<NZ>::SV], double2 (&u)[ZW3<NZ>::PV], int l, double2* T,
                                         const double2* tw) {
     using S = ZW3<NZ>;
-    constexpr int A = S::A, B = S::B, C = S::C;
+    constexpr int A = S::A, B = S::B, C = S::C, P1 = S::P1, P2 = S::P2;
     auto turn = [&](double2 x, int i) {
         double2 t = tw[i];
         if (SIGN > 0) t.y = -t.y;
         return cmul(x, t);
     };
+    asm volatile("" : "+v"(l));  // addresses formed anew in each transform, not held between them
     dft_reg<C, SIGN>(v);
-    const int s = l < S::SL ? l : S::SL - 1, b = s / A, j = s - b * A;
+    const int b = (l < S::SL ? l : S::SL - 1) / A;
     wave_lds_sync();
     if (l < S::SL) {
-        T[j * S::BP + b] = v[0];
+        T[l] = v[0];
 #pragma unroll
-        for (int m1 = 1; m1 < C; ++m1) T[(m1 * A + j) * S::BP + b] = turn(v[m1], A * b * m1);
+        for (int m1 = 1; m1 < C; ++m1) T[m1 * P1 + l] = turn(v[m1], A * P2 + b * S::PT + m1);
     }
     wave_lds_sync();
     double2 w[S::QG][B];
-    const int q0 = l < S::QL ? l : S::QL - 1;
+    const int q = l < S::QL ? l : S::QL - 1, j0 = q / C, m1 = q - j0 * C;
 #pragma unroll
     for (int g = 0; g < S::QG; ++g) {
 #pragma unroll
-        for (int i = 0; i < B; ++i) w[g][i] = T[(q0 + S::QL * g) * S::BP + i];
+        for (int i = 0; i < B; ++i) w[g][i] = T[m1 * P1 + i * A + j0 + A / S::QG * g];
         dft_reg<B, SIGN>(w[g]);
     }
     wave_lds_sync();
     if (l < S::QL) {
 #pragma unroll
         for (int g = 0; g < S::QG; ++g) {
-            const int q = q0 + S::QL * g, m1 = q / A, jq = q - m1 * A;
+            const int at = (j0 + A / S::QG * g) * P2 + m1;
 #pragma unroll
-            for (int m2 = 0; m2 < B; ++m2) {
-                const int k1 = m1 + C * m2;
-                T[k1 * S::AP + jq] = turn(w[g][m2], jq * k1);
-            }
+            for (int m2 = 0; m2 < B; ++m2) T[at + C * m2] = turn(w[g][m2], at + C * m2);
         }
     }
     wave_lds_sync();
     const int p = l < S::PL ? l : S::PL - 1;
 #pragma unroll
-    for (int i = 0; i < A; ++i) u[i] = T[p * S::AP + i];
+    for (int i = 0; i < A; ++i) u[i] = T[i * P2 + p];
     dft_reg<A, SIGN>(u);
 }
 
@@ -590,44 +605,43 @@ template <int NZ, int SIGN>
 __device__ __forceinline__ void zw3_p2s(double2 (&u)[ZW3<NZ>::PV], double2 (&v)[ZW3<NZ>::SV], int l, double2* T,
                                         const double2* tw) {
     using S = ZW3<NZ>;
-    constexpr int A = S::A, B = S::B, C = S::C;
+    constexpr int A = S::A, B = S::B, C = S::C, P1 = S::P1, P2 = S::P2;
     auto turn = [&](double2 x, int i) {
         double2 t = tw[i];
         if (SIGN > 0) t.y = -t.y;
         return cmul(x, t);
     };
+    asm volatile("" : "+v"(l));  // addresses formed anew in each transform, not held between them
     dft_reg<A, SIGN>(u);
-    const int p = l < S::PL ? l : S::PL - 1;
     wave_lds_sync();
     if (l < S::PL) {
-        const int i1 = p % C, i2 = p / C;
-        T[i1 * A * S::BP + i2] = u[0];
+        T[l] = u[0];
 #pragma unroll
-        for (int q = 1; q < A; ++q) T[(i1 * A + q) * S::BP + i2] = turn(u[q], p * q);
+        for (int q = 1; q < A; ++q) T[q * P2 + l] = turn(u[q], q * P2 + l);
     }
     wave_lds_sync();
     double2 w[S::QG][B];
-    const int q0 = l < S::QL ? l : S::QL - 1;
+    const int q = l < S::QL ? l : S::QL - 1, j0 = q / C, i1 = q - j0 * C;
 #pragma unroll
     for (int g = 0; g < S::QG; ++g) {
 #pragma unroll
-        for (int i = 0; i < B; ++i) w[g][i] = T[(q0 + S::QL * g) * S::BP + i];
+        for (int i = 0; i < B; ++i) w[g][i] = T[(j0 + A / S::QG * g) * P2 + i1 + C * i];
         dft_reg<B, SIGN>(w[g]);
     }
     wave_lds_sync();
     if (l < S::QL) {
 #pragma unroll
         for (int g = 0; g < S::QG; ++g) {
-            const int vq = q0 + S::QL * g, i1 = vq / A, q = vq - i1 * A;
-            T[q * S::CP + i1] = w[g][0];
+            const int at = i1 * P1 + j0 + A / S::QG * g;
+            T[at] = w[g][0];
 #pragma unroll
-            for (int p1 = 1; p1 < B; ++p1) T[(p1 * A + q) * S::CP + i1] = turn(w[g][p1], A * i1 * p1);
+            for (int p1 = 1; p1 < B; ++p1) T[at + p1 * A] = turn(w[g][p1], A * P2 + p1 * S::PT + i1);
         }
     }
     wave_lds_sync();
     const int s = l < S::SL ? l : S::SL - 1;
 #pragma unroll
-    for (int i = 0; i < C; ++i) v[i] = T[s * S::CP + i];
+    for (int i = 0; i < C; ++i) v[i] = T[i * P1 + s];
     dft_reg<C, SIGN>(v);
 }
 

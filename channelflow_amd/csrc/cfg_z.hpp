@@ -23,6 +23,18 @@ size_t lds_budget();
 constexpr bool zsplit(int method, int nz) {
     return method == NL_CONV || method == NL_SKEW || nz <= (method == NL_ROT ? 32 : 24);
 }
+// Three steps per transform (ZW3) at Nz = 72 and from 96 on. What bounds the z
+// pass there is how few wavefronts a SIMD holds: with 6 physical values per lane
+// instead of 8 to 16 and transforms of at most 9 values, 2 or 3 of them fit the
+// registers where 1 did (skew-symmetric 96: 341 -> 162 registers, rotational
+// 192: 297 -> 131), at the price of a second transpose through LDS. us per
+// launch, two steps -> three: one 96^3 skew-symmetric field 59 -> 44, 128^3
+// convection 92 -> 70, rotational 49 -> 35, 192x129x192 rotational 95 -> 76,
+// 256x33x256 52 -> 48, 64x49x162 skew-symmetric 61 -> 32, 8 members of 32x49x72
+// 72 -> 53; with a component per wavefront (k_zsplit) 96^3 skew-symmetric 37 -> 34,
+// 128^3 convection 62 -> 52. At 48 and 64, where 2 wavefronts fit anyway, the second transpose
+// costs more than it gives in a batch (16 of 64^3 113 -> 127, 24 of 48^3 82 -> 88).
+constexpr bool zwave_three(int nz) { return nz == 72 || nz >= 96; }
 // real physical lines per (y, x) line the LDS z-pass of a form keeps
 int zpass_nphys(int method);
 // largest LDS z-pass lines per block that fit the LDS budget

@@ -386,18 +386,6 @@ __device__ __forceinline__ void zw_r2c(const ZWCtx& c, double2* __restrict__ zo,
     }
 }
 
-// Three steps per transform (ZW3) at Nz = 72 and from 96 on. What bounds the z
-// pass there is how few wavefronts a SIMD holds: with 6 physical values per lane
-// instead of 8 to 16 and transforms of at most 9 values, 2 or 3 of them fit the
-// registers where 1 did (skew-symmetric 96: 341 -> 162 registers, rotational
-// 192: 297 -> 131), at the price of a second transpose through LDS. us per
-// launch, two steps -> three: one 96^3 skew-symmetric field 59 -> 44, 128^3
-// convection 92 -> 70, rotational 49 -> 35, 192x129x192 rotational 95 -> 76,
-// 256x33x256 52 -> 48, 64x49x162 skew-symmetric 61 -> 32, 8 members of 32x49x72
-// 72 -> 53; with a component per wavefront (k_zsplit) 96^3 skew-symmetric 37 -> 34,
-// 128^3 convection 62 -> 52. At 48 and 64, where 2 wavefronts fit anyway, the second transpose
-// costs more than it gives in a batch (16 of 64^3 113 -> 127, 24 of 48^3 82 -> 88).
-constexpr bool zwave_three(int nz) { return nz == 72 || nz >= 96; }
 template <int NZ>
 using ZLine = std::conditional_t<zwave_three(NZ), ZW3<NZ>, ZW<NZ>>;
 
@@ -418,8 +406,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
     using S = ZLine<NZ>;
     constexpr int N1 = S::PV;
     extern __shared__ double2 lds[];
-    double2 *const tw_l = lds, *const T_l = lds + NZ;
-    for (int i = threadIdx.x; i < NZ; i += blockDim.x) tw_l[i] = twg[i];
+    double2 *const tw_l = lds, *const T_l = lds + S::TWN;
+    for (int i = threadIdx.x; i < S::TWN; i += blockDim.x) tw_l[i] = twg[S::tw_power(i)];
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const int nxc = (g.Nx + S::LPW - 1) / S::LPW;
@@ -514,7 +502,7 @@ constexpr size_t zsplit_lds() {
     using S = ZLine<NZ>;
     const size_t rows = (size_t)3 * S::LPW * S::LBUF * sizeof(double2);
     const size_t shared = (size_t)(METHOD == NL_ROT ? 6 : 3) * S::PV * 64 * sizeof(double);
-    return NZ * sizeof(double2) + (rows > shared ? rows : shared);
+    return S::TWN * sizeof(double2) + (rows > shared ? rows : shared);
 }
 template <int METHOD, int NZ>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(1, 8)))
@@ -523,16 +511,16 @@ k_zsplit(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ t
     using S = ZLine<NZ>;
     constexpr int PV = S::PV;
     extern __shared__ double2 lds[];
-    double2* const T_l = lds + NZ;
+    double2* const T_l = lds + S::TWN;
     double* const ex = reinterpret_cast<double*>(T_l);  // [shared field][value][lane]
-    constexpr int NTW = (NZ + 191) / 192;
+    constexpr int NTW = (S::TWN + 191) / 192;
     dvec2 twr[NTW];
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) twr[i] = gmem(reinterpret_cast<const dvec2*>(twg))[min((int)threadIdx.x + 192 * i, NZ - 1)];
+    for (int i = 0; i < NTW; ++i) twr[i] = gmem(reinterpret_cast<const dvec2*>(twg))[S::tw_power(min((int)threadIdx.x + 192 * i, S::TWN - 1))];
     auto twiddles = [&] {  // behind the first loads of bins
 #pragma unroll
         for (int i = 0; i < NTW; ++i)
-            if ((int)threadIdx.x + 192 * i < NZ) reinterpret_cast<dvec2*>(lds)[threadIdx.x + 192 * i] = twr[i];
+            if ((int)threadIdx.x + 192 * i < S::TWN) reinterpret_cast<dvec2*>(lds)[threadIdx.x + 192 * i] = twr[i];
         __syncthreads();
     };
     const int cc = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
@@ -678,7 +666,7 @@ void launch_z_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, in
             k_zsplit<METHOD, NZ><<<dim3((unsigned)waves, n), 192, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
         } else {
             const int wb = tn.zwb > 0 ? tn.zwb : 4;
-            const size_t lds = (size_t)(NZ + wb * S::LPW * S::LBUF) * sizeof(double2);
+            const size_t lds = (size_t)(S::TWN + wb * S::LPW * S::LBUF) * sizeof(double2);
             const dim3 grid((unsigned)((waves + wb - 1) / wb), n);
             allow_lds(k_zwave<METHOD, NZ>, lds);
             k_zwave<METHOD, NZ><<<grid, 64 * wb, lds, st>>>(g, pz.tw, tab, want_g, xp, zo, sx);
