@@ -140,10 +140,10 @@ constexpr int yinv_tail(int cls) { return 2 * 64 * cls + 8; }  // per matrix
 constexpr int yfwd_tail(int cls) { return 2 * 64 * cls + 4; }
 
 // Per-mode tau data for one lambda_t, mode-major: array k (TAU_NA of them:
-// pband pup pinvd vband vup vinvd Pp Pm vp vm P0 v0) of mode m is the Ny-vector
+// pband pup pinvd vband vup vinvd Pp vp P0 v0) of mode m is the Ny-vector
 // at coef + (m*TAU_NA + k)*Ny; scalars i00 i01 i10 i11 sigma0_Nb1 sigma0_Nb at
 // scal + m*6.
-constexpr int TAU_NA = 12;
+constexpr int TAU_NA = 10;
 struct TauSet {
     double* coef;
     double* scal;

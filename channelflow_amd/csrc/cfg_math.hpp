@@ -215,7 +215,11 @@ CFG_HD void helm_solve(const HelmholtzView& h, SV u, SV f, double ua, double ub)
 struct TauView {
     HelmholtzView ph;  // pressure: lambda = kappa^2, nu = 1
     HelmholtzView vh;  // velocity: lambda = lambda_t + nu kappa^2
-    SV Pp, Pm, vp, vm, P0, v0;
+    // The homogeneous solutions: P+ = 1 at y = b, 0 at y = a, v+ its velocity; P-,
+    // v- with the walls exchanged are their mirrors, P-_n = (-1)^n P+_n, v-_n =
+    // -(-1)^n v+_n, in every rounding (the even and the odd systems are solved apart).
+    SV Pp, vp, P0, v0;
+    SV Pm{nullptr, 0}, vm{nullptr, 0};  // filled by tau_setup where given, not read
     double* scal;  // i00 i01 i10 i11 sigma0_Nb1 sigma0_Nb, at scal[k * sstride]
     long sstride;
     double nu, a, b, kx2pi, kz2pi;  // 2 pi kx/Lx, 2 pi kz/Lz
@@ -238,8 +242,9 @@ CFG_HD void tau_influence(const TauView& t, SV P, SV v, SV tmp) {  // tausolver.
     const double delta_plus = -sc[0 * ss] * dp - sc[1 * ss] * dm;
     const double delta_minus = -sc[2 * ss] * dp - sc[3 * ss] * dm;
     for (int i = 0; i < N; ++i) {
-        P[i] += delta_plus * t.Pp[i] + delta_minus * t.Pm[i];
-        v[i] += delta_plus * t.vp[i] + delta_minus * t.vm[i];
+        const double mP = (i & 1) ? -t.Pp[i] : t.Pp[i], mv = (i & 1) ? t.vp[i] : -t.vp[i];
+        P[i] += delta_plus * t.Pp[i] + delta_minus * mP;
+        v[i] += delta_plus * t.vp[i] + delta_minus * mv;
     }
 }
 
@@ -256,17 +261,18 @@ CFG_HD void tau_setup(const TauView& t, SV s0, SV s1) {
     helm_solve(t.ph, t.Pp, s0, 0.0, 1.0);
     cheb_diff(t.Pp, s1, N, L);
     helm_solve(t.vh, t.vp, s1, 0.0, 0.0);
-    helm_solve(t.ph, t.Pm, s0, 1.0, 0.0);
-    cheb_diff(t.Pm, s1, N, L);
-    helm_solve(t.vh, t.vm, s1, 0.0, 0.0);
+    for (int n = 0; n < N && t.Pm.p; ++n) {
+        t.Pm[n] = (n & 1) ? -t.Pp[n] : t.Pp[n];
+        t.vm[n] = (n & 1) ? t.vp[n] : -t.vp[n];
+    }
     if (t.zero_mode) {  // influence matrix is singular for kx=kz=0 and unused
         for (int k = 0; k < 6; ++k) sc[k * ss] = 0.0;
         for (int n = 0; n < N; ++n) { t.P0[n] = 0.0; t.v0[n] = 0.0; }
         return;
     }
-    double A, B, C, D;
+    double A, C;
     cheb_diff_ends(t.vp, s1, N, L, A, C);
-    cheb_diff_ends(t.vm, s1, N, L, B, D);
+    const double B = C, D = A;  // dv-/dy at b and a, by the mirror symmetry
     const double disc = A * D - B * C;
     sc[0 * ss] = D / disc;
     sc[1 * ss] = -B / disc;

@@ -41,11 +41,9 @@ __device__ TauView make_view(const Geom& g, const TauSet& s, int m, double nu, b
     t.ph = HelmholtzView{A(0), A(1), A(2), kappa2, g.Ny};
     t.vh = HelmholtzView{A(3), A(4), A(5), lambda, g.Ny};
     t.Pp = A(6);
-    t.Pm = A(7);
-    t.vp = A(8);
-    t.vm = A(9);
-    t.P0 = A(10);
-    t.v0 = A(11);
+    t.vp = A(7);
+    t.P0 = A(8);
+    t.v0 = A(9);
     t.scal = s.scal + (long)m * 6;
     t.sstride = 1;
     t.nu = nu;
@@ -59,7 +57,7 @@ __device__ TauView make_view(const Geom& g, const TauSet& s, int m, double nu, b
 }
 
 // TauSolver constructor per mode (tausolver.cpp:81-176), T modes per block,
-// one thread each. ALL: the mode's whole working set in LDS, its 12 tau
+// one thread each. ALL: the mode's whole working set in LDS, its 10 tau
 // profiles (array a at element (a*Ny + n)*T + t), 6 scalars and 2 scratch
 // profiles, copied to the mode-major tau set with contiguous writes at the end.
 // Otherwise (tall grids, where a block of 64 KB would hold fewer than 8 such
@@ -85,14 +83,12 @@ __global__ void k_tau_setup(Geom g, TauSet s, double nu, int taucorr) {
             v.vh.up = A(4);
             v.vh.invd = A(5);
             v.Pp = A(6);
-            v.Pm = A(7);
-            v.vp = A(8);
-            v.vm = A(9);
-            v.P0 = A(10);
-            v.v0 = A(11);
-            v.scal = sl + 14 * arr + t;
+            v.vp = A(7);
+            v.P0 = A(8);
+            v.v0 = A(9);
+            v.scal = sl + (TAU_NA + 2) * arr + t;
             v.sstride = T;
-            tau_setup(v, A(12), A(13));
+            tau_setup(v, A(TAU_NA), A(TAU_NA + 1));
         } else {
             tau_setup(v, A(0), A(1));
         }
@@ -106,15 +102,15 @@ __global__ void k_tau_setup(Geom g, TauSet s, double nu, int taucorr) {
             coef[i] = sl[a * arr + (long)n * T + mm];
         }
         __attribute__((address_space(1))) double* scal = gmem_w(s.scal) + (long)m0 * 6;
-        for (int i = t; i < nm * 6; i += T) scal[i] = sl[14 * arr + (long)(i % 6) * T + i / 6];
+        for (int i = t; i < nm * 6; i += T) scal[i] = sl[(TAU_NA + 2) * arr + (long)(i % 6) * T + i / 6];
     }
 }
 
 // modes per block of the set-up within 64 KB of LDS, at most 64: whole working
-// sets (14 profiles and 6 scalars each) where 8 or more fit, else scratch
+// sets (12 profiles and 6 scalars each) where 8 or more fit, else scratch
 // profiles only (2 each)
 static int tau_setup_modes(int Ny, bool* all) {
-    const long whole = (14L * Ny + 6) * (long)sizeof(double), scratch = 2L * Ny * (long)sizeof(double);
+    const long whole = ((TAU_NA + 2L) * Ny + 6) * (long)sizeof(double), scratch = 2L * Ny * (long)sizeof(double);
     const long T = (64L * 1024) / whole;
     *all = T >= 8;
     return (int)std::max(1L, std::min(64L, (64L * 1024) / (*all ? whole : scratch)));
@@ -125,7 +121,7 @@ void launch_tau_setup(const Geom& g, const TauSet& s, double nu, bool taucorr, h
     const int T = tau_setup_modes(g.Ny, &all);
     const dim3 grid((g.M + T - 1) / T);
     if (all) {
-        const size_t lds = (size_t)(14L * g.Ny + 6) * T * sizeof(double);
+        const size_t lds = (size_t)((TAU_NA + 2L) * g.Ny + 6) * T * sizeof(double);
         k_tau_setup<true><<<grid, T, lds, st>>>(g, s, nu, taucorr ? 1 : 0);
     } else {
         const size_t lds = (size_t)2 * g.Ny * T * sizeof(double);
@@ -221,8 +217,10 @@ constexpr int tau_waves(int K, int W) { return W == 16 && K <= 5 ? (K == 1 ? 4 :
 //
 // What bounds it: for one field the instruction chain of a wave, for a batch
 // HBM and that chain (24 x 32^3: 63 MB in 20.8 us, one round of blocks), for
-// one large field HBM (192x129x192: 450 MB in 120.8 us, 3.7 TB/s, of which the
-// right-hand-side rows are 256-byte pieces 130 KB apart). Against a segment per
+// one large field HBM (192x129x192: 434 MB in 116 us, 3.7 TB/s, of which the
+// right-hand-side rows are 256-byte pieces 130 KB apart). The set keeps P+ and v+
+// only: with P- and v- stored and loaded too 128^3 took 47.2 us, not 44.4,
+// 192x129x192 121.0, 96^3 23.6, not 22.4, 4 of 96^3 85.6, not 83.3. Against a segment per
 // complex mode with the scan multipliers recomputed for every right-hand side
 // and every lane past a system masked (8557 instructions at K = 3, now about
 // 2200): one 32^3 field 20.5 -> 9.2 us, 64^3 31.3 -> 14.6, 96^3 39.5 -> 23.5,
@@ -374,17 +372,17 @@ k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMembe
         const gcdouble sc = gmem(s.scal) + 6L * m;
         const double dplus = -sc[0] * dvb[0] - sc[1] * dva[0];
         const double dminus = -sc[2] * dvb[0] - sc[3] * dva[0];
-        const WV<K> Pp = wfac<K, W>(coef, Ny, 6, fo, c), Pm = wfac<K, W>(coef, Ny, 7, fo, c);
-        const WV<K> vp = wfac<K, W>(coef, Ny, 8, fo, c), vm = wfac<K, W>(coef, Ny, 9, fo, c);
+        // P- and v- are the mirrors of P+ and v+: (e, -o) and (-e, o)
+        const WV<K> Pp = wfac<K, W>(coef, Ny, 6, fo, c), vp = wfac<K, W>(coef, Ny, 7, fo, c);
         for (int k = 0; k < K; ++k) {
-            P[0].e[k] += dplus * Pp.e[k] + dminus * Pm.e[k];
-            P[0].o[k] += dplus * Pp.o[k] + dminus * Pm.o[k];
-            v[0].e[k] += dplus * vp.e[k] + dminus * vm.e[k];
-            v[0].o[k] += dplus * vp.o[k] + dminus * vm.o[k];
+            P[0].e[k] += dplus * Pp.e[k] + dminus * Pp.e[k];
+            P[0].o[k] += dplus * Pp.o[k] - dminus * Pp.o[k];
+            v[0].e[k] += dplus * vp.e[k] - dminus * vp.e[k];
+            v[0].o[k] += dplus * vp.o[k] + dminus * vp.o[k];
         }
         if (taucorr) {
             const int Nb = c.Nb;
-            const WV<K> P0 = wfac<K, W>(coef, Ny, 10, fo, c), v0 = wfac<K, W>(coef, Ny, 11, fo, c);
+            const WV<K> P0 = wfac<K, W>(coef, Ny, 8, fo, c), v0 = wfac<K, W>(coef, Ny, 9, fo, c);
             const double sigma1_Nb = lambda * wtop<K, W>(v[0], c) - Sy[Nb];
             double sigma1_Nb1 = lambda * wtop1<K, W>(v[0], c) - Sy[Nb - 1];
             sigma1_Nb1 += (4.0 / c.L) * Nb * wtop<K, W>(P[0], c);

@@ -181,11 +181,9 @@ struct cfg_tausolver {
         t.ph = HelmholtzView{A(0), A(1), A(2), kappa2, Ny};
         t.vh = HelmholtzView{A(3), A(4), A(5), lambda, Ny};
         t.Pp = A(6);
-        t.Pm = A(7);
-        t.vp = A(8);
-        t.vm = A(9);
-        t.P0 = A(10);
-        t.v0 = A(11);
+        t.vp = A(7);
+        t.P0 = A(8);
+        t.v0 = A(9);
         t.scal = cm + (long)TAU_NA * N;
         t.sstride = 1;
         t.nu = nu;
