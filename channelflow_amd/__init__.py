@@ -476,7 +476,7 @@ class Batch:
 
     def __del__(self):
         h = getattr(self, "_h", None)
-        if h:
+        if h and _lib is not None:
             library().cfg_batch_destroy(h)
             self._h = None
 
@@ -510,6 +510,12 @@ class Batch:
         _check(library().cfg_batch_get_state(self._h, int(member), _ptr(u.view(np.float64)),
                                              _ptr(q.view(np.float64))))
         return u, q
+
+    def velocity(self, member):
+        """The velocity of state(member), without the pressure."""
+        u = np.zeros(self._shapes[member], dtype=np.complex128)
+        _check(library().cfg_batch_get_state(self._h, int(member), _ptr(u.view(np.float64)), None))
+        return u
 
     def set_state(self, member, fields):
         u = _f64(fields[0].data)

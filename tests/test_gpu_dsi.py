@@ -149,3 +149,26 @@ def test_residual_variable_dt_matches_single_and_oracle(gpu):
         assert ms.dts[i] == dt.dt()
         assert rel(g, us, o.state()[0]) <= 1e-10
     assert any(x != COUETTE["dt"] for x in ms.dts)  # dt did adapt
+
+
+@pytest.mark.parametrize("case", ["skew", "alternating", "variable"])
+def test_repeated_calls_match_new_objects(gpu, case):
+    """A MultiShooting's later calls run in the batch of its first one: residuals for
+    other shots, other counts of members and the first shots again equal those of new
+    objects bit for bit, and so do a copy's."""
+    import copy
+    fl = cfa.DNSFlags(**dict(COUETTE, **{"alternating": dict(nonlinearity="Alternating"),
+                                         "variable": dict(variabledt=True)}.get(case, {})))
+    new = lambda: MultiShooting(NX, NY, NZ, LX_C, LZ_C, fl, 0.14)  # noqa: E731 (7 steps: an odd number)
+    shots, dirs = shots_and_dirs(3, 1)
+    other = [random_field(NX, NY, NZ, LX_C, LZ_C, norm=0.2, decay=0.4, seed=500 + i) for i in range(3)]
+    ms = new()
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots), new().eval(shots)))
+    dts = list(ms.dts)
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(other), new().eval(other)))
+    G, J, _ = ms.eval_with_jacobians(shots, dirs)
+    Gn, Jn, _ = new().eval_with_jacobians(shots, dirs)
+    assert all(np.array_equal(a, b) for a, b in zip(G + J[0], Gn + Jn[0]))
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots[:1]), new().eval(shots[:1])))
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots), new().eval(shots))) and ms.dts == dts
+    assert all(np.array_equal(a, b) for a, b in zip(copy.deepcopy(ms).eval(other), new().eval(other)))
