@@ -286,7 +286,7 @@ inline YTiles y_tiles(int N, const YTables& yt) {
     if (cls == 0) return o;
     const int ci = yinv_chunks(N), ns = yinv_split(cls), rows = yinv_rows(cls) * 16;
     const int ti = yinv_tile(yinv_rows(cls)), li = yinv_tail(yinv_rows(cls));
-    o.inv.assign((size_t)ns * 2 * (ci * ti + li), 0.0);
+    o.inv.assign((size_t)yinv_doubles(N), 0.0);
     for (int sp = 0; sp < ns; ++sp)
         for (int c = 0; c < ci; ++c)
             for (int a = 0; a < 2; ++a)
@@ -309,7 +309,7 @@ inline YTiles y_tiles(int N, const YTables& yt) {
                         (a == 0 ? yt.T : yt.TD)[(size_t)row * N + k];
                 }
     const int cf = yfwd_chunks(nh), tf = yfwd_tile(cls), lf = yfwd_tail(cls);
-    o.fwd.assign((size_t)2 * (cf * tf + lf), 0.0);
+    o.fwd.assign((size_t)yfwd_doubles(N), 0.0);
     for (int c = 0; c < cf; ++c)
         for (int a = 0; a < 2; ++a)
             for (int slot = 0; slot <= 2 * cls * 16; ++slot)

@@ -138,6 +138,15 @@ constexpr int yfwd_chunks(int nh) {
 }
 constexpr int yinv_tail(int cls) { return 2 * 64 * cls + 8; }  // per matrix
 constexpr int yfwd_tail(int cls) { return 2 * 64 * cls + 4; }
+// doubles of the staged matrices of a grid (y_tiles)
+constexpr long yinv_doubles(int Ny) {
+    const int cls = yw_class(Ny), rows = cls ? yinv_rows(cls) : 0;
+    return cls ? 2L * yinv_split(cls) * (yinv_chunks(Ny) * yinv_tile(rows) + yinv_tail(rows)) : 0;
+}
+constexpr long yfwd_doubles(int Ny) {
+    const int cls = yw_class(Ny);
+    return cls ? 2L * (yfwd_chunks((Ny + 1) / 2) * yfwd_tile(cls) + yfwd_tail(cls)) : 0;
+}
 
 // Per-mode tau data for one lambda_t, mode-major: array k (TAU_NA of them:
 // pband pup pinvd vband vup vinvd Pp vp P0 v0) of mode m is the Ny-vector

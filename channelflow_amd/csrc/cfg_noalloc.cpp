@@ -19,9 +19,19 @@ namespace {
 
 constexpr size_t kScratchBytes = size_t(48) << 20;  // 48 MiB per device
 constexpr size_t kScratchDoubles = kScratchBytes / sizeof(double);
+// the staged copies of the y operators lie behind it, so that they take nothing
+// from the grids that fit
+constexpr size_t tile_doubles() {
+    long most = 0;
+    for (int Ny = 5; Ny <= 385; Ny += 2) {
+        const long n = yinv_doubles(Ny) + yfwd_doubles(Ny);
+        most = n > most ? n : most;
+    }
+    return (size_t)most + 64;  // two 256-byte boundaries
+}
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) double scratch[kScratchDoubles];
+__device__ __align__(256) double scratch[kScratchDoubles + tile_doubles()];
 
 double* g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
 
@@ -73,10 +83,6 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
         const size_t o_twz = carve(off, 2 * (size_t)g.Nz);
         const size_t nyy = (size_t)g.Ny * g.Ny;
         const size_t o_T = carve(off, nyy), o_TD = carve(off, nyy), o_Ti = carve(off, nyy), o_DTi = carve(off, nyy);
-        const int cls = yw_class(g.Ny);
-        const size_t n_inv = cls ? (size_t)((g.Ny + YINV_KC - 1) / YINV_KC) * 2 * yinv_split(cls) * yinv_tile(yinv_rows(cls)) : 0;
-        const size_t n_fwd = cls ? (size_t)(((g.Ny + 1) / 2 + YFWD_KC - 1) / YFWD_KC) * 2 * yfwd_tile(cls) : 0;
-        const size_t o_inv = carve(off, n_inv), o_fwd = carve(off, n_fwd);
         const size_t o_base = carve(off, 4 * (size_t)g.Ny);
         const size_t ny = (size_t)nlwork_y_doubles(g), nx = (size_t)nlwork_x_doubles(g);
         const size_t o_yp = carve(off, ny), o_fo = carve(off, ny), o_xp = carve(off, nx), o_zo = carve(off, nx);
@@ -85,6 +91,7 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
                                          std::to_string(g.Nz) + " needs " + std::to_string(off * 8) +
                                          " scratch bytes; cfg_nonlinear_noalloc holds " +
                                          std::to_string(kScratchBytes));
+        const size_t o_inv = carve(off, (size_t)yinv_doubles(g.Ny)), o_fwd = carve(off, (size_t)yfwd_doubles(g.Ny));
         init_device_limits();
         double* S = scratch_ptr();
         hipStream_t st = static_cast<hipStream_t>(stream);
@@ -110,7 +117,7 @@ extern "C" int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flag
         put(o_Ti, yt.Ti.data(), nyy * 8);
         put(o_DTi, yt.DTi.data(), nyy * 8);
         const YTiles tiles = y_tiles(g.Ny, yt);
-        if (cls) {
+        if (!tiles.inv.empty()) {
             put(o_inv, tiles.inv.data(), tiles.inv.size() * 8);
             put(o_fwd, tiles.fwd.data(), tiles.fwd.size() * 8);
         }
