@@ -186,12 +186,12 @@ def kernel_bytes(grid, method):
 
 
 def tau_factor_bytes(grid):
-    """Bytes of one tau set (one lambda) of a grid class: 12 Ny-vectors of
+    """Bytes of one tau set (one lambda) of a grid class: 10 Ny-vectors of
     doubles and 6 scalars per live mode, read by every tau launch of the
     class whatever its member count."""
     Nx, Ny, Nz = grid
     M = (2 * (Nx // 3 - 1) + 1) * (Nz // 3)
-    return 8.0 * (12 * Ny * M + 6 * M)
+    return 8.0 * (10 * Ny * M + 6 * M)
 
 
 # ---------------------------------------------------------------------------
