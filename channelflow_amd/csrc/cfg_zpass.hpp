@@ -286,11 +286,19 @@ __device__ __forceinline__ Bins zw_bins(const ZWCtx& c) {
 }
 
 // c2r of two real fields at once (fa -> pa, fb -> pb; fb < 0: none), from the
-// live bins kz < nkz of xp; dza / dzb apply d/dz. As in FFTW's c2r, the
-// imaginary part of bin 0 is ignored.
-template <class S, class Then>
-__device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
-                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV], Then&& issued) {
+// live bins kz < nkz of xp. DZ: pb is d/dz of field fa, from the same loads. SB: pb
+// passes through the transform at 1/SB of its size, a power of two and so exact: both
+// halves of a transform share its rounding, and a derivative is some times larger
+// than its field (with u_c and du_c/dz, du_c/dx and du_c/dy paired at full size the
+// convection form's w was off by 8.2e-16 of its norm, at 1/8 by 4.7e-16, as with
+// every field paired as loaded). The scale enters as the multiplier of an fma: as a
+// product of the loaded value the compiler moves it under the load's condition, where
+// every load gets a wait of its own (16 of 64^3 90 -> 108 us). As in FFTW's c2r, the
+// imaginary part of bin 0 is ignored. issued is called once the loads are under way.
+template <class S, bool DZ, int SB, class Then>
+__device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, int fb,
+                                       double (&pa)[S::PV], double (&pb)[S::PV], Then&& issued) {
+    constexpr double sb = 1.0 / SB;
     constexpr int SL = S::SL, SV = S::SV, PV = S::PV;
     const int s = c.gi;
     // Value r of lane s is bin n = s + SL r. In the lower half of the r it can
@@ -310,22 +318,21 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
         }
     };
     fetch(fa, A);
-    if (fb >= 0) fetch(fb, B);
+    if (!DZ && fb >= 0) fetch(fb, B);
     issued();
     double2 v[SV];
     const double sd = s;
 #pragma unroll
     for (int r = 0; r < SV; ++r) {
         const bool up = 2 * r + 1 > SV || (2 * r + 1 == SV && SL * r >= bins.lo);  // the mirror of bin k
-        const double k = up ? (double)(SL * (SV - r)) - sd : sd + (double)(SL * r);
-        double2 a = A[r], b = fb >= 0 ? B[r] : make_double2(0.0, 0.0);
-        if (dza) a = imul(c.dk * k, a);
-        if (dzb) b = imul(c.dk * k, b);
+        const double2 a = A[r];
+        double2 b = !DZ && fb >= 0 ? B[r] : make_double2(0.0, 0.0);
+        if (DZ) b = imul(c.dk * (up ? (double)(SL * (SV - r)) - sd : sd + (double)(SL * r)), a);
         if (up) {
-            v[r] = make_double2(a.x + b.y, b.x - a.y);  // conj(A) + i conj(B) (zero in the gap)
+            v[r] = make_double2(fma(sb, b.y, a.x), fma(sb, b.x, -a.y));  // conj(A) + i conj(B) (zero in the gap)
         } else {
-            v[r] = make_double2(a.x - b.y, a.y + b.x);  // A + iB
-            if (r == 0 && s == 0) v[r] = make_double2(a.x, b.x);
+            v[r] = make_double2(fma(-sb, b.y, a.x), fma(sb, b.x, a.y));  // A + iB
+            if (r == 0 && s == 0) v[r] = make_double2(a.x, sb * b.x);
         }
     }
     double2 u[PV];
@@ -333,14 +340,13 @@ __device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict
 #pragma unroll
     for (int m = 0; m < PV; ++m) {
         pa[m] = u[m].x;
-        pb[m] = u[m].y;
+        pb[m] = SB * u[m].y;
     }
 }
-
 template <class S>
-__device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, bool dza, int fb,
-                                       bool dzb, double (&pa)[S::PV], double (&pb)[S::PV]) {
-    zw_c2r<S>(c, xp, fa, dza, fb, dzb, pa, pb, [] {});
+__device__ __forceinline__ void zw_c2r(const ZWCtx& c, const double2* __restrict__ xp, int fa, int fb,
+                                       double (&pa)[S::PV], double (&pb)[S::PV]) {
+    zw_c2r<S, false, 1>(c, xp, fa, fb, pa, pb, [] {});
 }
 
 // r2c of pa (and pb when TWO) -> zo fields ga (and gb), bins kz < nkz.
@@ -430,9 +436,9 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
     double2* __restrict__ zo = zo0 + blockIdx.y * sx;
     if constexpr (METHOD == NL_ROT) {
         double u0[N1], u1[N1], u2[N1], w0[N1], w1[N1], w2[N1];
-        zw_c2r<S>(c, xp, 0, false, 1, false, u0, u1);
-        zw_c2r<S>(c, xp, 2, false, 3, false, u2, w0);
-        zw_c2r<S>(c, xp, 4, false, 5, false, w1, w2);
+        zw_c2r<S>(c, xp, 0, 1, u0, u1);
+        zw_c2r<S>(c, xp, 2, 3, u2, w0);
+        zw_c2r<S>(c, xp, 4, 5, w1, w2);
         double f0[N1], f1[N1], f2[N1];
 #pragma unroll
         for (int m = 0; m < N1; ++m) {  // cross(vort, u) (diffops.cpp:2598-2605)
@@ -449,8 +455,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
         zw_r2c<S, false>(c, zo, f2, f2, 2, -1);
     } else {
         double u0[N1], u1[N1], u2[N1], pa[N1], pb[N1];
-        zw_c2r<S>(c, xp, 0, false, 1, false, u0, u1);
-        zw_c2r<S>(c, xp, 2, false, -1, false, u2, pa);
+        zw_c2r<S>(c, xp, 0, 1, u0, u1);
+        zw_c2r<S>(c, xp, 2, -1, u2, pa);
         if (want_g) {  // DIV with rotation: g = rotation terms only
 #pragma unroll
             for (int m = 0; m < N1; ++m) {
@@ -496,6 +502,9 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
 // 76 us). The first bins are requested before the twiddles are waited for. Two such
 // groups of lines per block, or blocks in XCD order, are slower (16 of 64^3 100 ->
 // 115, 107; the chain of barriers couples six wavefronts).
+// u_c and du_c/dz come from one load of u_c: 9 fields are read, not 12 (16 of 64^3
+// 95.8 -> 89.8, 24 of 48^3 65.6 -> 63.7, 24 of 32^3 22.2 -> 21.7, 128^3 convection 43.3
+// -> 42.7).
 // LDS of a block: the twiddles, then the line rows of the three wavefronts, which also carry the shared values
 template <int METHOD, int NZ>
 constexpr size_t zsplit_lds() {
@@ -547,7 +556,7 @@ k_zsplit(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ t
     auto get = [&](int f, int m) { return ex[(f * PV + m) * 64 + lane]; };
     if constexpr (METHOD == NL_ROT) {
         double u[PV], w[PV];
-        zw_c2r<S>(c, xp, cc, false, 3 + cc, false, u, w, twiddles);
+        zw_c2r<S, false, 1>(c, xp, cc, 3 + cc, u, w, twiddles);
         __syncthreads();
         share(cc, u);
         share(3 + cc, w);
@@ -586,8 +595,8 @@ k_zsplit(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ t
         constexpr bool SK = (METHOD == NL_SKEW);
         constexpr double s = SK ? 0.5 : 1.0, us = SK ? 2.0 : 1.0;
         double h[PV], dx[PV], dy[PV], dz[PV], f[PV];
-        zw_c2r<S>(c, xp, cc, false, 6 + cc, false, h, dx, twiddles);
-        zw_c2r<S>(c, xp, 3 + cc, false, cc, true, dy, dz);
+        zw_c2r<S, true, 8>(c, xp, cc, -1, h, dz, twiddles);      // u_c, du_c/dz
+        zw_c2r<S, false, 8>(c, xp, 6 + cc, 3 + cc, dx, dy, [] {});  // du_c/dx, du_c/dy
         if constexpr (SK) {
 #pragma unroll
             for (int m = 0; m < PV; ++m) h[m] *= s;
@@ -633,7 +642,7 @@ k_zsplit(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ t
         }
     } else {
         double u[PV], pa[PV], pb[PV], ga[PV], gb[PV];
-        zw_c2r<S>(c, xp, cc, false, -1, false, u, pa, twiddles);
+        zw_c2r<S, false, 1>(c, xp, cc, -1, u, pa, twiddles);
         __syncthreads();
         share(cc, u);
         __syncthreads();
