@@ -57,6 +57,61 @@ __global__ void __launch_bounds__(256) k_zcfl(Geom g, FFTPlan pz, int XB, const 
     }
 }
 
+// The same with a wavefront per group of lines, for the wavefront FFT lengths: the
+// transforms have no block barriers, and a line's largest value is divided instead of
+// every value (division by a positive spacing is monotone, so the result is the same).
+// us per launch, LDS lines -> wavefront lines: 48x35x48 12.6 -> 6.5 (and 5.7 -> 1.7 for
+// the reduction of its fewer blocks), 32^3 9.0 -> 5.2, 64^3 12.5 -> 6.2, 96^3 31.3 -> 11.2,
+// 128^3 63 -> 18, 192x129x192 128 -> 32.
+template <int NZ>
+__global__ void __launch_bounds__(256) k_zcfl_w(Geom g, const double2* __restrict__ twg,
+                                                const NLMember* __restrict__ tab, const double2* __restrict__ xp0,
+                                                long sx, double* __restrict__ part) {
+    using S = ZLine<NZ>;
+    constexpr int PV = S::PV;
+    extern __shared__ double2 lds[];
+    __shared__ double red[4];
+    for (int i = threadIdx.x; i < S::TWN; i += 256) lds[i] = twg[S::tw_power(i)];
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int nxc = (g.Nx + S::LPW - 1) / S::LPW;
+    const int wg = min((int)blockIdx.x * 4 + wave, g.Ny * nxc - 1);  // the last block may repeat a group
+    const int y = wg / nxc, L = lane / S::G, x = (wg - y * nxc) * S::LPW + L;
+    ZWCtx c;
+    c.gi = lane % S::G;
+    c.line_ok = x < g.Nx;
+    c.base = ((long)y * g.Nx + (c.line_ok ? x : 0)) * g.nkz;
+    c.fsz = (long)g.Ny * g.Nx * g.nkz;
+    c.nkz = g.nkz;
+    c.dk = 2 * PI / g.Lz;
+    c.T = lds + S::TWN + (wave * S::LPW + L) * S::LBUF;
+    c.tw = lds;
+    const double2* __restrict__ xp = xp0 + blockIdx.y * sx;
+    double u0[PV], u1[PV], u2[PV], none[PV];
+    zw_c2r<S>(c, xp, 0, 1, u0, u1);
+    zw_c2r<S>(c, xp, 2, -1, u2, none);
+    const int Ny = g.Ny;
+    const double piN = PI / (Ny - 1), rad = (g.b - g.a) / 2, cen = (g.b + g.a) / 2;
+    auto yc = [&](int j) { return cen + rad * cos(j * piN); };
+    const double dy = (y == 0 || y == Ny - 1) ? yc(0) - yc(1) : (yc(y - 1) - yc(y + 1)) / 2.0;
+    double m = 0.0;
+    if (c.line_ok && c.gi < S::PL) {
+        const double vs = tab[blockIdx.y].Vsuck;
+        double m0 = u0[0], m1 = u1[0] + vs, m2 = u2[0];
+#pragma unroll
+        for (int k = 1; k < PV; ++k) {
+            m0 = fmax(m0, u0[k]);
+            m1 = fmax(m1, u1[k] + vs);
+            m2 = fmax(m2, u2[k]);
+        }
+        m = fmax(fmax(m, m0 / (g.Lx / g.Nx)), fmax(m1 / dy, m2 / (g.Lz / g.Nz)));
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) part[(long)blockIdx.y * gridDim.x + blockIdx.x] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
 __global__ void __launch_bounds__(256) k_cfl_reduce(int nb, const double* __restrict__ part, double* __restrict__ out) {
     __shared__ double red[4];
     const double* p = part + (long)blockIdx.x * nb;
@@ -112,28 +167,36 @@ void launch_z_any(int method, const Geom& g, const FFTPlan& pz, int n, const NLM
     }
 }
 
+// returns the partial maxima per member
 template <int NZ>
-static void launch_zcfl_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, const double2* xp, long sx,
-                          double* part, int XB, hipStream_t st) {
-    const size_t lds = (size_t)g.Nz * sizeof(double2) +
-                       (size_t)XB * (2 * lpitch(g.Nz) * sizeof(double2) + (size_t)g.Nz * 3 * sizeof(double));
-    const dim3 grid(g.Ny * ((g.Nx + XB - 1) / XB), n);
-    allow_lds(k_zcfl<NZ>, lds);
-    k_zcfl<NZ><<<grid, 256, lds, st>>>(g, pz, XB, tab, xp, sx, part);
+static int launch_zcfl_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, const double2* xp, long sx,
+                         double* part, hipStream_t st) {
+    if constexpr (zwave_size(NZ)) {
+        using S = ZLine<NZ>;
+        const int nb = (g.Ny * ((g.Nx + S::LPW - 1) / S::LPW) + 3) / 4;
+        constexpr size_t lds = (size_t)(S::TWN + 4 * S::LPW * S::LBUF) * sizeof(double2);
+        allow_lds(k_zcfl_w<NZ>, lds);
+        k_zcfl_w<NZ><<<dim3((unsigned)nb, n), 256, lds, st>>>(g, pz.tw, tab, xp, sx, part);
+        return nb;
+    } else {
+        const int XB = zpass_xb_max(g, 3), nb = g.Ny * ((g.Nx + XB - 1) / XB);
+        const size_t lds = (size_t)g.Nz * sizeof(double2) +
+                           (size_t)XB * (2 * lpitch(g.Nz) * sizeof(double2) + (size_t)g.Nz * 3 * sizeof(double));
+        allow_lds(k_zcfl<NZ>, lds);
+        k_zcfl<NZ><<<dim3((unsigned)nb, n), 256, lds, st>>>(g, pz, XB, tab, xp, sx, part);
+        return nb;
+    }
 }
 
 int launch_zcfl(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, const double2* xp, long sx, double* part,
                 hipStream_t st) {
-    const int XB = zpass_xb_max(g, 3);
-    const int nb = g.Ny * ((g.Nx + XB - 1) / XB);
     switch (g.Nz) {
 #define CASE_Z(N) \
-    case N: launch_zcfl_t<N>(g, pz, n, tab, xp, sx, part, XB, st); break;
+    case N: return launch_zcfl_t<N>(g, pz, n, tab, xp, sx, part, st);
         CFG_FFT_SIZES(CASE_Z)
 #undef CASE_Z
-        default: launch_zcfl_t<0>(g, pz, n, tab, xp, sx, part, XB, st);
+        default: return launch_zcfl_t<0>(g, pz, n, tab, xp, sx, part, st);
     }
-    return nb;
 }
 
 void launch_cfl_reduce(int n, int nb, const double* part, double* out, hipStream_t st) {

@@ -292,6 +292,20 @@ def test_cfl_matches_oracle(gpu, case):
     assert abs(c6_gpu - c6_ref) <= 1e-12 * abs(c6_ref)
 
 
+@pytest.mark.parametrize("Nz", [16, 18, 32, 48, 64, 72, 96, 162, 192, 256])
+def test_cfl_line_lengths(gpu, Nz):
+    """The CFL factor's wavefront lines, two- and three-step, with line counts that do
+    not fill the last group and block, where the x (36 points), y (Ny = 65) or z spacing
+    decides; the 1e-12 bar of test_cfl_matches_oracle."""
+    for Nx, Ny in ((6, 9), (36, 9), (6, 65)):
+        u0 = random_field(Nx, Ny, Nz, LX_C, LZ_C, norm=0.5, decay=0.6, seed=Nz, dealias=False)
+        flags = dict(C1_FLAGS, dealiasing="NoDealiasing", Vsuck=0.01)
+        _, _, _, _, _, ref, dns = run_pair(Nx, Ny, Nz, LX_C, LZ_C, flags, u0, 0)
+        r, v = ref.cfl(), dns.CFL()
+        print(Nx, Ny, Nz, "CFL oracle", r, "gpu", v, flush=True)
+        assert abs(v - r) <= 1e-12 * abs(r)
+
+
 def test_variable_dt_loop(gpu):
     """simulateflow's loop (programs/simulateflow.cpp:131-142): advance n steps, CFL,
     TimeStep.adjust, reset_dt on a change -- same dt sequence and states within
