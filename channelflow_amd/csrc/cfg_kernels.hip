@@ -583,8 +583,9 @@ __global__ void __launch_bounds__(256) k_yfwd_t(Geom g, YMats ym, int have_g, co
 // 17.0 -> 14.4, 19.1 -> 13.8; 128^3 convection 41 -> 35, 22 -> 19; 192x129x192 81 ->
 // 63, 44 -> 35; 16 of 64^3 52 -> 46, 51 -> 44. The inverse at 192x129x192 then takes
 // 24 us for its loads alone, 23 us of matrix products at their peak rate and writes
-// 96 MB (20 us at the copy rate), one after the other in each block; loading two or
-// three chunks ahead, or four waves per SIMD, changes nothing.
+// 96 MB (20 us at the copy rate), one after the other in each block. Loading two or
+// three chunks ahead is slower (67, 72), and so are two column tiles per wave (71: the
+// registers leave half the blocks).
 //
 // Both transforms use the mirror symmetry of the Chebyshev points,
 // y_{Ny-1-j} = -y_j: T[Ny-1-j][k] = (-1)^k T[j][k], and the derivative flips
@@ -638,8 +639,20 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
     const int sp = bid.x % NSP, rt0 = sp * NRT;  // this block's row tiles
     const long m0 = (long)(bid.x / NSP) * YW_MODES;
     const long mcol = m0 + (lr >> 1);
+    // Two and four row tiles load without conditions (modes past M read mode M - 1 and are
+    // dropped, coefficients past Ny meet zeros of the staged matrix) at a uniform base
+    // and a 32-bit lane offset: 80 registers, not 89, and so 6 wavefronts, four blocks
+    // (128^3 31.4 -> 29.9 us, convection 33.2 -> 31.0, 192x129x192 62.6 -> 57.5). Where the
+    // occupancy stays the same the condition saves the loads (one 32^3 field 4.7
+    // against 4.9, 96^3 14.2 against 14.5).
+    constexpr bool ALL = NRT % 2 == 0;
     const bool mok = mcol < M;
-    const gcdouble ucol = gmem(me.u) + 2 * ((long)c * Ny * M + mcol) + (l & 1);
+    const gbytes ub = reinterpret_cast<gbytes>(gmem(me.u) + 2 * (long)c * Ny * M);
+    const unsigned uoff = (unsigned)(2 * min(mcol, M - 1) + (l & 1)) * 8u;
+    auto coefficient = [&](int k) {
+        if (ALL) return *reinterpret_cast<gcdouble>(ub + (16L * min(k, Ny - 1) * M + uoff));
+        return (mok && k < Ny) ? *reinterpret_cast<gcdouble>(ub + (16L * k * M + uoff)) : 0.0;
+    };
     const int nch = yinv_chunks(Ny), kend = nch * KC;
     mfma4d ae[NRT], ao[NRT];
     double dmid = 0.0;
@@ -648,7 +661,7 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int k = k0 + 2 * (4 * (i & 1) + lk) + (i >> 1);
-            bn[i] = (mok && k < Ny) ? ucol[2L * k * M] : 0.0;
+            bn[i] = coefficient(k);
         }
     };
     dvec2 mv[NST];
@@ -666,7 +679,7 @@ __global__ void __launch_bounds__(METHOD == NL_DIV ? 192 : 384) __attribute__((a
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             const int k = kend + 2 * lk + p;
-            tb[p] = (mok && k < Ny) ? ucol[2L * k * M] : 0.0;
+            tb[p] = coefficient(k);
             tm[p] = tail[2 * 64 * NRT + 4 * p + lk];
 #pragma unroll
             for (int rt = 0; rt < NRT; ++rt) ta[rt][p] = tail[(rt * 2 + p) * 64 + l];
