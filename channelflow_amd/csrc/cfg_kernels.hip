@@ -820,7 +820,7 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     const int Ny = g.Ny, nh = (Ny + 1) / 2, nm = Ny / 2;
     const bool odd = Ny & 1;
     const long M = g.M;
-    const int c = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4, part = l & 1;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, lr = l & 15, lk = l >> 4, part = l & 1;
     const long mcol = (long)bid.x * YW_MODES + (lr >> 1);
     const bool mok = mcol < M;
     const double beta = (METHOD == NL_SKEW) ? 0.5 : 1.0;
@@ -839,14 +839,17 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     const bool XTERM = !(METHOD == NL_SKEW && xfold);
     const int f0 = c == 0 ? 3 : (c == 1 ? 4 : 5), f2 = c == 0 ? 5 : (c == 1 ? 7 : 8);
     const int f1 = XTERM ? (c == 0 ? 4 : (c == 1 ? 6 : 7)) : 3 + c;
-    const long rowst = 2 * M;
-    // columns past M read mode M - 1 (every field of fo has Ny x M modes); the
-    // values are masked where they are used
-    const long mcl = mok ? mcol : M - 1;
-    const double* __restrict__ pg = fo + 2 * ((long)c * Ny * M + mcl) + part;
-    const double* __restrict__ p0 = fo + 2 * ((long)f0 * Ny * M + mcl) + (1 - part);
-    const double* __restrict__ p1 = fo + 2 * ((long)f1 * Ny * M + mcl) + part;
-    const double* __restrict__ p2 = fo + 2 * ((long)f2 * Ny * M + mcl) + (1 - part);
+    // Every access is at a component's uniform base and a 32-bit lane offset; with a
+    // 64-bit pointer per field and lane two to four row tiles held 16 registers more,
+    // a wavefront per SIMD less (us per launch, before -> after: 192x129x192 34.1 ->
+    // 28.4, 128^3 18.2 -> 17.3, 16 of 64^3 45.0 -> 42.3, 4 of 96^3 40.1 -> 38.4, 54x57x72
+    // 8.8 -> 8.1). Columns past M read mode M - 1 (every field of fo has Ny x M modes);
+    // the values are masked where they are used.
+    const unsigned rowb = (unsigned)M * 16u, mcl = (unsigned)(mok ? mcol : M - 1);
+    const unsigned own = (2 * mcl + part) * 8u, other = (2 * mcl + 1 - part) * 8u;
+    auto field = [&](int i) { return reinterpret_cast<gbytes>(gmem(fo) + 2 * (long)i * Ny * M); };
+    const gbytes pg = field(c), p0 = field(f0), p1 = field(f1), p2 = field(f2);
+    auto at = [](gbytes b, unsigned o) { return *reinterpret_cast<gcdouble>(b + o); };
     const int nch = yfwd_chunks(nh), yend = nch * KC;
     mfma4d ae[NRT], ao[NRT];
     double dlast = 0.0;
@@ -860,18 +863,19 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     double rv[NS][NR];
     auto fetch1 = [&](int y0, double (&r)[NR]) {
         const int y = min(y0 + lk, nh - 1), ymr = Ny - 1 - y;
-        r[0] = pg[y * rowst];
-        r[1] = pg[ymr * rowst];
+        const unsigned u = y * rowb, d = ymr * rowb;
+        r[0] = at(pg, u + own);
+        r[1] = at(pg, d + own);
         if (DIVF) {
-            r[2] = p1[y * rowst];
-            r[3] = p1[ymr * rowst];
+            r[2] = at(p1, u + own);
+            r[3] = at(p1, d + own);
             if (XTERM) {
-                r[4] = p0[y * rowst];
-                r[5] = p0[ymr * rowst];
+                r[4] = at(p0, u + other);
+                r[5] = at(p0, d + other);
             }
             if (ZTERM) {
-                r[6] = p2[y * rowst];
-                r[7] = p2[ymr * rowst];
+                r[6] = at(p2, u + other);
+                r[7] = at(p2, d + other);
             }
         }
     };
@@ -992,19 +996,20 @@ __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(yw_wav
     dlast += __shfl_xor(dlast, 16);
     dlast += __shfl_xor(dlast, 32);
     if (!mok) return;
-    __attribute__((address_space(1))) double* __restrict__ fc = f + 2 * ((long)c * Ny * M + mcol) + part;
+    const gbytes_w fc = reinterpret_cast<gbytes_w>(f + 2 * (long)c * Ny * M);
+    auto put = [&](int k, double v) { *reinterpret_cast<__attribute__((address_space(1))) double*>(fc + (k * rowb + own)) = v; };
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = rt * 16 + 4 * r + lk;
             if (i < nm) {
-                fc[2 * i * rowst] = ae[rt][r];
-                fc[(2 * i + 1) * rowst] = ao[rt][r];
+                put(2 * i, ae[rt][r]);
+                put(2 * i + 1, ao[rt][r]);
             }
         }
     }
-    if (odd && lk == 0) fc[(Ny - 1) * rowst] = dlast;
+    if (odd && lk == 0) put(Ny - 1, dlast);
 }
 
 // Row-tile count classes with a wave-column kernel; above the last one the
