@@ -783,7 +783,7 @@ def _counter_rows(path, counter):
             if r["Counter_Name"] != counter:
                 continue
             name = r["Kernel_Name"]
-            m = re.search(r"cfg::(k_\w+?)(?:_wave|_w|_t)?(?:<|\()", name)  # variants count as their kernel
+            m = re.search(r"cfg::(k_\w+?)(?:_wave|_w|_tall|_t)?(?:<|\()", name)  # variants count as their kernel
             short = m.group(1) if m else name.split("(")[0].strip()
             rows.append((KERNEL_ALIAS.get(short, short), float(r["Counter_Value"])))
     return rows

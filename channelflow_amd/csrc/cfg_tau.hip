@@ -201,14 +201,83 @@ __device__ __forceinline__ void tau_stage(const TauMember& me, const Geom& g, in
 // [mode][part][comp] of tau_pitch(Ny) doubles, then the rows of B (3 of 2KW
 // doubles, zero past Ny).
 __host__ __device__ constexpr int tau_pitch(int Ny) { return Ny + 1; }  // even (Ny is odd): 16-byte pairs
-constexpr size_t tau_lds(int Ny, int K, int W, int MPB) {
-    return ((size_t)MPB * 6 * tau_pitch(Ny) + (size_t)3 * 2 * K * W) * sizeof(double);
+// Doubles of a row per lane (wrow_pos): padded above 16 lanes at K = 4 (128x193x128 with
+// 8 doubles 120 us, with 10 107)
+constexpr int tau_lp(int K) { return K == 4 ? 2 * K + 2 : 2 * K; }
+template <int K>
+__host__ __device__ constexpr int tau_row(int Ny) { return (wrow_pos<K, tau_lp(K)>(Ny) + 2) / 2 * 2; }
+constexpr size_t tau_lds(int row, int lane, int W, int MPB) {
+    return ((size_t)MPB * 6 * row + (size_t)3 * lane * W) * sizeof(double);
 }
 
 // Waves per SIMD a variant is compiled for, where its registers fit without
 // spilling more than a few values (K = 5: 256 registers; a third wave at K = 3
 // spills 164 bytes, one 64^3 field 14.6 -> 21.3 us).
-constexpr int tau_waves(int K, int W) { return W == 16 && K <= 5 ? (K == 1 ? 4 : K == 2 ? 3 : 2) : 1; }
+constexpr int tau_waves(int K) { return K == 1 ? 4 : K == 2 ? 3 : K <= 5 ? 2 : 1; }
+
+// The kx = kz = 0 mode: P from Ry', v = 0, u and w from the velocity operator; real
+// parts only. For a whole block, c and seg as in the kernels below.
+template <int K, int W, int NTHR, int LP, class Op>
+__device__ __forceinline__ void tau_mean_mode(const Geom& g, const TauMember& me, const TauSet& s, double nu,
+                                              const gcdouble coef, double* const R, int RP, int seg, const WCtx& c,
+                                              __attribute__((address_space(1))) dvec2* __restrict__ u,
+                                              __attribute__((address_space(1))) dvec2* __restrict__ q) {
+    const int Ny = g.Ny;
+    auto at = [&](int row) { return LP == 2 * K ? row + row / Ny * (RP - Ny) : row / Ny * RP + wrow_pos<K, LP>(row % Ny); };
+    for (int row = threadIdx.x; row < 3 * Ny; row += NTHR) {
+        double acc = 0.0;
+        for (int j = 0; j < me.nterms; ++j) acc += me.coef[j] * gmem(me.in[j])[2L * row * g.M];
+        R[at(row)] = acc;
+    }
+    __syncthreads();
+    const SolveConst zc = me.sc;
+    // segment 0 solves for P, the first two from the next wavefront on for u and w
+    constexpr int U0 = 64 / W;
+    static_assert(NTHR / W >= U0 + 2, "the block has these segments");
+    if (seg == 0) {
+        const Op op(coef, Ny, 0, 0u, 0.0, c);
+        WV<K> y[1], f[1], x[1];
+        y[0] = wrow_load<K, W, LP>(R + RP, c);
+        wdiff_n<K, W, 1>(y, c, f);
+        op.template solve<1>(f, c, x);
+        wrow_store<K, W, LP>(R + RP, c, x[0]);
+    } else if (seg == U0 || seg == U0 + 1) {
+        const int cc = seg - U0;
+        double* const S = R + 2 * cc * RP;
+        const Op op(coef, Ny, 3, 0u, s.lambda_t, c);
+        const WV<K> r = wrow_load<K, W, LP>(S, c);
+        const WV<K> Byy = wload<K, W>(gmem(cc == 0 ? zc.nuUbaseyy : zc.nuWbaseyy), c);
+        WV<K> f[1], x[1];  // nse.cpp:505-527: nu U'' (nu W''), and a fixed mean gradient
+        for (int i = 0; i < K; ++i) {
+            f[0].e[i] = -(r.e[i] + Byy.e[i]);
+            f[0].o[i] = -(r.o[i] + Byy.o[i]);
+        }
+        if (zc.bulk) {  // bulk-velocity constraint (tausolver.cpp:404-450, helmholtz.cpp:158-213)
+            WV<K> two[2], sol[2];
+            two[0] = f[0];
+            two[1] = wzero<K, W>();
+            if (c.lane == 0) two[1].e[0] = nu;
+            op.template solve<2>(two, c, sol);
+            const double uamean = wmean<K, W>(sol[0], c), ucmean = wmean<K, W>(sol[1], c);
+            const double mu = nu * ((cc == 0 ? zc.umean : zc.wmean) - uamean) / ucmean;
+            if (c.lane == 0) {
+                f[0].e[0] += mu;
+                *(cc == 0 ? zc.dPdx_out : zc.dPdz_out) = mu;
+            }
+        } else if (c.lane == 0) {
+            f[0].e[0] += cc == 0 ? zc.dPdxRef : zc.dPdzRef;
+        }
+        op.template solve<1>(f, c, x);
+        wrow_store<K, W, LP>(S, c, x[0]);
+    }
+    __syncthreads();
+    for (int row = threadIdx.x; row < 3 * Ny; row += NTHR) {
+        const double v = R[at(row)];
+        const bool mid = row >= Ny && row < 2 * Ny;
+        if (mid) q[(long)(row - Ny) * g.M] = dvec2{v, 0.0};
+        u[(long)row * g.M] = dvec2{mid ? 0.0 : v, 0.0};
+    }
+}
 
 // Blocks of a launch, in XCD order: per member the block of the kx = kz = 0
 // mode alone (its mean-flow solves would run one after the other with the
@@ -226,7 +295,7 @@ constexpr int tau_waves(int K, int W) { return W == 16 && K <= 5 ? (K == 1 ? 4 :
 // 2200): one 32^3 field 20.5 -> 9.2 us, 64^3 31.3 -> 14.6, 96^3 39.5 -> 23.5,
 // 128^3 66.7 -> 48.0, 192x129x192 138.7 -> 120.8, 24 x 32^3 26.8 -> 20.8.
 template <int K, int W, int MPB>
-__global__ void __launch_bounds__(2 * W * MPB) __attribute__((amdgpu_waves_per_eu(tau_waves(K, W))))
+__global__ void __launch_bounds__(2 * W * MPB) __attribute__((amdgpu_waves_per_eu(tau_waves(K))))
 k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMember* __restrict__ tab) {
     extern __shared__ double2 lds2[];
     double* const lds = reinterpret_cast<double*>(lds2);
@@ -259,61 +328,8 @@ k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMembe
     const gcdouble coef = gmem(s.coef);
     const double pi2 = PI * PI;
 
-    if (mblk == 0) {  // kx = kz = 0: P from Ry', v = 0, u and w from the velocity operator; real parts only
-        double* const R = lds;  // [comp][RP]
-        for (int row = threadIdx.x; row < 3 * Ny; row += nthr) {
-            double acc = 0.0;
-            for (int j = 0; j < me.nterms; ++j) acc += me.coef[j] * gmem(me.in[j])[2L * row * g.M];
-            R[row + row / Ny * (RP - Ny)] = acc;
-        }
-        __syncthreads();
-        const SolveConst zc = me.sc;
-        // segment 0 solves for P, the first two of the next wavefront for u and w
-        constexpr int U0 = 64 / W;
-        static_assert(U0 >= 2 && 2 * MPB >= U0 + 2, "two segments in a wavefront, two wavefronts in a block");
-        if (seg == 0) {
-            const HelmOp<K, W> op(wfac3<K, W>(coef, Ny, 0, 0u, c), 0.0, c);
-            WV<K> y[1], f[1], x[1];
-            y[0] = wrow_load<K, W>(R + RP, c);
-            wdiff_n<K, W, 1>(y, c, f);
-            op.template solve<1>(f, c, x);
-            wrow_store<K, W>(R + RP, c, x[0]);
-        } else if (seg == U0 || seg == U0 + 1) {
-            const int cc = seg - U0;
-            double* const S = R + 2 * cc * RP;
-            const HelmOp<K, W> op(wfac3<K, W>(coef, Ny, 3, 0u, c), s.lambda_t, c);
-            const WV<K> r = wrow_load<K, W>(S, c);
-            const WV<K> Byy = wload<K, W>(gmem(cc == 0 ? zc.nuUbaseyy : zc.nuWbaseyy), c);
-            WV<K> f[1], x[1];  // nse.cpp:505-527: nu U'' (nu W''), and a fixed mean gradient
-            for (int i = 0; i < K; ++i) {
-                f[0].e[i] = -(r.e[i] + Byy.e[i]);
-                f[0].o[i] = -(r.o[i] + Byy.o[i]);
-            }
-            if (zc.bulk) {  // bulk-velocity constraint (tausolver.cpp:404-450, helmholtz.cpp:158-213)
-                WV<K> two[2], sol[2];
-                two[0] = f[0];
-                two[1] = wzero<K, W>();
-                if (c.lane == 0) two[1].e[0] = nu;
-                op.template solve<2>(two, c, sol);
-                const double uamean = wmean<K, W>(sol[0], c), ucmean = wmean<K, W>(sol[1], c);
-                const double mu = nu * ((cc == 0 ? zc.umean : zc.wmean) - uamean) / ucmean;
-                if (c.lane == 0) {
-                    f[0].e[0] += mu;
-                    *(cc == 0 ? zc.dPdx_out : zc.dPdz_out) = mu;
-                }
-            } else if (c.lane == 0) {
-                f[0].e[0] += cc == 0 ? zc.dPdxRef : zc.dPdzRef;
-            }
-            op.template solve<1>(f, c, x);
-            wrow_store<K, W>(S, c, x[0]);
-        }
-        __syncthreads();
-        for (int row = threadIdx.x; row < 3 * Ny; row += nthr) {
-            const double v = R[row + row / Ny * (RP - Ny)];
-            const bool mid = row >= Ny && row < 2 * Ny;
-            if (mid) q[(long)(row - Ny) * g.M] = dvec2{v, 0.0};
-            u[(long)row * g.M] = dvec2{mid ? 0.0 : v, 0.0};
-        }
+    if (mblk == 0) {
+        tau_mean_mode<K, W, nthr, 2 * K, HelmOp<K, W>>(g, me, s, nu, coef, lds, RP, seg, c, u, q);
         return;
     }
 
@@ -428,6 +444,204 @@ k_tau_solve_wave(Geom g, const double* __restrict__ hb, int nmem, const TauMembe
     }
     __syncthreads();
     wrow_store<K, W>(Sy, c, P[0]);
+    __syncthreads();
+    for (int row = Ny + threadIdx.x / MPB; row < 2 * Ny; row += nthr / MPB) {
+        const double a = lds[slot(ww, 0, row)], b = lds[slot(ww, 1, row)];
+        if (out) q[(long)(row - Ny) * g.M + mm] = dvec2{a, b};
+    }
+}
+
+// The same above Ny = 191, where a mode's profiles take 32 or 64 lanes. A block of 4
+// modes (64-byte pieces of a row) is 4 wavefronts, and what decides is how many blocks
+// a compute unit holds, so that one loads its rows while another solves: the velocity
+// operator is not held from v's solve to u's and w's, but formed one parity system at a
+// time (HelmParts), which leaves 2 wavefronts per SIMD. Held, K = 4 on 32 lanes took 298
+// registers and K = 6 408: a block alone on its compute unit. NP: real parts per
+// segment. At NP = 2 (K = 3 on 64 lanes, above Ny = 255) both parts of a mode share its
+// operators, and a block of 4 modes still has 4 wavefronts. LP: doubles of an LDS row
+// per lane (wrow_pos).
+// us per launch, SBDF3: a segment per complex mode / this kernel's shapes with the
+// operator held / now. Ny = 193: one field of 32xNyx32 37.0 / 25.4 / 25.0, 128xNyx128 107.0 /
+// 128.4 / 98.9, 8 of 32xNyx32 54.6 / 59.1 / 44.1, 24 of them 142.1 / 176.4 / 143.5; Ny = 257:
+// 43.0 / 30.2 / 31.8, 138.7 / 162.5 / 132.8, 65.1 / 74.0 / 63.7, 196.1 / 223.9 / 194.4; Ny = 321:
+// 45.4 / 33.4 / 34.6, 158.5 / 182.1 / 151.2, 76.5 / 86.6 / 73.9, 228.7 / 264.2 / 231.0.
+template <int K, int W, int MPB, int NP>
+__global__ void __launch_bounds__(2 * W * MPB / NP) __attribute__((amdgpu_waves_per_eu(2)))
+k_tau_solve_tall(Geom g, const double* __restrict__ hb, int nmem, const TauMember* __restrict__ tab) {
+    extern __shared__ double2 lds2[];
+    double* const lds = reinterpret_cast<double*>(lds2);
+    constexpr int nthr = 2 * W * MPB / NP, LP = tau_lp(K), HP = LP * W;
+    using Op = HelmParts<K, W, LP>;
+    auto pos = [](int n) { return wrow_pos<K, LP>(n); };
+    int mblk, mem;
+    xcd_block(nmem, mblk, mem);
+    const TauMember& me = tab[mem];
+    const TauSet s = me.set;
+    const double nu = me.nu;
+    const int taucorr = me.taucorr;
+    __attribute__((address_space(1))) dvec2* __restrict__ u = gmem_w(reinterpret_cast<dvec2*>(me.u));
+    __attribute__((address_space(1))) dvec2* __restrict__ q = gmem_w(reinterpret_cast<dvec2*>(me.q));
+    const int Ny = g.Ny, RP = tau_row<K>(Ny);
+    double* const hbl = lds + MPB * 6 * RP;
+    for (int i = threadIdx.x; i < 3 * HP; i += nthr) {
+        const int r = i / HP, at = i % HP, n = at % LP < 2 * K ? 2 * K * (at / LP) + at % LP : Ny;
+        hbl[i] = n < Ny ? hb[r * Ny + n] : 0.0;
+    }
+    for (int i = threadIdx.x; i < 6 * MPB; i += nthr) lds[i * RP + pos(Ny)] = 0.0;  // the rows' padding
+    WCtx c;
+    c.N = Ny;
+    c.Me = (Ny + 1) / 2;
+    c.Mo = (Ny - 1) / 2;
+    c.Nb = Ny - 1;
+    c.Nc = Ny - 1;
+    c.lane = threadIdx.x % W;
+    c.L = g.b - g.a;
+    c.hb = hbl;
+    const int seg = threadIdx.x / W;
+    const gcdouble coef = gmem(s.coef);
+    if (mblk == 0) {
+        tau_mean_mode<K, W, nthr, LP, Op>(g, me, s, nu, coef, lds, RP, seg, c, u, q);
+        return;
+    }
+
+    const int m0 = (mblk - 1) * MPB;
+    // the segment's mode and its first part: part 0 takes Ry.re, Rx.im, Rz.im; part 1 Ry.im, Rx.re, Rz.re
+    const int w = NP == 2 ? seg : seg >> 1, part = NP == 2 ? 0 : seg & 1;
+    const int m = min(m0 + w, g.M - 1);
+    auto slot = [&](int ww, int pt, int row) {
+        const int comp = (row >= Ny) + (row >= 2 * Ny);
+        return ((ww * 2 + pt) * 3 + comp) * RP + pos(row - comp * Ny);
+    };
+    const unsigned fo = (unsigned)m * (TAU_NA * Ny);  // this mode's factors
+    tau_stage<MPB>(me, g, m0, nthr, [&](int ww, int row, dvec2 v) {
+        const bool mid = row >= Ny && row < 2 * Ny;
+        lds[slot(ww, 0, row)] = mid ? v.x : v.y;
+        lds[slot(ww, 1, row)] = mid ? v.y : v.x;
+    });
+    __syncthreads();
+    const int ikx = m % g.nkx, ikz = m / g.nkx;
+    const int kx = kx_of(g, ikx), kz = ikz;
+    const double kk = (kx / g.Lx) * (kx / g.Lx) + (kz / g.Lz) * (kz / g.Lz);
+    const double kappa2 = 4 * (PI * PI) * kk;
+    const double lambda = s.lambda_t + (4.0 * (PI * PI) * nu) * kk;
+    auto each = [](auto&& fn) {  // for each of the segment's parts
+        fn(0);
+        if constexpr (NP == 2) fn(1);
+    };
+    double ax[NP], az[NP];
+    double *Sx[NP], *Sy[NP], *Sz[NP];
+    each([&](int p) {
+        const double sgn = part + p ? -1.0 : 1.0;
+        ax[p] = sgn * (2 * PI * kx / g.Lx);
+        az[p] = sgn * (2 * PI * kz / g.Lz);
+        Sx[p] = lds + ((seg * NP + p) * 3 + 0) * RP;
+        Sy[p] = lds + ((seg * NP + p) * 3 + 1) * RP;
+        Sz[p] = lds + ((seg * NP + p) * 3 + 2) * RP;
+    });
+    WV<K> P[NP], v[NP];
+    {
+        WV<K> f[NP], t[NP];
+        each([&](int p) { t[p] = wrow_load<K, W, LP>(Sy[p], c); });
+        wdiff_n<K, W, NP>(t, c, f);
+        each([&](int p) {
+            const WV<K> X = wrow_load<K, W, LP>(Sx[p], c), Z = wrow_load<K, W, LP>(Sz[p], c);
+            for (int k = 0; k < K; ++k) {
+                f[p].e[k] -= ax[p] * X.e[k] + az[p] * Z.e[k];
+                f[p].o[k] -= ax[p] * X.o[k] + az[p] * Z.o[k];
+            }
+        });
+        const Op op(coef, Ny, 0, fo, kappa2, c);
+        op.template solve<NP>(f, c, P);
+    }
+    const Op vop(coef, Ny, 3, fo, lambda, c);  // velocity operator: v, then u and w
+    {
+        WV<K> f[NP], t[NP];
+        wdiff_n<K, W, NP>(P, c, f);
+        each([&](int p) {
+            t[p] = wrow_load<K, W, LP>(Sy[p], c);
+            for (int k = 0; k < K; ++k) {
+                f[p].e[k] -= t[p].e[k];
+                f[p].o[k] -= t[p].o[k];
+            }
+        });
+        vop.template solve<NP>(f, c, v);
+        // influence-matrix correction (tausolver.cpp:178-191)
+        double dvb[NP], dva[NP];
+        wdiff_n<K, W, NP>(v, c, f);
+        wends_n<K, W, NP>(f, c, dvb, dva);
+        const gcdouble sc = gmem(s.scal) + 6L * m;
+        double dplus[NP], dminus[NP];
+        each([&](int p) {
+            dplus[p] = -sc[0] * dvb[p] - sc[1] * dva[p];
+            dminus[p] = -sc[2] * dvb[p] - sc[3] * dva[p];
+        });
+        // P- and v- are the mirrors of P+ and v+: (e, -o) and (-e, o)
+        const WV<K> Pp = wfac<K, W>(coef, Ny, 6, fo, c), vp = wfac<K, W>(coef, Ny, 7, fo, c);
+        each([&](int p) {
+            for (int k = 0; k < K; ++k) {
+                P[p].e[k] += dplus[p] * Pp.e[k] + dminus[p] * Pp.e[k];
+                P[p].o[k] += dplus[p] * Pp.o[k] - dminus[p] * Pp.o[k];
+                v[p].e[k] += dplus[p] * vp.e[k] - dminus[p] * vp.e[k];
+                v[p].o[k] += dplus[p] * vp.o[k] + dminus[p] * vp.o[k];
+            }
+        });
+        if (taucorr) {
+            const int Nb = c.Nb;
+            const WV<K> P0 = wfac<K, W>(coef, Ny, 8, fo, c), v0 = wfac<K, W>(coef, Ny, 9, fo, c);
+            each([&](int p) {
+                const double sigma1_Nb = lambda * wtop<K, W>(v[p], c) - Sy[p][pos(Nb)];
+                double sigma1_Nb1 = lambda * wtop1<K, W>(v[p], c) - Sy[p][pos(Nb - 1)];
+                sigma1_Nb1 += (4.0 / c.L) * Nb * wtop<K, W>(P[p], c);
+                const double sigmaNb = sigma1_Nb / (1.0 - sc[5]);
+                const double sigmaNb1 = sigma1_Nb1 / (1.0 - sc[4]);
+                for (int k = 0; k < K; ++k) {
+                    P[p].e[k] += sigmaNb1 * P0.e[k];
+                    P[p].o[k] += sigmaNb * P0.o[k];
+                    v[p].e[k] += sigmaNb * v0.e[k];
+                    v[p].o[k] += sigmaNb1 * v0.o[k];
+                }
+            });
+        }
+    }
+    each([&](int p) { wrow_store<K, W, LP>(Sy[p], c, v[p]); });  // the rows are this segment's alone
+    // u and w, one parity at a time (fewer live registers)
+    auto solve_uw = [&](double (WV<K>::*const Pk)[K], int par, int M) {
+        double f[2 * NP][K], x[2 * NP][K];
+        const HelmPar<K, W> op = vop.part(par, M, c);
+        each([&](int p) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int n = pos(2 * min(K * c.lane + k, M - 1) + par);
+                f[2 * p][k] = ax[p] * (P[p].*Pk)[k] - Sx[p][n];
+                f[2 * p + 1][k] = az[p] * (P[p].*Pk)[k] - Sz[p][n];
+            }
+        });
+        op.template solve<2 * NP>(f, hbl + LP * c.lane + par, HP, c, x);
+        each([&](int p) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int i = K * c.lane + k, at = wrow_own<K, LP>(c.lane, i, k) + par;
+                if (i < M) {
+                    Sx[p][at] = x[2 * p][k];
+                    Sz[p][at] = x[2 * p + 1][k];
+                }
+            }
+        });
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    solve_uw(&WV<K>::e, 0, c.Me);
+    __builtin_amdgcn_sched_barrier(0);
+    solve_uw(&WV<K>::o, 1, c.Mo);
+    __syncthreads();
+    const int ww = threadIdx.x % MPB, mm = m0 + ww;
+    const bool out = mm > 0 && mm < g.M;
+    for (int row = threadIdx.x / MPB; row < 3 * Ny; row += nthr / MPB) {
+        const double a = lds[slot(ww, 0, row)], b = lds[slot(ww, 1, row)];
+        const bool mid = row >= Ny && row < 2 * Ny;
+        if (out) u[(long)row * g.M + mm] = mid ? dvec2{a, b} : dvec2{b, a};
+    }
+    __syncthreads();
+    each([&](int p) { wrow_store<K, W, LP>(Sy[p], c, P[p]); });
     __syncthreads();
     for (int row = Ny + threadIdx.x / MPB; row < 2 * Ny; row += nthr / MPB) {
         const double a = lds[slot(ww, 0, row)], b = lds[slot(ww, 1, row)];
@@ -558,15 +772,17 @@ void launch_pressure(const Geom& g, const YMats& ym, const double* hb, const Pre
 
 void launch_tau_solve(const Geom& g, const double* hb, int n, const TauMember* tab, hipStream_t st) {
     const int Me = (g.Ny + 1) / 2;  // even coefficients: at most K per lane of a W-lane segment
-    auto go = [&](auto kern, int k, int w, int mpb) {
+    auto launch = [&](auto kern, int mpb, int threads, size_t lds) {
         const long nblk = ((long)((g.M + mpb - 1) / mpb) + 1) * n;
         if (nblk > 0x7fffffffL) throw std::runtime_error("tau solve: too many blocks in one launch");
-        const size_t lds = tau_lds(g.Ny, k, w, mpb);
         allow_lds(kern, lds);
-        kern<<<dim3((unsigned)nblk), 2 * w * mpb, lds, st>>>(g, hb, n, tab);
+        kern<<<dim3((unsigned)nblk), threads, lds, st>>>(g, hb, n, tab);
+    };
+    auto go = [&](auto kern, int k, int w, int mpb) {
+        launch(kern, mpb, 2 * w * mpb, tau_lds(tau_pitch(g.Ny), 2 * k, w, mpb));
     };
     // 16-lane segments (every shuffle a DPP row move) as far as their
-    // coefficients fit the registers, 32 lanes above. 8 modes per block: with 16
+    // coefficients fit the registers, 32 and 64 lanes above. 8 modes per block: with 16
     // a lone 32^3 field took 12.4 us, not 9.2, 64^3 17.1, not 14.6, and 24 of
     // 32^3 26.7, not 20.8. At 65-80 coefficients, where a block of 8 leaves
     // half-filled 256-byte runs of every row, 16 modes per block are faster once
@@ -580,8 +796,8 @@ void launch_tau_solve(const Geom& g, const double* hb, int n, const TauMember* t
     else if (Me <= 80 && g.M >= 192 * 16) go(k_tau_solve_wave<5, 16, 16>, 5, 16, 16);
     else if (Me <= 80) go(k_tau_solve_wave<5, 16, 8>, 5, 16, 8);
     else if (Me <= 96) go(k_tau_solve_wave<6, 16, 8>, 6, 16, 8);
-    else if (Me <= 128) go(k_tau_solve_wave<4, 32, 4>, 4, 32, 4);
-    else go(k_tau_solve_wave<6, 32, 4>, 6, 32, 4);
+    else if (Me <= 128) launch(k_tau_solve_tall<4, 32, 4, 1>, 4, 256, tau_lds(tau_row<4>(g.Ny), tau_lp(4), 32, 4));
+    else launch(k_tau_solve_tall<3, 64, 4, 2>, 4, 256, tau_lds(tau_row<3>(g.Ny), tau_lp(3), 64, 4));
 }
 
 // ===========================================================================
@@ -720,12 +936,16 @@ void launch_linear(const Geom& g, int n, const LinearMember* tab, hipStream_t st
     };
     // 16-lane segments and 8 modes per block as far as in the tau solve; above, 4 modes
     // keep a block within 100 KB of LDS, at 64-byte pieces of a row (at 65 coefficients,
-    // 32 lanes and 4 modes against 16 and 8: 128^3 26.3 -> 18.5 us, 192x129x192 54 -> 37)
+    // 32 lanes and 4 modes against 16 and 8: 128^3 26.3 -> 18.5 us, 192x129x192 54 -> 37).
+    // At 81-96 coefficients 8 modes on 16 lanes are the faster ones where one field fills
+    // the chip with their blocks (128x161x128 30.7 us, 32.7 with 4 modes; 32x161x32 10.8
+    // against 9.2, 24 of them 43.4 against 40.7).
     if (Me <= 16) go(k_linear_wave<1, 16, 8>, 16, 8);
     else if (Me <= 32) go(k_linear_wave<2, 16, 8>, 16, 8);
     else if (Me <= 48) go(k_linear_wave<3, 16, 8>, 16, 8);
     else if (Me <= 64) go(k_linear_wave<4, 16, 8>, 16, 8);
     else if (Me <= 80) go(k_linear_wave<5, 16, 8>, 16, 8);
+    else if (Me <= 96 && g.M >= 192 * 16) go(k_linear_wave<6, 16, 8>, 16, 8);
     else if (Me <= 96) go(k_linear_wave<3, 32, 4>, 32, 4);
     else if (Me <= 128) go(k_linear_wave<4, 32, 4>, 32, 4);
     else if (Me <= 192) go(k_linear_wave<6, 32, 4>, 32, 4);

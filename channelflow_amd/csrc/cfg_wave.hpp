@@ -647,25 +647,37 @@ __device__ __forceinline__ void wends_n(const WV<K> (&v)[NR], const WCtx& c, dou
 // A profile in a row of doubles: pairs (row[2i], row[2i+1]), the row 16-byte
 // aligned and row[N] (N is odd) finite. Lanes past the profile hold its last
 // pair: finite values that the operators' zero entries cancel (HelmPar).
-template <int K, int W>
+// LP: doubles of a row per lane, 2K or, padded, 2K + 2: at K = 4 the lanes' accesses
+// are 64 bytes apart otherwise, on a quarter of the LDS banks. wrow_pos: the place of
+// coefficient n.
+template <int K, int LP = 2 * K>
+__host__ __device__ constexpr int wrow_pos(int n) {
+    return LP == 2 * K ? n : n + (LP - 2 * K) * (n / (2 * K));
+}
+// and of a lane's pair k, pair i = K lane + k of the row
+template <int K, int LP>
+__device__ __forceinline__ int wrow_own(int lane, int i, int k) {
+    return LP == 2 * K ? 2 * i : LP * lane + 2 * k;
+}
+template <int K, int W, int LP = 2 * K>
 __device__ __forceinline__ WV<K> wrow_load(const double* row, const WCtx& c) {
     WV<K> v;
     const dvec2* p = reinterpret_cast<const dvec2*>(row);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const dvec2 a = p[min(K * c.lane + k, c.Me - 1)];
+        const dvec2 a = p[wrow_pos<K, LP>(2 * min(K * c.lane + k, c.Me - 1)) / 2];
         v.e[k] = a.x;
         v.o[k] = a.y;
     }
     return v;
 }
-template <int K, int W>
+template <int K, int W, int LP = 2 * K>
 __device__ __forceinline__ void wrow_store(double* row, const WCtx& c, const WV<K>& v) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int i = K * c.lane + k;
-        if (i < c.Me) row[2 * i] = v.e[k];
-        if (i < c.Mo) row[2 * i + 1] = v.o[k];
+        if (i < c.Me) row[wrow_own<K, LP>(c.lane, i, k)] = v.e[k];
+        if (i < c.Mo) row[wrow_own<K, LP>(c.lane, i, k) + 1] = v.o[k];
     }
 }
 // Array k of a tau set's mode (coef + off: the mode's first array), loaded at a
@@ -855,6 +867,8 @@ struct HelmOp {
         e.init(lambda, hb, 2, c.Me, c);
         o.init(lambda, hb + 1, 2, c.Mo, c);
     }
+    __device__ __forceinline__ HelmOp(const gcdouble coef, int Ny, int arr, unsigned off, double lambda, const WCtx& c)
+        : HelmOp(wfac3<K, W>(coef, Ny, arr, off, c), lambda, c) {}
     template <int NR>
     __device__ __forceinline__ void solve(const WV<K> (&f)[NR], const WCtx& c, WV<K> (&x)[NR]) const {
         double fe[NR][K], fo[NR][K], xe[NR][K], xo[NR][K];
@@ -875,6 +889,55 @@ struct HelmOp {
                 x[r].e[k] = xe[r][k];
                 x[r].o[k] = xo[r][k];
             }
+    }
+};
+
+// HelmOp of arrays arr, arr + 1, arr + 2 of a mode with one parity system at a time,
+// loaded (the second time from the caches) and formed where it is used: the same
+// values in half the registers.
+template <int K, int W, int LP>
+struct HelmParts {
+    const gcdouble coef;
+    const int Ny, arr;
+    const unsigned off;
+    const double lambda;
+    __device__ __forceinline__ HelmParts(const gcdouble coef, int Ny, int arr, unsigned off, double lambda, const WCtx&)
+        : coef(coef), Ny(Ny), arr(arr), off(off), lambda(lambda) {}
+    __device__ __forceinline__ HelmPar<K, W> part(int par, int M, const WCtx& c) const {
+        HelmPar<K, W> h;
+        const gcdouble b = coef + (long)arr * Ny;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const unsigned at = off + (unsigned)(2 * min(K * c.lane + k, M - 1) + par);
+            h.band[k] = b[at];
+            h.up[k] = b[at + (unsigned)Ny];
+            h.invd[k] = b[at + (unsigned)(2 * Ny)];
+        }
+        h.init(lambda, c.hb + LP * c.lane + par, 2, M, c);
+        return h;
+    }
+    template <int NR>
+    __device__ __forceinline__ void solve(const WV<K> (&f)[NR], const WCtx& c, WV<K> (&x)[NR]) const {
+        double y[NR][K], z[NR][K];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int k = 0; k < K; ++k) y[r][k] = f[r].e[k];
+        part(0, c.Me, c).template solve<NR>(y, c.hb + LP * c.lane, LP * W, c, z);
+        __builtin_amdgcn_sched_barrier(0);  // the next one's loads stay behind this solve
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                x[r].e[k] = z[r][k];
+                y[r][k] = f[r].o[k];
+            }
+        part(1, c.Mo, c).template solve<NR>(y, c.hb + LP * c.lane + 1, LP * W, c, z);
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int k = 0; k < K; ++k) x[r].o[k] = z[r][k];
+        __builtin_amdgcn_sched_barrier(0);
     }
 };
 

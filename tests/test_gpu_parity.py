@@ -263,6 +263,20 @@ def test_dns_linear_segments(gpu, constraint, Ny):
     assert np.all(eu <= 1e-10), eu
 
 
+@pytest.mark.parametrize("Ny", [161, 191])
+def test_dns_linear_eight_modes(gpu, Ny):
+    """NSE::linear and the tau solve at 81-96 even coefficients with 95 x 36 modes, enough
+    that the first takes 8 modes per block; the last block is not full (3420 modes).
+    The same 1e-10 bar as test_dns_schemes."""
+    flags = dict(C1_FLAGS, nonlinearity="Rotational", timestepping="CNRK2", initstepping="CNRK2", dt=0.005,
+                 dealiasing="NoDealiasing")
+    u0 = random_field(96, Ny, 72, LX_C, LZ_C, norm=0.1, decay=0.3, seed=Ny)
+    g, ur, qr, ug, qg, ref, dns = run_pair(96, Ny, 72, LX_C, LZ_C, flags, u0, 1)
+    eu = rel_l2_per_component(g, ug, ur)
+    print(Ny, "rel L2", eu, flush=True)
+    assert np.all(eu <= 1e-10), eu
+
+
 CFL_CASES = {
     "couette_skew": (C1_FLAGS, (24, 25, 24)),
     "poiseuille_rot_nodealias": (dict(baseflow="LaminarBase", constraint="PressureGradient", dPdx=-3.0 / 2000,
