@@ -14,7 +14,7 @@ LIB = os.path.join(HERE, "libcfgpu.so")
 
 SOURCES = ["cfg_kernels.hip", "cfg_z_skew.hip", "cfg_z_conv.hip", "cfg_z_rot.hip", "cfg_z_div.hip", "cfg_z.hip", "cfg_tau.hip",
            "cfg_step.cpp", "cfg_runtime.cpp", "cfg_batch.cpp", "cfg_noalloc.cpp", "cfg_tausolver.cpp"]
-HEADERS = ["cfg_dev.hpp", "cfg_fft.hpp", "cfg_z.hpp", "cfg_zpass.hpp", "cfg_kernels.hpp", "cfg_math.hpp", "cfg_wave.hpp",
+HEADERS = ["cfg_dev.hpp", "cfg_lds.hpp", "cfg_fft.hpp", "cfg_z.hpp", "cfg_zpass.hpp", "cfg_kernels.hpp", "cfg_math.hpp", "cfg_wave.hpp",
            "cfg_host.hpp", "cfg_step.hpp"]
 
 # Packed FP32 instructions are disabled in every HIP compile of this project.

@@ -1,14 +1,11 @@
-// What the kernel files share: complex arithmetic, the mode numbering, the
-// XCD block order and the dynamic-LDS opt-in.
+// What the kernel files share: complex arithmetic, the mode numbering and the
+// XCD block order.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include <map>
-#include <stdexcept>
-#include <string>
-
 #include "cfg_kernels.hpp"
+#include "cfg_lds.hpp"
 
 namespace cfg {
 
@@ -41,22 +38,6 @@ __device__ __forceinline__ BlockId xcd_grid() {
     const unsigned p = x * q + (x < r ? x : r) + L / NXCD;
     const unsigned t = p / gx;
     return BlockId{(int)(p - t * gx), (int)(t % gy), (int)(t / gy)};
-}
-
-// Raises a kernel's dynamic-LDS limit once per (kernel, size), so that launches
-// recorded into a graph make no attribute calls.
-template <class K>
-inline void allow_lds(K kernel, size_t bytes) {
-    if (bytes <= 64 * 1024) return;
-    static std::map<const void*, size_t> done;
-    size_t& d = done[(const void*)kernel];
-    if (d >= bytes) return;
-    const hipError_t e =
-        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess)  // the launch that follows would fail without saying why
-        throw std::runtime_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize, " + std::to_string(bytes) +
-                                 " B): " + hipGetErrorString(e));
-    d = bytes;
 }
 
 }  // namespace cfg

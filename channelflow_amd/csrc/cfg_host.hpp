@@ -42,6 +42,12 @@ struct Error : std::runtime_error {
         if (e_ != hipSuccess) throw Error(CFG_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+inline int current_device() {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    return dev;
+}
+
 // ---------------------------------------------------------------------------
 // device buffers
 // ---------------------------------------------------------------------------
@@ -496,10 +502,8 @@ inline int guarded(F&& f) {
 inline void init_device_limits() {
     static bool done = false;
     if (done) return;
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
     hipDeviceProp_t p;
-    HIPCHK(hipGetDeviceProperties(&p, dev));
+    HIPCHK(hipGetDeviceProperties(&p, current_device()));
     size_t b = p.sharedMemPerBlockOptin ? p.sharedMemPerBlockOptin : p.sharedMemPerBlock;
     set_lds_budget(std::min<size_t>(b, 160 * 1024));
     done = true;
@@ -574,11 +578,12 @@ class DevPool {
 };
 
 // Device copy of a small constant table, shared by every user with the same
-// contents (the base-flow constants of the members of one grid, base flow and
-// nu). Expired entries are swept as the cache grows.
+// contents on one device (the base-flow constants of the members of one grid,
+// base flow and nu). Expired entries are swept as the cache grows.
 inline std::shared_ptr<DBuf> shared_consts(const std::vector<double>& h) {
-    static std::map<std::vector<double>, std::weak_ptr<DBuf>> cache;
-    auto it = cache.find(h);
+    static std::map<std::pair<int, std::vector<double>>, std::weak_ptr<DBuf>> cache;
+    const std::pair<int, std::vector<double>> k(current_device(), h);
+    auto it = cache.find(k);
     if (it != cache.end()) {
         if (auto sp = it->second.lock()) return sp;
         cache.erase(it);
@@ -587,7 +592,7 @@ inline std::shared_ptr<DBuf> shared_consts(const std::vector<double>& h) {
         for (auto jt = cache.begin(); jt != cache.end();) jt = jt->second.expired() ? cache.erase(jt) : std::next(jt);
     auto sp = std::make_shared<DBuf>(h.size());
     HIPCHK(hipMemcpy(sp->p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
-    cache[h] = sp;
+    cache[k] = sp;
     return sp;
 }
 
@@ -670,7 +675,9 @@ class TableCache {
 };
 
 // ---------------------------------------------------------------------------
-// Per-grid constants shared by every field on that grid (process-wide)
+// Per-grid constants shared by every field on that grid (process-wide, per device:
+// what is cached lies in the memory of the device it was made on, and what keeps
+// it alive outlasts a change of the current device)
 // ---------------------------------------------------------------------------
 struct GridKey {
     int Nx, Ny, Nz, dealias;
@@ -684,8 +691,8 @@ inline GridKey grid_key(const cfg_grid& g, bool dealias) {
 }
 
 inline std::shared_ptr<Geometry> geometry_for(const cfg_grid& gr, bool dealias) {
-    static std::map<GridKey, std::weak_ptr<Geometry>> cache;
-    const GridKey k = grid_key(gr, dealias);
+    static std::map<std::pair<int, GridKey>, std::weak_ptr<Geometry>> cache;
+    const std::pair<int, GridKey> k(current_device(), grid_key(gr, dealias));
     auto it = cache.find(k);
     if (it != cache.end())
         if (auto sp = it->second.lock()) return sp;
@@ -745,11 +752,11 @@ inline size_t tau_set_bytes(const Geom& g) {
 
 inline std::shared_ptr<TauStore> tau_for(const Geometry& geo, double nu, double lambda_t, bool taucorr,
                                          hipStream_t st, DevPool& pool, KTimer* kt) {
-    using Key = std::tuple<GridKey, double, double, int>;
+    using Key = std::tuple<int, GridKey, double, double, int>;
     static std::map<Key, std::weak_ptr<TauStore>> cache;
     const Geom& g = geo.g;
     const GridKey gk{g.Nx, g.Ny, g.Nz, geo.dealias, g.Lx, g.Lz, g.a, g.b};
-    const Key k{gk, nu, lambda_t, taucorr ? 1 : 0};
+    const Key k{current_device(), gk, nu, lambda_t, taucorr ? 1 : 0};
     auto it = cache.find(k);
     if (it != cache.end()) {
         if (auto sp = it->second.lock()) {
