@@ -33,7 +33,7 @@ EXPORTED = ("cfg_last_error", "cfg_device_count", "cfg_dns_create", "cfg_dns_des
             "cfg_batch_create", "cfg_batch_destroy", "cfg_batch_add", "cfg_batch_remove", "cfg_batch_advance",
             "cfg_batch_size", "cfg_batch_get_state", "cfg_batch_set_state", "cfg_batch_time", "cfg_batch_finite",
             "cfg_batch_dpdx",
-            "cfg_batch_cfl", "cfg_batch_reset_dt", "cfg_batch_advance_members", "cfg_batch_profile", "cfg_batch_kernel_times", "cfg_batch_set_graphs", "cfg_batch_graph_stats", "cfg_batch_tick_stats",
+            "cfg_batch_cfl", "cfg_batch_reset_dt", "cfg_batch_advance_members", "cfg_batch_profile", "cfg_batch_kernel_times", "cfg_batch_set_graphs", "cfg_batch_graph_stats", "cfg_batch_tick_stats", "cfg_batch_memory",
             "cfg_server_create", "cfg_server_destroy", "cfg_server_submit", "cfg_server_step", "cfg_server_result",
             "cfg_server_memory", "cfg_tausolver_create", "cfg_tausolver_destroy", "cfg_tausolver_solve",
             "cfg_tausolver_solve_bulk", "cfg_tausolver_verify", "cfg_tausolver_verify_bulk")
@@ -122,6 +122,7 @@ def library():
         "cfg_batch_set_graphs": ([v, i], i),
         "cfg_batch_graph_stats": ([v, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)], i),
         "cfg_batch_tick_stats": ([v, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong), C.POINTER(C.c_double)], i),
+        "cfg_batch_memory": ([v, P, C.POINTER(C.c_int)], i),
         "cfg_server_create": ([d, C.POINTER(v)], i),
         "cfg_server_destroy": ([v], i),
         "cfg_server_submit": ([v, G, F, P, P, i, C.POINTER(C.c_longlong)], i),
@@ -586,6 +587,14 @@ class Batch:
         t, g, h = C.c_longlong(), C.c_longlong(), C.c_double()
         _check(library().cfg_batch_tick_stats(self._h, C.byref(t), C.byref(g), C.byref(h)))
         return t.value, g.value, h.value
+
+
+    def memory(self):
+        """(device bytes held for the members, whether the batch was made on the
+        current device)."""
+        b, here = C.c_double(), C.c_int()
+        _check(library().cfg_batch_memory(self._h, C.byref(b), C.byref(here)))
+        return b.value, bool(here.value)
 
 
 class PressureSolver:

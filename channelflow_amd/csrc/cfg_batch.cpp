@@ -48,6 +48,7 @@ enum GraphMode { GRAPHS_OFF = 0, GRAPHS_PER_CLASS = 1, GRAPHS_WHOLE = 2 };
 class Batch {
    public:
     Batch() {
+        dev_ = current_device();
         HIPCHK(hipStreamCreate(&bst_));
         HIPCHK(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&after_, hipEventDisableTiming));
@@ -225,6 +226,7 @@ class Batch {
         for (const TauStore* t : tau) b += t->bytes;
         return b;
     }
+    int device() const { return dev_; }  // the one its streams and memory belong to
     // a class left without members hands its free blocks and work buffers
     // back to HIP
     void trim_if_empty(BatchClass* c) {
@@ -341,6 +343,7 @@ class Batch {
 
     static constexpr size_t kMaxWholeKeys = 256;
     GraphMode mode_ = GRAPHS_PER_CLASS;
+    int dev_ = 0;
     hipStream_t bst_ = nullptr;
     hipEvent_t fork_ = nullptr, after_ = nullptr;
     std::unordered_map<std::string, hipGraphExec_t> whole_;
@@ -780,6 +783,14 @@ int cfg_batch_tick_stats(const cfg_batch* b, long long* ticks, long long* graph_
     return guarded([&] {
         if (!b) throw Error(CFG_ERR_ARG, "null batch");
         b->b.tick_stats(ticks, graph_launches, host_us);
+    });
+}
+
+int cfg_batch_memory(const cfg_batch* b, double* held_bytes, int* on_current_device) {
+    return guarded([&] {
+        if (!b) throw Error(CFG_ERR_ARG, "null batch");
+        if (held_bytes) *held_bytes = (double)b->b.held_bytes();
+        if (on_current_device) *on_current_device = b->b.device() == current_device() ? 1 : 0;
     });
 }
 

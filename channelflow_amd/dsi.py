@@ -129,24 +129,29 @@ class MultiShooting:
     # over the last one's batch and replaces its members one by one: nothing of their
     # state stays, and a result is that of a new batch, bit for bit. Building and
     # freeing them anew was 5 of the 34 ms of a residual of 16 shots of 32x49x32 over
-    # 200 steps (now 29). A batch is kept up to about 2 GiB of device memory, and freed with
-    # this object or when a call has another number of members.
+    # 200 steps (now 29). A batch is kept if it holds at most KEEP_BYTES of device memory
+    # (Batch.memory: states, work buffers and tau sets; a grid's fixed tables, some MB,
+    # come on top), and freed by release(), with this object, or when a call has another
+    # number of members, fails, or runs on another device.
     KEEP_BYTES = 2 << 30
 
     def _take_batch(self, n):
         from . import Batch
         try:
             batch, ids = self._kept.pop()  # one caller gets it; others build their own
-            if len(ids) == n:
+            if len(ids) == n and batch.memory()[1]:
                 return batch, ids
         except IndexError:
             pass
         return Batch(), []
 
     def _keep_batch(self, batch, ids):
-        # state and work buffers: 40 to 50 real fields of the full grid per member
-        if len(ids) * 400 * self.Nx * self.Ny * self.Nz <= self.KEEP_BYTES:
+        if batch.memory()[0] <= self.KEEP_BYTES:
             self._kept[:] = [(batch, ids)]
+
+    def release(self):
+        """Frees the device memory kept for the next call."""
+        self._kept.clear()
 
     def __getstate__(self):  # copies start without one
         return {**self.__dict__, "_kept": []}

@@ -251,6 +251,11 @@ int cfg_batch_graph_stats(const cfg_batch* b, long long* captures, long long* re
  * its target), graph launches among them, and host microseconds spent in them
  * (planning, launch tables, launches). No counterpart in the reference. */
 int cfg_batch_tick_stats(const cfg_batch* b, long long* ticks, long long* graph_launches, double* host_us);
+/* Device bytes the batch holds for its members, counted as cfg_server_memory
+ * counts them, and whether the calling thread's current device is the one the
+ * batch was made on. Either pointer may be NULL. No counterpart in the
+ * reference. */
+int cfg_batch_memory(const cfg_batch* b, double* held_bytes, int* on_current_device);
 
 /* ---- Serving ----------------------------------------------------------------
  * Continuous batching of integration requests (no counterpart in the

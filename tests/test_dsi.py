@@ -91,3 +91,61 @@ def test_multishooting_time_fit():
     assert ms.variable and ms.timestep.N() * ms.timestep.dT() == pytest.approx(1.0, rel=1e-14)
     with pytest.raises(ValueError):
         MultiShooting(16, 17, 16, 1.0, 1.0, cfa.DNSFlags(dt=0.02), -1.0)
+
+
+class BookBatch:
+    """Batch's calls as MultiShooting makes them, without a device: f^T(u) = 2 u."""
+    made = 0
+    held, here, fails = 0.0, True, False
+
+    def __init__(self):
+        BookBatch.made += 1
+        self.members, self.next = {}, 0
+
+    def add(self, fields, flags):
+        self.members[self.next] = fields[0].data
+        self.next += 1
+        return self.next - 1
+
+    def remove(self, m):
+        del self.members[m]
+
+    def advance(self, n):
+        if BookBatch.fails:
+            raise cfa.CfgError("velocity not finite", cfa.ERR_NONFINITE)
+
+    def velocity(self, m):
+        return 2 * self.members[m]
+
+    def memory(self):
+        return BookBatch.held, BookBatch.here
+
+
+@pytest.mark.parametrize("case", ["kept", "too large", "other device", "released", "failed", "other count"])
+def test_multishooting_keeps_only_what_it_may(monkeypatch, case):
+    """The batch of a call serves the next one only while it holds at most KEEP_BYTES by its
+    own account and the current device is its own; release(), a call that raises and
+    another member count let go of it."""
+    monkeypatch.setattr(cfa, "Batch", BookBatch)
+    for k, v in dict(made=0, held=float(MultiShooting.KEEP_BYTES), here=True, fails=False).items():
+        monkeypatch.setattr(BookBatch, k, v)
+    ms = MultiShooting(16, 9, 16, 2.0, 1.0, cfa.DNSFlags(dt=0.02, variabledt=False), 0.2)
+    shots = [np.full((3, 9, 16, 9), 1.0 + i, dtype=np.complex128) for i in range(2)]
+    if case == "too large":
+        BookBatch.held += 1
+    G = ms.eval(shots)
+    assert np.array_equal(G[0], 2 * shots[0] - shots[1]) and np.array_equal(G[1], 2 * shots[1] - shots[0])
+    if case == "other device":
+        BookBatch.here = False
+    elif case == "released":
+        ms.release()
+    elif case == "failed":
+        BookBatch.fails = True
+        with pytest.raises(cfa.CfgError):
+            ms.eval(shots)
+        BookBatch.fails = False
+    assert len(ms._kept) == (0 if case in ("too large", "released", "failed") else 1)
+    again = shots[:1] if case == "other count" else shots
+    made = BookBatch.made
+    assert np.array_equal(ms.eval(again)[0], 2 * again[0] - again[-1 if len(again) > 1 else 0])
+    assert BookBatch.made == made + (0 if case == "kept" else 1)

@@ -172,3 +172,32 @@ def test_repeated_calls_match_new_objects(gpu, case):
     assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots[:1]), new().eval(shots[:1])))
     assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots), new().eval(shots))) and ms.dts == dts
     assert all(np.array_equal(a, b) for a, b in zip(copy.deepcopy(ms).eval(other), new().eval(other)))
+
+
+def test_kept_batch_memory_and_failed_call(gpu, monkeypatch):
+    """A kept batch reports the memory it holds and its device; nothing is kept above
+    KEEP_BYTES, after release() or after a call whose integrations blew up, and the next
+    results are those of new objects bit for bit, also with members at different dt."""
+    shots, _ = shots_and_dirs(3, 0)
+    fl = cfa.DNSFlags(**COUETTE)
+    ref = MultiShooting(NX, NY, NZ, LX_C, LZ_C, fl, 0.14).eval(shots)
+    ms = MultiShooting(NX, NY, NZ, LX_C, LZ_C, fl, 0.14)
+    ms.eval(shots)
+    held, here = ms._kept[0][0].memory()
+    live = 3 * NY * 9 * 5 * 16  # a velocity field's live modes
+    assert here and held >= 3 * (1 + 3 + 3) * live  # u, and SBDF3's histories of u and f, per member
+    with pytest.raises(cfa.CfgError) as e:
+        ms.eval([1e200 * u for u in shots])
+    assert e.value.code == cfa.ERR_NONFINITE and not ms._kept
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots), ref)) and ms._kept
+    ms.release()
+    assert not ms._kept
+    monkeypatch.setattr(MultiShooting, "KEEP_BYTES", 0)
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(shots), ref)) and not ms._kept
+    monkeypatch.undo()
+    var = cfa.DNSFlags(**dict(COUETTE, variabledt=True, dT=0.1, dtmax=0.05))
+    scaled = [shots[0], 4 * shots[1], 0.1 * shots[2]]
+    ms = MultiShooting(NX, NY, NZ, LX_C, LZ_C, var, 0.4)
+    first = ms.eval(scaled)
+    assert len(set(ms.dts)) > 1 and ms._kept
+    assert all(np.array_equal(a, b) for a, b in zip(ms.eval(scaled), first))
