@@ -1306,7 +1306,7 @@ NLTune tune_nonlinear(const Geom& g, const YMats& ym, const FFTPlan& px, const F
     if (zwave_size(g.Nx) && want_g) {  // the forward wavefront x-FFT on its own (it folds the skew form)
         const int nzf = method == NL_SKEW ? 8 : (method == NL_DIV ? 9 : 3);  // as launch_nonlinear
         std::vector<NLTune> fc;
-        for (int wb = 1; wb <= 4; wb *= 2) {
+        for (int wb = method == NL_SKEW ? 2 : 1; wb <= 4; wb *= 2) {  // the fold runs in pairs
             NLTune c;
             c.xwbf = wb;
             fc.push_back(c);

@@ -310,3 +310,19 @@ def test_server_backfills_past_a_large_request(gpu):
     assert len(order) == 4
     assert order.index(ids[2]) < order.index(ids[1])  # a small request passed the large one
     assert held_max <= 7.0e6
+
+
+def test_tuner_candidates_differ(gpu, monkeypatch, capfd):
+    """Every candidate that the tuner times is a launch of its own: the skew-symmetric
+    forward x-FFT runs in pairs of wavefronts, so its blocks have two or four."""
+    import re
+    monkeypatch.setenv("CFGPU_TUNE_LOG", "1")
+    b = cfa.Batch()
+    for i, nl in enumerate(("SkewSymmetric", "Rotational")):
+        u0 = random_field(16, 17, 16, LX_C, LZ_C, norm=0.05, decay=0.4, seed=500 + i)
+        b.add(fields((16, 17, 16), u0), cfa.DNSFlags(**dict(COUETTE, nonlinearity=nl)))
+    b.advance(1)
+    lines = [x for x in capfd.readouterr().err.splitlines() if x.startswith("cfg tune xfwd ")]
+    blocks = [[int(v) for v in re.findall(r"xwbf (\d+)", x)] for x in lines]
+    print(lines, flush=True)
+    assert sorted(blocks) == [[1, 2, 4], [2, 4]]
