@@ -102,7 +102,6 @@ __device__ __forceinline__ void stockham_bfly(const double2* __restrict__ s, dou
     for (int r = 0; r < R; ++r) d[pidx(o + r * NS)] = v[r];
 }
 
-// runtime length (plan in P)
 template <int SIGN>
 __device__ double2* fft_lds(double2* a, double2* b, const FFTPlan& P, const double2* tw, int nlines) {
     double2* src = a;
@@ -129,114 +128,6 @@ __device__ double2* fft_lds(double2* a, double2* b, const FFTPlan& P, const doub
         Ns *= R;
     }
     return src;
-}
-
-// compile-time length: every divisor is a constant. Radices 4, 2, 3 in that
-// order; with r8, radix 8 first where that takes fewer passes (ties: 4). The
-// z-pass gains from the fewer passes; the x-FFTs, with fewer lines per block,
-// lose more to the smaller number of butterflies per pass.
-constexpr int fft_passes_from(int n, bool eight) {
-    int c = 0;
-    while (eight && n % 8 == 0) n /= 8, ++c;
-    while (n % 4 == 0) n /= 4, ++c;
-    while (n % 2 == 0) n /= 2, ++c;
-    while (n % 3 == 0) n /= 3, ++c;
-    return c;
-}
-constexpr int fft_radix(int n, int p, bool r8) {
-    const bool eight = r8 && fft_passes_from(n, true) < fft_passes_from(n, false);
-    int c = 0;
-    while (eight && n % 8 == 0) {
-        if (c == p) return 8;
-        n /= 8;
-        ++c;
-    }
-    while (n % 4 == 0) {
-        if (c == p) return 4;
-        n /= 4;
-        ++c;
-    }
-    while (n % 2 == 0) {
-        if (c == p) return 2;
-        n /= 2;
-        ++c;
-    }
-    while (n % 3 == 0) {
-        if (c == p) return 3;
-        n /= 3;
-        ++c;
-    }
-    return 0;
-}
-constexpr int fft_npass(int n, bool r8) {
-    int c = 0;
-    while (fft_radix(n, c, r8) != 0) ++c;
-    return c;
-}
-constexpr int fft_ns(int n, int p, bool r8) {
-    int s = 1;
-    for (int q = 0; q < p; ++q) s *= fft_radix(n, q, r8);
-    return s;
-}
-
-// Threads per block of every kernel that runs the compile-time FFTs.
-constexpr int FFT_BLOCK = 256;
-
-// One Stockham pass per recursion level. A thread keeps the same butterfly
-// index j in every line it visits (FFT_BLOCK / NR lines per sweep), so its
-// padded source and destination offsets and its twiddles are computed once
-// per pass; a twiddle of 1 (k = 0) multiplies exactly.
-template <int N, int SIGN, int P, bool R8>
-__device__ __forceinline__ double2* fft_ct(double2* a, double2* b, const double2* tw, int nlines) {
-    if constexpr (P == fft_npass(N, R8)) {
-        return a;
-    } else {
-        constexpr int R = fft_radix(N, P, R8), NR = N / R, NS = fft_ns(N, P, R8), TSTEP = N / (NS * R);
-        constexpr int LPI = FFT_BLOCK / NR, LP = lpitch(N);
-        static_assert(LPI >= 1, "FFT line longer than the block");
-        const int j = threadIdx.x % NR, l0 = threadIdx.x / NR;
-        if (l0 < LPI) {
-            const int k = j % NS;
-            const int o = (j / NS) * NS * R + k;
-            int so[R], dof[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                so[r] = pidx(j + r * NR);
-                dof[r] = pidx(o + r * NS);
-            }
-            double2 t[R];
-            if constexpr (NS > 1) {
-#pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    t[r] = tw[r * k * TSTEP];
-                    if (SIGN > 0) t[r].y = -t[r].y;
-                }
-            }
-            for (int line = l0; line < nlines; line += LPI) {
-                const double2* __restrict__ src = a + line * LP;
-                double2* __restrict__ dst = b + line * LP;
-                double2 v[R == 8 ? 8 : 4];
-#pragma unroll
-                for (int r = 0; r < R; ++r) v[r] = src[so[r]];
-                if constexpr (NS > 1) {
-#pragma unroll
-                    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], t[r]);
-                }
-                dft_small<R, SIGN>(v);
-#pragma unroll
-                for (int r = 0; r < R; ++r) dst[dof[r]] = v[r];
-            }
-        }
-        __syncthreads();
-        return fft_ct<N, SIGN, P + 1, R8>(b, a, tw, nlines);
-    }
-}
-
-// N == 0 selects the runtime-length path
-template <int N, int SIGN, bool R8 = false>
-__device__ __forceinline__ double2* fft_any(double2* a, double2* b, const FFTPlan& P, const double2* tw, int nlines) {
-    if constexpr (N == 0) return fft_lds<SIGN>(a, b, P, tw, nlines);
-    else return fft_ct<N, SIGN, 0, R8>(a, b, tw, nlines);
 }
 
 // stage the twiddle table of P into LDS
@@ -346,10 +237,12 @@ struct ZW3 {
 };
 
 // the lengths with a wavefront FFT
+#define CFG_FFT_SIZES(X) \
+    X(16) X(18) X(24) X(32) X(36) X(48) X(54) X(64) X(72) X(96) X(108) X(128) X(144) X(162) X(192) X(256)
 constexpr bool zwave_size(int n) {
-    for (int m : {16, 18, 24, 32, 36, 48, 54, 64, 72, 96, 108, 128, 144, 162, 192, 256})
-        if (n == m) return true;
-    return false;
+#define CFG_IS_SIZE(N) || n == N
+    return false CFG_FFT_SIZES(CFG_IS_SIZE);
+#undef CFG_IS_SIZE
 }
 
 // Orders the LDS accesses of one wavefront (its lanes read what other lanes of
@@ -660,8 +553,5 @@ __device__ __forceinline__ void line_p2s(double2 (&u)[S::PV], double2 (&v)[S::SV
     if constexpr (three_step<S>) zw3_p2s<S::N, SIGN>(u, v, l, T, tw);
     else zw_b2a<S::N, SIGN>(u, v, l, T, tw);
 }
-
-#define CFG_FFT_SIZES(X) \
-    X(16) X(18) X(24) X(32) X(36) X(48) X(54) X(64) X(72) X(96) X(108) X(128) X(144) X(162) X(192) X(256)
 
 }  // namespace cfg

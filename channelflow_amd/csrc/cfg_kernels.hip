@@ -88,7 +88,6 @@ void launch_nonfinite(int nfields, const double* const* fields, long n, double* 
 // ===========================================================================
 // inverse x-FFT: yp [F][Ny][nkz][nkx] -> xp [Fo][Ny][Nx][nkz]; output f >= nsrc is
 // d/dx of source field f - nsrc. XL kz-lines per block.
-template <int NX>
 __global__ void __launch_bounds__(256) k_xinv(Geom g, FFTPlan px, int XL, int nsrc, const double2* __restrict__ yp0,
                                               long sy, double2* __restrict__ xp0, long sx) {
     extern __shared__ double2 lds[];
@@ -120,7 +119,7 @@ __global__ void __launch_bounds__(256) k_xinv(Geom g, FFTPlan px, int XL, int ns
         a[l * P + pidx(j)] = v;
     }
     __syncthreads();
-    double2* r = fft_any<NX, +1>(a, b, px, tw, nl);
+    double2* r = fft_lds<+1>(a, b, px, tw, nl);
     double2* out = xp + (((long)fo * Ny + y) * Nx) * nkz + ikz0;
     for (int w = threadIdx.x; w < nl * Nx; w += blockDim.x) {
         const int x = w / nl, l = w - x * nl;
@@ -129,7 +128,6 @@ __global__ void __launch_bounds__(256) k_xinv(Geom g, FFTPlan px, int XL, int ns
 }
 
 // forward x-FFT: zo [G][Ny][Nx][nkz] -> fo [G][Ny][nkz][nkx], scaled by 1/(Nx Nz)
-template <int NX>
 __global__ void __launch_bounds__(256) k_xfwd(Geom g, FFTPlan px, int XL, const double2* __restrict__ zo0, long sx,
                                               double2* __restrict__ fo0, long sy) {
     extern __shared__ double2 lds[];
@@ -151,7 +149,7 @@ __global__ void __launch_bounds__(256) k_xfwd(Geom g, FFTPlan px, int XL, const 
         a[l * P + pidx(x)] = in[(long)x * nkz + l];
     }
     __syncthreads();
-    double2* r = fft_any<NX, -1>(a, b, px, tw, nl);
+    double2* r = fft_lds<-1>(a, b, px, tw, nl);
     const double scale = 1.0 / ((double)g.Nx * g.Nz);
     for (int w = threadIdx.x; w < nl * nkx; w += blockDim.x) {
         const int l = w / nkx, ikx = w - l * nkx;
@@ -1105,11 +1103,11 @@ static bool launch_x(bool inverse, const Geom& g, const FFTPlan& px, int nsrc, i
         const size_t lds = (size_t)(g.Nx + 2 * XL * lpitch(g.Nx)) * sizeof(double2);
         const dim3 grid(g.Ny * nchunk, nf, n);
         if (inverse) {
-            allow_lds(k_xinv<NX>, lds);
-            k_xinv<NX><<<grid, 256, lds, st>>>(g, px, XL, nsrc, in, sin, out, sout);
+            allow_lds(k_xinv, lds);
+            k_xinv<<<grid, 256, lds, st>>>(g, px, XL, nsrc, in, sin, out, sout);
         } else {
-            allow_lds(k_xfwd<NX>, lds);
-            k_xfwd<NX><<<grid, 256, lds, st>>>(g, px, XL, in, sin, out, sout);
+            allow_lds(k_xfwd, lds);
+            k_xfwd<<<grid, 256, lds, st>>>(g, px, XL, in, sin, out, sout);
         }
         return false;
     }

@@ -129,12 +129,6 @@ void launch_tau_setup(const Geom& g, const TauSet& s, double nu, bool taucorr, h
     }
 }
 
-__device__ __forceinline__ CV cview(double* base, const Geom& g, int comp, int m) {
-    const long S2 = 2L * g.M;
-    double* p = base + 2L * ((long)comp * g.Ny * g.M + m);
-    return CV{SV{p, S2}, SV{p + 1, S2}};
-}
-
 // Tau solve (NSE::solve, nse.cpp:479-575; TauSolver::solve, tausolver.cpp:347-450,
 // with solve_P_and_v :193-251). The operators of a mode are real, and the real
 // and imaginary parts of its equations couple only as (v, P real; u, w

@@ -273,61 +273,16 @@ __device__ __forceinline__ void wends(const WV<K>& v, const WCtx& c, double& at_
     at_a = se - so;
 }
 
-// Affine suffix scan: x_i = cc_i + aa_i x_{i+1}; maps past the chain end are
-// the identity (cc = 0, aa = 1) and the last real map is constant (aa = 0).
-// On return cc[k] holds x_i.
-template <int K, int W>
-__device__ __forceinline__ void waff_suffix(double (&cc)[K], const double (&aa)[K], int lane) {
-    double Fc[K], Fa[K];
-    double xc = 0.0, xa = 1.0;
-    for (int k = K - 1; k >= 0; --k) {
-        xc = cc[k] + aa[k] * xc;
-        xa = aa[k] * xa;
-        Fc[k] = xc;
-        Fa[k] = xa;
-    }
-    for (int d = 1; d < W; d <<= 1) {
-        const double yc = wdn<W>(xc, d), ya = wdn1<W>(xa, d);
-        if (wrow<W>() || lane + d < W) {
-            xc = xc + xa * yc;
-            xa = xa * ya;
-        }
-    }
-    double ec = wdn<W>(xc, 1);
-    if (!wrow<W>() && lane == W - 1) ec = 0.0;
-    for (int k = 0; k < K; ++k) cc[k] = Fc[k] + Fa[k] * ec;
-}
-
-// Affine prefix scan: y_i = cc_i + aa_i y_{i-1}; the first map is constant.
-template <int K, int W>
-__device__ __forceinline__ void waff_prefix(double (&cc)[K], const double (&aa)[K], int lane) {
-    double Gc[K], Ga[K];
-    double xc = 0.0, xa = 1.0;
-    for (int k = 0; k < K; ++k) {
-        xc = cc[k] + aa[k] * xc;
-        xa = aa[k] * xa;
-        Gc[k] = xc;
-        Ga[k] = xa;
-    }
-    for (int d = 1; d < W; d <<= 1) {
-        const double yc = wup<W>(xc, d), ya = wup1<W>(xa, d);
-        if (wrow<W>() || lane >= d) {
-            xc = xc + xa * yc;
-            xa = xa * ya;
-        }
-    }
-    double ec = wup<W>(xc, 1);
-    if (!wrow<W>() && lane == 0) ec = 0.0;
-    for (int k = 0; k < K; ++k) cc[k] = Gc[k] + Ga[k] * ec;
-}
-
 // ---- several right-hand sides per scan ----------------------------------------
 // The Chebyshev-tau operators are real, so the real and imaginary parts of a
 // mode (and u and w, which share the velocity operator) are solved together:
 // one affine scan carries NR constant terms with a shared multiplier, which
-// keeps the arithmetic of each right-hand side exactly that of the one-RHS
-// routines above while the dependent shuffle chains are shared.
+// keeps the arithmetic of each right-hand side what it would be alone while the
+// dependent shuffle chains are shared.
 
+// Affine suffix scan: x_i = cc_i + aa_i x_{i+1}; maps past the chain end are
+// the identity (cc = 0, aa = 1) and the last real map is constant (aa = 0).
+// On return cc[r][k] holds x_i.
 template <int K, int W, int NR>
 __device__ __forceinline__ void waff_suffix_n(double (&cc)[NR][K], const double (&aa)[K], int lane) {
     double Fc[NR][K], Fa[K];
@@ -365,6 +320,7 @@ __device__ __forceinline__ void waff_suffix_n(double (&cc)[NR][K], const double 
     }
 }
 
+// Affine prefix scan: y_i = cc_i + aa_i y_{i-1}; the first map is constant.
 template <int K, int W, int NR>
 __device__ __forceinline__ void waff_prefix_n(double (&cc)[NR][K], const double (&aa)[K], int lane) {
     double Gc[NR][K], Ga[K];

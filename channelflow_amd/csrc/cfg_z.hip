@@ -14,7 +14,6 @@ namespace cfg {
 // velocity comes from the divergence form's inverse transforms, which add U, W
 // and -Vsuck to the (0,0) mode; Vsuck is added back for v. One partial maximum
 // per block, then one per member.
-template <int NZ>
 __global__ void __launch_bounds__(256) k_zcfl(Geom g, FFTPlan pz, int XB, const NLMember* __restrict__ tab,
                                               const double2* __restrict__ xp0, long sx, double* __restrict__ part) {
     extern __shared__ double2 lds[];
@@ -34,8 +33,8 @@ __global__ void __launch_bounds__(256) k_zcfl(Geom g, FFTPlan pz, int XB, const 
     c.wb = c.wa + XB * lpitch(g.Nz);
     c.phys = reinterpret_cast<double*>(c.wb + XB * lpitch(g.Nz));
     stage_tw(c.tw, pz);
-    zc2r_pair<NZ>(c, xp, 0, false, 0, 1, false, 1);
-    zc2r_pair<NZ>(c, xp, 2, false, 2, -1, false, -1);
+    zc2r_pair(c, xp, 0, false, 0, 1, false, 1);
+    zc2r_pair(c, xp, 2, false, 2, -1, false, -1);
     const int Ny = g.Ny, y = c.y;
     const double piN = PI / (Ny - 1), rad = (g.b - g.a) / 2, cen = (g.b + g.a) / 2;  // chebypoints (chebyshev.cpp:746-754)
     auto yc = [&](int j) { return cen + rad * cos(j * piN); };
@@ -182,8 +181,8 @@ static int launch_zcfl_t(const Geom& g, const FFTPlan& pz, int n, const NLMember
         const int XB = zpass_xb_max(g, 3), nb = g.Ny * ((g.Nx + XB - 1) / XB);
         const size_t lds = (size_t)g.Nz * sizeof(double2) +
                            (size_t)XB * (2 * lpitch(g.Nz) * sizeof(double2) + (size_t)g.Nz * 3 * sizeof(double));
-        allow_lds(k_zcfl<NZ>, lds);
-        k_zcfl<NZ><<<dim3((unsigned)nb, n), 256, lds, st>>>(g, pz, XB, tab, xp, sx, part);
+        allow_lds(k_zcfl, lds);
+        k_zcfl<<<dim3((unsigned)nb, n), 256, lds, st>>>(g, pz, XB, tab, xp, sx, part);
         return nb;
     }
 }

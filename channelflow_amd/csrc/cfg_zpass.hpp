@@ -27,8 +27,7 @@ __device__ __forceinline__ double* physf(const ZCtx& c, int f) { return c.phys +
 // c2r of two real fields at once: field fa -> phys[da], fb -> phys[db]
 // (fb < 0: none). dza/dzb apply d/dz. Imag parts of kz = 0 are ignored, as
 // FFTW's c2r does. The unused middle bins are zeroed in the same sweep.
-template <int NZ>
-__device__ void zc2r_pair(const ZCtx& c, const double2* __restrict__ xp, int fa, bool dza, int da, int fb, bool dzb,
+__device__ inline void zc2r_pair(const ZCtx& c, const double2* __restrict__ xp, int fa, bool dza, int da, int fb, bool dzb,
                           int db) {
     const Geom& g = c.g;
     const int Nz = g.Nz, nkz = g.nkz;
@@ -59,7 +58,7 @@ __device__ void zc2r_pair(const ZCtx& c, const double2* __restrict__ xp, int fa,
         }
     }
     __syncthreads();
-    double2* r = fft_any<NZ, +1, true>(c.wa, c.wb, c.pz, c.tw, c.nl);
+    double2* r = fft_lds<+1>(c.wa, c.wb, c.pz, c.tw, c.nl);
     double* pa = physf(c, da);
     double* pb = db >= 0 ? physf(c, db) : nullptr;
     for (int w = threadIdx.x; w < c.nl * Nz; w += blockDim.x) {
@@ -75,8 +74,7 @@ __device__ void zc2r_pair(const ZCtx& c, const double2* __restrict__ xp, int fa,
 // fold != 0 (with sb >= 0): field ga receives A + fold i kz B instead of A,
 // kz = 2 pi k / Lz, A and B the spectra of phys[sa] and phys[sb]; gb < 0 then
 // drops B.
-template <int NZ>
-__device__ void zr2c_pair(const ZCtx& c, double2* __restrict__ zo, int sa, int ga, int sb, int gb,
+__device__ inline void zr2c_pair(const ZCtx& c, double2* __restrict__ zo, int sa, int ga, int sb, int gb,
                           double fold = 0.0) {
     const Geom& g = c.g;
     const int Nz = g.Nz, nkz = g.nkz;
@@ -88,7 +86,7 @@ __device__ void zr2c_pair(const ZCtx& c, double2* __restrict__ zo, int sa, int g
         c.wa[l * P + pidx(zz)] = make_double2(pa[w], pb ? pb[w] : 0.0);
     }
     __syncthreads();
-    double2* r = fft_any<NZ, -1, true>(c.wa, c.wb, c.pz, c.tw, c.nl);
+    double2* r = fft_lds<-1>(c.wa, c.wb, c.pz, c.tw, c.nl);
     const long fsz = (long)g.Ny * g.Nx * nkz;
     for (int w = threadIdx.x; w < c.nl * nkz; w += blockDim.x) {
         const int l = w / nkz, k = w - l * nkz;
@@ -113,7 +111,7 @@ __device__ void zr2c_pair(const ZCtx& c, double2* __restrict__ zo, int sa, int g
 // u.grad u / omega x u part and the rotation term) then uu00 uu01 uu02 uu11
 // uu12 uu22 for DIV; for SKEW g_i + i kz u_i u_2 / 2 then uu00 uu01 uu02 uu11
 // uu12 (8 fields).
-template <int METHOD, int NZ>
+template <int METHOD>
 __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const NLMember* __restrict__ tab,
                                                int want_g, const double2* __restrict__ xp0, double2* __restrict__ zo0,
                                                long sx) {
@@ -137,9 +135,9 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
     const int Nz = g.Nz;
     const int npts = c.nl * Nz;
     if (METHOD == NL_ROT) {
-        zc2r_pair<NZ>(c, xp, 0, false, 0, 1, false, 1);
-        zc2r_pair<NZ>(c, xp, 2, false, 2, 3, false, 3);
-        zc2r_pair<NZ>(c, xp, 4, false, 4, 5, false, 5);
+        zc2r_pair(c, xp, 0, false, 0, 1, false, 1);
+        zc2r_pair(c, xp, 2, false, 2, 3, false, 3);
+        zc2r_pair(c, xp, 4, false, 4, 5, false, 5);
         double *u0 = physf(c, 0), *u1 = physf(c, 1), *u2 = physf(c, 2);
         double *w0 = physf(c, 3), *w1 = physf(c, 4), *w2 = physf(c, 5);
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {  // cross(vort, u) (diffops.cpp:2598-2605)
@@ -156,8 +154,8 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
             w2[w] = f2;
         }
         __syncthreads();
-        zr2c_pair<NZ>(c, zo, 3, 0, 4, 1);
-        zr2c_pair<NZ>(c, zo, 5, 2, -1, -1);
+        zr2c_pair(c, zo, 3, 0, 4, 1);
+        zr2c_pair(c, zo, 5, 2, -1, -1);
         return;
     }
     double *u0 = physf(c, 0), *u1 = physf(c, 1), *u2 = physf(c, 2);
@@ -171,10 +169,10 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
         const double s = SK ? 0.5 : 1.0;
         double *fa = physf(c, 5), *fb = physf(c, 6);
         auto su = [&](const double* uj, int w) { return SK ? s * uj[w] : uj[w]; };
-        zc2r_pair<NZ>(c, xp, 0, false, 0, 1, false, 1);  // u, v
-        zc2r_pair<NZ>(c, xp, 2, false, 2, 6, false, 3);  // w, du/dx
+        zc2r_pair(c, xp, 0, false, 0, 1, false, 1);  // u, v
+        zc2r_pair(c, xp, 2, false, 2, 6, false, 3);  // w, du/dx
         for (int w = threadIdx.x; w < npts; w += blockDim.x) fa[w] = 0.0 + su(u0, w) * pa[w];
-        zc2r_pair<NZ>(c, xp, 3, false, 3, 0, true, 4);   // du/dy, du/dz
+        zc2r_pair(c, xp, 3, false, 3, 0, true, 4);   // du/dy, du/dz
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             fa[w] += su(u1, w) * pa[w];
             fa[w] += su(u2, w) * pb[w];
@@ -183,19 +181,19 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
         }
         __syncthreads();
         // skew-symmetric: f0 + i kz u0u2 / 2 and u0u2 (the layout of k_zsplit)
-        zr2c_pair<NZ>(c, zo, 5, 0, SK ? 4 : -1, SK ? 5 : -1, SK ? 0.5 : 0.0);
-        zc2r_pair<NZ>(c, xp, 7, false, 3, 4, false, 4);  // dv/dx, dv/dy
+        zr2c_pair(c, zo, 5, 0, SK ? 4 : -1, SK ? 5 : -1, SK ? 0.5 : 0.0);
+        zc2r_pair(c, xp, 7, false, 3, 4, false, 4);  // dv/dx, dv/dy
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             fa[w] = 0.0 + su(u0, w) * pa[w];
             fa[w] += su(u1, w) * pb[w];
         }
-        zc2r_pair<NZ>(c, xp, 1, true, 3, 8, false, 4);   // dv/dz, dw/dx
+        zc2r_pair(c, xp, 1, true, 3, 8, false, 4);   // dv/dz, dw/dx
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             fa[w] += su(u2, w) * pa[w];
             if (rotation != 0.0) fa[w] += rotation * u0[w];
             fb[w] = 0.0 + su(u0, w) * pb[w];
         }
-        zc2r_pair<NZ>(c, xp, 5, false, 3, 2, true, 4);   // dw/dy, dw/dz
+        zc2r_pair(c, xp, 5, false, 3, 2, true, 4);   // dw/dy, dw/dz
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             fb[w] += su(u1, w) * pa[w];
             fb[w] += su(u2, w) * pb[w];
@@ -209,33 +207,33 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
                 pb[w] = u2[w] * u2[w];
             }
             __syncthreads();
-            zr2c_pair<NZ>(c, zo, 5, 1, 3, 7, 0.5);
-            zr2c_pair<NZ>(c, zo, 6, 2, 4, -1, 0.5);
+            zr2c_pair(c, zo, 5, 1, 3, 7, 0.5);
+            zr2c_pair(c, zo, 6, 2, 4, -1, 0.5);
             for (int w = threadIdx.x; w < npts; w += blockDim.x) {
                 pa[w] = u0[w] * u0[w];
                 pb[w] = u0[w] * u1[w];
             }
             __syncthreads();
-            zr2c_pair<NZ>(c, zo, 3, 3, 4, 4);
+            zr2c_pair(c, zo, 3, 3, 4, 4);
             for (int w = threadIdx.x; w < npts; w += blockDim.x) pa[w] = u1[w] * u1[w];
             __syncthreads();
-            zr2c_pair<NZ>(c, zo, 3, 6, -1, -1);
+            zr2c_pair(c, zo, 3, 6, -1, -1);
         } else {
-            zr2c_pair<NZ>(c, zo, 5, 1, 6, 2);  // f1, f2
+            zr2c_pair(c, zo, 5, 1, 6, 2);  // f1, f2
         }
     } else {
-        zc2r_pair<NZ>(c, xp, 0, false, 0, 1, false, 1);
-        zc2r_pair<NZ>(c, xp, 2, false, 2, -1, false, -1);
+        zc2r_pair(c, xp, 0, false, 0, 1, false, 1);
+        zc2r_pair(c, xp, 2, false, 2, -1, false, -1);
         if (want_g) {  // DIV with rotation: g = rotation terms only
             for (int w = threadIdx.x; w < npts; w += blockDim.x) {
                 pa[w] = -(rotation * u1[w]);
                 pb[w] = rotation * u0[w];
             }
             __syncthreads();
-            zr2c_pair<NZ>(c, zo, 3, 0, 4, 1);
+            zr2c_pair(c, zo, 3, 0, 4, 1);
             for (int w = threadIdx.x; w < npts; w += blockDim.x) pa[w] = 0.0;
             __syncthreads();
-            zr2c_pair<NZ>(c, zo, 3, 2, -1, -1);
+            zr2c_pair(c, zo, 3, 2, -1, -1);
         }
         // outer(u, u) (diffops.cpp:2336-2388), two entries per r2c
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
@@ -243,19 +241,19 @@ __global__ void __launch_bounds__(256) k_zpass(Geom g, FFTPlan pz, int XB, const
             pb[w] = u0[w] * u1[w];
         }
         __syncthreads();
-        zr2c_pair<NZ>(c, zo, 3, 3, 4, 4);
+        zr2c_pair(c, zo, 3, 3, 4, 4);
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             pa[w] = u0[w] * u2[w];
             pb[w] = u1[w] * u1[w];
         }
         __syncthreads();
-        zr2c_pair<NZ>(c, zo, 3, 5, 4, 6);
+        zr2c_pair(c, zo, 3, 5, 4, 6);
         for (int w = threadIdx.x; w < npts; w += blockDim.x) {
             pa[w] = u1[w] * u2[w];
             pb[w] = u2[w] * u2[w];
         }
         __syncthreads();
-        zr2c_pair<NZ>(c, zo, 3, 7, 4, 8);
+        zr2c_pair(c, zo, 3, 7, 4, 8);
     }
 }
 
@@ -686,8 +684,8 @@ void launch_z_t(const Geom& g, const FFTPlan& pz, int n, const NLMember* tab, in
         const size_t lds = (size_t)g.Nz * sizeof(double2) +
                            (size_t)XB * (2 * lpitch(g.Nz) * sizeof(double2) + (size_t)g.Nz * nphys * sizeof(double));
         const dim3 grid(g.Ny * ((g.Nx + XB - 1) / XB), n);
-        allow_lds(k_zpass<METHOD, NZ>, lds);
-        k_zpass<METHOD, NZ><<<grid, 256, lds, st>>>(g, pz, XB, tab, want_g, xp, zo, sx);
+        allow_lds(k_zpass<METHOD>, lds);
+        k_zpass<METHOD><<<grid, 256, lds, st>>>(g, pz, XB, tab, want_g, xp, zo, sx);
     }
 }
 
