@@ -579,7 +579,7 @@ __global__ void __launch_bounds__(256) k_yfwd_t(Geom g, YMats ym, int have_g, co
 // instructions; us per launch, before -> after (inverse, forward): one 32^3 field
 // 5.4 -> 4.8, 6.0 -> 4.7; 64^3 10.8 -> 6.9 (with the row split), 11.6 -> 8.6; 96^3
 // 17.0 -> 14.4, 19.1 -> 13.8; 128^3 convection 41 -> 35, 22 -> 19; 192x129x192 81 ->
-// 63, 44 -> 35; 16 of 64^3 52 -> 46, 51 -> 44. The inverse at 192x129x192 then takes
+// 63, 44 -> 35 (57.5 and 28.4 with the addressing below); 16 of 64^3 52 -> 46, 51 -> 44. The inverse at 192x129x192 then takes
 // 24 us for its loads alone, 23 us of matrix products at their peak rate and writes
 // 96 MB (20 us at the copy rate), one after the other in each block. Loading two or
 // three chunks ahead is slower (67, 72), and so are two column tiles per wave (71: the

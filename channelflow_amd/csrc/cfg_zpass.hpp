@@ -493,8 +493,8 @@ k_zwave(Geom g, const double2* __restrict__ twg, const NLMember* __restrict__ ta
 // gradient, or the vorticity component w_c), hands the velocity (and w) to the other
 // two through LDS and forms its part of the products. Each wavefront's transforms are
 // a serial chain through LDS, so what bounds the pass is how many wavefronts a SIMD
-// holds: 32 bins take 126 registers here against 180 in one wavefront, 64 bins 162
-// against 238, 192 bins 116 against 200. The shared values lie in the wavefronts'
+// holds: 32 bins take 122 registers here against 180 in one wavefront, 64 bins 162
+// against 238, 192 bins 101 against 200. The shared values lie in the wavefronts'
 // line rows, which are free between the inverse and the forward transforms; in space
 // of their own they cost a third of the occupancy (rotational 192x129x192 93 against
 // 76 us). The first bins are requested before the twiddles are waited for. Two such

@@ -137,11 +137,12 @@ int cfg_solve(const cfg_grid* grid, const cfg_flags* flags, double lambda_t, con
  *          DealiasXZ, Nx/2-1, Nz/2-1 without).
  *   stream a hipStream_t, or NULL for the null stream; the call is ordered
  *          after the caller's work on it and returns once f_dev is written.
- * Work buffers and tables live in one fixed device array of
- * CFG_NOALLOC_SCRATCH_BYTES per device (held until the process ends). A grid
- * that needs more (64x65x64 fits, 96x97x96 does not) is rejected with
- * CFG_ERR_ARG. Calls on one device share that array: calls that overlap on one
- * device race. */
+ * Work buffers and tables live in one fixed device array per device (held
+ * until the process ends): CFG_NOALLOC_SCRATCH_BYTES, and behind them about
+ * 1.2 MB for the y operators in the order in which the kernels stage them. A
+ * grid that needs more than the first part (64x65x64 fits, 96x97x96 does not)
+ * is rejected with CFG_ERR_ARG. Calls on one device share that array: calls
+ * that overlap on one device race. */
 #define CFG_NOALLOC_SCRATCH_BYTES (48u << 20)
 int cfg_nonlinear_noalloc(const cfg_grid* grid, const cfg_flags* flags, const double* u_dev, double* f_dev,
                           void* stream);
