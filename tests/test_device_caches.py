@@ -11,9 +11,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 @pytest.fixture(scope="module")
 def lib(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("caches") / "libdevicecaches.so")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__",
-                    "-Wl,-Bsymbolic", "-fno-gnu-unique", "-I/opt/rocm/include", "-o", so, os.path.join(ROOT, "tests", "hostmath", "device_caches.cpp")],
-                   check=True)
+    src = os.path.join(ROOT, "tests", "hostmath", "device_caches.cpp")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", "-Wl,-Bsymbolic",
+                    "-fno-gnu-unique", "-I/opt/rocm/include", "-o", so, src], check=True)
     return C.CDLL(so)
 
 
